@@ -114,6 +114,20 @@ def load(path: str | None = None) -> ctypes.CDLL:
     return lib
 
 
+_HOST = None
+
+
+def host():
+    """The C++ host path (csrc/host.cpp), imported on first use; raises if it has not been built."""
+    global _HOST
+    if _HOST is None:
+        load()
+        import torch  # noqa: F401  (its libraries are the module's)
+        from . import _host
+        _HOST = _host
+    return _HOST
+
+
 def strerror(code: int) -> str:
     return load().evoattn_strerror(code).decode()
 

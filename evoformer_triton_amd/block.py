@@ -104,13 +104,12 @@ class _Projections(torch.autograd.Function):
 
 class _Linear(torch.autograd.Function):
     """x W^T + b with the weight gradient summed over slices of the rows (see _row_slices); forward and
-    input gradient are the library's GEMMs as torch.nn.functional.linear calls them."""
+    input gradient are the library's GEMMs as torch.nn.functional.linear calls them.  What the tracer sees."""
 
     @staticmethod
-    def forward(ctx, x, weight, bias, dx_place=None):
+    def forward(ctx, x, weight, bias):
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
-        ctx.dx_place = dx_place          # where the input gradient is to be written (shaped like x, rows may lie apart)
         # (as a matrix: for an input of more dimensions whose rows lie apart torch multiplies and then adds the
         # bias in a pass of its own)
         y = torch.nn.functional.linear(x.reshape(-1, x.shape[-1]), weight, bias)
@@ -122,103 +121,46 @@ class _Linear(torch.autograd.Function):
         dy2, x2 = dy.reshape(-1, dy.shape[-1]), x.reshape(-1, x.shape[-1])
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
-            if ctx.dx_place is not None:
-                dx = ctx.dx_place
-                torch.mm(dy2, weight, out=dx.view(-1, x.shape[-1]))
-            else:
-                dx = (dy2 @ weight).view(x.shape)
+            dx = (dy2 @ weight).view(x.shape)
         if ctx.needs_input_grad[1]:
             dw = _weight_grad(dy2, x2)
         if ctx.has_bias and ctx.needs_input_grad[2]:
             db = _bias_grad(dy2)
-        return dx, dw, db, None
+        return dx, dw, db
 
 
 def _linear(layer: nn.Linear, x: torch.Tensor, dx_place: Optional[torch.Tensor] = None) -> torch.Tensor:
-    return _Linear.apply(x, layer.weight, layer.bias, dx_place)
+    if torch.compiler.is_compiling():
+        return _Linear.apply(x, layer.weight, layer.bias)
+    return _lib.host().linear(x, layer.weight, layer.bias, dx_place)      # (the same in C++)
 
 
-class _StackedProjection(torch.autograd.Function):
+class _StackedProjection:
     """The Q, K, V (and gate) projections of one input as a single GEMM with their weights stacked:
-    forward(x, gate_bias, w0, w1, ...) -> x [w0; w1; ...]^T (+ gate_bias on the last layer's columns), shaped
+    apply(x, gate_bias, w0, w1, ...) -> x [w0; w1; ...]^T (+ gate_bias on the last layer's columns), shaped
     [..., n * out].  The input is read once instead of n times, its gradient is one GEMM over the whole
     gradient of the result (no additions of n partial gradients), and so is the weight gradient (summed over
     slices of the rows, see _row_slices), cut into the layers' pieces afterwards."""
 
     @staticmethod
-    def forward(ctx, x, gate_bias, *weights):
-        w = torch.cat(weights, 0)
-        bias = None
-        if gate_bias is not None:
-            bias = torch.cat([gate_bias.new_zeros(w.shape[0] - gate_bias.shape[0]), gate_bias])
-        ctx.save_for_backward(x, w)
-        ctx.sizes = [t.shape[0] for t in weights]
-        ctx.has_bias = gate_bias is not None
-        return torch.nn.functional.linear(x, w, bias)
-
-    @staticmethod
-    def backward(ctx, dp):
-        x, w = ctx.saved_tensors
-        dp2, x2 = dp.reshape(-1, dp.shape[-1]), x.reshape(-1, x.shape[-1])
-        dx = (dp2 @ w).view(x.shape) if ctx.needs_input_grad[0] else None
-        db = _bias_grad(dp2[:, dp2.shape[1] - ctx.sizes[-1]:]) if ctx.has_bias and ctx.needs_input_grad[1] else None
-        dws = [None] * len(ctx.sizes)
-        if any(ctx.needs_input_grad[2:]):
-            dws = list(_weight_grad(dp2, x2).split(ctx.sizes, 0))
-        return (dx, db, *dws)
+    def apply(x, gate_bias, *weights):
+        return _lib.host().stacked_projection(x, gate_bias, weights)
 
 
-
-class _LayerNorm(torch.autograd.Function):
+class _LayerNorm:
     """LayerNorm over the last dimension through the library's kernels (evoattn_layernorm_fwd / _bwd): x and y
     cross HBM once in the forward, x, dy and dx once in the backward; the gradients of weight and bias are summed
-    in a fixed order."""
+    in a fixed order.  None where those kernels do not take the call."""
 
     @staticmethod
-    def forward(ctx, x, weight, bias, eps):
-        lib = _lib.load()
-        xc = x.contiguous()
-        cols = xc.shape[-1]
-        rows = xc.numel() // cols
-        w = None if weight is None else weight.contiguous()
-        b = None if bias is None else bias.contiguous()
-        with _on_device(xc.device):
-            y = torch.empty_like(xc)
-            mean = torch.empty((rows,), device=xc.device, dtype=torch.float32)
-            rstd = torch.empty((rows,), device=xc.device, dtype=torch.float32)
-            _lib.check(lib.evoattn_layernorm_fwd(_ptr(xc), _ptr(w), _ptr(b), _ptr(y), _ptr(mean), _ptr(rstd), rows, cols,
-                                                 _DTYPES[xc.dtype], float(eps), _stream(xc.device)), "evoattn_layernorm_fwd")
-        ctx.save_for_backward(xc, w, mean, rstd)
-        ctx.has_bias = bias is not None
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        lib = _lib.load()
-        xc, w, mean, rstd = ctx.saved_tensors
-        cols = xc.shape[-1]
-        rows = xc.numel() // cols
-        dyc = dy.contiguous()
-        need_x, need_w, need_b = ctx.needs_input_grad[0], w is not None and ctx.needs_input_grad[1], ctx.has_bias and ctx.needs_input_grad[2]
-        if not (need_x or need_w or need_b):
-            return None, None, None, None
-        with _on_device(xc.device):
-            dx = torch.empty_like(xc) if need_x else None
-            dw = torch.empty((cols,), device=xc.device, dtype=xc.dtype) if need_w else None
-            db = torch.empty((cols,), device=xc.device, dtype=xc.dtype) if need_b else None
-            ws = _alloc_bytes(lib.evoattn_layernorm_bwd_workspace_bytes(rows, cols, _DTYPES[xc.dtype]), xc.device) if need_w or need_b else None
-            _lib.check(lib.evoattn_layernorm_bwd(_ptr(dyc), _ptr(xc), _ptr(w), _ptr(mean), _ptr(rstd), _ptr(dx), _ptr(dw), _ptr(db),
-                                                 _ptr(ws), 0 if ws is None else ws.numel(), rows, cols, _DTYPES[xc.dtype],
-                                                 _stream(xc.device)), "evoattn_layernorm_bwd")
-        return dx, dw, db, None
+    def apply(x, weight, bias, eps):
+        return _lib.host().layer_norm(x, weight, bias, eps)
 
 
 def _layer_norm(layer: nn.LayerNorm, x: torch.Tensor) -> torch.Tensor:
-    w, b = layer.weight, layer.bias
-    if torch.compiler.is_compiling() or x.numel() == 0 or x.dtype not in _DTYPES or (w is not None and w.dtype != x.dtype) \
-            or _lib.load().evoattn_layernorm_bwd_workspace_bytes(1, x.shape[-1], _DTYPES[x.dtype]) == 0:
-        return layer(x)          # under the tracer, no rows, mixed dtypes, or a row length the kernels do not take: the framework's
-    return _LayerNorm.apply(x, w, b, layer.eps)
+    # under the tracer, no rows, mixed dtypes, or a row length the kernels do not take: the framework's
+    y = None if torch.compiler.is_compiling() else _LayerNorm.apply(x, layer.weight, layer.bias, layer.eps)
+    return layer(x) if y is None else y
 
 
 class GatedAttentionBlock(nn.Module):

@@ -1,10 +1,11 @@
-"""Builds libevoattn.so (gfx950) in-tree with hipcc.
+"""Builds libevoattn.so (gfx950) in-tree with hipcc, and _host.so (the operator's host path in C++) on top of it.
 
     python -m evoformer_triton_amd.build [--force]
 
 One object per (kernel file, head dim) so that the objects compile in parallel; the result
 is evoformer_triton_amd/libevoattn.so, a plain C-ABI library (include/evoattn.h) that links
-against the HIP runtime only.
+against the HIP runtime only.  evoformer_triton_amd/_host.so is a Python module that links
+against that library and torch.
 """
 from __future__ import annotations
 
@@ -18,6 +19,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libevoattn.so")
+HOST = os.path.join(HERE, "_host.so")
 HEAD_DIMS = (8, 16, 32, 64)
 
 # -packed-fp32-ops off: packed fp32 VALU forms are not used on this hardware pool.
@@ -71,6 +73,22 @@ def _compile(unit, extra=(), obj_dir=None):
     return out, err
 
 
+def _build_host():
+    """csrc/host.cpp against torch's headers and libraries, next to the kernels' library."""
+    import sysconfig
+    import torch
+    tdir = os.path.dirname(torch.__file__)
+    inc = [os.path.join(tdir, "include"), os.path.join(tdir, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+           sysconfig.get_paths()["include"], os.path.join(ROOT, "include")]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-isystem{d}" for d in inc),
+           os.path.join(CSRC, "host.cpp"), "-o", HOST, "-L" + os.path.join(tdir, "lib"), "-L" + HERE, "-ltorch", "-ltorch_cpu", "-ltorch_hip",
+           "-ltorch_python", "-lc10", "-lc10_hip", "-l:libevoattn.so", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building _host.so failed:\n" + r.stderr)
+
+
 def build(force: bool = True, verbose: bool = False, jobs: int | None = None, extra=(), lib_path: str | None = None,
           obj_dir: str | None = None) -> str:
     """Compile every HIP source for gfx950 and link the shared library.  `extra` adds compiler
@@ -78,10 +96,10 @@ def build(force: bool = True, verbose: bool = False, jobs: int | None = None, ex
     lib_out = lib_path or LIB
     os.makedirs(obj_dir or OBJ, exist_ok=True)
     units = _units()
-    if not force and not extra and os.path.exists(LIB):
+    if not force and not extra and os.path.exists(LIB) and os.path.exists(HOST):
         newest = max(os.path.getmtime(os.path.join(r, f)) for r, _, fs in os.walk(CSRC) for f in fs)
         newest = max(newest, os.path.getmtime(os.path.join(ROOT, "include", "evoattn.h")))
-        if os.path.getmtime(LIB) >= newest:
+        if min(os.path.getmtime(LIB), os.path.getmtime(HOST)) >= newest:
             return LIB
     jobs = jobs or min(8, os.cpu_count() or 1)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
@@ -95,6 +113,8 @@ def build(force: bool = True, verbose: bool = False, jobs: int | None = None, ex
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr)
+    if lib_out == LIB:
+        _build_host()
     return lib_out
 
 

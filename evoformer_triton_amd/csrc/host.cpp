@@ -1,0 +1,688 @@
+// The host side of the operator in C++: what a call does between Python and the C ABI - looking the
+// tensors over, allocating results and scratch with torch, the autograd node - without the interpreter.
+//
+// A small call is bound by its host, not by its kernels: through Python (an autograd.Function, ctypes
+// structures, the backward taking the GIL in the engine's thread) a forward took 26 us and a forward +
+// backward 165 us of host time, the kernels of a small step 30 us.  The nodes below do the same work
+// in C++; the backward runs in the engine's thread without the GIL.
+//
+// A function here returns None for a call it does not take (tensors that are not plain GPU tensors, head
+// dims that need padding, empty problems, anything invalid): the caller in Python then goes its own
+// way, which also words the error messages.
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <optional>
+#include <string>
+#include <vector>
+
+#include "evoattn.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+void check(int rc, const char *where) {
+    TORCH_CHECK(rc == EVO_OK, where, " failed: ", evoattn_strerror(rc), " (code ", rc, ")");
+}
+
+int evo_dtype(at::ScalarType t) {
+    switch (t) {
+        case at::kBFloat16: return EVO_BF16;
+        case at::kHalf: return EVO_F16;
+        case at::kFloat: return EVO_F32;
+        default: return EVO_NONE;
+    }
+}
+
+bool head_dim_built(int64_t D) { return D == 8 || D == 16 || D == 32 || D == 64 || D == 128; }
+
+// An ordinary tensor with memory of its own kind: no subclass or mode with a dispatch in Python, no functorch wrapper
+// and no lazily negated or conjugated view, whose data pointer would not be what it stands for.
+bool plain(const Tensor &t) {
+    static const auto special = c10::DispatchKeySet({
+        c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::FuncTorchBatched,
+        c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate,
+        c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
+    return t.layout() == at::kStrided && !t.key_set().has_any(special);
+}
+
+bool plain_modes() {
+    const auto tls = c10::impl::tls_local_dispatch_key_set();
+    return !tls.included_.has(c10::DispatchKey::Python) && !tls.included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+hipStream_t stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+Tensor scratch(size_t bytes, const Tensor &like) {
+    return at::empty({(int64_t)std::max<size_t>(bytes, 256)}, like.options().dtype(at::kByte));
+}
+
+size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+
+// What a call's backward needs besides the tensors: the parameter block (its pointers are set anew) and the
+// caller's mask and bias as they came, whose shape and dtype their gradients take.
+struct Call {
+    EvoAttnParams p;
+    int64_t mask_b, mask_s, bias_b;
+    at::ScalarType mask_dtype, bias_dtype;
+    bool gated;
+};
+
+// The mask and the bias as the kernels read them; false where they do not fit the shape of Q.
+bool operands(Call &c, const Tensor &q, OptTensor &mask, OptTensor &bias) {
+    EvoAttnParams &p = c.p;
+    p.mask_kind = EVO_MASK_NONE;
+    p.bias_dtype = EVO_NONE;
+    const auto qdev = q.device();
+    if (mask && mask->defined()) {
+        Tensor m = *mask;
+        if (!plain(m) || m.device() != qdev || m.dim() != 5) return false;
+        const auto sz = m.sizes();
+        if (sz[2] != 1 || sz[3] != 1 || sz[4] != p.N || (sz[0] != 1 && sz[0] != p.B) || (sz[1] != 1 && sz[1] != p.S)) return false;
+        c.mask_b = sz[0];
+        c.mask_s = sz[1];
+        c.mask_dtype = m.scalar_type();
+        switch (m.scalar_type()) {
+            case at::kBool: case at::kByte: p.mask_kind = EVO_MASK_BOOL; break;
+            case at::kFloat: p.mask_kind = EVO_MASK_F32; break;
+            case at::kBFloat16: p.mask_kind = EVO_MASK_BF16; break;
+            case at::kHalf: p.mask_kind = EVO_MASK_F16; break;
+            default:
+                if (!at::isFloatingType(m.scalar_type()) && !at::isIntegralType(m.scalar_type(), true)) return false;
+                p.mask_kind = m.is_floating_point() ? EVO_MASK_F32 : EVO_MASK_BOOL;
+                m = m.is_floating_point() ? m.to(at::kFloat) : m.ne(0);
+        }
+        if (m.stride(4) != 1) m = m.contiguous();
+        p.mask_stride_b = m.size(0) == p.B && p.B > 1 ? m.stride(0) : 0;
+        p.mask_stride_s = m.size(1) == p.S && p.S > 1 ? m.stride(1) : 0;
+        p.mask = m.data_ptr();
+        mask = m;
+    } else {
+        mask = Tensor();
+    }
+    if (bias && bias->defined()) {
+        Tensor b = *bias;
+        if (!plain(b) || b.device() != qdev || b.dim() != 5 || !b.is_floating_point()) return false;
+        const auto sz = b.sizes();
+        if (sz[1] != 1 || sz[2] != p.H || sz[3] != p.N || sz[4] != p.N || (sz[0] != 1 && sz[0] != p.B)) return false;
+        c.bias_b = sz[0];
+        c.bias_dtype = b.scalar_type();
+        if (b.scalar_type() != at::kFloat && b.scalar_type() != q.scalar_type()) b = b.to(at::kFloat);
+        if (b.stride(4) != 1 || b.stride(3) < p.N) b = b.contiguous();
+        p.bias_dtype = evo_dtype(b.scalar_type());
+        p.bias_stride_b = b.size(0) == p.B && p.B > 1 ? b.stride(0) : 0;
+        p.bias_stride_h = b.stride(2);
+        p.bias_stride_row = b.stride(3);
+        p.bias = b.data_ptr();
+        bias = b;
+    } else {
+        bias = Tensor();
+    }
+    return true;
+}
+
+// LSE and the prepared operands share one allocation: [LSE | prep].
+struct Aux {
+    size_t lse_bytes;
+    explicit Aux(const EvoAttnParams &p) : lse_bytes(align256((size_t)p.B * p.H * p.S * p.N * sizeof(float))) {}
+    void place(EvoAttnParams &p, const Tensor &aux) const {
+        char *base = (char *)aux.data_ptr();
+        p.lse = (float *)base;
+        p.prep = base + lse_bytes;
+        p.prep_bytes = (size_t)aux.numel() - lse_bytes;
+    }
+};
+
+Tensor finish_dbias(Tensor d, const Call &c) {
+    const EvoAttnParams &p = c.p;
+    d = d.view({p.B, 1, p.H, p.N, p.N});
+    if (c.bias_b == 1 && p.B > 1) d = d.sum(0, true);
+    return d.scalar_type() == c.bias_dtype ? d : d.to(c.bias_dtype);
+}
+
+Tensor finish_dmask(Tensor d, const Call &c) {
+    const EvoAttnParams &p = c.p;
+    d = d.view({p.B, p.S, 1, 1, p.N});
+    if (c.mask_b == 1 && p.B > 1) d = d.sum(0, true);
+    if (c.mask_s == 1 && p.S > 1) d = d.sum(1, true);
+    return d.scalar_type() == c.mask_dtype ? d : d.to(c.mask_dtype);
+}
+
+// The backward's scratch and results beside dQ, dK, dV: allocates dBias, dMask and the workspace, sets their
+// pointers in `p`, and enqueues the backward.
+void enqueue_backward(EvoAttnParams &p, const Tensor &like, const Tensor &bias, bool want_dbias, bool want_dmask, Tensor &dbias,
+                      Tensor &dmask) {
+    if (want_dbias) {
+        dbias = at::empty({p.B, p.H, p.N, p.N}, bias.options());
+        p.dbias = dbias.data_ptr();
+        p.dbias_dtype = p.bias_dtype;
+    }
+    if (want_dmask) {
+        dmask = at::empty({p.B, p.S, p.N}, like.options().dtype(at::kFloat));
+        p.dmask = (float *)dmask.data_ptr();
+    }
+    Tensor ws = scratch(evoattn_bwd_workspace_bytes(&p), like);
+    p.workspace = ws.data_ptr();
+    p.workspace_bytes = (size_t)ws.numel();
+    p.flags |= EVO_FLAG_PREP_VALID;   // same bias and mask as the forward
+    check(evoattn_bwd(&p, stream_of(like)), "evoattn_bwd");
+}
+
+// Gradients of gradients are not formed: as torch's once_differentiable does, results of a backward that is itself
+// recorded become inputs of a node that says so when it is differentiated.
+variable_list once_differentiable(variable_list outs, bool recorded) {
+    if (!recorded) return outs;
+    std::vector<size_t> at_;
+    variable_list defined;
+    for (size_t i = 0; i < outs.size(); ++i)
+        if (outs[i].defined()) {
+            at_.push_back(i);
+            defined.push_back(outs[i].detach().set_requires_grad(true));
+        }
+    torch::autograd::DelayedError err("trying to differentiate twice a function that was marked with @once_differentiable",
+                                      (int64_t)defined.size());
+    variable_list wrapped = err.apply(std::move(defined));
+    for (size_t i = 0; i < at_.size(); ++i) outs[at_[i]] = wrapped[i];
+    return outs;
+}
+
+// A node whose saved tensors lie in one list.
+struct SavingNode : Node {
+    std::vector<SavedVariable> saved;
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (auto &s : saved) s.reset_data();
+    }
+    void save(const Tensor &t, bool is_output = false) { saved.emplace_back(t, is_output); }
+    template <typename... T>
+    static bool wanted(const T &...t) {
+        return at::GradMode::is_enabled() && ((t.defined() && t.requires_grad()) || ...);
+    }
+};
+
+template <typename N, typename... T>
+std::shared_ptr<N> make_node(const T &...inputs) {
+    std::shared_ptr<N> node(new N(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(inputs...));
+    return node;
+}
+
+// ------------------------------------------------------------------ attention
+
+struct AttentionNode : SavingNode {
+    Call c{};
+    std::string name() const override { return c.gated ? "GatedAttentionBackward" : "EvoformerAttentionBackward"; }
+
+    // grads[0]: the gradient of the output; results: Q, K, V, mask, bias, gate
+    variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        const bool rec = at::GradMode::is_enabled();
+        variable_list out(6);
+        {
+            at::AutoDispatchBelowADInplaceOrView guard;
+            const Tensor q = saved[0].unpack(), k = saved[1].unpack(), v = saved[2].unpack(), mask = saved[3].unpack(),
+                         bias = saved[4].unpack(), aux = saved[5].unpack(), o = saved[6].unpack(shared_from_this());
+            const Tensor gate = c.gated ? saved[7].unpack() : Tensor();
+            c10::DeviceGuard on(q.device());
+            Tensor dO = grads[0].defined() ? grads[0].contiguous() : at::zeros_like(q);
+            if (dO.scalar_type() != q.scalar_type()) dO = dO.to(q.scalar_type());
+            EvoAttnParams p = c.p;
+            Aux(p).place(p, aux);
+            p.q = q.data_ptr();
+            p.k = k.data_ptr();
+            p.v = v.data_ptr();
+            p.mask = mask.defined() ? mask.data_ptr() : nullptr;
+            p.bias = bias.defined() ? bias.data_ptr() : nullptr;
+            p.dout = dO.data_ptr();
+            Tensor dbias, dmask;
+            for (int i = 0; i < 3; ++i) out[i] = at::empty_like(q);
+            p.dq = out[0].data_ptr();
+            p.dk = out[1].data_ptr();
+            p.dv = out[2].data_ptr();
+            if (c.gated) {   // o is the gated output, dO its gradient
+                out[5] = at::empty_like(q);
+                p.o = nullptr;
+                p.o_gated = o.data_ptr();
+                p.gate = gate.data_ptr();
+                p.dgate = out[5].data_ptr();
+            } else {
+                p.o = o.data_ptr();
+            }
+            const bool want_dmask = mask.defined() && mask.is_floating_point() && task_should_compute_output(3);
+            const bool want_dbias = bias.defined() && task_should_compute_output(4);
+            enqueue_backward(p, q, bias, want_dbias, want_dmask, dbias, dmask);
+            if (want_dbias) out[4] = finish_dbias(dbias, c);
+            if (want_dmask) out[3] = finish_dmask(dmask, c);
+        }
+        return once_differentiable(std::move(out), rec);
+    }
+};
+
+// The attention on dense [B,S,N,H,D] tensors with the reference's flat-reshape heads or (per_head) true ones, with a
+// gate sigmoid(gate) * O; none where this path does not take the call.
+OptTensor attention(const Tensor &Q, const Tensor &K, const Tensor &V, OptTensor mask, OptTensor bias, const OptTensor &gate, bool per_head,
+                    int64_t flags) {
+    if (!plain(Q) || !plain(K) || !plain(V) || !Q.is_cuda() || Q.dim() != 5 || !plain_modes()) return std::nullopt;
+    if (!K.sizes().equals(Q.sizes()) || !V.sizes().equals(Q.sizes()) || K.device() != Q.device() || V.device() != Q.device()) return std::nullopt;
+    const auto dt = Q.scalar_type();
+    if (K.scalar_type() != dt || V.scalar_type() != dt || evo_dtype(dt) == EVO_NONE || Q.numel() == 0 || !head_dim_built(Q.size(4)))
+        return std::nullopt;
+    for (int i = 0; i < 5; ++i)
+        if (Q.size(i) > INT32_MAX) return std::nullopt;
+    const bool gated = gate && gate->defined();
+    if (gated && (!plain(*gate) || !gate->sizes().equals(Q.sizes()) || gate->scalar_type() != dt || gate->device() != Q.device())) return std::nullopt;
+
+    Call c{};
+    EvoAttnParams &p = c.p;
+    p.B = (int32_t)Q.size(0);
+    p.S = (int32_t)Q.size(1);
+    p.N = (int32_t)Q.size(2);
+    p.H = (int32_t)Q.size(3);
+    p.D = (int32_t)Q.size(4);
+    p.dtype = evo_dtype(dt);
+    p.dbias_dtype = EVO_F32;
+    p.flags = (int32_t)flags;
+    p.scale = (float)(1.0 / std::sqrt((double)p.D));
+    const int64_t row = (int64_t)p.N * p.D;
+    p.stride_b = (int64_t)p.S * p.H * row;
+    p.stride_h = per_head ? p.D : p.S * row;
+    p.stride_s = per_head ? p.H * row : row;
+    p.stride_n = per_head ? (int64_t)p.H * p.D : p.D;
+    c.gated = gated;
+
+    OptTensor mask_in = mask, bias_in = bias;
+    const Tensor mask0 = mask ? *mask : Tensor(), bias0 = bias ? *bias : Tensor(), gate0 = gated ? *gate : Tensor();
+    Tensor q, k, v, g, o, aux;
+    {
+        at::AutoDispatchBelowADInplaceOrView guard;
+        if (!operands(c, Q, mask, bias)) return std::nullopt;
+        c10::DeviceGuard on(Q.device());
+        q = Q.contiguous();
+        k = K.contiguous();
+        v = V.contiguous();
+        o = at::empty_like(q);
+        const Aux layout(p);
+        aux = scratch(layout.lse_bytes + evoattn_prep_bytes(&p), q);
+        layout.place(p, aux);
+        p.q = q.data_ptr();
+        p.k = k.data_ptr();
+        p.v = v.data_ptr();
+        if (gated) {   // only the gated output is written: the backward's gate pass forms delta from it
+            g = gate0.contiguous();
+            p.gate = g.data_ptr();
+            p.o_gated = o.data_ptr();
+        } else {
+            p.o = o.data_ptr();
+        }
+        if (evoattn_fwd(&p, stream_of(q)) != EVO_OK) return std::nullopt;
+    }
+    if (SavingNode::wanted(Q, K, V, mask0, bias0, gate0)) {
+        auto node = make_node<AttentionNode>(Q, K, V, mask0, bias0, gate0);
+        node->c = c;
+        node->c.p.gate = nullptr;
+        torch::autograd::set_history(o, node);
+        node->saved.reserve(gated ? 8 : 7);
+        node->save(q);
+        node->save(k);
+        node->save(v);
+        node->save(*mask);
+        node->save(*bias);
+        node->save(aux);
+        node->save(o, true);
+        if (gated) node->save(g);
+    }
+    return o;
+}
+
+// Q, K, V (and the gate) as slots of one [B,S,N,W,H,D] tensor (`_SlotAttention` in evoformer.py describes the buffers).
+struct SlotAttention : torch::autograd::Function<SlotAttention> {
+    static void strides(EvoAttnParams &p, const Tensor &P) {
+        const int64_t W = P.size(3), tok = W * p.H * p.D;
+        p.stride_b = (int64_t)p.S * p.N * tok;
+        p.stride_h = p.D;
+        p.stride_s = p.N * tok;
+        p.stride_n = tok;
+    }
+    static char *slot(const Tensor &t, const EvoAttnParams &p, int i) {
+        return (char *)t.data_ptr() + (size_t)i * p.H * p.D * t.element_size();
+    }
+
+    static variable_list forward(AutogradContext *ctx, const Tensor &P, OptTensor mask, OptTensor bias, bool gated) {
+        Call c{};
+        EvoAttnParams &p = c.p;
+        p.B = (int32_t)P.size(0);
+        p.S = (int32_t)P.size(1);
+        p.N = (int32_t)P.size(2);
+        p.H = (int32_t)P.size(4);
+        p.D = (int32_t)P.size(5);
+        p.dtype = evo_dtype(P.scalar_type());
+        p.dbias_dtype = EVO_F32;
+        p.scale = (float)(1.0 / std::sqrt((double)p.D));
+        strides(p, P);
+        c.gated = gated;
+        TORCH_CHECK_VALUE(operands(c, P, mask, bias), "the mask must be [B,S,1,1,N] and the pair bias [B,1,H,N,N] (B and the mask's S may be 1), on P's device");
+        c10::DeviceGuard on(P.device());
+        Tensor ob = at::empty_like(P);
+        const Aux layout(p);
+        Tensor aux = scratch(layout.lse_bytes + evoattn_prep_bytes(&p), P);
+        layout.place(p, aux);
+        p.q = slot(P, p, 0);
+        p.k = slot(P, p, 1);
+        p.v = slot(P, p, 2);
+        if (gated) {   // the gated output alone: slot 0 stays unwritten
+            p.gate = slot(P, p, 3);
+            p.o_gated = slot(ob, p, 1);
+        } else {
+            p.o = slot(ob, p, 0);
+        }
+        check(evoattn_fwd(&p, stream_of(P)), "evoattn_fwd");
+        Tensor out = ob.select(3, gated ? 1 : 0);
+        // `out` is what the backward reads: saved like any output, so that a consumer who changes it in place is told so
+        // by autograd's version check.  Slot 2 alone is kept under a version counter of its own: the consumer
+        // writes the incoming gradient there in place, which must not look like a change of `out` (the same memory object).
+        Tensor grad_slot = ob.variable_data().select(3, 2);
+        ctx->save_for_backward({P, *mask, *bias, aux, out});
+        ctx->saved_data["slot"] = grad_slot;
+        p.gate = nullptr;
+        p.o_gated = nullptr;
+        ctx->saved_data["call"] = std::string((const char *)&c, sizeof c);
+        ctx->mark_non_differentiable({grad_slot});
+        ctx->set_materialize_grads(false);   // (no tensor of zeros for the second output's gradient, which nobody has)
+        return {out, grad_slot};
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const bool rec = at::GradMode::is_enabled();
+        variable_list res(4);
+        {
+            at::AutoDispatchBelowADInplaceOrView guard;
+            const auto saved = ctx->get_saved_variables();
+            const Tensor &P = saved[0], &mask = saved[1], &bias = saved[2], &aux = saved[3], &out = saved[4];
+            Call c;
+            const std::string bytes = ctx->saved_data["call"].toStringRef();
+            memcpy(&c, bytes.data(), sizeof c);
+            const Tensor slot2 = ctx->saved_data["slot"].toTensor();
+            if (!grads[0].defined()) {   // the output took no part in what is differentiated
+                res[0] = at::zeros_like(P);
+                return res;
+            }
+            const Tensor &dout = grads[0];
+            bool in_place = dout.data_ptr() == slot2.data_ptr() && dout.scalar_type() == slot2.scalar_type() && dout.sizes().equals(slot2.sizes());
+            for (int i = 0; in_place && i < 5; ++i) in_place = slot2.size(i) == 1 || dout.stride(i) == slot2.stride(i);
+            c10::DeviceGuard on(P.device());
+            if (!in_place) const_cast<Tensor &>(slot2).copy_(dout);
+            // (edges are those of the tensors that were given)
+            size_t edge = 1;
+            const bool want_dmask = mask.defined() && ctx->needs_input_grad(edge) && mask.is_floating_point();
+            if (mask.defined()) ++edge;
+            const bool want_dbias = bias.defined() && ctx->needs_input_grad(edge);
+            Tensor DP = P.size(3) == (c.gated ? 4 : 3) ? at::empty_like(P) : at::zeros_like(P);
+            EvoAttnParams p = c.p;
+            Aux(p).place(p, aux);
+            p.q = slot(P, p, 0);
+            p.k = slot(P, p, 1);
+            p.v = slot(P, p, 2);
+            p.mask = mask.defined() ? mask.data_ptr() : nullptr;
+            p.bias = bias.defined() ? bias.data_ptr() : nullptr;
+            p.dout = slot2.data_ptr();
+            p.dq = slot(DP, p, 0);
+            p.dk = slot(DP, p, 1);
+            p.dv = slot(DP, p, 2);
+            if (c.gated) {   // slot 2 is this node's own memory: the gradient of the ungated output takes its place
+                p.o = nullptr;
+                p.gate = slot(P, p, 3);
+                p.dgate = slot(DP, p, 3);
+                p.o_gated = out.data_ptr();
+                p.flags |= EVO_FLAG_GATE_DOUT_INPLACE;
+            } else {
+                p.o = out.data_ptr();
+            }
+            Tensor dbias, dmask;
+            enqueue_backward(p, P, bias, want_dbias, want_dmask, dbias, dmask);
+            res[0] = DP;
+            if (want_dmask) res[1] = finish_dmask(dmask, c);
+            if (want_dbias) res[2] = finish_dbias(dbias, c);
+        }
+        return once_differentiable(std::move(res), rec);
+    }
+};
+
+variable_list slot_attention(const Tensor &P, const OptTensor &mask, const OptTensor &bias, bool gated) {
+    TORCH_CHECK_VALUE(plain(P) && P.is_cuda() && P.dim() == 6 && P.numel() > 0 && P.is_contiguous() && P.size(3) >= (gated ? 4 : 3) &&
+                          (P.scalar_type() == at::kBFloat16 || P.scalar_type() == at::kHalf) && head_dim_built(P.size(5)),
+                      "P must be a contiguous 16-bit [B,S,N,W,H,D] tensor with W >= 3 (4 with a gate) and a head dim the library is built for");
+    return SlotAttention::apply(P, mask, bias, gated);
+}
+
+// ------------------------------------------------------------------ the layers of the block around the attention
+
+// Slices of the rows that a weight gradient is summed over (`_row_slices` in block.py: the same rule, and why).
+int64_t row_slices(int64_t rows, int64_t n_out, int64_t n_in) {
+    const int64_t tiles = ((n_out + 127) / 128) * ((n_in + 127) / 128);
+    int64_t g = 1;
+    while (g * tiles < 512 && rows % (2 * g) == 0 && rows / (2 * g) >= 256) g *= 2;
+    return g;
+}
+
+Tensor weight_grad(const Tensor &dy2, const Tensor &x2) {
+    const int64_t rows = dy2.size(0), g = row_slices(rows, dy2.size(1), x2.size(1));
+    if (g == 1) return dy2.t().mm(x2);
+    return at::bmm(dy2.view({g, rows / g, -1}).transpose(1, 2), x2.view({g, rows / g, -1})).sum(0);
+}
+
+Tensor bias_grad(const Tensor &dy2) {
+    const int64_t rows = dy2.size(0), cols = dy2.size(1);
+    const int dt = evo_dtype(dy2.scalar_type());
+    if (rows && dy2.is_cuda() && dt != EVO_NONE && cols <= INT32_MAX && dy2.stride(1) == 1 && dy2.stride(0) >= cols && dy2.stride(0) % 8 == 0 &&
+        (uintptr_t)dy2.data_ptr() % 16 == 0) {
+        if (const size_t bytes = evoattn_colsum_workspace_bytes(rows, (int32_t)cols, dt)) {
+            c10::DeviceGuard on(dy2.device());
+            Tensor out = at::empty({cols}, dy2.options()), ws = scratch(bytes, dy2);
+            check(evoattn_colsum(dy2.data_ptr(), dy2.stride(0), out.data_ptr(), ws.data_ptr(), (size_t)ws.numel(), rows, (int32_t)cols, dt,
+                                 stream_of(dy2)), "evoattn_colsum");
+            return out;
+        }
+    }
+    return dy2.sum(0);
+}
+
+Tensor as_rows(const Tensor &t) { return t.reshape({-1, t.size(-1)}); }
+
+struct LinearNode : SavingNode {
+    bool has_bias = false;
+    Tensor dx_place;
+    std::string name() const override { return "LinearBackward"; }
+    variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        const bool rec = at::GradMode::is_enabled();
+        variable_list out(3);
+        if (!grads[0].defined()) return out;
+        {
+            at::AutoDispatchBelowADInplaceOrView guard;
+            const Tensor x = saved[0].unpack(), w = saved[1].unpack(), dy2 = as_rows(grads[0]);
+            if (task_should_compute_output(0)) {
+                if (dx_place.defined()) {
+                    Tensor rows = dx_place.view({-1, x.size(-1)});
+                    at::mm_out(rows, dy2, w);
+                    out[0] = dx_place;
+                } else {
+                    out[0] = dy2.mm(w).view(x.sizes());
+                }
+            }
+            if (task_should_compute_output(1)) out[1] = weight_grad(dy2, as_rows(x));
+            if (has_bias && task_should_compute_output(2)) out[2] = bias_grad(dy2);
+        }
+        return once_differentiable(std::move(out), rec);
+    }
+};
+
+// x W^T + b with the weight gradient summed over slices of the rows; `dx_place` (shaped like x, rows may lie apart): where
+// the input gradient is to be written.
+Tensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, const OptTensor &dx_place) {
+    Tensor y;
+    {
+        at::AutoDispatchBelowADInplaceOrView guard;
+        // (as a matrix: for an input of more dimensions whose rows lie apart torch multiplies and then adds the
+        // bias in a pass of its own)
+        y = at::linear(as_rows(x), weight, bias);
+        auto shape = x.sizes().vec();
+        shape.back() = weight.size(0);
+        y = y.view(shape);
+    }
+    const Tensor b = bias ? *bias : Tensor();
+    if (SavingNode::wanted(x, weight, b)) {
+        auto node = make_node<LinearNode>(x, weight, b);
+        node->has_bias = b.defined();
+        if (dx_place) node->dx_place = *dx_place;
+        torch::autograd::set_history(y, node);
+        node->save(x);
+        node->save(weight);
+    }
+    return y;
+}
+
+struct StackedNode : SavingNode {
+    std::vector<int64_t> sizes;
+    bool has_bias = false;
+    std::string name() const override { return "StackedProjectionBackward"; }
+    // results: x, gate_bias, the weights
+    variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        const bool rec = at::GradMode::is_enabled();
+        variable_list out(2 + sizes.size());
+        if (!grads[0].defined()) return out;
+        {
+            at::AutoDispatchBelowADInplaceOrView guard;
+            const Tensor x = saved[0].unpack(), w = saved[1].unpack(), dp2 = as_rows(grads[0]);
+            if (task_should_compute_output(0)) out[0] = dp2.mm(w).view(x.sizes());
+            if (has_bias && task_should_compute_output(1)) out[1] = bias_grad(dp2.narrow(1, dp2.size(1) - sizes.back(), sizes.back()));
+            bool any = false;
+            for (size_t i = 0; i < sizes.size(); ++i) any |= task_should_compute_output(2 + i);
+            if (any) {
+                auto parts = weight_grad(dp2, as_rows(x)).split_with_sizes(sizes, 0);
+                for (size_t i = 0; i < sizes.size(); ++i) out[2 + i] = parts[i];
+            }
+        }
+        return once_differentiable(std::move(out), rec);
+    }
+};
+
+// Several projections of one input as one GEMM with their weights stacked; `gate_bias` is added on the last layer's columns.
+Tensor stacked_projection(const Tensor &x, const OptTensor &gate_bias, const std::vector<Tensor> &weights) {
+    Tensor y, w;
+    const Tensor gb = gate_bias ? *gate_bias : Tensor();
+    {
+        at::AutoDispatchBelowADInplaceOrView guard;
+        w = at::cat(weights, 0);
+        OptTensor bias;
+        if (gb.defined()) bias = at::constant_pad_nd(gb, {w.size(0) - gb.size(0), 0});
+        y = at::linear(x, w, bias);
+    }
+    bool needed = SavingNode::wanted(x, gb);
+    for (const auto &t : weights) needed |= SavingNode::wanted(t);
+    if (needed) {
+        std::shared_ptr<StackedNode> node(new StackedNode(), torch::autograd::deleteNode);
+        variable_list inputs{x, gb};
+        inputs.insert(inputs.end(), weights.begin(), weights.end());
+        node->set_next_edges(torch::autograd::collect_next_edges(inputs));
+        for (const auto &t : weights) node->sizes.push_back(t.size(0));
+        node->has_bias = gb.defined();
+        torch::autograd::set_history(y, node);
+        node->save(x);
+        node->save(w);
+    }
+    return y;
+}
+
+struct LayerNormNode : SavingNode {
+    bool has_bias = false;
+    std::string name() const override { return "LayerNormBackward"; }
+    variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        const bool rec = at::GradMode::is_enabled();
+        variable_list out(3);
+        if (!grads[0].defined()) return out;
+        {
+            at::AutoDispatchBelowADInplaceOrView guard;
+            const Tensor x = saved[0].unpack(), w = saved[1].unpack(), stats = saved[2].unpack(), dy = grads[0].contiguous();
+            const int64_t cols = x.size(-1), rows = x.numel() / cols;
+            const bool need_x = task_should_compute_output(0), need_w = w.defined() && task_should_compute_output(1),
+                       need_b = has_bias && task_should_compute_output(2);
+            c10::DeviceGuard on(x.device());
+            const int dt = evo_dtype(x.scalar_type());
+            Tensor ws;
+            if (need_x) out[0] = at::empty_like(x);
+            if (need_w) out[1] = at::empty({cols}, x.options());
+            if (need_b) out[2] = at::empty({cols}, x.options());
+            if (need_w || need_b) ws = scratch(evoattn_layernorm_bwd_workspace_bytes(rows, (int32_t)cols, dt), x);
+            const float *mean = (const float *)stats.data_ptr();
+            auto ptr = [](const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; };
+            if (need_x || need_w || need_b)
+                check(evoattn_layernorm_bwd(dy.data_ptr(), x.data_ptr(), ptr(w), mean, mean + (rows + 3) / 4 * 4, ptr(out[0]), ptr(out[1]), ptr(out[2]),
+                                            ptr(ws), ws.defined() ? (size_t)ws.numel() : 0, rows, (int32_t)cols, dt, stream_of(x)),
+                      "evoattn_layernorm_bwd");
+        }
+        return once_differentiable(std::move(out), rec);
+    }
+};
+
+// LayerNorm over the last dimension through the library's kernels: x and y cross HBM once in the forward, x, dy and dx once in
+// the backward.  None for rows, dtypes or devices that those kernels do not take.
+OptTensor layer_norm(const Tensor &x, const OptTensor &weight, const OptTensor &bias, double eps) {
+    const int dt = evo_dtype(x.scalar_type());
+    const Tensor w0 = weight ? *weight : Tensor(), b0 = bias ? *bias : Tensor();
+    if (!plain(x) || !plain_modes() || !x.is_cuda() || x.dim() < 1 || x.numel() == 0 || dt == EVO_NONE || x.size(-1) > INT32_MAX) return std::nullopt;
+    for (const Tensor &t : {w0, b0})
+        if (t.defined() && (!plain(t) || t.scalar_type() != x.scalar_type() || t.device() != x.device() || t.dim() != 1 || t.size(0) != x.size(-1)))
+            return std::nullopt;
+    if (evoattn_layernorm_bwd_workspace_bytes(1, (int32_t)x.size(-1), dt) == 0) return std::nullopt;
+    Tensor y, xc, w, b, stats;
+    {
+        at::AutoDispatchBelowADInplaceOrView guard;
+        c10::DeviceGuard on(x.device());
+        xc = x.contiguous();
+        w = w0.defined() ? w0.contiguous() : Tensor();
+        b = b0.defined() ? b0.contiguous() : Tensor();
+        const int64_t cols = xc.size(-1), rows = xc.numel() / cols, rows4 = (rows + 3) / 4 * 4;
+        y = at::empty_like(xc);
+        stats = at::empty({2 * rows4}, xc.options().dtype(at::kFloat));   // mean, then 1 / deviation, each on a 16-byte boundary
+        float *mean = (float *)stats.data_ptr();
+        check(evoattn_layernorm_fwd(xc.data_ptr(), w.defined() ? w.data_ptr() : nullptr, b.defined() ? b.data_ptr() : nullptr, y.data_ptr(), mean,
+                                    mean + rows4, rows, (int32_t)cols, dt, (float)eps, stream_of(xc)), "evoattn_layernorm_fwd");
+    }
+    if (SavingNode::wanted(x, w0, b0)) {
+        auto node = make_node<LayerNormNode>(x, w0, b0);
+        node->has_bias = b0.defined();
+        torch::autograd::set_history(y, node);
+        node->save(xc);
+        node->save(w);
+        node->save(stats);
+    }
+    return y;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+    namespace py = pybind11;
+    const py::call_guard<py::gil_scoped_release> no_gil;
+    m.def("attention", &attention, no_gil, py::arg("Q"), py::arg("K"), py::arg("V"), py::arg("res_mask"), py::arg("pair_bias"), py::arg("gate"),
+          py::arg("per_head"), py::arg("flags"));
+    m.def("slot_attention", &slot_attention, no_gil, py::arg("P"), py::arg("res_mask"), py::arg("pair_bias"), py::arg("gated"));
+    m.def("linear", &linear, no_gil, py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("dx_place"));
+    m.def("stacked_projection", &stacked_projection, no_gil, py::arg("x"), py::arg("gate_bias"), py::arg("weights"));
+    m.def("layer_norm", &layer_norm, no_gil, py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("eps"));
+}

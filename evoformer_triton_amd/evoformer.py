@@ -472,6 +472,15 @@ def _op_gated_backward(ctx, dOg, dlse, dprep, dseen):
 _op_fwd_gated.register_autograd(_op_gated_backward, setup_context=_op_gated_setup_context)
 
 
+def _native(Q, K, V, res_mask, pair_bias, gate, per_head):
+    """The call through the C++ host path (csrc/host.cpp: checks, allocations, launches and the autograd node without
+    the interpreter), or None where that path does not take it: under the tracer, where the device work is the
+    registered operator, and for empty problems, head dims that need padding and invalid arguments."""
+    if torch.compiler.is_compiling():
+        return None
+    return _lib.host().attention(Q, K, V, res_mask, pair_bias, gate, per_head, FLAGS)
+
+
 class EvoformerAttention(torch.autograd.Function):
     """`EvoformerAttention.apply(Q, K, V, res_mask, pair_bias)` (evoformer.py:633-862).
 
@@ -480,6 +489,11 @@ class EvoformerAttention(torch.autograd.Function):
     dense tensor is reinterpreted as [Batch, Head, N_seq, N_res, Dim] by a flat reshape
     (evoformer.py:648-650), and the output is reshaped back the same way (:735).
     """
+
+    @classmethod
+    def apply(cls, Q, K, V, res_mask=None, pair_bias=None):
+        out = _native(Q, K, V, res_mask, pair_bias, None, False)
+        return super().apply(Q, K, V, res_mask, pair_bias) if out is None else out
 
     @staticmethod
     def forward(ctx, Q, K, V, res_mask=None, pair_bias=None):
@@ -494,6 +508,11 @@ class EvoformerAttention(torch.autograd.Function):
 
 class _PerHeadAttention(torch.autograd.Function):
     """Same kernels with true per-head semantics: head h of problem (b,s) is Q[b,s,:,h,:]."""
+
+    @classmethod
+    def apply(cls, Q, K, V, res_mask=None, pair_bias=None):
+        out = _native(Q, K, V, res_mask, pair_bias, None, True)
+        return super().apply(Q, K, V, res_mask, pair_bias) if out is None else out
 
     @staticmethod
     def forward(ctx, Q, K, V, res_mask=None, pair_bias=None):
@@ -511,6 +530,11 @@ class _GatedAttention(torch.autograd.Function):
     returns O ungated, evoformer.py:735).  `gate`: the gate logits, shaped like Q.  No ungated O is written:
     the gated output is kept for the backward, which returns the gate's gradient as a sixth value.  Under torch.compile the
     same work goes through torch.ops.evoattn.fwd_gated / .bwd_gated."""
+
+    @classmethod
+    def apply(cls, Q, K, V, res_mask, pair_bias, gate, layout):
+        out = _native(Q, K, V, res_mask, pair_bias, gate, layout == "ds4sci")
+        return super().apply(Q, K, V, res_mask, pair_bias, gate, layout) if out is None else out
 
     @staticmethod
     def forward(ctx, Q, K, V, res_mask, pair_bias, gate, layout):
@@ -560,7 +584,7 @@ def _finish_dmask(dmask, mask_orig, B, S, N):
     return dmask.to(dtype)
 
 
-class _SlotAttention(torch.autograd.Function):
+class _SlotAttention:
     """Per-head attention on Q, K, V (and the gate's logits) that are the slots 0, 1, 2 (and 3) of one
     contiguous tensor P [B,S,N,W,H,D]: the result of one projection GEMM with the weights of the three or
     four Linear layers stacked, which reads the block's input once instead of W times.  The kernels take the
@@ -582,90 +606,8 @@ class _SlotAttention(torch.autograd.Function):
     the projection's input and weight gradients are single GEMMs over it."""
 
     @staticmethod
-    def forward(ctx, P, res_mask, pair_bias, gated):
-        lib = _lib.load()
-        B, S, N, W, H, D = P.shape
-        if not P.is_contiguous() or W < (4 if gated else 3) or P.dtype not in (torch.bfloat16, torch.float16) or D not in _HEAD_DIMS:
-            raise ValueError("P must be a contiguous 16-bit [B,S,N,W,H,D] tensor with W >= 3 (4 with a gate) and a head dim the library is built for")
-        mask, mask_kind, mstr = _prep_mask(res_mask, B, S, N, P.device)
-        bias, bias_dt, bstr = _prep_bias(pair_bias, B, H, N, P.dtype, P.device)
-        with _on_device(P.device):
-            OB = torch.empty_like(P)
-            lse = torch.empty((B, H, S, N), device=P.device, dtype=torch.float32)
-            p = _SlotAttention._params(P, OB, mask, mask_kind, mstr, bias, bias_dt, bstr, lse)
-            prep = _alloc_bytes(lib.evoattn_prep_bytes(ctypes.byref(p)), P.device)
-            p.prep, p.prep_bytes = _ptr(prep), prep.numel()
-            if gated:         # the gated output alone: slot 0 stays unwritten
-                p.o = None
-                p.gate, p.o_gated = _ptr(P[:, :, :, 3]), _ptr(OB[:, :, :, 1])
-            _lib.check(lib.evoattn_fwd(ctypes.byref(p), _stream(P.device)), "evoattn_fwd")
-        out = OB[:, :, :, 1 if gated else 0]
-        # `out` is what the backward reads (O, or with a gate sigmoid(g) * O): saved like any output, so that a
-        # consumer who changes it in place is told so by autograd's version check.  Slot 2 alone is kept under a
-        # version counter of its own (`.data`): the consumer writes the incoming gradient there in place, which
-        # must not look like a change of `out` (the same memory object) to whoever saved `out` for its backward.
-        grad_slot = OB.data[:, :, :, 2]
-        ctx.save_for_backward(P, mask, bias, lse, prep, out)
-        ctx.grad_slot = grad_slot
-        ctx.gated = bool(gated)
-        ctx.mask_meta = (mask_kind, mstr, None if res_mask is None else (tuple(res_mask.shape), res_mask.dtype))
-        ctx.bias_meta = (bias_dt, bstr, None if pair_bias is None else (tuple(pair_bias.shape), pair_bias.dtype))
-        ctx.mark_non_differentiable(grad_slot)
-        ctx.set_materialize_grads(False)      # (no tensor of zeros for the second output's gradient, which nobody has)
-        return out, grad_slot
-
-    @staticmethod
-    def _params(P, OB, mask, mask_kind, mstr, bias, bias_dt, bstr, lse):
-        """OB: the buffer of outputs (its slot 0 is O), or None where the caller sets `o` / `o_gated` itself."""
-        B, S, N, W, H, D = P.shape
-        p = _params(P[:, :, :, 0], P[:, :, :, 1], P[:, :, :, 2], mask, mask_kind, mstr, bias, bias_dt, bstr,
-                    None if OB is None else OB[:, :, :, 0], lse, "ds4sci")
-        p.stride_b, p.stride_h, p.stride_s, p.stride_n = S * N * W * H * D, D, N * W * H * D, W * H * D
-        return p
-
-    @staticmethod
-    def backward(ctx, dout, _unused):
-        lib = _lib.load()
-        P, mask, bias, lse, prep, out = ctx.saved_tensors
-        B, S, N, W, H, D = P.shape
-        mask_kind, mstr, mask_orig = ctx.mask_meta
-        bias_dt, bstr, bias_orig = ctx.bias_meta
-        slot = ctx.grad_slot
-        if dout is None:                      # the output took no part in what is differentiated
-            return torch.zeros_like(P), None, None, None
-        in_place = dout.data_ptr() == slot.data_ptr() and dout.dtype == slot.dtype and dout.shape == slot.shape and all(
-            n == 1 or a == b for n, a, b in zip(slot.shape, dout.stride(), slot.stride()))
-        if not in_place:
-            slot.copy_(dout)
-        want_dmask = bool(ctx.needs_input_grad[1] and mask is not None and mask.is_floating_point())
-        want_dbias = bool(ctx.needs_input_grad[2] and bias is not None)
-        with _on_device(P.device):
-            DP = torch.empty_like(P) if W == (4 if ctx.gated else 3) else torch.zeros_like(P)
-            p = _SlotAttention._params(P, None, mask, mask_kind, mstr, bias, bias_dt, bstr, lse)
-            p.dout, p.dq, p.dk, p.dv = _ptr(slot), _ptr(DP[:, :, :, 0]), _ptr(DP[:, :, :, 1]), _ptr(DP[:, :, :, 2])
-            if ctx.gated:     # slot 2 is this Function's own memory: the gradient of the ungated output takes its place
-                # (delta and the gate's gradient come from the gated output, which is `out`; no ungated O exists)
-                p.gate, p.dgate, p.o_gated = _ptr(P[:, :, :, 3]), _ptr(DP[:, :, :, 3]), _ptr(out)
-                p.flags |= _lib.EVO_FLAG_GATE_DOUT_INPLACE
-            else:
-                p.o = _ptr(out)
-            dbias = dmask = None
-            if want_dbias:
-                dbias = torch.empty((B, H, N, N), device=P.device, dtype=bias.dtype)
-                p.dbias, p.dbias_dtype = _ptr(dbias), _DTYPES[bias.dtype]
-            if want_dmask:
-                dmask = torch.empty((B, S, N), device=P.device, dtype=torch.float32)
-                p.dmask = _ptr(dmask)
-            ws = _alloc_bytes(lib.evoattn_bwd_workspace_bytes(ctypes.byref(p)), P.device)
-            p.workspace, p.workspace_bytes = _ptr(ws), ws.numel()
-            p.prep, p.prep_bytes = _ptr(prep), prep.numel()
-            p.flags |= _lib.EVO_FLAG_PREP_VALID
-            _lib.check(lib.evoattn_bwd(ctypes.byref(p), _stream(P.device)), "evoattn_bwd")
-        if dbias is not None:
-            dbias = _finish_dbias(dbias, bias_orig, B, H, N)
-        if dmask is not None:
-            dmask = _finish_dmask(dmask, mask_orig, B, S, N)
-        return DP, dmask, dbias, None
+    def apply(P, res_mask, pair_bias, gated):
+        return _lib.host().slot_attention(P, res_mask, pair_bias, bool(gated))
 
 
 def slot_attention(P, res_mask=None, pair_bias=None, gated: bool = False):

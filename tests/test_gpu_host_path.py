@@ -1,0 +1,71 @@
+"""The C++ host path of the operator against the Python one: same kernels, same bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # B, S, N, H, D, mask, bias, per_head, gated, dtype
+    (1, 1, 1, 1, 8, None, None, False, False, torch.bfloat16),
+    (2, 3, 33, 2, 32, "f64", "f16", False, False, torch.bfloat16),      # operands of foreign dtypes, widened
+    (2, 3, 40, 2, 16, "one", "shared", True, False, torch.float16),     # broadcast over the batch and the rows
+    (1, 4, 200, 3, 64, "bool", "strided", True, True, torch.bfloat16),
+    (2, 2, 24, 2, 128, "int", "same", False, True, torch.float32),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_both_host_paths_give_the_same_bits(gpu_device, case, monkeypatch):
+    import evoformer_triton_amd.evoformer as E
+    B, S, N, H, D, mask, bias, per_head, gated, dt = case
+    g = torch.Generator().manual_seed(3)
+    q, k, v, gate, dO = (torch.randn((B, S, N, H, D), generator=g).to(dt).to(gpu_device) for _ in range(5))
+    keep = torch.rand((1 if mask == "one" else B, 1 if mask == "one" else S, 1, 1, N), generator=g) < 0.8
+    keep[..., 0] = True
+    m = None if mask is None else {"bool": keep, "int": keep.long(), "f64": torch.where(keep, 0.25, -1e9).double(),
+                                   "one": torch.where(keep, 0.5, -1e9)}[mask].to(gpu_device)
+    b = None
+    if bias is not None:
+        b = torch.randn((1 if bias == "shared" else B, 1, H, N, N * (2 if bias == "strided" else 1)), generator=g)
+        b = b.to(torch.float16 if bias == "f16" else dt).to(gpu_device)
+        b = b[..., ::2] if bias == "strided" else b
+    fmask = m is not None and m.is_floating_point()
+
+    def run():
+        leaves = [t.detach().clone().requires_grad_() for t in (q, k, v)] + ([gate.detach().clone().requires_grad_()] if gated else [])
+        bb = None if b is None else b.detach().requires_grad_()
+        mm = m.detach().requires_grad_() if fmask else m
+        o = E.evoformer_attention(*leaves[:3], mm, bb, layout="ds4sci" if per_head else "reference", gate=leaves[3] if gated else None)
+        return [o, *torch.autograd.grad(o, leaves + ([] if bb is None else [bb]) + ([mm] if fmask else []), dO)]
+
+    got = run()
+    monkeypatch.setattr(E, "_native", lambda *a: None)
+    want = run()
+    for a, w in zip(got, want):
+        assert a.shape == w.shape and a.dtype == w.dtype and torch.equal(a, w)
+
+
+def test_the_native_node_is_once_differentiable(gpu_device):
+    import evoformer_triton_amd.evoformer as E
+    q = torch.randn((1, 2, 32, 2, 32), device=gpu_device).requires_grad_()
+    o = E.EvoformerAttention.apply(q, q, q, None, None)
+    (dq,) = torch.autograd.grad(o, q, torch.ones_like(o), create_graph=True)
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        dq.sum().backward()
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(o, q, torch.ones_like(o))
+        torch.autograd.grad(o, q, torch.ones_like(o))
+
+
+def test_what_the_native_path_does_not_take(gpu_device):
+    """Head dims that need padding go the Python way; invalid arguments keep their errors."""
+    import evoformer_triton_amd.evoformer as E
+    q = torch.randn((1, 2, 32, 2, 24), device=gpu_device, dtype=torch.bfloat16).requires_grad_()
+    o = E.EvoformerAttention.apply(q, q, q)
+    assert o.shape == q.shape and torch.isfinite(torch.autograd.grad(o, q, torch.ones_like(o))[0]).all()
+    p = torch.randn((1, 2, 32, 2, 32), device=gpu_device, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="res_mask"):
+        E.EvoformerAttention.apply(p, p, p, torch.zeros(1, 2, 1, 1, 31, device=gpu_device), None)
+    with pytest.raises(ValueError, match="pair_bias"):
+        E.EvoformerAttention.apply(p, p, p, None, torch.zeros(1, 1, 3, 32, 32, device=gpu_device))
+    with pytest.raises(RuntimeError, match="same device"):
+        E.EvoformerAttention.apply(p, p, p, torch.zeros(1, 2, 1, 1, 32), None)
