@@ -97,6 +97,23 @@ static bool mfma_ok(const EvoAttnParams &p, int pass) {
     return true;
 }
 
+// fp32 on the fp32 matrix instruction (f32.hip): rows and their strides in whole 16-byte pieces.  Anything else in fp32 (and 16-bit tensors at odd addresses) takes the plain
+// kernels, one row per thread on the vector ALU.
+static bool f32_ok(const EvoAttnParams &p, int pass) {
+    if (p.dtype != EVO_F32 || (p.flags & EVO_FLAG_FORCE_GENERIC)) return false;
+    if (p.stride_b % 4 || p.stride_h % 4 || p.stride_s % 4 || p.stride_n % 4) return false;
+    if (!aligned(p.q, 16) || !aligned(p.k, 16) || !aligned(p.v, 16) || !aligned(p.o, 16)) return false;
+    // (a problem's rows, whole tiles of them, and a bias matrix lie within 32-bit byte offsets)
+    if ((int64_t)(p.N + 64) * p.stride_n + p.D >= ((int64_t)1 << 30)) return false;
+    if (p.bias && (int64_t)p.N * p.bias_stride_row >= ((int64_t)1 << 30)) return false;
+    const int64_t nb = (p.N + 63) / 64;
+    if (pass == EVO_PASS_BWD) {
+        if (!aligned(p.dout, 16) || !aligned(p.dq, 16) || !aligned(p.dk, 16) || !aligned(p.dv, 16)) return false;
+        if (p.dbias && nb * nb * p.B * p.H * f32_dbias_chunks(p) > (int64_t)0x7fffffff) return false;
+    }
+    return true;
+}
+
 static int bias_vec_ok(const EvoAttnParams &p) {
     if (!p.bias) return 0;
     const size_t a = p.bias_dtype == EVO_F32 ? 16 : 8;
@@ -192,6 +209,12 @@ static bool dq_writes_dbias(const EvoAttnParams &p) { return p.dbias && p.S == 1
 // per workgroup, rounds and partials (below).
 static void chunking(const EvoAttnParams &p, int *n_chunks, int *chunk) {
     const int64_t NT = (p.N + 31) / 32;
+    if (p.dtype == EVO_F32) {
+        const int want = f32_dbias_chunks(p);
+        *chunk = (p.S + want - 1) / want;
+        *n_chunks = (p.S + *chunk - 1) / *chunk;
+        return;
+    }
     if (dq_split_ok(p)) {
         // the dBias kernel: one workgroup per block of 128 queries x 128 keys (64 at head dim 64), (b, h) and chunk, two
         // workgroups per CU (256 CUs) at a time; among the chunk counts that give one to four rounds
@@ -411,6 +434,7 @@ static int launch_dq(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
 
 const char *evoattn_kernels(const EvoAttnParams *p, int pass) {
     if (!p) return "invalid";
+    if (f32_ok(*p, pass)) return pass == EVO_PASS_FWD ? "f32_fwd" : p->dbias ? "f32_dq+f32_dbias,f32_dkdv" : "f32_dq,f32_dkdv";
     if (!mfma_ok(*p, pass)) return "generic";
     if (pass == EVO_PASS_FWD) return fwd_ring_ok(*p) ? "mfma_fwd_ring" : "mfma_fwd";
     const bool kvr = kv_ring_ok(*p);
@@ -435,6 +459,7 @@ int evoattn_fwd(const EvoAttnParams *p, void *hip_stream) {
     int rc = evoattn_check(p, EVO_PASS_FWD);
     if (rc) return rc;
     hipStream_t st = (hipStream_t)hip_stream;
+    if (f32_ok(*p, EVO_PASS_FWD)) return launch_f32_fwd(*p, st);
     if (!mfma_ok(*p, EVO_PASS_FWD)) return launch_generic_fwd(*p, st);
     if ((rc = check_prep(*p))) return rc;
     return fwd_launches(*p, st);
@@ -460,7 +485,8 @@ int evoattn_fwd_static(const EvoAttnParams *p, void *hip_stream) {
     int rc = evoattn_check(p, EVO_PASS_FWD);
     if (rc) return rc;
     hipStream_t st = (hipStream_t)hip_stream;
-    if (!mfma_ok(*p, EVO_PASS_FWD)) return launch_generic_fwd(*p, st);   // those kernels take no prepared operands
+    if (f32_ok(*p, EVO_PASS_FWD)) return launch_f32_fwd(*p, st);         // (these kernels take no prepared operands,
+    if (!mfma_ok(*p, EVO_PASS_FWD)) return launch_generic_fwd(*p, st);   // nor do those)
     if (prep_layout(*p).total > (size_t)EVOATTN_STATIC_PREP_BYTES) return EVO_EWORKSPACE;
     EvoAttnParams q = *p;
     if ((rc = static_prep(&q.prep))) return rc;
@@ -509,6 +535,7 @@ int evoattn_bwd(const EvoAttnParams *p0, void *hip_stream) {
     e.shift = (float *)(ws + w.shift);
     e.dmask_part = (float *)(ws + w.dmask_part);
     e.dbias_part = (float *)(ws + w.dbias_part);
+    if (f32_ok(*p, EVO_PASS_BWD)) return launch_f32_bwd(*p, e, st);
     if (!mfma_ok(*p, EVO_PASS_BWD)) return launch_generic_bwd(*p, e, st);
     if ((rc = check_prep(*p))) return rc;
     fill_prep(*p, e);

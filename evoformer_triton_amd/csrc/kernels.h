@@ -8,6 +8,9 @@ namespace evo {
 
 int launch_generic_fwd(const EvoAttnParams &p, hipStream_t st);
 int launch_generic_bwd(const EvoAttnParams &p, const Extra &e, hipStream_t st);
+int launch_f32_fwd(const EvoAttnParams &p, hipStream_t st);
+int launch_f32_bwd(const EvoAttnParams &p, const Extra &e, hipStream_t st);
+int f32_dbias_chunks(const EvoAttnParams &p);  // chunks of S rows that those kernels split a dBias sum into
 int launch_delta_generic(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_dmask_reduce(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_dbias_reduce(const EvoAttnParams &p, const Extra &e, hipStream_t st);

@@ -40,7 +40,7 @@ enum {
     EVO_NONE = -1,
     EVO_BF16 = 0,
     EVO_F16  = 1,
-    EVO_F32  = 2   /* "check mode": every product and sum in fp32, no matrix cores */
+    EVO_F32  = 2   /* every product and sum in fp32, on the fp32 matrix instruction where rows lie in whole 16-byte pieces */
 };
 
 /* row-mask encodings; mask is indexed [b][s][key], key contiguous */
@@ -202,11 +202,11 @@ int evoattn_fwd_static(const EvoAttnParams *p, void *hip_stream);
 int evoattn_bwd(const EvoAttnParams *p, void *hip_stream);
 
 /* Name of the kernel family evoattn_fwd/evoattn_bwd would run for these parameters
- * ("mfma" or "generic"); for tests and reports. */
+ * ("mfma": 16-bit operands on the matrix cores, or "generic": the rest); for tests and reports. */
 const char *evoattn_path(const EvoAttnParams *p, int pass);
 
 /* Names of the main kernels that pass would launch, comma separated (e.g. "mfma_fwd_ring",
- * "mfma_dq_ring,mfma_dkdv", "mfma_dq_wide,mfma_dkdv", "generic"); for reports and profiles. */
+ * "mfma_dq_ring,mfma_dkdv", "mfma_dq_wide,mfma_dkdv", "f32_dq+f32_dbias,f32_dkdv", "generic"); for reports and profiles. */
 const char *evoattn_kernels(const EvoAttnParams *p, int pass);
 
 /* ---- LayerNorm of the block around the attention -------------------------------------------
