@@ -294,9 +294,23 @@ typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 struct Tile16 {
     u32x4_t w[2];
 };
+// In memory a tile lies in pieces of 16 bytes per lane, lane after lane: the first pieces of all lanes, then the second
+// ones, so that a load instruction of the wave covers 1 KB without gaps.  (With a lane's pieces side by side, every
+// instruction touched all of the tile's cache lines and used a half, of fp32 tiles a quarter, of each: the CU's
+// vector cache then carries two to four times the lookups; fp32 bias, B = 1, S = 200, N = 640, H = 5, head dim 64, step
+// 1181 -> 1136 us.)
+// `lane_tile`: the tile's first element + lane * 8.
 __device__ __forceinline__ void load_tile16(const unsigned short *lane_tile, Tile16 &t) {
     t.w[0] = *reinterpret_cast<const u32x4_t *>(lane_tile);
-    t.w[1] = *reinterpret_cast<const u32x4_t *>(lane_tile + 8);
+    t.w[1] = *reinterpret_cast<const u32x4_t *>(lane_tile + 512);
+}
+// The same for a tile prepared in fp32, four pieces of four entries.  `lane_tile`: the tile's first element + lane * 4.
+__device__ __forceinline__ void load_tile32(const float *lane_tile, f32x16 &dst) {
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(lane_tile + 256 * rr);
+        dst[4 * rr] = v[0]; dst[4 * rr + 1] = v[1]; dst[4 * rr + 2] = v[2]; dst[4 * rr + 3] = v[3];
+    }
 }
 template <typename T>
 __device__ __forceinline__ void unpack_tile16(const Tile16 &t, float mul, f32x16 &dst) {

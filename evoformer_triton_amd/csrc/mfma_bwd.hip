@@ -84,8 +84,8 @@ __global__ void __launch_bounds__(256) mfma_dq(EvoAttnParams p, Extra e) {
 
     const int bb = e.bias_batches > 1 ? b : 0;
     const int64_t tile0 = ((((int64_t)bb * p.H + h) * NT + qt) * NT) * 1024;
-    const float *btile0 = e.bq + tile0 + lane * 16;
-    const float *ztile = e.bq + e.zero_tile + lane * 16;
+    const float *btile0 = e.bq + tile0 + lane * 4;
+    const float *ztile = e.bq + e.zero_tile + lane * 4;
     // or, for a bias that is used too few times to pay for the tiles, this lane's row of the
     // caller's tensor
     const bool bdirect = HAS_BIAS && e.bias_direct;
@@ -102,16 +102,12 @@ __global__ void __launch_bounds__(256) mfma_dq(EvoAttnParams p, Extra e) {
         }
         if (e.bq16) {   // uniform: a bias in the dtype of q is prepared as given, 16 bits per entry
             Tile16 t;
-            load_tile16(e.bq16 + (dead_row ? e.zero_tile : tile0 + (int64_t)kt * 1024) + lane * 16, t);
+            load_tile16(e.bq16 + (dead_row ? e.zero_tile : tile0 + (int64_t)kt * 1024) + lane * 8, t);
             unpack_tile16<T>(t, dead_row ? 0.0f : kLog2e, dst);
             return;
         }
         const float *src = dead_row ? ztile : btile0 + (int64_t)kt * 1024;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-            const f32x4 v = *reinterpret_cast<const f32x4 *>(src + 4 * rr);
-            dst[4 * rr] = v[0]; dst[4 * rr + 1] = v[1]; dst[4 * rr + 2] = v[2]; dst[4 * rr + 3] = v[3];
-        }
+        load_tile32(src, dst);
     };
     f32x16 bres[NRES];
     if (BIAS_RESIDENT) {
@@ -407,8 +403,8 @@ __global__ void __launch_bounds__(NW * 64, D >= 64 ? 2 : NW == 8 ? 4 : 3) mfma_d
 
     const int bb = e.bias_batches > 1 ? pr.b : 0;
     const int ktc = min(key0 >> 5, NT - 1);
-    const float *btile = dead ? e.bk + e.zero_tile + lane * 16
-                              : e.bk + (((int64_t)bb * p.H + pr.h) * NT * NT + ktc) * 1024 + lane * 16;
+    const float *btile = dead ? e.bk + e.zero_tile + lane * 4
+                              : e.bk + (((int64_t)bb * p.H + pr.h) * NT * NT + ktc) * 1024 + lane * 4;
     const int64_t bstep = dead ? 0 : (int64_t)NT * 1024;  // next query tile, same key tile
     // or, for a bias that is used too few times to pay for the tiles, this lane's column of
     // the caller's tensor
@@ -417,8 +413,8 @@ __global__ void __launch_bounds__(NW * 64, D >= 64 ? 2 : NW == 8 ? 4 : 3) mfma_d
     const char *bmat = (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h) * (bf32 ? 4 : 2);
     const float bmul = dead ? 0.0f : kLog2e;
     const unsigned short *btile16 = !TILE16 ? nullptr
-                                    : dead  ? e.bk16 + e.zero_tile + lane * 16
-                                            : e.bk16 + (((int64_t)bb * p.H + pr.h) * NT * NT + ktc) * 1024 + lane * 16;
+                                    : dead  ? e.bk16 + e.zero_tile + lane * 8
+                                            : e.bk16 + (((int64_t)bb * p.H + pr.h) * NT * NT + ktc) * 1024 + lane * 8;
     auto cval = [&](const CTile &t) -> f32x16 {
         if constexpr (TILE16) {
             f32x16 v;
@@ -436,11 +432,7 @@ __global__ void __launch_bounds__(NW * 64, D >= 64 ? 2 : NW == 8 ? 4 : 3) mfma_d
             else bias_tile_cols<T, false>(bmat, keyc, min(qt, NT - 1) * 32, p.N, (unsigned)p.bias_stride_row, g, bmul, dst);
         } else if (HAS_BIAS) {
             const float *src = btile + (int64_t)min(qt, NT - 1) * bstep;
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(src + 4 * rr);
-                dst[4 * rr] = v[0]; dst[4 * rr + 1] = v[1]; dst[4 * rr + 2] = v[2]; dst[4 * rr + 3] = v[3];
-            }
+            load_tile32(src, dst);
         }
     };
 

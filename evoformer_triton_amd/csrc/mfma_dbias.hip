@@ -81,16 +81,12 @@ __global__ void __launch_bounds__(256, 2) mfma_dbias(EvoAttnParams p, Extra e) {
 #pragma unroll
     for (int j = 0; j < TPW; ++j) {
         const int kt = min(k0 / 32 + j, NT - 1);
-        const int64_t o = ((((int64_t)bb * p.H + h) * NT + qtc) * NT + kt) * 1024 + lane * 16;
+        const int64_t o = ((((int64_t)bb * p.H + h) * NT + qtc) * NT + kt) * 1024;
         if constexpr (BF32) {
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(e.bq + o + 4 * rr);
-                bres32[j][4 * rr] = v[0]; bres32[j][4 * rr + 1] = v[1]; bres32[j][4 * rr + 2] = v[2]; bres32[j][4 * rr + 3] = v[3];
-            }
+            load_tile32(e.bq + o + lane * 4, bres32[j]);
         } else {
             Tile16 t;
-            load_tile16(e.bq16 + o, t);
+            load_tile16(e.bq16 + o + lane * 8, t);
 #pragma unroll
             for (int i = 0; i < 8; ++i) bres[j][i] = t.w[i >> 2][i & 3];
         }

@@ -80,15 +80,15 @@ __global__ void __launch_bounds__(NW * 64, D >= 128 ? 1 : NW == 8 ? (D <= 32 ? 4
     // this lane's row of the caller's tensor where no tiles were prepared
     const int bb = e.bias_batches > 1 ? pr.b : 0;
     const int qtc = min(q0 >> 5, NT - 1);
-    const float *btile0 = e.bq + ((((int64_t)bb * p.H + pr.h) * NT + qtc) * NT) * 1024 + lane * 16;
-    const float *ztile = e.bq + e.zero_tile + lane * 16;
+    const float *btile0 = e.bq + ((((int64_t)bb * p.H + pr.h) * NT + qtc) * NT) * 1024 + lane * 4;
+    const float *ztile = e.bq + e.zero_tile + lane * 4;
     const bool bdirect = HAS_BIAS && e.bias_direct;
     const bool bf32 = p.bias_dtype == EVO_F32;
     const char *brow = (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h +
                                                (int64_t)qrow * p.bias_stride_row) * (bf32 ? 4 : 2);
     const unsigned short *btile16 = !TILE16 ? nullptr
-                                    : dead  ? e.bq16 + e.zero_tile + lane * 16
-                                            : e.bq16 + ((((int64_t)bb * p.H + pr.h) * NT + qtc) * NT) * 1024 + lane * 16;
+                                    : dead  ? e.bq16 + e.zero_tile + lane * 8
+                                            : e.bq16 + ((((int64_t)bb * p.H + pr.h) * NT + qtc) * NT) * 1024 + lane * 8;
     auto load_btile = [&](int kt, f32x16 &dst) {
         if constexpr (TILE16) {
             Tile16 t;
@@ -103,11 +103,7 @@ __global__ void __launch_bounds__(NW * 64, D >= 128 ? 1 : NW == 8 ? (D <= 32 ? 4
             return;
         }
         const float *src = dead ? ztile : btile0 + (int64_t)kt * 1024;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-            const f32x4 v = *reinterpret_cast<const f32x4 *>(src + 4 * rr);
-            dst[4 * rr] = v[0]; dst[4 * rr + 1] = v[1]; dst[4 * rr + 2] = v[2]; dst[4 * rr + 3] = v[3];
-        }
+        load_tile32(src, dst);
     };
 
     // this lane's half of the query row: Q (scaled), dO, and delta = <dO, O>

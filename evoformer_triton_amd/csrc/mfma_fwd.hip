@@ -116,8 +116,8 @@ __global__ void __launch_bounds__(NW * 64, D >= 64 ? 2 : NW == 8 ? 4 : 3) mfma_f
     // bias tiles of this wave's query rows; a dead problem reads the all-zero tile instead
     const int bb = e.bias_batches > 1 ? pr.b : 0;
     const int qt = min(q0 >> 5, NT - 1);
-    const float *btile = dead ? e.bq + e.zero_tile + lane * 16
-                              : e.bq + ((((int64_t)bb * p.H + pr.h) * NT + qt) * NT) * 1024 + lane * 16;
+    const float *btile = dead ? e.bq + e.zero_tile + lane * 4
+                              : e.bq + ((((int64_t)bb * p.H + pr.h) * NT + qt) * NT) * 1024 + lane * 4;
     const int64_t bstep = dead ? 0 : 1024;
     // or, for a bias that is used too few times to pay for the tiles, this lane's row of the
     // caller's tensor
@@ -127,8 +127,8 @@ __global__ void __launch_bounds__(NW * 64, D >= 64 ? 2 : NW == 8 ? 4 : 3) mfma_f
                                                (int64_t)qrow * p.bias_stride_row) * (bf32 ? 4 : 2);
     const float bmul = dead ? 0.0f : kLog2e;
     const unsigned short *btile16 = !TILE16 ? nullptr
-                                    : dead  ? e.bq16 + e.zero_tile + lane * 16
-                                            : e.bq16 + ((((int64_t)bb * p.H + pr.h) * NT + qt) * NT) * 1024 + lane * 16;
+                                    : dead  ? e.bq16 + e.zero_tile + lane * 8
+                                            : e.bq16 + ((((int64_t)bb * p.H + pr.h) * NT + qt) * NT) * 1024 + lane * 8;
 
     float m = LAZY ? 0.0f : -INFINITY, mf = 0.0f, l = 0.0f;
     f32x16 oacc[DT];
@@ -147,11 +147,7 @@ __global__ void __launch_bounds__(NW * 64, D >= 64 ? 2 : NW == 8 ? 4 : 3) mfma_f
             else bias_tile_rows<T, false>(brow, min(kt, NT - 1) * 32, p.N, g, bmul, dst);
         } else if (HAS_BIAS) {
             const float *src = btile + (int64_t)min(kt, NT - 1) * bstep;
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(src + 4 * rr);
-                dst[4 * rr] = v[0]; dst[4 * rr + 1] = v[1]; dst[4 * rr + 2] = v[2]; dst[4 * rr + 3] = v[3];
-            }
+            load_tile32(src, dst);
         }
     };
 

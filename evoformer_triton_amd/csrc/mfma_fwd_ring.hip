@@ -138,20 +138,16 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     if (BIASK == 1) {
         const int bb = e.bias_batches > 1 ? b : 0;
         // (tiles of a bias in the dtype of q are prepared as given, 16 bits per entry: log2 units here)
-        const int64_t tile0 = ((((int64_t)bb * p.H + h) * NT + min(wave, NT - 1)) * NT) * 1024 + lane * 16;
+        const int64_t tile0 = ((((int64_t)bb * p.H + h) * NT + min(wave, NT - 1)) * NT) * 1024;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int64_t o = tile0 + (int64_t)min(j, NT - 1) * 1024;
             if (e.bq16) {   // uniform
                 Tile16 t;
-                load_tile16(e.bq16 + o, t);
+                load_tile16(e.bq16 + o + lane * 8, t);
                 unpack_tile16<T>(t, kLog2e, btile[j]);
             } else {
-#pragma unroll
-                for (int rr = 0; rr < 4; ++rr) {
-                    const f32x4 v = *reinterpret_cast<const f32x4 *>(e.bq + o + 4 * rr);
-                    btile[j][4 * rr] = v[0]; btile[j][4 * rr + 1] = v[1]; btile[j][4 * rr + 2] = v[2]; btile[j][4 * rr + 3] = v[3];
-                }
+                load_tile32(e.bq + o + lane * 4, btile[j]);
             }
         }
     }

@@ -3,7 +3,7 @@
 // hot loops consume without any per-score arithmetic.
 //
 //  * bias -> two copies in 32x32 accumulator-tile order (64 lanes x 16 registers contiguous
-//    per tile), one with lane = query (for S^T = K Q^T tiles) and one with lane = key (for
+//    per tile, in 16-byte pieces), one with lane = query (for S^T = K Q^T tiles) and one with lane = key (for
 //    S = Q K^T tiles): the bias add of the reference (evoformer.py:68, :450, :594) becomes
 //    the C operand of the score matmul.  An fp32 bias is stored as fp32 scaled by log2(e) and
 //    a kernel loads a tile straight into the MFMA accumulator; a bias in the dtype of q is
@@ -98,13 +98,13 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
                     wq[r] = sm[li][tl * 32 + a];     // lane = query, register = key
                     wk[r] = sm[a][tl * 32 + li];     // lane = key, register = query
                 }
-                const int64_t o = ((tile0 + tl) * 64 + lane) * 16;
+                const int64_t o = (tile0 + tl) * 1024 + lane * 8;   // (16-byte pieces, lane after lane: see load_tile16)
                 uint4 *dq = reinterpret_cast<uint4 *>(e.bq16 + o), *dk = reinterpret_cast<uint4 *>(e.bk16 + o);
 #pragma unroll
                 for (int hh = 0; hh < 2; ++hh) {
-                    dq[hh] = make_uint4(wq[8 * hh] | ((unsigned)wq[8 * hh + 1] << 16), wq[8 * hh + 2] | ((unsigned)wq[8 * hh + 3] << 16),
+                    dq[64 * hh] = make_uint4(wq[8 * hh] | ((unsigned)wq[8 * hh + 1] << 16), wq[8 * hh + 2] | ((unsigned)wq[8 * hh + 3] << 16),
                                         wq[8 * hh + 4] | ((unsigned)wq[8 * hh + 5] << 16), wq[8 * hh + 6] | ((unsigned)wq[8 * hh + 7] << 16));
-                    dk[hh] = make_uint4(wk[8 * hh] | ((unsigned)wk[8 * hh + 1] << 16), wk[8 * hh + 2] | ((unsigned)wk[8 * hh + 3] << 16),
+                    dk[64 * hh] = make_uint4(wk[8 * hh] | ((unsigned)wk[8 * hh + 1] << 16), wk[8 * hh + 2] | ((unsigned)wk[8 * hh + 3] << 16),
                                         wk[8 * hh + 4] | ((unsigned)wk[8 * hh + 5] << 16), wk[8 * hh + 6] | ((unsigned)wk[8 * hh + 7] << 16));
                 }
             }
@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
             }
             __syncthreads();
             if (tl < ntile) {
-                const int64_t o = ((tile0 + tl) * 64 + lane) * 16;
+                const int64_t o = (tile0 + tl) * 1024 + lane * 4;
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
                     f32x4 vq, vk;
@@ -158,8 +158,8 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
                         vq[i] = sm[li][tl * 32 + a];
                         vk[i] = sm[a][tl * 32 + li];
                     }
-                    *reinterpret_cast<f32x4 *>(e.bq + o + 4 * m) = vq;
-                    *reinterpret_cast<f32x4 *>(e.bk + o + 4 * m) = vk;
+                    *reinterpret_cast<f32x4 *>(e.bq + o + 256 * m) = vq;
+                    *reinterpret_cast<f32x4 *>(e.bk + o + 256 * m) = vk;
                 }
             }
         }
