@@ -168,11 +168,12 @@ static bool dq_wide_grid_ok(const EvoAttnParams &p) {
 // bf16, H = 4, head dim 32, one kernel / the pair: N = 320 (S = 128) 92 / 110 us; N = 352, 448, 480 (S = 256)
 // 177 / 190, 259 / 274, 277 / 291 us; N = 576, 704, 736 (S = 256) 459 / 436, 633 / 623, 660 / 654 us; N = 640
 // (B = 2, S = 256) 1.06 / 0.99 ms; head dim 16, H = 8, S = 512: N = 576 1.51 / 1.46 ms, N = 640 1.72 / 1.63 ms,
-// N = 704 2.01 / 2.06 ms.
+// N = 704 2.01 / 2.06 ms.  At head dim 128 the one kernel is the one-workgroup-per-problem form, one workgroup per CU without
+// a prefetch: dQ and dBias, H = 4, N = 512, S = 64 245 / 172 us, N = 201, S = 32 58 / 38 us.
 // EVO_FLAG_DEBUG_NO_DQ_SPLIT selects the one kernel, for comparison.
 static bool dq_split_ok(const EvoAttnParams &p) {
-    const int min_n = p.D == 64 ? 128 : 512;
-    if (p.D > 64) return false;   // the dBias kernel is not built for head dim 128
+    if (p.D == 128 && p.N > 2048) return false;   // (rows that long keep the plain kernels at that head dim)
+    const int min_n = p.D == 128 ? 32 : p.D == 64 ? 128 : 512;
     const int rem = p.N % 256;
     const bool full_blocks = rem == 0 || rem >= (p.D == 32 ? 224 : 192);
     const bool ring = dq_ring_ok(p);
@@ -187,7 +188,7 @@ static bool dq_split_ok(const EvoAttnParams &p) {
     // 185 / 215; N = 2048, S = 4 / 7 331 / 600 against 444 / 826; D = 8, S = 7 472 against 730; D = 64, B = 4, H = 32,
     // N = 1024, S = 4 1.89 against 2.33 ms; at N = 640..768 with S = 5, 6 the one kernel stays ahead, 76 / 103
     // against 88 / 111).  Beyond 2048 keys that kernel has no form either.
-    const int min_s = p.N >= 1024 ? 2 : !ring ? (p.D == 64 ? 16 : 8) : p.D == 32 && p.N > 512 ? 8 : 64;
+    const int min_s = p.D == 128 ? 2 : p.N >= 1024 ? 2 : !ring ? (p.D == 64 ? 16 : 8) : p.D == 32 && p.N > 512 ? 8 : 64;
     if (!p.dbias || p.S < min_s || p.N <= min_n || (p.flags & EVO_FLAG_DEBUG_NO_DQ_SPLIT) || bias_direct(p) || !dq_wide_grid_ok(p)) return false;
     return p.bias_dtype == p.dtype || p.bias_dtype == EVO_F32;   // (the dBias kernel keeps 16-bit pairs or fp32 tiles)
 }
@@ -216,11 +217,11 @@ static void chunking(const EvoAttnParams &p, int *n_chunks, int *chunk) {
         return;
     }
     if (dq_split_ok(p)) {
-        // the dBias kernel: one workgroup per block of 128 queries x 128 keys (64 at head dim 64), (b, h) and chunk, two
-        // workgroups per CU (256 CUs) at a time; among the chunk counts that give one to four rounds
+        // the dBias kernel: one workgroup per block of 128 queries x 128 keys (64 from head dim 64 on), (b, h) and chunk, two
+        // (head dim 128: one) workgroups per CU (256 CUs) at a time; among the chunk counts that give one to four rounds
         // the one that leaves the fewest slots idle in the last round (near ties: the fewest chunks)
-        const int64_t kb = p.D == 64 ? 64 : 128;   // keys per block
-        const int64_t base = (int64_t)((p.N + 127) / 128) * ((p.N + kb - 1) / kb) * p.B * p.H, slots = 512;
+        const int64_t kb = p.D >= 64 ? 64 : 128;   // keys per block
+        const int64_t base = (int64_t)((p.N + 127) / 128) * ((p.N + kb - 1) / kb) * p.B * p.H, slots = p.D == 128 ? 256 : 512;
         const int64_t lo = slots / base > 0 ? slots / base : 1, hi = (4 * slots + base - 1) / base;
         int64_t want = lo;
         double best = -1.0;

@@ -21,16 +21,16 @@ EVO_DECL(16)
 EVO_DECL(32)
 EVO_DECL(64)
 #undef EVO_DECL
-// head dim 128: the one-workgroup-per-problem kernels only
+// head dim 128: no kernels over a chunk of rows but the one that sums dBias
 int launch_mfma_fwd_d128(const EvoAttnParams &, const Extra &, hipStream_t);
 int launch_mfma_dq_d128(const EvoAttnParams &, const Extra &, hipStream_t);
 int launch_mfma_dkdv_d128(const EvoAttnParams &, const Extra &, hipStream_t);
 int launch_mfma_dqw_d128(const EvoAttnParams &, const Extra &, hipStream_t);
+int launch_mfma_dbias_d128(const EvoAttnParams &, const Extra &, hipStream_t);
 static int unbuilt(const EvoAttnParams &, const Extra &, hipStream_t) { return EVO_EUNSUPPORTED; }
 #define launch_mfma_fwdr_d128 unbuilt
 #define launch_mfma_dqr_d128 unbuilt
 #define launch_mfma_kvr_d128 unbuilt
-#define launch_mfma_dbias_d128 unbuilt
 
 #define EVO_ROUTE(name)                                                       \
     int launch_mfma_##name(const EvoAttnParams &p, const Extra &e, hipStream_t st) { \

@@ -1,5 +1,5 @@
 // Backward kernels for gfx950 on the bf16/fp16 32x32x16 matrix-core instruction.
-// Compiled once per head dim (-DEVO_D=8|16|32|64).
+// Compiled once per head dim (-DEVO_D=8|16|32|64|128; dK/dV up to 32, 64 and 128: mfma_stream.hip).
 //
 // They replace the reference's `_attn_bwd_preprocess` (evoformer.py:299-326),
 // `_attn_bwd_dq` (:329-476) and `_attn_bwd_dk_dv` (:479-630).  Both kernels recompute
@@ -319,7 +319,7 @@ template <int D>
 struct KvGeo {
     static constexpr int C = D / 8;                          // 16-byte chunks per row
     static constexpr int RPB = 16 / C > 0 ? 16 / C : 1;      // rows per 256 bytes
-    static constexpr int BQS = D <= 32 ? 256 : 128;          // query rows staged per round
+    static constexpr int BQS = 256;                          // query rows staged per round
     static constexpr bool RESID = D <= 16;
     // LDS layout for `rows` staged query rows (BQS, or 128 where a problem has no more):
     //   [Q scaled][Q as given][dO]([rounding residue of Q scaled] for RESID)[-LSE columns][-delta columns]
@@ -343,7 +343,7 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 // tiles of a bias in the dtype of q as given (half the bytes per tile, 8 registers in flight
 // instead of 16; unpacked and multiplied by log2 e right before they are used)
 template <typename T, int D, int BT, int NW, int ROWS>
-__global__ void __launch_bounds__(NW * 64, D >= 64 ? 2 : NW == 8 ? 4 : 3) mfma_dkdv(EvoAttnParams p, Extra e) {
+__global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_dkdv(EvoAttnParams p, Extra e) {
     typedef Geo<D> G;
     typedef KvGeo<D> R;
     constexpr bool HAS_BIAS = BT != 0, TILE16 = BT == 2;
@@ -660,16 +660,16 @@ static int dq_bias(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     return p.bias_dtype == EVO_NONE ? dq_ntw<T, D, false>(p, e, st) : dq_ntw<T, D, true>(p, e, st);
 }
 
+int EVO_CAT(launch_mfma_dq_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    return p.dtype == EVO_BF16 ? dq_bias<bf16_t, EVO_D>(p, e, st) : dq_bias<f16_t, EVO_D>(p, e, st);
+}
+
+#if EVO_D < 64   // (head dims 64 and 128: mfma_stream.hip)
 template <typename T, int D, int BT, int NW, int ROWS>
 static int dkdv_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const unsigned grid = (unsigned)((p.N + NW * 32 - 1) / (NW * 32)) * (unsigned)(p.B * p.H * p.S);
-    constexpr int lds = KvGeo<D>::lds_bytes(ROWS);   // at most 56 KB up to head dim 64, 100 KB at 128
-    auto kern = mfma_dkdv<T, D, BT, NW, ROWS>;
-    if constexpr (lds > 64 * 1024) {
-        static PerDevice done{};
-        if (const int rc = ensure_dynamic_lds((const void *)kern, lds, done, nullptr)) return rc;
-    }
-    kern<<<grid, NW * 64, lds, st>>>(p, e);
+    constexpr int lds = KvGeo<D>::lds_bytes(ROWS);   // at most 56 KB
+    mfma_dkdv<T, D, BT, NW, ROWS><<<grid, NW * 64, lds, st>>>(p, e);
     return hip_rc();
 }
 
@@ -702,12 +702,9 @@ static int dkdv_waves(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     return wide ? dkdv_bias<T, D, 8>(p, e, st) : dkdv_bias<T, D, 4>(p, e, st);
 }
 
-int EVO_CAT(launch_mfma_dq_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
-    return p.dtype == EVO_BF16 ? dq_bias<bf16_t, EVO_D>(p, e, st) : dq_bias<f16_t, EVO_D>(p, e, st);
-}
-
 int EVO_CAT(launch_mfma_dkdv_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     return p.dtype == EVO_BF16 ? dkdv_waves<bf16_t, EVO_D>(p, e, st) : dkdv_waves<f16_t, EVO_D>(p, e, st);
 }
+#endif
 
 }  // namespace evo

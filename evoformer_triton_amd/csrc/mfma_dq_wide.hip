@@ -1,6 +1,6 @@
 // dQ (and delta) for problems whose dBias is not a sum over S rows: no pair bias, a bias that
 // takes no gradient, or a single S row per (batch, head), where dBias is dS itself and is
-// written as it is formed.  Compiled once per head dim (-DEVO_D=8|16|32|64).
+// written as it is formed.  Compiled once per head dim (-DEVO_D=8|16|32; 64 and 128: mfma_stream.hip).
 //
 // Replaces the reference's `_attn_bwd_preprocess` (evoformer.py:299-326) and `_attn_bwd_dq`
 // (:329-476) for that case: P = exp(score - LSE) recomputed (:452), dS = P * (dP - delta)
@@ -29,7 +29,7 @@ template <int D>
 struct DqWideGeo {
     static constexpr int C = D / 8;                          // 16-byte chunks per row
     static constexpr int RPB = 16 / C > 0 ? 16 / C : 1;      // rows per 256 bytes
-    static constexpr int ROWS = D <= 32 ? 256 : 128;         // keys staged per round
+    static constexpr int ROWS = 256;                         // keys staged per round
     // [K][V][mask columns of K]
     static constexpr int OFF_K = 0, OFF_V = ROWS * D * 2, OFF_AK = 2 * ROWS * D * 2;
     static constexpr int LDS_BYTES = OFF_AK + ROWS * 16;
@@ -42,7 +42,7 @@ typedef short s16x4w __attribute__((ext_vector_type(4)));
 // tiles of a bias in the dtype of q as given (half the bytes per tile; unpacked and multiplied by
 // log2 e as they arrive)
 template <typename T, int D, int BT, int NW, bool WRITE_DS>
-__global__ void __launch_bounds__(NW * 64, D >= 128 ? 1 : NW == 8 ? (D <= 32 ? 4 : 2) : 3) mfma_dq_wide(EvoAttnParams p, Extra e) {
+__global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_dq_wide(EvoAttnParams p, Extra e) {
     constexpr bool HAS_BIAS = BT != 0, TILE16 = BT == 2;
     typedef Geo<D> G;
     typedef DqWideGeo<D> R;

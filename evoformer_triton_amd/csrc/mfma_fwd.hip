@@ -1,5 +1,5 @@
 // Flash-style forward for gfx950 on the bf16/fp16 32x32x16 matrix-core instruction.
-// Compiled once per head dim (-DEVO_D=8|16|32|64).
+// Compiled once per head dim (-DEVO_D=8|16|32; 64 and 128: mfma_stream.hip).
 //
 // Replaces the reference's `_attn_fwd` / `_attn_fwd_inner` (evoformer.py:23-297): bias add
 // and mask fused before the running max (:68-71), online softmax (:71-89), P cast to the
@@ -36,20 +36,17 @@ namespace evo {
 // tiles of a bias in the dtype of q as given (half the bytes per tile, 8 registers in flight
 // instead of 16; unpacked and multiplied by log2 e right before they are used)
 template <typename T, int D, int BT, int NW>
-__global__ void __launch_bounds__(NW * 64, D >= 64 ? 2 : NW == 8 ? 4 : 3) mfma_fwd(EvoAttnParams p, Extra e) {
+__global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_fwd(EvoAttnParams p, Extra e) {
     constexpr bool HAS_BIAS = BT != 0, TILE16 = BT == 2;
     typedef typename std::conditional<TILE16, Tile16, f32x16>::type CTile;   // a bias tile on its way
     // The softmax that skips the search for the maximum after a problem's first 64 keys keeps a
     // second copy of the score code for the rare step that has to be redone; with fp32 bias
-    // tiles in flight that does not fit 128 registers (8 waves) or 256 at head dim 128, and in
-    // the 4-wave forms it measured no better on balance (B = 4, S = 1, H = 32, D = 64, fp32 bias
-    // read from the caller's rows: N = 1024 136 against 130 TFLOP/s, N = 768 107 against 130):
-    // the forms with an fp32 bias keep the plain online softmax, and so do head dims 64 and 128
-    // (no bias, B = 4, S = 1, H = 32, D = 64, N = 1024: 72 against 62 us).
-    constexpr bool LAZY = BT != 1 && D <= 32;
+    // tiles in flight that does not fit 128 registers (8 waves): the forms with an fp32 bias keep the
+    // plain online softmax.
+    constexpr bool LAZY = BT != 1;
     constexpr int NTH = NW * 64;                  // threads per workgroup
     constexpr int BQ = NW * 32;                   // query rows per workgroup
-    constexpr int BKV = D <= 32 ? 256 : 128;      // keys staged per round
+    constexpr int BKV = 256;                      // keys staged per round
     constexpr int SPS = BKV / 64;                 // 64-key steps per stage
     constexpr bool AUG_IN_PAD = D == 8;           // mask columns fit the zero padding of k-step 0
     constexpr int KW = AUG_IN_PAD ? 16 : D + 16;  // K row: data, 3 mask columns, zeros

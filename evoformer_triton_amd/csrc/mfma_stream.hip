@@ -1,0 +1,847 @@
+// Forward, dQ and dK/dV for head dims 64 and 128: one workgroup per block of rows of a problem (b, h, s), the other side's
+// rows streamed through LDS.  Compiled once per head dim (-DEVO_D=64|128).
+//
+// The arithmetic is that of the one-workgroup-per-problem kernels for smaller head dims (mfma_fwd.hip, mfma_bwd.hip,
+// mfma_dq_wide.hip: every additive term of the score rides in the matrix instruction, the scaled Q rounded once in the
+// same way everywhere), and so is a wave's part: 32 rows, and 32 x 32 tiles against the other side.  What differs is how the
+// other side arrives.  At these head dims a wave keeps 110 to 250 registers, a SIMD two to four waves, and kernels that staged
+// 128 rows at a time between two barriers waited 60 to 85 % of their time for memory with every unit less than 35 %
+// busy.  Here
+//   * rows go from memory into LDS by the load path itself (`buffer_load_dwordx4 ... lds`), no register in between, a stage of
+//     64 (head dim 128 in the dK/dV kernel: 32) rows ahead of the one that is computed on: one barrier per stage, and the
+//     wait before it finds the rows there;
+//   * V, K, dO and Q lie row-major; the operands that need them transposed read them by `ds_read_b64_tr_b16`;
+//   * a lane's 16-byte piece of a row is stored at chunk c ^ x(row), x the row's low bits reversed: reads of one chunk of
+//     consecutive rows and transposing reads of four chunks of eight rows both touch all banks evenly (with the bits in
+//     order the eight rows met in half of the banks).
+#include <type_traits>
+
+#include "bwd_common.h"
+#include "kernels.h"
+
+#ifndef EVO_D
+#error "compile with -DEVO_D=<head dim>"
+#endif
+
+namespace evo {
+
+typedef short s16x4s __attribute__((ext_vector_type(4)));
+
+template <int D>
+struct StreamGeo {
+    static constexpr int C = D / 8, ROW = D * 2;   // 16-byte chunks, bytes per row
+    // the low bits of the row reversed (head dim 64: of every second row, two rows share the 64 banks)
+    static __device__ __forceinline__ int x(int r) {
+        return D == 64 ? ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1)
+                       : (r & 1) << 3 | ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1);
+    }
+    static __device__ __forceinline__ int at(int r, int c) { return r * ROW + ((c ^ x(r)) << 4); }
+};
+
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void wait_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, unsigned char *dst, int off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16, off, 0, 0, 0);
+}
+
+// Rows r0 .. r0 + ROWS - 1 of two arrays that share their strides, into LDS at `dst` and `dst` + ROWS rows: this wave's share
+// of the 1 KB pieces.  Rows at or beyond N repeat the last one (their keys carry the mask floor, their queries
+// probability zero).
+template <int D, int ROWS, int NW>
+__device__ __forceinline__ void dma_rows(__amdgpu_buffer_rsrc_t a, __amdgpu_buffer_rsrc_t b, unsigned char *dst, int r0, int N, int sn2,
+                                         int wave, int lane) {
+    typedef StreamGeo<D> G;
+    constexpr int PIECES = ROWS * G::ROW / 1024, RPP = 1024 / G::ROW;   // rows per piece
+#pragma unroll
+    for (int i = 0; i < (PIECES + NW - 1) / NW; ++i) {
+        const int m = wave + i * NW;
+        if (PIECES % NW != 0 && m >= PIECES) break;   // (uniform over the wave)
+        const int r = m * RPP + lane / G::C, c = (lane % G::C) ^ G::x(r);
+        const int off = min(r0 + r, N - 1) * sn2 + c * 16;
+        dma16(a, dst + m * 1024, off);
+        dma16(b, dst + ROWS * G::ROW + m * 1024, off);
+    }
+}
+
+// A operand of a product that contracts over 32 staged rows (kb .. kb + 31): row 32 dt + li of the transpose, the eight rows
+// that step `ts` of an accumulator tile holds.
+template <typename T, int D>
+__device__ __forceinline__ typename Mfma<T>::v8 transposed(const unsigned char *tile, int kb, int ts, int dt, int lane) {
+    typedef StreamGeo<D> G;
+    const int g = lane >> 5, col = dt * 32 + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    typename Mfma<T>::v8 r;
+#pragma unroll
+    for (int h2 = 0; h2 < 2; ++h2) {
+        const int row = kb + 16 * ts + 8 * h2 + 4 * g + ((lane & 15) >> 2);
+        const s16x4s w = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (s16x4s __attribute__((address_space(3))) *)(tile + G::at(row, col >> 3) + (col & 7) * 2));
+        const typename Mfma<T>::v4 v = __builtin_bit_cast(typename Mfma<T>::v4, w);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[4 * h2 + i] = v[i];
+    }
+    return r;
+}
+
+// The bias tiles of one wave: its 32 rows (or, COLS, its 32 columns) against the tiles of the other side.
+// BT: 1 prepared fp32 tiles (times log2 e), 2 prepared 16-bit tiles as given, 3 the caller's rows (few S rows).
+template <typename T, int BT, bool COLS>
+struct BiasStream {
+    typedef typename std::conditional<BT == 2, Tile16, f32x16>::type Tile;
+    const float *t32;
+    const unsigned short *t16;
+    const char *mat;
+    int64_t step;
+    unsigned col, row_stride;
+    float mul;
+    int NT, N, g;
+    bool f32;
+    __device__ __forceinline__ BiasStream(const EvoAttnParams &p, const Extra &e, const Prob &pr, int own_tile, int own_row, bool dead, int lane) {
+        NT = (p.N + 31) / 32;
+        N = p.N;
+        g = lane >> 5;
+        mul = dead ? 0.0f : kLog2e;
+        const int bb = e.bias_batches > 1 ? pr.b : 0;
+        if (BT == 3) {
+            f32 = p.bias_dtype == EVO_F32;
+            row_stride = (unsigned)p.bias_stride_row;
+            col = (unsigned)own_row;
+            mat = (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h + (COLS ? 0 : (int64_t)own_row * p.bias_stride_row)) * (f32 ? 4 : 2);
+        } else {
+            const int64_t first = (((int64_t)bb * p.H + pr.h) * NT * NT + (COLS ? own_tile : own_tile * NT)) * 1024;
+            step = dead ? 0 : COLS ? (int64_t)NT * 1024 : 1024;
+            if (BT == 1) t32 = (COLS ? e.bk : e.bq) + (dead ? e.zero_tile : first) + lane * 4;
+            if (BT == 2) t16 = (COLS ? e.bk16 : e.bq16) + (dead ? e.zero_tile : first) + lane * 8;
+        }
+    }
+    // tile t of the other side on its way; past the last one that one again (not used)
+    __device__ __forceinline__ void load(int t, Tile &dst) const {
+        t = min(t, NT - 1);
+        if constexpr (BT == 1) load_tile32(t32 + t * step, dst);
+        if constexpr (BT == 2) load_tile16(t16 + t * step, dst);
+        if constexpr (BT == 3) {
+            if (COLS) {
+                if (f32) bias_tile_cols<T, true>(mat, col, t * 32, N, row_stride, g, mul, dst);
+                else bias_tile_cols<T, false>(mat, col, t * 32, N, row_stride, g, mul, dst);
+            } else {
+                if (f32) bias_tile_rows<T, true>(mat, t * 32, N, g, mul, dst);
+                else bias_tile_rows<T, false>(mat, t * 32, N, g, mul, dst);
+            }
+        }
+    }
+    // as the C operand of the score product, log2 units
+    __device__ __forceinline__ f32x16 value(const Tile &t) const {
+        if constexpr (BT == 2) {
+            f32x16 v;
+            unpack_tile16<T>(t, mul, v);
+            return v;
+        } else {
+            return t;
+        }
+    }
+};
+template <typename T, bool COLS>
+struct BiasStream<T, 0, COLS> {
+    struct Tile {};
+    __device__ __forceinline__ BiasStream(const EvoAttnParams &, const Extra &, const Prob &, int, int, bool, int) {}
+    __device__ __forceinline__ void load(int, Tile &) const {}
+    __device__ __forceinline__ f32x16 value(const Tile &) const {
+        f32x16 z;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[r] = 0.0f;
+        return z;
+    }
+};
+
+// ------------------------------------------------------------------ forward
+
+template <int D>
+struct FwdStream {
+    static constexpr int ROWS = 64, OFF_V = ROWS * D * 2, OFF_A = 2 * ROWS * D * 2, BYTES = OFF_A + ROWS * 16;
+};
+
+template <typename T, int D, int BT>
+__global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_fwd(EvoAttnParams p, Extra e) {
+    typedef StreamGeo<D> G;
+    typedef FwdStream<D> R;
+    constexpr int NW = 4, KSD = D / 16, KS = KSD + 1, DT = D / 32;
+    typedef typename Mfma<T>::v8 v8;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2][R::BYTES];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, g = lane >> 5;
+    const int NT = (p.N + 31) / 32, nqb = (p.N + 127) / 128;
+    const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+    const Prob pr = walk_problem(p, lid / nqb);
+    const int q0 = (lid % nqb) * 128 + wave * 32, qrow = min(q0 + li, p.N - 1);
+    const bool active = q0 < p.N;   // wave-uniform
+    const bool dead = e.dead[pr.b * p.S + pr.s] != 0;
+    const int sn2 = (int)p.stride_n * 2, valid = (p.N - 1) * sn2 + D * 2;
+    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.k + pr.base), 0, valid, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.v + pr.base), 0, valid, 0x00020000);
+    const int np256 = (p.N + 255) / 256 * 256;
+    const __amdgpu_buffer_rsrc_t mrs =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(e.m2a + ((int64_t)pr.b * p.S + pr.s) * np256), 0, np256 * 16, 0x00020000);
+    auto fetch = [&](int stage) {
+        unsigned char *dst = lds[stage & 1];
+        dma_rows<D, R::ROWS, NW>(krs, vrs, dst, stage * R::ROWS, p.N, sn2, wave, lane);
+        if (wave == 0) dma16(mrs, dst + R::OFF_A, (stage * R::ROWS + lane) * 16);
+    };
+    fetch(0);
+
+    // Q operand: data times scale * log2(e), rounded once; ones against the mask columns
+    const float c = p.scale * kLog2e;
+    v8 qf[KS];
+    {
+        const T *Q = (const T *)p.q + pr.base + (int64_t)qrow * p.stride_n;
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) qf[ks] = dead ? zero8<T>() : scaled8<T>(ld8(Q + ks * 16 + g * 8), c);
+        qf[KSD] = zero8<T>();
+        if (g == 0) qf[KSD][0] = qf[KSD][1] = qf[KSD][2] = (T)1.0f;
+    }
+    const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, dead, lane);
+    typename BiasStream<T, BT, false>::Tile ct;
+    bias.load(0, ct);
+
+    // m: the maximum the probabilities are relative to; mf: what the mask step subtracts inside the product (m, or 0 while
+    // m is unknown or too large for three 16-bit columns): after the first tile the scores arrive relative to m, and
+    // a later tile searches its maximum only when its sums show that it stands far above (see mfma_fwd.hip).
+    float m = 0.0f, mf = 0.0f, l = 0.0f;
+    f32x16 o[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
+
+    auto score = [&](const unsigned char *buf, int kb, const f32x16 &init, f32x16 &a) {
+        a = init;
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + G::at(kb + li, 2 * ks + g)), qf[ks], a);
+        a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (kb + li) * 16), qf[KSD], a);   // (zero in the step's upper half)
+    };
+    auto settle = [&](bool first, f32x16 &a, float used) {
+        float mloc = a[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mloc = fmaxf(mloc, a[r]);
+        const unsigned u = __float_as_uint(mloc);
+        auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        const float cand = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) + used;
+        const bool grow = first || cand > m + 8.0f;   // (moved only when it grows by more than 2^8)
+        if (__any(grow || m != used)) {
+            const float mn = grow ? cand : m;
+            if (!first) {
+                const float alpha = fast_exp2(m - mn);
+                l *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+            }
+            m = mn;
+            const float dsub = m - used;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) a[r] -= dsub;
+            mf = fabsf(m) <= 1024.0f ? m : 0.0f;
+            const v8 qa = aug8<T>(ones3<T>(), pack_split3<T>(-mf));
+            if (g == 0) qf[KSD] = qa;
+        }
+    };
+    auto probs = [&](f32x16 &a, v8 (&pf)[2]) {
+        float s = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            a[r] = fast_exp2(a[r]);
+            s += a[r];
+        }
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pf[ts][i] = (T)a[8 * ts + i];
+        return s;
+    };
+    auto tile = [&](const unsigned char *buf, int kt, int kb) {
+        const float used = mf;
+        f32x16 a;
+        score(buf, kb, bias.value(ct), a);
+        bias.load(kt + 1, ct);
+        const bool lazy = kt != 0 && !__any(m != used);
+        if (!lazy) settle(kt == 0, a, used);
+        v8 pf[2];
+        float s = probs(a, pf);
+        if (__builtin_expect(lazy && __any(!(s <= 8192.0f)), 0)) {   // some score stands far above m: once more, the long way
+            typename BiasStream<T, BT, false>::Tile again;
+            bias.load(kt, again);
+            score(buf, kb, bias.value(again), a);
+            settle(false, a, used);
+            s = probs(a, pf);
+        }
+        l += s;
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] = Mfma<T>::mma(transposed<T, D>(buf + R::OFF_V, kb, ts, dt, lane), pf[ts], o[dt]);
+    };
+
+    const int nst = (p.N + R::ROWS - 1) / R::ROWS;
+    wait_loads();
+    wait_lds_barrier();
+    for (int s = 0; s < nst; ++s) {
+        if (s + 1 < nst) fetch(s + 1);
+        if (active) {
+            const unsigned char *buf = lds[s & 1];
+            tile(buf, 2 * s, 0);
+            if (2 * s + 1 < NT) tile(buf, 2 * s + 1, 32);
+        }
+        if (s + 1 < nst) {
+            wait_loads();
+            wait_lds_barrier();
+        }
+    }
+
+    if (!active) return;
+    l += __shfl_xor(l, 32);
+    const float inv = 1.0f / l;
+    if (q0 + li >= p.N) return;
+    if (g == 0) p.lse[pr.row0 + q0 + li] = (m + __log2f(l)) * kLn2;
+    const int64_t off = pr.base + (int64_t)(q0 + li) * p.stride_n;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        if (p.o) store_row_tile<T>((T *)p.o + off, dt * 32, D, o[dt], inv, g);
+        if (p.gate) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[dt][r] *= inv;
+            gate_row_tile<T>((const T *)p.gate + off, dt * 32, D, o[dt], g);
+            store_row_tile<T>((T *)p.o_gated + off, dt * 32, D, o[dt], 1.0f, g);
+        }
+    }
+}
+
+// ------------------------------------------------------------------ dQ
+
+// As mfma_dq_wide.hip, whose place it takes at these head dims: where dBias is no sum over S rows, or its sum comes from a
+// kernel of its own.  A wave has 32 queries for all keys; with WRITE_DS (S = 1) dBias is dS and goes out as it is formed.
+template <typename T, int D, int BT, bool WRITE_DS>
+__global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_dq(EvoAttnParams p, Extra e) {
+    typedef StreamGeo<D> G;
+    typedef FwdStream<D> R;
+    constexpr int NW = 4, KSD = D / 16, KS = KSD + 1, DT = D / 32;
+    typedef typename Mfma<T>::v8 v8;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2][R::BYTES];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, g = lane >> 5;
+    const int NT = (p.N + 31) / 32, nqb = (p.N + 127) / 128;
+    const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+    const Prob pr = walk_problem(p, lid / nqb);
+    const int q0 = (lid % nqb) * 128 + wave * 32, qrow = min(q0 + li, p.N - 1);
+    const bool active = q0 < p.N;
+    const bool dead = e.dead[pr.b * p.S + pr.s] != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
+    const int sn2 = (int)p.stride_n * 2, valid = (p.N - 1) * sn2 + D * 2;
+    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.k + pr.base), 0, valid, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.v + pr.base), 0, valid, 0x00020000);
+    const int np256 = (p.N + 255) / 256 * 256;
+    const __amdgpu_buffer_rsrc_t mrs =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(e.m2a + ((int64_t)pr.b * p.S + pr.s) * np256), 0, np256 * 16, 0x00020000);
+    auto fetch = [&](int stage) {
+        unsigned char *dst = lds[stage & 1];
+        dma_rows<D, R::ROWS, NW>(krs, vrs, dst, stage * R::ROWS, p.N, sn2, wave, lane);
+        if (wave == 0) dma16(mrs, dst + R::OFF_A, (stage * R::ROWS + lane) * 16);
+    };
+    fetch(0);
+
+    // this lane's half of the query row: Q (scaled), dO, and delta = <dO, O>
+    const float cs = p.scale * kLog2e;
+    v8 qf[KS], gf[KS];
+    float dl = 0.0f;
+    {
+        const int64_t row = pr.base + (int64_t)qrow * p.stride_n + g * 8;
+        // (where delta is given, by the gate's pass, there may be no ungated O: dO is read in its place and the sum dropped)
+        const T *O = e.delta_given ? (const T *)p.dout : (const T *)p.o;
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) {
+            qf[ks] = dead ? zero8<T>() : scaled8<T>(ld8((const T *)p.q + row + ks * 16), cs);
+            gf[ks] = ld8((const T *)p.dout + row + ks * 16);
+            dl = dot8<T>(gf[ks], ld8(O + row + ks * 16), dl);
+        }
+        dl += __shfl_xor(dl, 32);
+        if (e.delta_given) dl = e.delta[pr.row0 + qrow];
+        else if (g == 0 && q0 + li < p.N) e.delta[pr.row0 + q0 + li] = dl;
+        const float lse2 = p.lse[pr.row0 + qrow] * kLog2e;
+        const uint2 one3 = ones3<T>(), zero3 = {0u, 0u};
+        qf[KSD] = g == 0 ? aug8<T>(one3, pack_split3<T>(-lse2)) : zero8<T>();   // ones x mask, -lse x ones
+        gf[KSD] = g == 0 ? aug8<T>(pack_split3<T>(-dl), zero3) : zero8<T>();    // -delta x ones
+    }
+    const v8 vaug = aug8<T>(ones3<T>(), {0u, 0u});
+    const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, dead, lane);
+    typename BiasStream<T, BT, false>::Tile ct;
+    bias.load(0, ct);
+
+    // S = 1: this lane's row of dBias[b][h]
+    const int64_t dsrow = (((int64_t)pr.b * p.H + pr.h) * p.N + qrow) * p.N;
+    const bool ds_vec = (p.N & 3) == 0 && ((uintptr_t)p.dbias & 15) == 0, ds_f32 = p.dbias_dtype == EVO_F32;
+
+    f32x16 dq[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dq[dt][r] = 0.0f;
+
+    auto tile = [&](const unsigned char *buf, int kt, int kb) {
+        f32x16 a = bias.value(ct), dp;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) {
+            const int o = G::at(kb + li, 2 * ks + g);
+            a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + o), qf[ks], a);                  // log2 P^T
+            dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_V + o), gf[ks], dp);     // dP^T - delta
+        }
+        a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (kb + li) * 16), qf[KSD], a);
+        dp = Mfma<T>::mma(vaug, gf[KSD], dp);
+        bias.load(kt + 1, ct);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) a[r] = fast_exp2(a[r]) * dp[r];
+        if (kill) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) a[r] = 0.0f;
+        }
+        if (WRITE_DS && q0 + li < p.N) {
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+                const int kg = kt * 32 + 8 * rr + 4 * g;   // registers 4 rr .. 4 rr + 3 hold keys kg .. kg + 3
+                if (ds_vec && kg + 4 <= p.N) {
+                    if (ds_f32) {
+                        f32x4 v;
+                        v[0] = a[4 * rr]; v[1] = a[4 * rr + 1]; v[2] = a[4 * rr + 2]; v[3] = a[4 * rr + 3];
+                        *reinterpret_cast<f32x4 *>((float *)p.dbias + dsrow + kg) = v;
+                    } else {
+                        store4<T>((T *)p.dbias + dsrow + kg, a[4 * rr], a[4 * rr + 1], a[4 * rr + 2], a[4 * rr + 3]);
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (kg + i < p.N) {
+                            if (ds_f32) ((float *)p.dbias)[dsrow + kg + i] = a[4 * rr + i];
+                            else ((T *)p.dbias)[dsrow + kg + i] = (T)a[4 * rr + i];
+                        }
+                }
+            }
+        }
+        v8 ds[2];
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ds[ts][i] = (T)a[8 * ts + i];
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) dq[dt] = Mfma<T>::mma(transposed<T, D>(buf, kb, ts, dt, lane), ds[ts], dq[dt]);
+    };
+
+    const int nst = (p.N + R::ROWS - 1) / R::ROWS;
+    wait_loads();
+    wait_lds_barrier();
+    for (int s = 0; s < nst; ++s) {
+        if (s + 1 < nst) fetch(s + 1);
+        if (active) {
+            const unsigned char *buf = lds[s & 1];
+            tile(buf, 2 * s, 0);
+            if (2 * s + 1 < NT) tile(buf, 2 * s + 1, 32);
+        }
+        if (s + 1 < nst) {
+            wait_loads();
+            wait_lds_barrier();
+        }
+    }
+    if (active && q0 + li < p.N) {
+        T *dQ = (T *)p.dq + pr.base + (int64_t)(q0 + li) * p.stride_n;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) store_row_tile<T>(dQ, dt * 32, D, dq[dt], p.scale, g);
+    }
+}
+
+// ------------------------------------------------------------------ dK and dV
+
+// A wave has 32 keys, the queries stream by.  The score product wants Q scaled and rounded, dK wants it as given: a wave
+// scales the pieces it has fetched itself, from LDS to LDS, between the wait and the barrier.  At head dim 128 the keys'
+// K operand lies in LDS (next to V, dK and dV it would not fit the registers of two waves per SIMD).
+template <int D, int NW>
+struct KvStream {
+    static constexpr int ROWS = D == 64 ? 64 : 32, BLK = ROWS * D * 2;
+    static constexpr bool K_LDS = D == 128;
+    static constexpr int OFF_G = BLK, OFF_QS = 2 * BLK, OFF_AQ = 3 * BLK, OFF_AG = OFF_AQ + ROWS * 16, STAGE = (OFF_AG + ROWS * 16 + 1023) / 1024 * 1024;
+    static constexpr int OFF_K = 2 * STAGE, BYTES = OFF_K + (K_LDS ? NW * 32 * D * 2 : 0);
+};
+
+template <typename T, int D, int BT, int NW>
+__global__ void __launch_bounds__(NW * 64, 2) stream_dkdv(EvoAttnParams p, Extra e) {
+    typedef StreamGeo<D> G;
+    typedef KvStream<D, NW> R;
+    constexpr int KSD = D / 16, DT = D / 32, ROWS = R::ROWS;
+    typedef typename Mfma<T>::v8 v8;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, g = lane >> 5;
+    const int NT = (p.N + 31) / 32, nkb = (p.N + NW * 32 - 1) / (NW * 32);
+    const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+    const Prob pr = walk_problem(p, lid / nkb);
+    const int key0 = (lid % nkb) * NW * 32 + wave * 32, key = key0 + li, keyc = min(key, p.N - 1);
+    const bool active = key0 < p.N;
+    const bool dead = e.dead[pr.b * p.S + pr.s] != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
+    const bool want_dm = e.dmask_part != nullptr && p.dmask != nullptr;
+    const float cs = p.scale * kLog2e;
+    const uint2 one3 = ones3<T>(), zero3 = {0u, 0u};
+    const int sn2 = (int)p.stride_n * 2, valid = (p.N - 1) * sn2 + D * 2;
+    const __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.q + pr.base), 0, valid, 0x00020000);
+    const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.dout + pr.base), 0, valid, 0x00020000);
+
+    float nl = 0.0f, nd = 0.0f;   // -LSE log2(e) and -delta of a row of the stage on its way (threads 0 .. ROWS - 1)
+    auto fetch = [&](int stage) {
+        dma_rows<D, ROWS, NW>(qrs, grs, lds + (stage & 1) * R::STAGE, stage * ROWS, p.N, sn2, wave, lane);
+        const int q = stage * ROWS + (int)threadIdx.x;
+        if (threadIdx.x < ROWS) {   // rows at and beyond N: probability zero
+            nl = q < p.N ? -p.lse[pr.row0 + q] * kLog2e : kMaskFloor;
+            nd = q < p.N ? -e.delta[pr.row0 + q] : 0.0f;
+        }
+    };
+    auto finish = [&](int stage) {   // what this wave fetched is there: its pieces of Q scaled, the extra columns
+        unsigned char *buf = lds + (stage & 1) * R::STAGE;
+        wait_loads();
+        constexpr int PIECES = R::BLK / 1024;
+#pragma unroll
+        for (int i = 0; i < (PIECES + NW - 1) / NW; ++i) {
+            const int m = wave + i * NW;
+            if (PIECES % NW != 0 && m >= PIECES) break;
+            const v8 a = *reinterpret_cast<const v8 *>(buf + m * 1024 + lane * 16);
+            *reinterpret_cast<v8 *>(buf + R::OFF_QS + m * 1024 + lane * 16) = scaled8<T>(a, cs);
+        }
+        if (threadIdx.x < ROWS) {
+            *reinterpret_cast<v8 *>(buf + R::OFF_AQ + threadIdx.x * 16) = aug8<T>(one3, pack_split3<T>(nl));
+            *reinterpret_cast<v8 *>(buf + R::OFF_AG + threadIdx.x * 16) = aug8<T>(pack_split3<T>(nd), zero3);
+        }
+        wait_lds_barrier();
+    };
+    fetch(0);
+
+    // this wave's keys: K with the mask columns, V with ones against -delta
+    v8 kf[R::K_LDS ? 1 : KSD], vf[KSD], kaug, vaug;
+    {
+        const int64_t row = pr.base + (int64_t)keyc * p.stride_n + g * 8;
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) {
+            const v8 k = dead ? zero8<T>() : ld8((const T *)p.k + row + ks * 16);
+            if constexpr (R::K_LDS) *reinterpret_cast<v8 *>(lds + R::OFF_K + wave * 32 * G::ROW + G::at(li, 2 * ks + g)) = k;
+            else kf[ks] = k;
+            vf[ks] = ld8((const T *)p.v + row + ks * 16);
+        }
+        const uint2 mraw = e.m2[((int64_t)pr.b * p.S + pr.s) * (NT * 32) + min(key, NT * 32 - 1)];
+        kaug = g == 0 ? aug8<T>(mraw, one3) : zero8<T>();     // mask x ones, ones x -lse
+        vaug = g == 0 ? aug8<T>(one3, zero3) : zero8<T>();    // ones x -delta
+    }
+    const BiasStream<T, BT, true> bias(p, e, pr, min(key0 >> 5, NT - 1), keyc, dead, lane);
+    typename BiasStream<T, BT, true>::Tile ct;
+    bias.load(0, ct);
+    // (the dBias partials of the kernels before this one, summed on the way in where the caller asks for it)
+    if (e.dbias_chunks > 0) sum_dbias_partials<NW * 64>(p, e, threadIdx.x);
+
+    f32x16 dk[DT], dv[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dk[dt][r] = dv[dt][r] = 0.0f;
+    float dm = 0.0f;
+
+    auto tile = [&](const unsigned char *buf, int qt, int qb) {
+        f32x16 a = bias.value(ct), dp;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) {
+            const int o = G::at(qb + li, 2 * ks + g);
+            v8 k;
+            if constexpr (R::K_LDS) k = *reinterpret_cast<const v8 *>(lds + R::OFF_K + wave * 32 * G::ROW + G::at(li, 2 * ks + g));
+            else k = kf[ks];
+            a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_QS + o), k, a);          // log2 P
+            dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_G + o), vf[ks], dp);    // dP - delta
+        }
+        a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_AQ + (qb + li) * 16), kaug, a);
+        dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_AG + (qb + li) * 16), vaug, dp);
+        bias.load(qt + 1, ct);
+        v8 pf[2], ds[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            a[r] = fast_exp2(a[r]);
+            dp[r] *= a[r];
+        }
+        if (kill) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
+        }
+        if (want_dm) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) dm += dp[r];
+        }
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                pf[ts][i] = (T)a[8 * ts + i];
+                ds[ts][i] = (T)dp[8 * ts + i];
+            }
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                dv[dt] = Mfma<T>::mma(transposed<T, D>(buf + R::OFF_G, qb, ts, dt, lane), pf[ts], dv[dt]);
+                dk[dt] = Mfma<T>::mma(transposed<T, D>(buf, qb, ts, dt, lane), ds[ts], dk[dt]);
+            }
+    };
+
+    const int nst = (p.N + ROWS - 1) / ROWS;
+    finish(0);
+    for (int s = 0; s < nst; ++s) {
+        if (s + 1 < nst) fetch(s + 1);
+        if (active) {
+            const unsigned char *buf = lds + (s & 1) * R::STAGE;
+            tile(buf, s * (ROWS / 32), 0);
+            if (ROWS == 64 && 2 * s + 1 < NT) tile(buf, 2 * s + 1, 32);
+        }
+        if (s + 1 < nst) finish(s + 1);
+    }
+
+    if (!active) return;
+    if (want_dm) {
+        dm += __shfl_xor(dm, 32);
+        if (g == 0 && key < p.N) e.dmask_part[pr.row0 + key] = dm;
+    }
+    if (key < p.N) {
+        T *dK = (T *)p.dk + pr.base + (int64_t)key * p.stride_n, *dV = (T *)p.dv + pr.base + (int64_t)key * p.stride_n;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            store_row_tile<T>(dK, dt * 32, D, dk[dt], p.scale, g);
+            store_row_tile<T>(dV, dt * 32, D, dv[dt], 1.0f, g);
+        }
+    }
+}
+
+// ------------------------------------------------------------------ dBias partials
+
+// What mfma_dbias.hip is for the smaller head dims: dS a second time, summed over a chunk of S rows in registers.  A
+// workgroup has 128 queries x 64 keys of one (b, h), a wave 32 queries x 2 key tiles.  Keys (K, V, mask columns) are shared and
+// double-buffered in LDS; a wave's own rows of Q and dO come into LDS of its own, which it reads into registers at the
+// top of a row and refills at once, so they need no second buffer and no barrier.
+template <int D>
+struct DbStream {
+    static constexpr int KB = 64, QB = 128, BLK = KB * D * 2;
+    static constexpr int OFF_V = BLK, OFF_A = 2 * BLK, KEYS = OFF_A + KB * 16;
+    static constexpr int OFF_Q = 2 * KEYS, WAVE = 2 * 32 * D * 2, BYTES = OFF_Q + 4 * WAVE;
+};
+
+template <typename T, int D, bool BF32>
+__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) stream_dbias(EvoAttnParams p, Extra e) {
+    typedef StreamGeo<D> G;
+    typedef DbStream<D> R;
+    constexpr int KSD = D / 16, KS = KSD + 1;
+    typedef typename Mfma<T>::v8 v8;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, g = lane >> 5;
+    const int NT = (p.N + 31) / 32, nqb = (p.N + R::QB - 1) / R::QB, nkb = (p.N + R::KB - 1) / R::KB;
+    const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+    const int kbi = lid % nkb, qbi = (lid / nkb) % nqb;
+    const unsigned bh = (lid / (nkb * nqb)) % (unsigned)(p.B * p.H);
+    const int c = lid / (nkb * nqb) / (unsigned)(p.B * p.H), b = bh / p.H, h = bh % p.H;
+    const int q0 = qbi * R::QB + wave * 32, k0 = kbi * R::KB, qrow = min(q0 + li, p.N - 1);
+    const bool active = q0 < p.N, two = k0 + 32 < p.N;   // wave-uniform; a second key tile exists
+    const int sn2 = (int)p.stride_n * 2, valid = (p.N - 1) * sn2 + D * 2, np256 = (p.N + 255) / 256 * 256;
+    const float cs = p.scale * kLog2e;
+    const uint2 one3 = ones3<T>(), zero3 = {0u, 0u};
+    const v8 vaug = aug8<T>(one3, zero3);
+
+    // the bias of the wave's two tiles, resident: 16-bit pairs as given or fp32 in log2 units
+    const int bb = e.bias_batches > 1 ? b : 0;
+    Tile16 b16[2];
+    f32x16 b32[BF32 ? 2 : 1], sum[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int64_t o = ((((int64_t)bb * p.H + h) * NT + min(q0 >> 5, NT - 1)) * NT + min(k0 / 32 + j, NT - 1)) * 1024;
+        if constexpr (BF32) load_tile32(e.bq + o + lane * 4, b32[j]);
+        else load_tile16(e.bq16 + o + lane * 8, b16[j]);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[j][r] = 0.0f;
+    }
+    const int s_begin = c * e.chunk, s_end = min(p.S, s_begin + e.chunk);
+    if (s_begin >= s_end) return;   // uniform over the workgroup
+
+    unsigned char *const own = lds + R::OFF_Q + wave * R::WAVE;
+    float lse_n = 0.0f, delta_n = 0.0f;
+    auto fetch_keys = [&](int s) {
+        const Prob pr = decode_problem(p, bh * (unsigned)p.S + s);
+        const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.k + pr.base), 0, valid, 0x00020000);
+        const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.v + pr.base), 0, valid, 0x00020000);
+        const __amdgpu_buffer_rsrc_t mrs = __builtin_amdgcn_make_buffer_rsrc((void *)(e.m2a + ((int64_t)b * p.S + s) * np256), 0, np256 * 16, 0x00020000);
+        unsigned char *dst = lds + ((s - s_begin) & 1) * R::KEYS;
+        dma_rows<D, R::KB, 4>(krs, vrs, dst, k0, p.N, sn2, wave, lane);
+        if (wave == 0) dma16(mrs, dst + R::OFF_A, (k0 + lane) * 16);
+    };
+    auto fetch_queries = [&](int s) {
+        const Prob pr = decode_problem(p, bh * (unsigned)p.S + s);
+        const __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.q + pr.base), 0, valid, 0x00020000);
+        const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.dout + pr.base), 0, valid, 0x00020000);
+        dma_rows<D, 32, 1>(qrs, grs, own, q0, p.N, sn2, 0, lane);
+        lse_n = p.lse[pr.row0 + qrow];
+        delta_n = e.delta[pr.row0 + qrow];
+    };
+    fetch_keys(s_begin);
+    fetch_queries(s_begin);
+    for (int s = s_begin; s < s_end; ++s) {
+        const bool dead = e.dead[b * p.S + s] != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
+        wait_loads();
+        wait_lds_barrier();
+        if (s + 1 < s_end) fetch_keys(s + 1);   // (everybody has left that buffer: it held row s - 1)
+        v8 qf[KS], gf[KS];
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) {
+            const int o = G::at(li, 2 * ks + g);
+            qf[ks] = *reinterpret_cast<const v8 *>(own + o);
+            gf[ks] = *reinterpret_cast<const v8 *>(own + 32 * G::ROW + o);
+        }
+        qf[KSD] = g == 0 ? aug8<T>(one3, pack_split3<T>(-lse_n * kLog2e)) : zero8<T>();
+        gf[KSD] = g == 0 ? aug8<T>(pack_split3<T>(-delta_n), zero3) : zero8<T>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (s + 1 < s_end) fetch_queries(s + 1);
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) qf[ks] = dead ? zero8<T>() : scaled8<T>(qf[ks], cs);
+        if (!active || kill) continue;
+        const unsigned char *buf = lds + ((s - s_begin) & 1) * R::KEYS;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if (j == 1 && !two) break;   // uniform
+            f32x16 a, dp;
+            if constexpr (BF32) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) a[r] = dead ? 0.0f : b32[j][r];   // (uniform)
+            } else {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)   // (unpacked anew for each row: expanded once the tiles would take twice the registers)
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) asm volatile("" : "+v"(b16[j].w[i][w]));
+                unpack_tile16<T>(b16[j], dead ? 0.0f : kLog2e, a);
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < KSD; ++ks) {
+                const int o = G::at(32 * j + li, 2 * ks + g);
+                a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + o), qf[ks], a);                  // log2 P^T
+                dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_V + o), gf[ks], dp);     // dP^T - delta
+            }
+            a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (32 * j + li) * 16), qf[KSD], a);
+            dp = Mfma<T>::mma(vaug, gf[KSD], dp);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[j][r] += fast_exp2(a[r]) * dp[r];
+        }
+    }
+    // the partial of this chunk: lane = query li, registers 4 rr .. 4 rr + 3 = keys 8 rr + 4 g ..
+    if (active && q0 + li < p.N) {
+        float *part = e.dbias_part + ((((int64_t)c * p.B + b) * p.H + h) * p.N + (q0 + li)) * p.N;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+                const int kg = k0 + 32 * j + 8 * rr + 4 * g;
+                if ((p.N & 3) == 0 && kg + 4 <= p.N) {
+                    f32x4 v;
+                    v[0] = sum[j][4 * rr]; v[1] = sum[j][4 * rr + 1]; v[2] = sum[j][4 * rr + 2]; v[3] = sum[j][4 * rr + 3];
+                    *reinterpret_cast<f32x4 *>(part + kg) = v;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (kg + i < p.N) part[kg + i] = sum[j][4 * rr + i];
+                }
+            }
+    }
+}
+
+// ------------------------------------------------------------------ launchers
+
+template <typename T, int D>
+static int fwd_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    const unsigned grid = (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H * p.S);
+    if (p.bias_dtype == EVO_NONE) stream_fwd<T, D, 0><<<grid, 256, 0, st>>>(p, e);
+    else if (e.bias_direct) stream_fwd<T, D, 3><<<grid, 256, 0, st>>>(p, e);
+    else if (e.bq16) stream_fwd<T, D, 2><<<grid, 256, 0, st>>>(p, e);
+    else stream_fwd<T, D, 1><<<grid, 256, 0, st>>>(p, e);
+    return hip_rc();
+}
+
+int EVO_CAT(launch_mfma_fwd_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    return p.dtype == EVO_BF16 ? fwd_launch<bf16_t, EVO_D>(p, e, st) : fwd_launch<f16_t, EVO_D>(p, e, st);
+}
+
+template <typename T, int D>
+static int dq_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    const unsigned grid = (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H * p.S);
+    const bool direct = e.bias_direct, t16 = e.bq16 != nullptr;
+    if (p.dbias && p.S != 1) return EVO_EUNSUPPORTED;   // (a sum over S rows is the other kernels' business)
+    if (p.bias_dtype == EVO_NONE) stream_dq<T, D, 0, false><<<grid, 256, 0, st>>>(p, e);
+    else if (!p.dbias && direct) stream_dq<T, D, 3, false><<<grid, 256, 0, st>>>(p, e);
+    else if (!p.dbias && t16) stream_dq<T, D, 2, false><<<grid, 256, 0, st>>>(p, e);
+    else if (!p.dbias) stream_dq<T, D, 1, false><<<grid, 256, 0, st>>>(p, e);
+    else if (direct) stream_dq<T, D, 3, true><<<grid, 256, 0, st>>>(p, e);
+    else if (t16) stream_dq<T, D, 2, true><<<grid, 256, 0, st>>>(p, e);
+    else stream_dq<T, D, 1, true><<<grid, 256, 0, st>>>(p, e);
+    return hip_rc();
+}
+
+int EVO_CAT(launch_mfma_dqw_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    return p.dtype == EVO_BF16 ? dq_launch<bf16_t, EVO_D>(p, e, st) : dq_launch<f16_t, EVO_D>(p, e, st);
+}
+
+template <typename T, int D, int BT, int NW>
+static int dkdv_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    const unsigned grid = (unsigned)((p.N + NW * 32 - 1) / (NW * 32)) * (unsigned)(p.B * p.H * p.S);
+    constexpr int lds = KvStream<D, NW>::BYTES;
+    auto kern = stream_dkdv<T, D, BT, NW>;
+    if constexpr (lds > 64 * 1024) {
+        static PerDevice done{};
+        if (const int rc = ensure_dynamic_lds((const void *)kern, lds, done, nullptr)) return rc;
+    }
+    kern<<<grid, NW * 64, lds, st>>>(p, e);
+    return hip_rc();
+}
+
+template <typename T, int D, int NW>
+static int dkdv_bias(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    if (p.bias_dtype == EVO_NONE) return dkdv_launch<T, D, 0, NW>(p, e, st);
+    if (e.bias_direct) return dkdv_launch<T, D, 3, NW>(p, e, st);
+    return e.bk16 ? dkdv_launch<T, D, 2, NW>(p, e, st) : dkdv_launch<T, D, 1, NW>(p, e, st);
+}
+
+template <typename T, int D>
+static int dkdv_waves(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    if constexpr (D == 128) {
+        if (p.N > 128) return dkdv_bias<T, D, 8>(p, e, st);
+    }
+    return dkdv_bias<T, D, 4>(p, e, st);
+}
+
+int EVO_CAT(launch_mfma_dkdv_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    return p.dtype == EVO_BF16 ? dkdv_waves<bf16_t, EVO_D>(p, e, st) : dkdv_waves<f16_t, EVO_D>(p, e, st);
+}
+
+template <typename T, int D, bool BF32>
+static int dbias_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    typedef DbStream<D> R;
+    const int64_t grid = (int64_t)((p.N + R::QB - 1) / R::QB) * ((p.N + R::KB - 1) / R::KB) * p.B * p.H * e.n_chunks;
+    if (grid <= 0 || grid > 0x7fffffff) return EVO_EOVERFLOW;
+    static PerDevice done{};
+    if (const int rc = ensure_dynamic_lds((const void *)&stream_dbias<T, D, BF32>, R::BYTES, done, nullptr)) return rc;
+    stream_dbias<T, D, BF32><<<(unsigned)grid, 256, R::BYTES, st>>>(p, e);
+    return hip_rc();
+}
+
+int EVO_CAT(launch_mfma_dbias_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    const bool f = p.bias_dtype == EVO_F32;
+    if (p.dtype == EVO_BF16) return f ? dbias_launch<bf16_t, EVO_D, true>(p, e, st) : dbias_launch<bf16_t, EVO_D, false>(p, e, st);
+    return f ? dbias_launch<f16_t, EVO_D, true>(p, e, st) : dbias_launch<f16_t, EVO_D, false>(p, e, st);
+}
+
+}  // namespace evo
