@@ -398,9 +398,28 @@ const char *evoattn_path(const EvoAttnParams *p, int pass) {
     return mfma_ok(*p, pass) ? "mfma" : "generic";
 }
 
+// Whether a kernel that walks over a chunk of S rows, one workgroup per CU with the head's bias resident, is ahead of one
+// whose workgroups take single problems and stream (head dim 32): it gains a quarter to a sixth per row of 225 to 256 keys
+// and pays `start` rows' worth per round and the rows that do not fill its last round; shorter rows leave waves of its eight
+// idle.  (Forward, H = 8: S = 512, N = 256 103 against 120 us; S = 300, N = 248 67 / 75; N = 216 65 / 66; S = 200,
+// N = 200, H = 4 32 / 30.  dK/dV: S = 512, N = 256 133 / 140; S = 300, N = 248 77 / 81; N = 216 67 / 66; S = 200,
+// N = 200, H = 4 35 / 31.)  Rows of exactly 256 keys keep it throughout: there the two are level from a few S rows per
+// workgroup on.
+static bool ring_pays(const EvoAttnParams &p, double start, double per_row) {
+    if (p.N == 256) return true;
+    if (p.N <= 224) return false;
+    const int64_t bh = (int64_t)p.B * p.H;
+    const int n = chunks_for_rounds(bh, p.S, 256, 0.0);
+    const double rounds = (double)((bh * n + 255) / 256), rows = (double)((p.S + n - 1) / n);
+    return per_row * rounds * (rows + start) * 256.0 < (double)bh * p.S;
+}
+
 // rows of 129..256 keys: a workgroup per chunk of S rows with the head's bias resident
 static bool fwd_ring_ok(const EvoAttnParams &p) {
     if ((p.flags & EVO_FLAG_PER_PROBLEM) || bias_direct(p) || p.N <= 128 || p.N > mfma_fwdr_max_n(p.D)) return false;
+    // (a gated call keeps it at every length: the bias of a block's pair norm has a gradient that is zero but for
+    // the rounding of O, and the two kernels round P against different maxima)
+    if (p.D == 32 && !p.gate && !ring_pays(p, 2.4, 0.72)) return false;
     // Resident, a bias in the dtype of q takes 64 registers, an fp32 bias 128, which fit the register file only at
     // head dim 8 without a gate; elsewhere most of them are spilled and the one-workgroup-per-problem forward, which
     // streams the tiles, serves an fp32 bias (B = 1, S = 512, N = 256, H = 8, D = 32: 130 against 214 us).
@@ -414,6 +433,7 @@ static bool fwd_ring_ok(const EvoAttnParams &p) {
 static bool kv_ring_ok(const EvoAttnParams &p) {
     if ((p.flags & (EVO_FLAG_PER_PROBLEM | EVO_FLAG_DEBUG_NO_KV_RING)) || p.N <= 128 || p.N > mfma_kvr_max_n(p.D) || p.N % 8) return false;
     if (!aligned(p.lse, 16) || bias_direct(p)) return false;   // LSE rows are read four values at a time
+    if (p.D == 32 && !ring_pays(p, 1.3, 0.82)) return false;
     return !p.bias || p.bias_dtype == p.dtype;
 }
 

@@ -684,6 +684,10 @@ static int dkdv_bias(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
          : bt == 2 ? dkdv_launch<T, D, 2, NW, R::BQS>(p, e, st) : dkdv_launch<T, D, 1, NW, R::BQS>(p, e, st);
 }
 
+#if EVO_D == 32
+int launch_stream_dkdv_d32(const EvoAttnParams &p, const Extra &e, hipStream_t st);   // four waves, rows streamed (mfma_stream.hip)
+#endif
+
 // 8 waves (256 keys) per workgroup stage Q and dO once for twice the keys: measured faster
 // wherever a problem has more than 128 keys (N = 256: 171 vs 191 us at S = 512, H = 8;
 // N = 384, D = 32: 127 vs 149 us; N = 384, D = 8 within 3 %).
@@ -695,11 +699,18 @@ static int dkdv_waves(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const int64_t wgs = (int64_t)((p.N + 255) / 256) * p.B * p.H * p.S;
     // ... and unless the last 256-key workgroup of a problem would be at most half full at a small head dim, where
     // staging Q and dO a second time is cheap (bf16, S = 1024, H = 8, N = 384: 444 vs 531 us at head dim 8, 535 vs
-    // 571 us at 16; N = 320, head dim 8: 171 vs 222 us; at head dim 32 the two forms are level, 124 vs 123 us)
+    // 571 us at 16; N = 320, head dim 8: 171 vs 222 us)
     const int rem = p.N % 256;
-    const bool half_empty = D <= 16 && rem > 0 && rem <= 128;
+    const bool half_empty = rem > 0 && rem <= 128;
     const bool wide = (p.N > 128 && wgs >= 1024 && !half_empty) != ((p.flags & EVO_FLAG_DEBUG_OTHER_WIDTH) != 0);
+    // At head dim 32 the narrow form is the one that streams its rows (N = 384, S = 384, H = 4 116 -> 107 us, N = 288,
+    // S = 288 73 -> 61, N = 200, S = 200 36 -> 31; where the wide form's workgroups are full and enough it is ahead,
+    // N = 768 667 against 747 us, N = 216, S = 300, H = 8 69 against 74).
+#if EVO_D == 32
+    return wide ? dkdv_bias<T, D, 8>(p, e, st) : launch_stream_dkdv_d32(p, e, st);
+#else
     return wide ? dkdv_bias<T, D, 8>(p, e, st) : dkdv_bias<T, D, 4>(p, e, st);
+#endif
 }
 
 int EVO_CAT(launch_mfma_dkdv_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {

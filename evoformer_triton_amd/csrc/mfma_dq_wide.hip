@@ -1,6 +1,6 @@
 // dQ (and delta) for problems whose dBias is not a sum over S rows: no pair bias, a bias that
 // takes no gradient, or a single S row per (batch, head), where dBias is dS itself and is
-// written as it is formed.  Compiled once per head dim (-DEVO_D=8|16|32; 64 and 128: mfma_stream.hip).
+// written as it is formed.  Compiled once per head dim (-DEVO_D=8|16; from 32 on: mfma_stream.hip).
 //
 // Replaces the reference's `_attn_bwd_preprocess` (evoformer.py:299-326) and `_attn_bwd_dq`
 // (:329-476) for that case: P = exp(score - LSE) recomputed (:452), dS = P * (dP - delta)

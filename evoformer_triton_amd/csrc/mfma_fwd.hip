@@ -1,5 +1,5 @@
 // Flash-style forward for gfx950 on the bf16/fp16 32x32x16 matrix-core instruction.
-// Compiled once per head dim (-DEVO_D=8|16|32; 64 and 128: mfma_stream.hip).
+// Compiled once per head dim (-DEVO_D=8|16; from 32 on: mfma_stream.hip).
 //
 // Replaces the reference's `_attn_fwd` / `_attn_fwd_inner` (evoformer.py:23-297): bias add
 // and mask fused before the running max (:68-71), online softmax (:71-89), P cast to the

@@ -1,5 +1,5 @@
-// Forward, dQ and dK/dV for head dims 64 and 128: one workgroup per block of rows of a problem (b, h, s), the other side's
-// rows streamed through LDS.  Compiled once per head dim (-DEVO_D=64|128).
+// Forward, dQ, dK/dV and dBias for head dims 32 (without dBias), 64 and 128: one workgroup per block of rows of a problem
+// (b, h, s), the other side's rows streamed through LDS.  Compiled once per head dim (-DEVO_D=32|64|128).
 //
 // The arithmetic is that of the one-workgroup-per-problem kernels for smaller head dims (mfma_fwd.hip, mfma_bwd.hip,
 // mfma_dq_wide.hip: every additive term of the score rides in the matrix instruction, the scaled Q rounded once in the
@@ -32,7 +32,7 @@ struct StreamGeo {
     static constexpr int C = D / 8, ROW = D * 2;   // 16-byte chunks, bytes per row
     // the low bits of the row reversed (head dim 64: of every second row, two rows share the 64 banks)
     static __device__ __forceinline__ int x(int r) {
-        return D == 64 ? ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1)
+        return D == 32 ? (r >> 2) & 3 : D == 64 ? ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1)
                        : (r & 1) << 3 | ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1);
     }
     static __device__ __forceinline__ int at(int r, int c) { return r * ROW + ((c ^ x(r)) << 4); }
@@ -160,10 +160,14 @@ struct FwdStream {
 };
 
 template <typename T, int D, int BT>
-__global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_fwd(EvoAttnParams p, Extra e) {
+__global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3 : 2) stream_fwd(EvoAttnParams p, Extra e) {
     typedef StreamGeo<D> G;
     typedef FwdStream<D> R;
     constexpr int NW = 4, KSD = D / 16, KS = KSD + 1, DT = D / 32;
+    constexpr int ST = D == 32 ? 2 : 1;
+    // ST: key tiles per step.  Wider heads leave no registers for a second tile of scores.  Two tiles
+    // add up exactly as in mfma_fwd.hip, so that a D = 32 row's result does not depend on which of the two forms it.
+    // (Three waves per SIMD: S = N = 384, H = 4 97 us; at four the second tile spills, 124 us; mfma_fwd.hip's form 124 us.)
     typedef typename Mfma<T>::v8 v8;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[2][R::BYTES];
 
@@ -198,12 +202,13 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_fwd(EvoAttnParams
         if (g == 0) qf[KSD][0] = qf[KSD][1] = qf[KSD][2] = (T)1.0f;
     }
     const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, dead, lane);
-    typename BiasStream<T, BT, false>::Tile ct;
-    bias.load(0, ct);
+    typename BiasStream<T, BT, false>::Tile ct[ST];
+#pragma unroll
+    for (int t = 0; t < ST; ++t) bias.load(t, ct[t]);
 
     // m: the maximum the probabilities are relative to; mf: what the mask step subtracts inside the product (m, or 0 while
-    // m is unknown or too large for three 16-bit columns): after the first tile the scores arrive relative to m, and
-    // a later tile searches its maximum only when its sums show that it stands far above (see mfma_fwd.hip).
+    // m is unknown or too large for three 16-bit columns): after the first step the scores arrive relative to m, and
+    // a later one searches its maximum only when its sums show that it stands far above (see mfma_fwd.hip).
     float m = 0.0f, mf = 0.0f, l = 0.0f;
     f32x16 o[DT];
 #pragma unroll
@@ -217,10 +222,12 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_fwd(EvoAttnParams
         for (int ks = 0; ks < KSD; ++ks) a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + G::at(kb + li, 2 * ks + g)), qf[ks], a);
         a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (kb + li) * 16), qf[KSD], a);   // (zero in the step's upper half)
     };
-    auto settle = [&](bool first, f32x16 &a, float used) {
-        float mloc = a[0];
+    auto settle = [&](bool first, f32x16 (&a)[ST], float used) {
+        float mloc = a[0][0];
 #pragma unroll
-        for (int r = 1; r < 16; ++r) mloc = fmaxf(mloc, a[r]);
+        for (int t = 0; t < ST; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, a[t][r]);
         const unsigned u = __float_as_uint(mloc);
         auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
         const float cand = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) + used;
@@ -238,46 +245,60 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_fwd(EvoAttnParams
             m = mn;
             const float dsub = m - used;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) a[r] -= dsub;
+            for (int t = 0; t < ST; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) a[t][r] -= dsub;
             mf = fabsf(m) <= 1024.0f ? m : 0.0f;
             const v8 qa = aug8<T>(ones3<T>(), pack_split3<T>(-mf));
             if (g == 0) qf[KSD] = qa;
         }
     };
-    auto probs = [&](f32x16 &a, v8 (&pf)[2]) {
+    auto probs = [&](f32x16 (&a)[ST], v8 (&pf)[2 * ST]) {
         float s = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            a[r] = fast_exp2(a[r]);
-            s += a[r];
+            float x = 0.0f;
+#pragma unroll
+            for (int t = 0; t < ST; ++t) {
+                a[t][r] = fast_exp2(a[t][r]);
+                x = t ? x + a[t][r] : a[t][r];
+            }
+            s += x;
         }
 #pragma unroll
-        for (int ts = 0; ts < 2; ++ts)
+        for (int ts = 0; ts < 2 * ST; ++ts)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) pf[ts][i] = (T)a[8 * ts + i];
+            for (int i = 0; i < 8; ++i) pf[ts][i] = (T)a[ts / 2][8 * (ts & 1) + i];
         return s;
     };
-    auto tile = [&](const unsigned char *buf, int kt, int kb) {
+    // ST tiles, from tile kt and row kb of the stage on
+    auto step = [&](const unsigned char *buf, int kt, int kb) {
         const float used = mf;
-        f32x16 a;
-        score(buf, kb, bias.value(ct), a);
-        bias.load(kt + 1, ct);
+        f32x16 a[ST];
+#pragma unroll
+        for (int t = 0; t < ST; ++t) score(buf, kb + 32 * t, bias.value(ct[t]), a[t]);
+#pragma unroll
+        for (int t = 0; t < ST; ++t) bias.load(kt + ST + t, ct[t]);
         const bool lazy = kt != 0 && !__any(m != used);
         if (!lazy) settle(kt == 0, a, used);
-        v8 pf[2];
+        v8 pf[2 * ST];
         float s = probs(a, pf);
         if (__builtin_expect(lazy && __any(!(s <= 8192.0f)), 0)) {   // some score stands far above m: once more, the long way
-            typename BiasStream<T, BT, false>::Tile again;
-            bias.load(kt, again);
-            score(buf, kb, bias.value(again), a);
+#pragma unroll
+            for (int t = 0; t < ST; ++t) {
+                typename BiasStream<T, BT, false>::Tile again;
+                bias.load(kt + t, again);
+                score(buf, kb + 32 * t, bias.value(again), a[t]);
+            }
             settle(false, a, used);
             s = probs(a, pf);
         }
         l += s;
 #pragma unroll
-        for (int ts = 0; ts < 2; ++ts)
+        for (int ts = 0; ts < 2 * ST; ++ts)
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) o[dt] = Mfma<T>::mma(transposed<T, D>(buf + R::OFF_V, kb, ts, dt, lane), pf[ts], o[dt]);
+            for (int dt = 0; dt < DT; ++dt)
+                o[dt] = Mfma<T>::mma(transposed<T, D>(buf + R::OFF_V, kb + (ts / 2) * 32, ts & 1, dt, lane), pf[ts], o[dt]);
     };
 
     const int nst = (p.N + R::ROWS - 1) / R::ROWS;
@@ -287,8 +308,8 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_fwd(EvoAttnParams
         if (s + 1 < nst) fetch(s + 1);
         if (active) {
             const unsigned char *buf = lds[s & 1];
-            tile(buf, 2 * s, 0);
-            if (2 * s + 1 < NT) tile(buf, 2 * s + 1, 32);
+            step(buf, 2 * s, 0);
+            if (ST == 1 && 2 * s + 1 < NT) step(buf, 2 * s + 1, 32);
         }
         if (s + 1 < nst) {
             wait_loads();
@@ -319,7 +340,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_fwd(EvoAttnParams
 // As mfma_dq_wide.hip, whose place it takes at these head dims: where dBias is no sum over S rows, or its sum comes from a
 // kernel of its own.  A wave has 32 queries for all keys; with WRITE_DS (S = 1) dBias is dS and goes out as it is formed.
 template <typename T, int D, int BT, bool WRITE_DS>
-__global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_dq(EvoAttnParams p, Extra e) {
+__global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 ? 3 : 2) stream_dq(EvoAttnParams p, Extra e) {
     typedef StreamGeo<D> G;
     typedef FwdStream<D> R;
     constexpr int NW = 4, KSD = D / 16, KS = KSD + 1, DT = D / 32;
@@ -367,6 +388,10 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_dq(EvoAttnParams 
         const uint2 one3 = ones3<T>(), zero3 = {0u, 0u};
         qf[KSD] = g == 0 ? aug8<T>(one3, pack_split3<T>(-lse2)) : zero8<T>();   // ones x mask, -lse x ones
         gf[KSD] = g == 0 ? aug8<T>(pack_split3<T>(-dl), zero3) : zero8<T>();    // -delta x ones
+        if (kill) {   // no gradient through replaced scores: dP - delta is then zero, and dS with it
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) gf[ks] = zero8<T>();
+        }
     }
     const v8 vaug = aug8<T>(ones3<T>(), {0u, 0u});
     const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, dead, lane);
@@ -398,10 +423,6 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_dq(EvoAttnParams 
         bias.load(kt + 1, ct);
 #pragma unroll
         for (int r = 0; r < 16; ++r) a[r] = fast_exp2(a[r]) * dp[r];
-        if (kill) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) a[r] = 0.0f;
-        }
         if (WRITE_DS && q0 + li < p.N) {
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
@@ -464,14 +485,14 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) stream_dq(EvoAttnParams 
 // K operand lies in LDS (next to V, dK and dV it would not fit the registers of two waves per SIMD).
 template <int D, int NW>
 struct KvStream {
-    static constexpr int ROWS = D == 64 ? 64 : 32, BLK = ROWS * D * 2;
+    static constexpr int ROWS = D <= 64 ? 64 : 32, BLK = ROWS * D * 2;
     static constexpr bool K_LDS = D == 128;
     static constexpr int OFF_G = BLK, OFF_QS = 2 * BLK, OFF_AQ = 3 * BLK, OFF_AG = OFF_AQ + ROWS * 16, STAGE = (OFF_AG + ROWS * 16 + 1023) / 1024 * 1024;
     static constexpr int OFF_K = 2 * STAGE, BYTES = OFF_K + (K_LDS ? NW * 32 * D * 2 : 0);
 };
 
 template <typename T, int D, int BT, int NW>
-__global__ void __launch_bounds__(NW * 64, 2) stream_dkdv(EvoAttnParams p, Extra e) {
+__global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnParams p, Extra e) {
     typedef StreamGeo<D> G;
     typedef KvStream<D, NW> R;
     constexpr int KSD = D / 16, DT = D / 32, ROWS = R::ROWS;
@@ -529,11 +550,11 @@ __global__ void __launch_bounds__(NW * 64, 2) stream_dkdv(EvoAttnParams p, Extra
             const v8 k = dead ? zero8<T>() : ld8((const T *)p.k + row + ks * 16);
             if constexpr (R::K_LDS) *reinterpret_cast<v8 *>(lds + R::OFF_K + wave * 32 * G::ROW + G::at(li, 2 * ks + g)) = k;
             else kf[ks] = k;
-            vf[ks] = ld8((const T *)p.v + row + ks * 16);
+            vf[ks] = kill ? zero8<T>() : ld8((const T *)p.v + row + ks * 16);   // (no gradient through replaced scores: dS is then zero)
         }
         const uint2 mraw = e.m2[((int64_t)pr.b * p.S + pr.s) * (NT * 32) + min(key, NT * 32 - 1)];
         kaug = g == 0 ? aug8<T>(mraw, one3) : zero8<T>();     // mask x ones, ones x -lse
-        vaug = g == 0 ? aug8<T>(one3, zero3) : zero8<T>();    // ones x -delta
+        vaug = g == 0 && !kill ? aug8<T>(one3, zero3) : zero8<T>();    // ones x -delta
     }
     const BiasStream<T, BT, true> bias(p, e, pr, min(key0 >> 5, NT - 1), keyc, dead, lane);
     typename BiasStream<T, BT, true>::Tile ct;
@@ -569,10 +590,6 @@ __global__ void __launch_bounds__(NW * 64, 2) stream_dkdv(EvoAttnParams p, Extra
         for (int r = 0; r < 16; ++r) {
             a[r] = fast_exp2(a[r]);
             dp[r] *= a[r];
-        }
-        if (kill) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
         }
         if (want_dm) {
 #pragma unroll
@@ -635,7 +652,7 @@ struct DbStream {
 };
 
 template <typename T, int D, bool BF32>
-__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) stream_dbias(EvoAttnParams p, Extra e) {
+__global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnParams p, Extra e) {
     typedef StreamGeo<D> G;
     typedef DbStream<D> R;
     constexpr int KSD = D / 16, KS = KSD + 1;
@@ -815,6 +832,7 @@ static int dkdv_bias(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     return e.bk16 ? dkdv_launch<T, D, 2, NW>(p, e, st) : dkdv_launch<T, D, 1, NW>(p, e, st);
 }
 
+// Eight waves share a stage of queries at head dim 128 (the keys' K operand takes their LDS then).
 template <typename T, int D>
 static int dkdv_waves(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     if constexpr (D == 128) {
@@ -823,10 +841,15 @@ static int dkdv_waves(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     return dkdv_bias<T, D, 4>(p, e, st);
 }
 
+#if EVO_D == 32   // (mfma_bwd.hip chooses between its kernel of eight waves and this one)
+int launch_stream_dkdv_d32(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+#else
 int EVO_CAT(launch_mfma_dkdv_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+#endif
     return p.dtype == EVO_BF16 ? dkdv_waves<bf16_t, EVO_D>(p, e, st) : dkdv_waves<f16_t, EVO_D>(p, e, st);
 }
 
+#if EVO_D >= 64
 template <typename T, int D, bool BF32>
 static int dbias_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     typedef DbStream<D> R;
@@ -843,5 +866,6 @@ int EVO_CAT(launch_mfma_dbias_d, EVO_D)(const EvoAttnParams &p, const Extra &e, 
     if (p.dtype == EVO_BF16) return f ? dbias_launch<bf16_t, EVO_D, true>(p, e, st) : dbias_launch<bf16_t, EVO_D, false>(p, e, st);
     return f ? dbias_launch<f16_t, EVO_D, true>(p, e, st) : dbias_launch<f16_t, EVO_D, false>(p, e, st);
 }
+#endif
 
 }  // namespace evo

@@ -1,4 +1,4 @@
-"""The kernels for head dims 64 and 128 (csrc/mfma_stream.hip) at the edges of their stages, against eager in fp32."""
+"""The kernels whose rows stream through LDS (csrc/mfma_stream.hip, head dims from 32 on) at the edges of their stages, against eager in fp32."""
 import pytest
 import torch
 
@@ -17,6 +17,12 @@ CASES = [  # B, S, N, H, D, mask, bias, layout, gated, dtype
     (4, 1, 200, 16, 64, "bool", "f32", "reference", False, torch.bfloat16),      # the caller's bias rows, dBias written as formed
     (1, 3, 257, 2, 128, "jump", "f32", "ds4sci", False, torch.float16),
     (4, 1, 320, 16, 128, "bool", "q", "reference", False, torch.bfloat16),
+    (1, 5, 1, 2, 32, "dead", None, "reference", False, torch.float16),
+    (1, 40, 33, 2, 32, "soft", "q", "reference", True, torch.bfloat16),          # a second tile of one key
+    (1, 33, 193, 1, 32, "jump", "q", "ds4sci", False, torch.bfloat16),
+    (1, 3, 232, 1, 32, "dead", "q", "reference", False, torch.float16),          # too few S rows for a resident bias
+    (1, 70, 232, 8, 32, "bool", "q", "reference", False, torch.bfloat16),
+    (1, 6, 264, 2, 32, "soft", "f32", "reference", True, torch.bfloat16),
 ]
 
 
