@@ -19,9 +19,8 @@ results out so that the attention kernels read them as they fall:
     backward (`evoformer_attention(..., gate=g)`), so sigmoid(g) * O never makes a round trip
     of its own;
   * the gated output [B,S,N,H,D] viewed as [B,S,N,H*D] is the input of the output projection;
-  * the pair bias Linear(z) [B,N,N,H] is permuted once to [B,1,H,N,N] (H*N*N elements, small
-    next to the S*N*H*D of the other operands) in the dtype of Q, so the kernels take it from
-    16-bit tiles.
+  * the pair bias Linear(LayerNorm(z)) comes from one kernel as [B,1,H,N,N] in the dtype of Q, so the attention kernels
+    take it from 16-bit tiles; for shapes that kernel does not take, from the separate steps and a permute.
 """
 from __future__ import annotations
 
@@ -163,6 +162,14 @@ def _layer_norm(layer: nn.LayerNorm, x: torch.Tensor) -> torch.Tensor:
     return layer(x) if y is None else y
 
 
+def _pair_bias(norm: nn.LayerNorm, layer: nn.Linear, z: torch.Tensor) -> Optional[torch.Tensor]:
+    """Linear(LayerNorm(z)) permuted to [B,1,H,N,N] in one pass over z (csrc/pair_bias.hip), with the results of the separate
+    steps.  None where that kernel does not take the call."""
+    if torch.compiler.is_compiling() or layer.bias is not None or z.dim() != 4:
+        return None
+    return _lib.host().pair_bias(z, norm.weight, norm.bias, norm.eps, layer.weight)
+
+
 class GatedAttentionBlock(nn.Module):
     """Row-wise gated self-attention with pair bias (the MSA row attention of an Evoformer
     block).
@@ -213,7 +220,9 @@ class GatedAttentionBlock(nn.Module):
     def _bias_and_mask(self, z, mask, dtype, shape, norm, lin):
         B, S, N = shape
         bias = add_mask = None
-        if z is not None and self.linear_z is not None:
+        if z is not None and self.linear_z is not None and norm is _layer_norm and lin is _linear and z.dtype == dtype:
+            bias = _pair_bias(self.layer_norm_z, self.linear_z, z)
+        if bias is None and z is not None and self.linear_z is not None:
             bias = lin(self.linear_z, norm(self.layer_norm_z, z)).permute(0, 3, 1, 2).unsqueeze(1).contiguous().to(dtype)
         if mask is not None:
             add_mask = (self.inf * (mask.to(torch.float32) - 1.0)).view(B, S, 1, 1, N)

@@ -674,6 +674,84 @@ OptTensor layer_norm(const Tensor &x, const OptTensor &weight, const OptTensor &
     return y;
 }
 
+struct PairBiasNode : SavingNode {
+    std::string name() const override { return "PairBiasBackward"; }
+    // results: z, the LayerNorm's weight and bias, the projection's weight
+    variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        const bool rec = at::GradMode::is_enabled();
+        variable_list out(4);
+        if (!grads[0].defined()) return out;
+        {
+            at::AutoDispatchBelowADInplaceOrView guard;
+            const Tensor z = saved[0].unpack(), lw = saved[1].unpack(), lb = saved[2].unpack(), w = saved[3].unpack(), stats = saved[4].unpack();
+            const Tensor db = grads[0].contiguous();
+            const int64_t B = z.size(0), pairs = z.size(1) * z.size(2), rows = B * pairs;
+            const int32_t C = (int32_t)z.size(3), H = (int32_t)w.size(0);
+            const int dt = evo_dtype(z.scalar_type());
+            c10::DeviceGuard on(z.device());
+            Tensor ws, dparams;
+            if (task_should_compute_output(0)) out[0] = at::empty_like(z);
+            if (task_should_compute_output(1) || task_should_compute_output(2) || task_should_compute_output(3)) {
+                dparams = at::empty({2 + H, C}, z.options());
+                ws = scratch(evoattn_pair_bias_workspace_bytes(B, pairs, C, H, dt), z);
+            }
+            const float *mean = (const float *)stats.data_ptr();
+            auto ptr = [](const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; };
+            if (out[0].defined() || dparams.defined())
+                check(evoattn_pair_bias_bwd(db.data_ptr(), z.data_ptr(), ptr(lw), ptr(lb), w.data_ptr(), mean, mean + rows, ptr(out[0]), ptr(dparams),
+                                            ptr(ws), ws.defined() ? (size_t)ws.numel() : 0, B, pairs, C, H, dt, stream_of(z)), "evoattn_pair_bias_bwd");
+            if (task_should_compute_output(1)) out[1] = dparams.select(0, 0);
+            if (task_should_compute_output(2)) out[2] = dparams.select(0, 1);
+            if (task_should_compute_output(3)) out[3] = dparams.narrow(0, 2, H);
+        }
+        return once_differentiable(std::move(out), rec);
+    }
+};
+
+// LayerNorm of the pair representation, its projection to heads and the permute to [B,1,H,N,N] in one pass.  None for what
+// the kernels do not take.
+OptTensor pair_bias(const Tensor &z, const OptTensor &ln_weight, const OptTensor &ln_bias, double eps, const Tensor &weight) {
+    const int dt = evo_dtype(z.scalar_type());
+    const Tensor lw0 = ln_weight ? *ln_weight : Tensor(), lb0 = ln_bias ? *ln_bias : Tensor();
+    if (!plain(z) || !plain_modes() || !z.is_cuda() || z.dim() != 4 || z.numel() == 0 || !plain(weight) || weight.dim() != 2 ||
+        weight.size(1) != z.size(3) || weight.size(1) > 4096 || weight.size(0) > 4096)
+        return std::nullopt;
+    for (const Tensor &t : {lw0, lb0, weight})
+        if (t.defined() && (!plain(t) || t.scalar_type() != z.scalar_type() || t.device() != z.device())) return std::nullopt;
+    for (const Tensor &t : {lw0, lb0})
+        if (t.defined() && (t.dim() != 1 || t.size(0) != z.size(3))) return std::nullopt;
+    const int64_t B = z.size(0), pairs = z.size(1) * z.size(2), rows = B * pairs;
+    const int32_t C = (int32_t)z.size(3), H = (int32_t)weight.size(0);
+    if (evoattn_pair_bias_workspace_bytes(B, pairs, C, H, dt) == 0) return std::nullopt;
+    Tensor out, zc, lw, lb, w, stats;
+    {
+        at::AutoDispatchBelowADInplaceOrView guard;
+        c10::DeviceGuard on(z.device());
+        zc = z.contiguous();
+        w = weight.contiguous();
+        lw = lw0.defined() ? lw0.contiguous() : Tensor();
+        lb = lb0.defined() ? lb0.contiguous() : Tensor();
+        auto aligned = [](const Tensor &t) { return !t.defined() || (uintptr_t)t.data_ptr() % 16 == 0; };
+        if (!aligned(zc) || !aligned(w) || !aligned(lw) || !aligned(lb)) return std::nullopt;
+        out = at::empty({B, 1, H, z.size(1), z.size(2)}, zc.options());
+        stats = at::empty({2 * rows}, zc.options().dtype(at::kFloat));   // mean, then 1 / deviation
+        float *mean = (float *)stats.data_ptr();
+        check(evoattn_pair_bias_fwd(zc.data_ptr(), lw.defined() ? lw.data_ptr() : nullptr, lb.defined() ? lb.data_ptr() : nullptr, w.data_ptr(),
+                                    out.data_ptr(), mean, mean + rows, B, pairs, C, H, dt, (float)eps, stream_of(zc)), "evoattn_pair_bias_fwd");
+    }
+    if (SavingNode::wanted(z, lw0, lb0, weight)) {
+        auto node = make_node<PairBiasNode>(z, lw0, lb0, weight);
+        torch::autograd::set_history(out, node);
+        node->save(zc);
+        node->save(lw);
+        node->save(lb);
+        node->save(w);
+        node->save(stats);
+    }
+    return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -685,4 +763,5 @@ PYBIND11_MODULE(_host, m) {
     m.def("linear", &linear, no_gil, py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("dx_place"));
     m.def("stacked_projection", &stacked_projection, no_gil, py::arg("x"), py::arg("gate_bias"), py::arg("weights"));
     m.def("layer_norm", &layer_norm, no_gil, py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("eps"));
+    m.def("pair_bias", &pair_bias, no_gil, py::arg("z"), py::arg("ln_weight"), py::arg("ln_bias"), py::arg("eps"), py::arg("weight"));
 }

@@ -32,5 +32,6 @@ int mfma_dqr_qrows(int D, int N);  // query rows per workgroup of the double-buf
 int launch_mfma_dkdv(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_dqw(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // dQ where no dBias is asked for
 int launch_mfma_dbias(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // dBias partials alone (reads delta)
+int launch_column_reduce(const float *part, int blocks, int cols, void *out, int dtype, hipStream_t st);  // out[c] = sum of part[.][c], fixed order
 
 }  // namespace evo

@@ -12,6 +12,7 @@
 // by a second small kernel in a fixed order: no atomics, bit-reproducible.
 #include "common.h"
 #include "bwd_common.h"
+#include "kernels.h"
 
 namespace evo {
 
@@ -354,6 +355,13 @@ static int colsum_launch(const void *a, void *out, float *part, int64_t rows, in
     }
     ln_reduce_kernel<T><<<(cols + kLnRedCols - 1) / kLnRedCols, kLnRedCols * kLnRedSlices, 0, st>>>(part, rows > 0 ? (int)grid : 0, 1, cols,
                                                                                                   (T *)out, (T *)nullptr);
+    return hip_rc();
+}
+
+int launch_column_reduce(const float *part, int blocks, int cols, void *out, int dtype, hipStream_t st) {
+    const unsigned grid = (cols + kLnRedCols - 1) / kLnRedCols;
+    if (dtype == EVO_BF16) ln_reduce_kernel<bf16_t><<<grid, kLnRedCols * kLnRedSlices, 0, st>>>(part, blocks, 1, cols, (bf16_t *)out, (bf16_t *)nullptr);
+    else ln_reduce_kernel<f16_t><<<grid, kLnRedCols * kLnRedSlices, 0, st>>>(part, blocks, 1, cols, (f16_t *)out, (f16_t *)nullptr);
     return hip_rc();
 }
 

@@ -237,6 +237,22 @@ size_t evoattn_colsum_workspace_bytes(int64_t rows, int32_t cols, int32_t dtype)
 int evoattn_colsum(const void *a, int64_t row_stride, void *out, void *workspace, size_t workspace_bytes, int64_t rows,
                    int32_t cols, int32_t dtype, void *hip_stream);
 
+/* The pair bias of the block around the attention (no counterpart in the reference's operator): LayerNorm over
+ * the last dimension of z [batches, pairs, cols], projection to `heads` channels by w [heads, cols], result [batches, heads,
+ * pairs], each step rounded to the dtype as the separate steps round.
+ *   dtype  EVO_BF16 / EVO_F16: everything but mean and rstd [batches * pairs] fp32, written by the forward, read by the backward
+ *   cols   64, 128 or 256;  heads  1 to 16
+ *   gamma, beta may be NULL (weight 1, bias 0); dz or dparams may be NULL (not wanted)
+ *   dparams  [2 + heads, cols]: the gradients of gamma, of beta and of w, summed through `workspace` in a fixed order
+ * evoattn_pair_bias_workspace_bytes() is 0 for what these entry points do not take.  z, gamma, beta, w, dz and the workspace
+ * 16-byte aligned.  Nothing is allocated or synchronised. */
+size_t evoattn_pair_bias_workspace_bytes(int64_t batches, int64_t pairs, int32_t cols, int32_t heads, int32_t dtype);
+int evoattn_pair_bias_fwd(const void *z, const void *gamma, const void *beta, const void *w, void *bias, float *mean, float *rstd,
+                          int64_t batches, int64_t pairs, int32_t cols, int32_t heads, int32_t dtype, float eps, void *hip_stream);
+int evoattn_pair_bias_bwd(const void *dbias, const void *z, const void *gamma, const void *beta, const void *w, const float *mean,
+                          const float *rstd, void *dz, void *dparams, void *workspace, size_t workspace_bytes, int64_t batches,
+                          int64_t pairs, int32_t cols, int32_t heads, int32_t dtype, void *hip_stream);
+
 #ifdef __cplusplus
 }
 #endif
