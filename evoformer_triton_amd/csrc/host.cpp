@@ -10,6 +10,7 @@
 // dims that need padding, empty problems, anything invalid): the caller in Python then goes its own
 // way, which also words the error messages.
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -501,6 +502,70 @@ Tensor bias_grad(const Tensor &dy2) {
 
 Tensor as_rows(const Tensor &t) { return t.reshape({-1, t.size(-1)}); }
 
+// The products of the Linear layers: through the library's kernels (csrc/linear.hip) where they take the operands, else torch's.
+bool lin_rows_ok(const Tensor &t, at::ScalarType dt) {
+    return plain(t) && t.is_cuda() && t.dim() == 2 && t.scalar_type() == dt && t.stride(1) == 1 && t.stride(0) % 8 == 0 && t.stride(0) >= t.size(1) &&
+           (uintptr_t)t.data_ptr() % 16 == 0;
+}
+// `a`: rows of a matrix to be multiplied by the stacked weights [n, k]
+bool lin_ok(const Tensor &a, const std::vector<Tensor> &w) {
+    const auto dt = a.scalar_type();
+    if ((dt != at::kBFloat16 && dt != at::kHalf) || w.empty() || w.size() > 4 || !plain_modes() || !lin_rows_ok(a, dt) || a.size(0) == 0) return false;
+    for (const Tensor &t : w)
+        if (!lin_rows_ok(t, dt) || t.device() != a.device() || !t.is_contiguous() || !t.sizes().equals(w[0].sizes())) return false;
+    const int64_t rows = w[0].size(0), n = rows * (int64_t)w.size(), k = w[0].size(1);
+    return n <= INT32_MAX && k <= INT32_MAX && rows % 64 == 0 && evoattn_linear_dw_workspace_bytes(a.size(0), (int32_t)n, (int32_t)k, evo_dtype(dt)) != 0;
+}
+struct WeightPtrs {
+    const void *p[4] = {};
+    explicit WeightPtrs(const std::vector<Tensor> &w) {
+        for (size_t i = 0; i < w.size(); ++i) p[i] = w[i].data_ptr();
+    }
+};
+
+// a w^T (+ bias on the last columns) as [rows, n]; not defined where the kernels do not take it
+Tensor lin_forward(const Tensor &a, const std::vector<Tensor> &w, const Tensor &bias) {
+    if (at::autocast::is_autocast_enabled(at::kCUDA) || !lin_ok(a, w) || a.size(1) != w[0].size(1)) return Tensor();
+    const int64_t n = w[0].size(0) * (int64_t)w.size();
+    const int64_t from = bias.defined() ? n - bias.numel() : 0;
+    if (bias.defined() && (!plain(bias) || bias.dim() != 1 || bias.scalar_type() != a.scalar_type() || bias.device() != a.device() || !bias.is_contiguous() ||
+                           from < 0 || from % 16 || (uintptr_t)bias.data_ptr() % 16))
+        return Tensor();
+    c10::DeviceGuard on(a.device());
+    Tensor y = at::empty({a.size(0), n}, a.options());
+    check(evoattn_linear_fwd(a.data_ptr(), a.stride(0), WeightPtrs(w).p, (int32_t)w.size(), (int32_t)w[0].size(0), bias.defined() ? bias.data_ptr() : nullptr,
+                             (int32_t)from, y.data_ptr(), n, a.size(0), (int32_t)n, (int32_t)a.size(1), evo_dtype(a.scalar_type()), stream_of(a)),
+          "evoattn_linear_fwd");
+    return y;
+}
+
+// dy w into `dx`, whose rows may lie apart; false where the kernels do not take it
+bool lin_input_grad(const Tensor &dy, const std::vector<Tensor> &w, const Tensor &dx) {
+    if (!lin_ok(dy, w) || !lin_rows_ok(dx, dy.scalar_type()) || dy.size(1) != w[0].size(0) * (int64_t)w.size() || dx.size(0) != dy.size(0) ||
+        dx.size(1) != w[0].size(1) || dx.device() != dy.device())
+        return false;
+    c10::DeviceGuard on(dy.device());
+    check(evoattn_linear_dx(dy.data_ptr(), dy.stride(0), WeightPtrs(w).p, (int32_t)w.size(), (int32_t)w[0].size(0), dx.data_ptr(), dx.stride(0), dy.size(0),
+                            (int32_t)dy.size(1), (int32_t)dx.size(1), evo_dtype(dy.scalar_type()), stream_of(dy)), "evoattn_linear_dx");
+    return true;
+}
+
+// dy^T x and, if asked for, the column sums of dy
+std::pair<Tensor, Tensor> lin_weight_grad(const Tensor &dy, const Tensor &x, bool sums) {
+    const auto dt = dy.scalar_type();
+    const int64_t rows = dy.size(0), n = dy.size(1), k = x.size(1);
+    size_t bytes = 0;
+    if ((dt == at::kBFloat16 || dt == at::kHalf) && plain_modes() && lin_rows_ok(dy, dt) && lin_rows_ok(x, dt) && x.device() == dy.device() &&
+        n <= INT32_MAX && k <= INT32_MAX)
+        bytes = evoattn_linear_dw_workspace_bytes(rows, (int32_t)n, (int32_t)k, evo_dtype(dt));
+    if (!bytes) return {weight_grad(dy, x), sums ? bias_grad(dy) : Tensor()};
+    c10::DeviceGuard on(dy.device());
+    Tensor out = at::empty({n * k + (sums ? n : 0)}, dy.options()), ws = scratch(bytes, dy);
+    check(evoattn_linear_dw(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), out.data_ptr(), sums, ws.data_ptr(), (size_t)ws.numel(), rows, (int32_t)n,
+                            (int32_t)k, evo_dtype(dt), stream_of(dy)), "evoattn_linear_dw");
+    return {out.narrow(0, 0, n * k).view({n, k}), sums ? out.narrow(0, n * k, n) : Tensor()};
+}
+
 struct LinearNode : SavingNode {
     bool has_bias = false;
     Tensor dx_place;
@@ -514,16 +579,13 @@ struct LinearNode : SavingNode {
             at::AutoDispatchBelowADInplaceOrView guard;
             const Tensor x = saved[0].unpack(), w = saved[1].unpack(), dy2 = as_rows(grads[0]);
             if (task_should_compute_output(0)) {
-                if (dx_place.defined()) {
-                    Tensor rows = dx_place.view({-1, x.size(-1)});
-                    at::mm_out(rows, dy2, w);
-                    out[0] = dx_place;
-                } else {
-                    out[0] = dy2.mm(w).view(x.sizes());
-                }
+                out[0] = dx_place.defined() ? dx_place : at::empty_like(x, at::MemoryFormat::Contiguous);
+                Tensor rows = out[0].view({-1, x.size(-1)});
+                if (!lin_input_grad(dy2, {w}, rows)) at::mm_out(rows, dy2, w);
             }
-            if (task_should_compute_output(1)) out[1] = weight_grad(dy2, as_rows(x));
-            if (has_bias && task_should_compute_output(2)) out[2] = bias_grad(dy2);
+            const bool sums = has_bias && task_should_compute_output(2);
+            if (task_should_compute_output(1)) std::tie(out[1], out[2]) = lin_weight_grad(dy2, as_rows(x), sums);
+            else if (sums) out[2] = bias_grad(dy2);
         }
         return once_differentiable(std::move(out), rec);
     }
@@ -537,7 +599,9 @@ Tensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, cons
         at::AutoDispatchBelowADInplaceOrView guard;
         // (as a matrix: for an input of more dimensions whose rows lie apart torch multiplies and then adds the
         // bias in a pass of its own)
-        y = at::linear(as_rows(x), weight, bias);
+        const Tensor rows = as_rows(x);
+        y = lin_forward(rows, {weight}, bias ? *bias : Tensor());
+        if (!y.defined()) y = at::linear(rows, weight, bias);
         auto shape = x.sizes().vec();
         shape.back() = weight.size(0);
         y = y.view(shape);
@@ -566,14 +630,24 @@ struct StackedNode : SavingNode {
         if (!grads[0].defined()) return out;
         {
             at::AutoDispatchBelowADInplaceOrView guard;
-            const Tensor x = saved[0].unpack(), w = saved[1].unpack(), dp2 = as_rows(grads[0]);
-            if (task_should_compute_output(0)) out[0] = dp2.mm(w).view(x.sizes());
-            if (has_bias && task_should_compute_output(1)) out[1] = bias_grad(dp2.narrow(1, dp2.size(1) - sizes.back(), sizes.back()));
+            const Tensor x = saved[0].unpack(), dp2 = as_rows(grads[0]);
+            std::vector<Tensor> w;
+            for (size_t i = 0; i < sizes.size(); ++i) w.push_back(saved[1 + i].unpack());
+            if (task_should_compute_output(0)) {
+                out[0] = at::empty_like(x, at::MemoryFormat::Contiguous);
+                Tensor rows = as_rows(out[0]);
+                if (!lin_input_grad(dp2, w, rows)) at::mm_out(rows, dp2, at::cat(w, 0));
+            }
+            const bool sums = has_bias && task_should_compute_output(1);
             bool any = false;
             for (size_t i = 0; i < sizes.size(); ++i) any |= task_should_compute_output(2 + i);
             if (any) {
-                auto parts = weight_grad(dp2, as_rows(x)).split_with_sizes(sizes, 0);
+                auto [dw, db] = lin_weight_grad(dp2, as_rows(x), sums);
+                auto parts = dw.split_with_sizes(sizes, 0);
                 for (size_t i = 0; i < sizes.size(); ++i) out[2 + i] = parts[i];
+                if (sums) out[1] = db.narrow(0, db.size(0) - sizes.back(), sizes.back());
+            } else if (sums) {
+                out[1] = bias_grad(dp2.narrow(1, dp2.size(1) - sizes.back(), sizes.back()));
             }
         }
         return once_differentiable(std::move(out), rec);
@@ -582,14 +656,21 @@ struct StackedNode : SavingNode {
 
 // Several projections of one input as one GEMM with their weights stacked; `gate_bias` is added on the last layer's columns.
 Tensor stacked_projection(const Tensor &x, const OptTensor &gate_bias, const std::vector<Tensor> &weights) {
-    Tensor y, w;
+    Tensor y;
     const Tensor gb = gate_bias ? *gate_bias : Tensor();
     {
         at::AutoDispatchBelowADInplaceOrView guard;
-        w = at::cat(weights, 0);
-        OptTensor bias;
-        if (gb.defined()) bias = at::constant_pad_nd(gb, {w.size(0) - gb.size(0), 0});
-        y = at::linear(x, w, bias);
+        y = lin_forward(as_rows(x), weights, gb);
+        if (y.defined()) {
+            auto shape = x.sizes().vec();
+            shape.back() = y.size(1);
+            y = y.view(shape);
+        } else {
+            const Tensor w = at::cat(weights, 0);
+            OptTensor bias;
+            if (gb.defined()) bias = at::constant_pad_nd(gb, {w.size(0) - gb.size(0), 0});
+            y = at::linear(x, w, bias);
+        }
     }
     bool needed = SavingNode::wanted(x, gb);
     for (const auto &t : weights) needed |= SavingNode::wanted(t);
@@ -602,7 +683,7 @@ Tensor stacked_projection(const Tensor &x, const OptTensor &gate_bias, const std
         node->has_bias = gb.defined();
         torch::autograd::set_history(y, node);
         node->save(x);
-        node->save(w);
+        for (const auto &t : weights) node->save(t);
     }
     return y;
 }
@@ -714,7 +795,7 @@ struct PairBiasNode : SavingNode {
 OptTensor pair_bias(const Tensor &z, const OptTensor &ln_weight, const OptTensor &ln_bias, double eps, const Tensor &weight) {
     const int dt = evo_dtype(z.scalar_type());
     const Tensor lw0 = ln_weight ? *ln_weight : Tensor(), lb0 = ln_bias ? *ln_bias : Tensor();
-    if (!plain(z) || !plain_modes() || !z.is_cuda() || z.dim() != 4 || z.numel() == 0 || !plain(weight) || weight.dim() != 2 ||
+    if (!plain(z) || !plain_modes() || at::autocast::is_autocast_enabled(at::kCUDA) || !z.is_cuda() || z.dim() != 4 || z.numel() == 0 || !plain(weight) || weight.dim() != 2 ||
         weight.size(1) != z.size(3) || weight.size(1) > 4096 || weight.size(0) > 4096)
         return std::nullopt;
     for (const Tensor &t : {lw0, lb0, weight})

@@ -237,6 +237,22 @@ size_t evoattn_colsum_workspace_bytes(int64_t rows, int32_t cols, int32_t dtype)
 int evoattn_colsum(const void *a, int64_t row_stride, void *out, void *workspace, size_t workspace_bytes, int64_t rows,
                    int32_t cols, int32_t dtype, void *hip_stream);
 
+/* The Linear layers of the block around the attention (no counterpart in the reference's operator), 16-bit, on the matrix
+ * cores with fp32 sums.  The weight [n, k] may be `nw` (1 to 4) matrices of w_rows rows each, stacked.
+ *   fwd  y [rows, n] = x [rows, k] w^T, plus bias on outputs bias_from .. n - 1 (bias may be NULL)
+ *   dx   dx [rows, k] = dy [rows, n] w
+ *   dw   out [n k (+ n)] = dy^T x, then (sums) the column sums of dy; through `workspace`, in a fixed order
+ *   dtype  EVO_BF16 / EVO_F16;  n, k and w_rows multiples of 64, bias_from of 16
+ * ld*: elements from one row to the next, multiples of 8.  All pointers 16-byte aligned.  evoattn_linear_dw_workspace_bytes() is 0
+ * for shapes that these entry points do not take.  Nothing is allocated or synchronised. */
+int evoattn_linear_fwd(const void *x, int64_t ldx, const void *const *w, int32_t nw, int32_t w_rows, const void *bias, int32_t bias_from,
+                       void *y, int64_t ldy, int64_t rows, int32_t n, int32_t k, int32_t dtype, void *hip_stream);
+int evoattn_linear_dx(const void *dy, int64_t lddy, const void *const *w, int32_t nw, int32_t w_rows, void *dx, int64_t lddx, int64_t rows,
+                      int32_t n, int32_t k, int32_t dtype, void *hip_stream);
+size_t evoattn_linear_dw_workspace_bytes(int64_t rows, int32_t n, int32_t k, int32_t dtype);
+int evoattn_linear_dw(const void *dy, int64_t lddy, const void *x, int64_t ldx, void *out, int32_t sums, void *workspace, size_t workspace_bytes,
+                      int64_t rows, int32_t n, int32_t k, int32_t dtype, void *hip_stream);
+
 /* The pair bias of the block around the attention (no counterpart in the reference's operator): LayerNorm over
  * the last dimension of z [batches, pairs, cols], projection to `heads` channels by w [heads, cols], result [batches, heads,
  * pairs], each step rounded to the dtype as the separate steps round.
