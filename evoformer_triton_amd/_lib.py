@@ -34,7 +34,7 @@ EXPORTS = ("evoattn_version", "evoattn_strerror", "evoattn_check", "evoattn_prep
            "evoattn_layernorm_fwd", "evoattn_layernorm_bwd_workspace_bytes", "evoattn_layernorm_bwd",
            "evoattn_colsum_workspace_bytes", "evoattn_colsum",
            "evoattn_pair_bias_workspace_bytes", "evoattn_pair_bias_fwd", "evoattn_pair_bias_bwd",
-           "evoattn_linear_fwd", "evoattn_linear_dx", "evoattn_linear_dw_workspace_bytes", "evoattn_linear_dw")
+           "evoattn_keep_mask", "evoattn_linear_fwd", "evoattn_linear_dx", "evoattn_linear_dw_workspace_bytes", "evoattn_linear_dw")
 EVOATTN_STATIC_PREP_BYTES = 16 << 20
 
 
@@ -108,6 +108,8 @@ def load(path: str | None = None) -> ctypes.CDLL:
     lib.evoattn_colsum_workspace_bytes.argtypes = [i64, i32, i32]
     lib.evoattn_colsum.restype = ctypes.c_int
     lib.evoattn_colsum.argtypes = [vp, i64, vp, vp, ctypes.c_size_t, i64, i32, i32, vp]
+    lib.evoattn_keep_mask.restype = ctypes.c_int
+    lib.evoattn_keep_mask.argtypes = [vp, vp, i64, ctypes.c_float, vp]
     lib.evoattn_linear_fwd.restype = ctypes.c_int
     lib.evoattn_linear_fwd.argtypes = [vp, i64, ctypes.POINTER(vp), i32, i32, vp, i32, vp, i64, i64, i32, i32, i32, vp]
     lib.evoattn_linear_dx.restype = ctypes.c_int

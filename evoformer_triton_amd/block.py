@@ -170,6 +170,10 @@ def _pair_bias(norm: nn.LayerNorm, layer: nn.Linear, z: torch.Tensor) -> Optiona
     return _lib.host().pair_bias(z, norm.weight, norm.bias, norm.eps, layer.weight)
 
 
+_NO_PARAMETERS = {"weight": None, "bias": None}
+_UNBIASED = ("linear_q", "linear_k", "linear_v", "linear_z")
+
+
 class GatedAttentionBlock(nn.Module):
     """Row-wise gated self-attention with pair bias (the MSA row attention of an Evoformer
     block).
@@ -230,14 +234,37 @@ class GatedAttentionBlock(nn.Module):
 
     def _slots_ok(self, m: torch.Tensor) -> bool:
         """Whether Q, K, V and the gate can come from one GEMM and reach the kernels as slots of its result."""
-        layers = [self.linear_q, self.linear_k, self.linear_v, self.linear_o] + ([self.linear_g] if self.linear_g is not None else [])
-        return (m.is_cuda and m.numel() > 0 and not torch.compiler.is_compiling() and m.dtype in (torch.bfloat16, torch.float16)
-                and self.c_hidden in _HEAD_DIMS and all(l.weight.dtype == m.dtype for l in layers)
-                and all(l.bias is None for l in layers[:3]))
+        if not m.is_cuda or m.dtype not in (torch.bfloat16, torch.float16) or m.numel() == 0 or torch.compiler.is_compiling() \
+                or self.c_hidden not in _HEAD_DIMS:
+            return False
+        mods = self._modules
+        layers = [mods["linear_q"], mods["linear_k"], mods["linear_v"], mods["linear_o"]] + ([mods["linear_g"]] if mods.get("linear_g") is not None else [])
+        return all(l.weight.dtype == m.dtype for l in layers) and all(l.bias is None for l in layers[:3])
+
+    def _native(self, m, z, mask):
+        """The block as one call and one autograd node (csrc/host.cpp); None where it does not take the call.  (Layers are
+        looked up as a module stores them: their attribute access alone takes 15 us of a 100 us forward.)"""
+        mods, with_z = self._modules, z is not None and self._modules.get("linear_z") is not None
+        inputs = [m, z if with_z else None]
+        for name, used in (("layer_norm_m", True), ("linear_q", True), ("linear_k", True), ("linear_v", True), ("linear_g", mods.get("linear_g") is not None),
+                           ("linear_o", True), ("layer_norm_z", with_z), ("linear_z", with_z)):
+            own = mods[name]._parameters if used else _NO_PARAMETERS
+            if "weight" not in own or "bias" not in own:
+                return None     # (a layer whose weight is formed from something else)
+            if name in _UNBIASED:
+                if own["bias"] is not None:
+                    return None
+                inputs.append(own["weight"])
+            else:
+                inputs += (own["weight"], own["bias"])
+        return _lib.host().block(inputs, mask, self.no_heads, mods["layer_norm_m"].eps, mods["layer_norm_z"].eps if with_z else 0.0, self.inf)
 
     def forward(self, m: torch.Tensor, z: Optional[torch.Tensor] = None, mask: Optional[torch.Tensor] = None):
         B, S, N, _ = m.shape
         if self._slots_ok(m):
+            out = self._native(m, z, mask)
+            if out is not None:
+                return out
             H, D = self.no_heads, self.c_hidden
             gated = self.linear_g is not None
             x = _layer_norm(self.layer_norm_m, m)

@@ -361,8 +361,15 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
         return (char *)t.data_ptr() + (size_t)i * p.H * p.D * t.element_size();
     }
 
-    static variable_list forward(AutogradContext *ctx, const Tensor &P, OptTensor mask, OptTensor bias, bool gated) {
+    // What the forward leaves for the backward.  `ob` [B,S,N,W,H,D]: slot 1 (gated, else 0) the output, slot 2 room for its gradient.
+    struct Run {
         Call c{};
+        Tensor ob, aux;
+        OptTensor mask, bias;
+    };
+    static Run enqueue(const Tensor &P, const OptTensor &mask, const OptTensor &bias, bool gated) {
+        Run r;
+        Call &c = r.c;
         EvoAttnParams &p = c.p;
         p.B = (int32_t)P.size(0);
         p.S = (int32_t)P.size(1);
@@ -374,31 +381,68 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
         p.scale = (float)(1.0 / std::sqrt((double)p.D));
         strides(p, P);
         c.gated = gated;
-        TORCH_CHECK_VALUE(operands(c, P, mask, bias), "the mask must be [B,S,1,1,N] and the pair bias [B,1,H,N,N] (B and the mask's S may be 1), on P's device");
+        r.mask = mask;
+        r.bias = bias;
+        TORCH_CHECK_VALUE(operands(c, P, r.mask, r.bias), "the mask must be [B,S,1,1,N] and the pair bias [B,1,H,N,N] (B and the mask's S may be 1), on P's device");
         c10::DeviceGuard on(P.device());
-        Tensor ob = at::empty_like(P);
+        r.ob = at::empty_like(P);
         const Aux layout(p);
-        Tensor aux = scratch(layout.lse_bytes + evoattn_prep_bytes(&p), P);
-        layout.place(p, aux);
+        r.aux = scratch(layout.lse_bytes + evoattn_prep_bytes(&p), P);
+        layout.place(p, r.aux);
         p.q = slot(P, p, 0);
         p.k = slot(P, p, 1);
         p.v = slot(P, p, 2);
         if (gated) {   // the gated output alone: slot 0 stays unwritten
             p.gate = slot(P, p, 3);
-            p.o_gated = slot(ob, p, 1);
+            p.o_gated = slot(r.ob, p, 1);
         } else {
-            p.o = slot(ob, p, 0);
+            p.o = slot(r.ob, p, 0);
         }
         check(evoattn_fwd(&p, stream_of(P)), "evoattn_fwd");
+        p.gate = nullptr;
+        p.o_gated = nullptr;
+        return r;
+    }
+    // the gradient of P; that of the output lies at `dout` (slot 2 of the forward's buffer)
+    static Tensor enqueue_gradients(const Call &c, const Tensor &P, const Tensor &mask, const Tensor &bias, const Tensor &aux, void *out, void *dout,
+                                    bool want_dbias, bool want_dmask, Tensor &dbias, Tensor &dmask) {
+        c10::DeviceGuard on(P.device());
+        Tensor DP = P.size(3) == (c.gated ? 4 : 3) ? at::empty_like(P) : at::zeros_like(P);
+        EvoAttnParams p = c.p;
+        Aux(p).place(p, aux);
+        p.q = slot(P, p, 0);
+        p.k = slot(P, p, 1);
+        p.v = slot(P, p, 2);
+        p.mask = mask.defined() ? mask.data_ptr() : nullptr;
+        p.bias = bias.defined() ? bias.data_ptr() : nullptr;
+        p.dout = dout;
+        p.dq = slot(DP, p, 0);
+        p.dk = slot(DP, p, 1);
+        p.dv = slot(DP, p, 2);
+        if (c.gated) {   // slot 2 is the node's own memory: the gradient of the ungated output takes its place
+            p.o = nullptr;
+            p.gate = slot(P, p, 3);
+            p.dgate = slot(DP, p, 3);
+            p.o_gated = out;
+            p.flags |= EVO_FLAG_GATE_DOUT_INPLACE;
+        } else {
+            p.o = out;
+        }
+        enqueue_backward(p, P, bias, want_dbias, want_dmask, dbias, dmask);
+        return DP;
+    }
+
+    static variable_list forward(AutogradContext *ctx, const Tensor &P, OptTensor mask, OptTensor bias, bool gated) {
+        const Run r = enqueue(P, mask, bias, gated);
+        const Call &c = r.c;
+        const Tensor &ob = r.ob, &aux = r.aux;
         Tensor out = ob.select(3, gated ? 1 : 0);
         // `out` is what the backward reads: saved like any output, so that a consumer who changes it in place is told so
         // by autograd's version check.  Slot 2 alone is kept under a version counter of its own: the consumer
         // writes the incoming gradient there in place, which must not look like a change of `out` (the same memory object).
         Tensor grad_slot = ob.variable_data().select(3, 2);
-        ctx->save_for_backward({P, *mask, *bias, aux, out});
+        ctx->save_for_backward({P, *r.mask, *r.bias, aux, out});
         ctx->saved_data["slot"] = grad_slot;
-        p.gate = nullptr;
-        p.o_gated = nullptr;
         ctx->saved_data["call"] = std::string((const char *)&c, sizeof c);
         ctx->mark_non_differentiable({grad_slot});
         ctx->set_materialize_grads(false);   // (no tensor of zeros for the second output's gradient, which nobody has)
@@ -430,30 +474,8 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
             const bool want_dmask = mask.defined() && ctx->needs_input_grad(edge) && mask.is_floating_point();
             if (mask.defined()) ++edge;
             const bool want_dbias = bias.defined() && ctx->needs_input_grad(edge);
-            Tensor DP = P.size(3) == (c.gated ? 4 : 3) ? at::empty_like(P) : at::zeros_like(P);
-            EvoAttnParams p = c.p;
-            Aux(p).place(p, aux);
-            p.q = slot(P, p, 0);
-            p.k = slot(P, p, 1);
-            p.v = slot(P, p, 2);
-            p.mask = mask.defined() ? mask.data_ptr() : nullptr;
-            p.bias = bias.defined() ? bias.data_ptr() : nullptr;
-            p.dout = slot2.data_ptr();
-            p.dq = slot(DP, p, 0);
-            p.dk = slot(DP, p, 1);
-            p.dv = slot(DP, p, 2);
-            if (c.gated) {   // slot 2 is this node's own memory: the gradient of the ungated output takes its place
-                p.o = nullptr;
-                p.gate = slot(P, p, 3);
-                p.dgate = slot(DP, p, 3);
-                p.o_gated = out.data_ptr();
-                p.flags |= EVO_FLAG_GATE_DOUT_INPLACE;
-            } else {
-                p.o = out.data_ptr();
-            }
             Tensor dbias, dmask;
-            enqueue_backward(p, P, bias, want_dbias, want_dmask, dbias, dmask);
-            res[0] = DP;
+            res[0] = enqueue_gradients(c, P, mask, bias, aux, out.data_ptr(), slot2.data_ptr(), want_dbias, want_dmask, dbias, dmask);
             if (want_dmask) res[1] = finish_dmask(dmask, c);
             if (want_dbias) res[2] = finish_dbias(dbias, c);
         }
@@ -688,6 +710,45 @@ Tensor stacked_projection(const Tensor &x, const OptTensor &gate_bias, const std
     return y;
 }
 
+// mean, then 1 / deviation of every row, each on a 16-byte boundary
+Tensor ln_stats(const Tensor &x, int64_t rows) { return at::empty({2 * ((rows + 3) / 4 * 4)}, x.options().dtype(at::kFloat)); }
+const void *ptr_or_null(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+bool ln_ok(const Tensor &x, const Tensor &w, const Tensor &b) {
+    const int dt = evo_dtype(x.scalar_type());
+    if (!plain(x) || !plain_modes() || !x.is_cuda() || x.dim() < 1 || x.numel() == 0 || dt == EVO_NONE || x.size(-1) > INT32_MAX) return false;
+    for (const Tensor *t : {&w, &b})
+        if (t->defined() && (!plain(*t) || t->scalar_type() != x.scalar_type() || t->device() != x.device() || t->dim() != 1 || t->size(0) != x.size(-1)))
+            return false;
+    return evoattn_layernorm_bwd_workspace_bytes(1, (int32_t)x.size(-1), dt) != 0;
+}
+// (x, w, b contiguous)
+Tensor ln_forward(const Tensor &x, const Tensor &w, const Tensor &b, double eps, const Tensor &stats) {
+    c10::DeviceGuard on(x.device());
+    const int64_t cols = x.size(-1), rows = x.numel() / cols;
+    Tensor y = at::empty_like(x);
+    float *mean = (float *)stats.data_ptr();
+    check(evoattn_layernorm_fwd(x.data_ptr(), ptr_or_null(w), ptr_or_null(b), y.data_ptr(), mean, mean + stats.numel() / 2, rows, (int32_t)cols,
+                                evo_dtype(x.scalar_type()), (float)eps, stream_of(x)), "evoattn_layernorm_fwd");
+    return y;
+}
+void ln_backward(const Tensor &dy, const Tensor &x, const Tensor &w, const Tensor &stats, bool need_x, bool need_w, bool need_b, Tensor &dx, Tensor &dw,
+                 Tensor &db) {
+    if (!need_x && !need_w && !need_b) return;
+    c10::DeviceGuard on(x.device());
+    const int64_t cols = x.size(-1), rows = x.numel() / cols;
+    const int dt = evo_dtype(x.scalar_type());
+    Tensor ws;
+    if (need_x) dx = at::empty_like(x);
+    if (need_w) dw = at::empty({cols}, x.options());
+    if (need_b) db = at::empty({cols}, x.options());
+    if (need_w || need_b) ws = scratch(evoattn_layernorm_bwd_workspace_bytes(rows, (int32_t)cols, dt), x);
+    const float *mean = (const float *)stats.data_ptr();
+    check(evoattn_layernorm_bwd(dy.data_ptr(), x.data_ptr(), ptr_or_null(w), mean, mean + stats.numel() / 2, const_cast<void *>(ptr_or_null(dx)),
+                                const_cast<void *>(ptr_or_null(dw)), const_cast<void *>(ptr_or_null(db)), const_cast<void *>(ptr_or_null(ws)),
+                                ws.defined() ? (size_t)ws.numel() : 0, rows, (int32_t)cols, dt, stream_of(x)), "evoattn_layernorm_bwd");
+}
+
 struct LayerNormNode : SavingNode {
     bool has_bias = false;
     std::string name() const override { return "LayerNormBackward"; }
@@ -698,23 +759,9 @@ struct LayerNormNode : SavingNode {
         if (!grads[0].defined()) return out;
         {
             at::AutoDispatchBelowADInplaceOrView guard;
-            const Tensor x = saved[0].unpack(), w = saved[1].unpack(), stats = saved[2].unpack(), dy = grads[0].contiguous();
-            const int64_t cols = x.size(-1), rows = x.numel() / cols;
-            const bool need_x = task_should_compute_output(0), need_w = w.defined() && task_should_compute_output(1),
-                       need_b = has_bias && task_should_compute_output(2);
-            c10::DeviceGuard on(x.device());
-            const int dt = evo_dtype(x.scalar_type());
-            Tensor ws;
-            if (need_x) out[0] = at::empty_like(x);
-            if (need_w) out[1] = at::empty({cols}, x.options());
-            if (need_b) out[2] = at::empty({cols}, x.options());
-            if (need_w || need_b) ws = scratch(evoattn_layernorm_bwd_workspace_bytes(rows, (int32_t)cols, dt), x);
-            const float *mean = (const float *)stats.data_ptr();
-            auto ptr = [](const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; };
-            if (need_x || need_w || need_b)
-                check(evoattn_layernorm_bwd(dy.data_ptr(), x.data_ptr(), ptr(w), mean, mean + (rows + 3) / 4 * 4, ptr(out[0]), ptr(out[1]), ptr(out[2]),
-                                            ptr(ws), ws.defined() ? (size_t)ws.numel() : 0, rows, (int32_t)cols, dt, stream_of(x)),
-                      "evoattn_layernorm_bwd");
+            const Tensor x = saved[0].unpack(), w = saved[1].unpack(), stats = saved[2].unpack();
+            ln_backward(grads[0].contiguous(), x, w, stats, task_should_compute_output(0), w.defined() && task_should_compute_output(1),
+                        has_bias && task_should_compute_output(2), out[0], out[1], out[2]);
         }
         return once_differentiable(std::move(out), rec);
     }
@@ -723,26 +770,15 @@ struct LayerNormNode : SavingNode {
 // LayerNorm over the last dimension through the library's kernels: x and y cross HBM once in the forward, x, dy and dx once in
 // the backward.  None for rows, dtypes or devices that those kernels do not take.
 OptTensor layer_norm(const Tensor &x, const OptTensor &weight, const OptTensor &bias, double eps) {
-    const int dt = evo_dtype(x.scalar_type());
     const Tensor w0 = weight ? *weight : Tensor(), b0 = bias ? *bias : Tensor();
-    if (!plain(x) || !plain_modes() || !x.is_cuda() || x.dim() < 1 || x.numel() == 0 || dt == EVO_NONE || x.size(-1) > INT32_MAX) return std::nullopt;
-    for (const Tensor &t : {w0, b0})
-        if (t.defined() && (!plain(t) || t.scalar_type() != x.scalar_type() || t.device() != x.device() || t.dim() != 1 || t.size(0) != x.size(-1)))
-            return std::nullopt;
-    if (evoattn_layernorm_bwd_workspace_bytes(1, (int32_t)x.size(-1), dt) == 0) return std::nullopt;
-    Tensor y, xc, w, b, stats;
+    if (!ln_ok(x, w0, b0)) return std::nullopt;
+    Tensor y, xc, w, stats;
     {
         at::AutoDispatchBelowADInplaceOrView guard;
-        c10::DeviceGuard on(x.device());
         xc = x.contiguous();
         w = w0.defined() ? w0.contiguous() : Tensor();
-        b = b0.defined() ? b0.contiguous() : Tensor();
-        const int64_t cols = xc.size(-1), rows = xc.numel() / cols, rows4 = (rows + 3) / 4 * 4;
-        y = at::empty_like(xc);
-        stats = at::empty({2 * rows4}, xc.options().dtype(at::kFloat));   // mean, then 1 / deviation, each on a 16-byte boundary
-        float *mean = (float *)stats.data_ptr();
-        check(evoattn_layernorm_fwd(xc.data_ptr(), w.defined() ? w.data_ptr() : nullptr, b.defined() ? b.data_ptr() : nullptr, y.data_ptr(), mean,
-                                    mean + rows4, rows, (int32_t)cols, dt, (float)eps, stream_of(xc)), "evoattn_layernorm_fwd");
+        stats = ln_stats(xc, xc.numel() / xc.size(-1));
+        y = ln_forward(xc, w, b0.defined() ? b0.contiguous() : Tensor(), eps, stats);
     }
     if (SavingNode::wanted(x, w0, b0)) {
         auto node = make_node<LayerNormNode>(x, w0, b0);
@@ -755,6 +791,61 @@ OptTensor layer_norm(const Tensor &x, const OptTensor &weight, const OptTensor &
     return y;
 }
 
+// The pair bias (csrc/pair_bias.hip): contiguous 16-byte aligned operands, and whether the kernels take them.
+struct PairOperands {
+    Tensor z, lw, lb, w;
+    int64_t B, pairs;
+    int32_t C, H;
+    int dt;
+    size_t workspace;
+    PairOperands(const Tensor &z_, const Tensor &lw_, const Tensor &lb_, const Tensor &w_) : z(z_), lw(lw_), lb(lb_), w(w_) {
+        B = z.size(0);
+        pairs = z.size(1) * z.size(2);
+        C = (int32_t)z.size(3);
+        H = (int32_t)w.size(0);
+        dt = evo_dtype(z.scalar_type());
+        workspace = evoattn_pair_bias_workspace_bytes(B, pairs, C, H, dt);
+    }
+    static bool ok(const Tensor &z, const Tensor &lw, const Tensor &lb, const Tensor &w) {
+        if (!plain(z) || !plain_modes() || at::autocast::is_autocast_enabled(at::kCUDA) || !z.is_cuda() || z.dim() != 4 || z.numel() == 0 || !plain(w) ||
+            w.dim() != 2 || w.size(1) != z.size(3) || w.size(1) > 4096 || w.size(0) > 4096)
+            return false;
+        for (const Tensor *t : {&lw, &lb, &w})
+            if (t->defined() && (!plain(*t) || t->scalar_type() != z.scalar_type() || t->device() != z.device())) return false;
+        for (const Tensor *t : {&lw, &lb})
+            if (t->defined() && (t->dim() != 1 || t->size(0) != z.size(3))) return false;
+        return evoattn_pair_bias_workspace_bytes(z.size(0), z.size(1) * z.size(2), (int32_t)z.size(3), (int32_t)w.size(0), evo_dtype(z.scalar_type())) != 0;
+    }
+    static Tensor ready(const Tensor &t) {
+        Tensor c = t.defined() ? t.contiguous() : t;
+        return c.defined() && (uintptr_t)c.data_ptr() % 16 ? c.clone() : c;
+    }
+    Tensor forward(double eps, Tensor &stats) const {
+        c10::DeviceGuard on(z.device());
+        Tensor out = at::empty({B, 1, H, z.size(1), z.size(2)}, z.options());
+        stats = at::empty({2 * B * pairs}, z.options().dtype(at::kFloat));   // mean, then 1 / deviation
+        float *mean = (float *)stats.data_ptr();
+        check(evoattn_pair_bias_fwd(z.data_ptr(), ptr_or_null(lw), ptr_or_null(lb), w.data_ptr(), out.data_ptr(), mean, mean + B * pairs, B, pairs, C, H, dt,
+                                    (float)eps, stream_of(z)), "evoattn_pair_bias_fwd");
+        return out;
+    }
+    // dparams [2 + H, C]: LayerNorm weight, LayerNorm bias, projection
+    void backward(const Tensor &dbias, const Tensor &stats, bool need_z, bool need_params, Tensor &dz, Tensor &dparams) const {
+        if (!need_z && !need_params) return;
+        c10::DeviceGuard on(z.device());
+        Tensor ws;
+        if (need_z) dz = at::empty_like(z);
+        if (need_params) {
+            dparams = at::empty({2 + H, C}, z.options());
+            ws = scratch(workspace, z);
+        }
+        const float *mean = (const float *)stats.data_ptr();
+        check(evoattn_pair_bias_bwd(dbias.data_ptr(), z.data_ptr(), ptr_or_null(lw), ptr_or_null(lb), w.data_ptr(), mean, mean + B * pairs,
+                                    const_cast<void *>(ptr_or_null(dz)), const_cast<void *>(ptr_or_null(dparams)), const_cast<void *>(ptr_or_null(ws)),
+                                    ws.defined() ? (size_t)ws.numel() : 0, B, pairs, C, H, dt, stream_of(z)), "evoattn_pair_bias_bwd");
+    }
+};
+
 struct PairBiasNode : SavingNode {
     std::string name() const override { return "PairBiasBackward"; }
     // results: z, the LayerNorm's weight and bias, the projection's weight
@@ -765,26 +856,13 @@ struct PairBiasNode : SavingNode {
         if (!grads[0].defined()) return out;
         {
             at::AutoDispatchBelowADInplaceOrView guard;
-            const Tensor z = saved[0].unpack(), lw = saved[1].unpack(), lb = saved[2].unpack(), w = saved[3].unpack(), stats = saved[4].unpack();
-            const Tensor db = grads[0].contiguous();
-            const int64_t B = z.size(0), pairs = z.size(1) * z.size(2), rows = B * pairs;
-            const int32_t C = (int32_t)z.size(3), H = (int32_t)w.size(0);
-            const int dt = evo_dtype(z.scalar_type());
-            c10::DeviceGuard on(z.device());
-            Tensor ws, dparams;
-            if (task_should_compute_output(0)) out[0] = at::empty_like(z);
-            if (task_should_compute_output(1) || task_should_compute_output(2) || task_should_compute_output(3)) {
-                dparams = at::empty({2 + H, C}, z.options());
-                ws = scratch(evoattn_pair_bias_workspace_bytes(B, pairs, C, H, dt), z);
-            }
-            const float *mean = (const float *)stats.data_ptr();
-            auto ptr = [](const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; };
-            if (out[0].defined() || dparams.defined())
-                check(evoattn_pair_bias_bwd(db.data_ptr(), z.data_ptr(), ptr(lw), ptr(lb), w.data_ptr(), mean, mean + rows, ptr(out[0]), ptr(dparams),
-                                            ptr(ws), ws.defined() ? (size_t)ws.numel() : 0, B, pairs, C, H, dt, stream_of(z)), "evoattn_pair_bias_bwd");
-            if (task_should_compute_output(1)) out[1] = dparams.select(0, 0);
-            if (task_should_compute_output(2)) out[2] = dparams.select(0, 1);
-            if (task_should_compute_output(3)) out[3] = dparams.narrow(0, 2, H);
+            const PairOperands o(saved[0].unpack(), saved[1].unpack(), saved[2].unpack(), saved[3].unpack());
+            const bool lw = task_should_compute_output(1), lb = task_should_compute_output(2), w = task_should_compute_output(3);
+            Tensor dparams;
+            o.backward(grads[0].contiguous(), saved[4].unpack(), task_should_compute_output(0), lw || lb || w, out[0], dparams);
+            if (lw) out[1] = dparams.select(0, 0);
+            if (lb) out[2] = dparams.select(0, 1);
+            if (w) out[3] = dparams.narrow(0, 2, o.H);
         }
         return once_differentiable(std::move(out), rec);
     }
@@ -793,44 +871,159 @@ struct PairBiasNode : SavingNode {
 // LayerNorm of the pair representation, its projection to heads and the permute to [B,1,H,N,N] in one pass.  None for what
 // the kernels do not take.
 OptTensor pair_bias(const Tensor &z, const OptTensor &ln_weight, const OptTensor &ln_bias, double eps, const Tensor &weight) {
-    const int dt = evo_dtype(z.scalar_type());
-    const Tensor lw0 = ln_weight ? *ln_weight : Tensor(), lb0 = ln_bias ? *ln_bias : Tensor();
-    if (!plain(z) || !plain_modes() || at::autocast::is_autocast_enabled(at::kCUDA) || !z.is_cuda() || z.dim() != 4 || z.numel() == 0 || !plain(weight) || weight.dim() != 2 ||
-        weight.size(1) != z.size(3) || weight.size(1) > 4096 || weight.size(0) > 4096)
-        return std::nullopt;
-    for (const Tensor &t : {lw0, lb0, weight})
-        if (t.defined() && (!plain(t) || t.scalar_type() != z.scalar_type() || t.device() != z.device())) return std::nullopt;
-    for (const Tensor &t : {lw0, lb0})
-        if (t.defined() && (t.dim() != 1 || t.size(0) != z.size(3))) return std::nullopt;
-    const int64_t B = z.size(0), pairs = z.size(1) * z.size(2), rows = B * pairs;
-    const int32_t C = (int32_t)z.size(3), H = (int32_t)weight.size(0);
-    if (evoattn_pair_bias_workspace_bytes(B, pairs, C, H, dt) == 0) return std::nullopt;
-    Tensor out, zc, lw, lb, w, stats;
+    const Tensor lw = ln_weight ? *ln_weight : Tensor(), lb = ln_bias ? *ln_bias : Tensor();
+    if (!PairOperands::ok(z, lw, lb, weight)) return std::nullopt;
+    std::optional<PairOperands> o;
+    Tensor out, stats;
     {
         at::AutoDispatchBelowADInplaceOrView guard;
-        c10::DeviceGuard on(z.device());
-        zc = z.contiguous();
-        w = weight.contiguous();
-        lw = lw0.defined() ? lw0.contiguous() : Tensor();
-        lb = lb0.defined() ? lb0.contiguous() : Tensor();
-        auto aligned = [](const Tensor &t) { return !t.defined() || (uintptr_t)t.data_ptr() % 16 == 0; };
-        if (!aligned(zc) || !aligned(w) || !aligned(lw) || !aligned(lb)) return std::nullopt;
-        out = at::empty({B, 1, H, z.size(1), z.size(2)}, zc.options());
-        stats = at::empty({2 * rows}, zc.options().dtype(at::kFloat));   // mean, then 1 / deviation
-        float *mean = (float *)stats.data_ptr();
-        check(evoattn_pair_bias_fwd(zc.data_ptr(), lw.defined() ? lw.data_ptr() : nullptr, lb.defined() ? lb.data_ptr() : nullptr, w.data_ptr(),
-                                    out.data_ptr(), mean, mean + rows, B, pairs, C, H, dt, (float)eps, stream_of(zc)), "evoattn_pair_bias_fwd");
+        o.emplace(PairOperands::ready(z), PairOperands::ready(lw), PairOperands::ready(lb), PairOperands::ready(weight));
+        out = o->forward(eps, stats);
     }
-    if (SavingNode::wanted(z, lw0, lb0, weight)) {
-        auto node = make_node<PairBiasNode>(z, lw0, lb0, weight);
+    if (SavingNode::wanted(z, lw, lb, weight)) {
+        auto node = make_node<PairBiasNode>(z, lw, lb, weight);
         torch::autograd::set_history(out, node);
-        node->save(zc);
-        node->save(lw);
-        node->save(lb);
-        node->save(w);
-        node->save(stats);
+        for (const Tensor *t : {&o->z, &o->lw, &o->lb, &o->w, &stats}) node->save(*t);
     }
     return out;
+}
+
+// ------------------------------------------------------------------ the whole block
+
+// Inputs of the block in the order of its node's results.
+enum BlockInput { kM, kZ, kNormMW, kNormMB, kQ, kK, kV, kG, kGBias, kO, kOBias, kNormZW, kNormZB, kZW, kBlockInputs };
+
+// One node for what the layers above do in five, with the tensors between them its own: a training step of a small block
+// spent a third of its host time between those nodes (the engine's bookkeeping, views, the interpreter).
+struct BlockNode : SavingNode {
+    Call c{};
+    // saved: the inputs, then
+    enum { kX = kBlockInputs, kStatsM, kP, kMask, kBias, kAux, kOut, kStatsZ, kSaved };
+    std::string name() const override { return "GatedAttentionBlockBackward"; }
+    variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        const bool rec = at::GradMode::is_enabled();
+        variable_list out(kBlockInputs);
+        if (!grads[0].defined()) return out;
+        {
+            at::AutoDispatchBelowADInplaceOrView guard;
+            Tensor t[kSaved];
+            for (int i = 0; i < kSaved; ++i) t[i] = saved[i].unpack();
+            bool want[kBlockInputs], inner = false;
+            for (int i = 0; i < kBlockInputs; ++i) {
+                want[i] = t[i].defined() && task_should_compute_output(i);
+                inner |= want[i] && i != kO && i != kOBias;
+            }
+            Tensor dy = grads[0].scalar_type() == t[kM].scalar_type() ? as_rows(grads[0]) : as_rows(grads[0].to(t[kM].scalar_type()));
+            const int64_t rows = dy.size(0), W = t[kP].size(3), hd = t[kP].size(4) * t[kP].size(5);
+            const Tensor slots = t[kOut].view({rows, W * hd}), o = slots.narrow(1, (c.gated ? 1 : 0) * hd, hd);
+            if (want[kO] || want[kOBias]) {
+                std::tie(out[kO], out[kOBias]) = lin_weight_grad(dy, o, want[kOBias]);
+                if (!want[kO]) out[kO] = Tensor();
+            }
+            if (inner) {
+                Tensor dout = slots.narrow(1, 2 * hd, hd), dbias, dmask;
+                if (!lin_input_grad(dy, {t[kO]}, dout)) at::mm_out(dout, dy, t[kO]);
+                const bool z_side = want[kZ] || want[kNormZW] || want[kNormZB] || want[kZW];
+                const Tensor DP = SlotAttention::enqueue_gradients(c, t[kP], t[kMask], t[kBias], t[kAux], o.data_ptr(), dout.data_ptr(), z_side, false, dbias,
+                                                                   dmask);
+                if (z_side) {
+                    Tensor dparams;
+                    PairOperands(t[kZ], t[kNormZW], t[kNormZB], t[kZW])
+                        .backward(dbias, t[kStatsZ], want[kZ], want[kNormZW] || want[kNormZB] || want[kZW], out[kZ], dparams);
+                    if (want[kNormZW]) out[kNormZW] = dparams.select(0, 0);
+                    if (want[kNormZB]) out[kNormZB] = dparams.select(0, 1);
+                    if (want[kZW]) out[kZW] = dparams.narrow(0, 2, dparams.size(0) - 2);
+                }
+                const Tensor dp2 = DP.view({rows, W * hd}), x2 = as_rows(t[kX]);
+                bool weights = want[kGBias];
+                for (int i = 0; i < W; ++i) weights |= want[kQ + i];
+                if (weights) {
+                    auto [dw, db] = lin_weight_grad(dp2, x2, want[kGBias]);
+                    for (int i = 0; i < W; ++i)
+                        if (want[kQ + i]) out[kQ + i] = dw.narrow(0, i * hd, hd);
+                    if (want[kGBias]) out[kGBias] = db.narrow(0, (W - 1) * hd, hd);
+                }
+                if (want[kM] || want[kNormMW] || want[kNormMB]) {
+                    Tensor dx = at::empty_like(x2);
+                    std::vector<Tensor> w(t + kQ, t + kQ + W);
+                    if (!lin_input_grad(dp2, w, dx)) at::mm_out(dx, dp2, at::cat(w, 0));
+                    ln_backward(dx, t[kM], t[kNormMW], t[kStatsM], want[kM], want[kNormMW], want[kNormMB], out[kM], out[kNormMW], out[kNormMB]);
+                }
+            }
+        }
+        return once_differentiable(std::move(out), rec);
+    }
+};
+
+// The block around the attention, in.size() == kBlockInputs (those that a block does not have undefined); `keep` [B,S,N], 1 where a
+// key counts.  None where some part of it does not take the call.
+OptTensor block(const std::vector<OptTensor> &in, const OptTensor &keep, int64_t heads, double eps_m, double eps_z, double inf) {
+    Tensor t[kBlockInputs];
+    TORCH_CHECK(in.size() == kBlockInputs, "block: wrong number of inputs");
+    for (int i = 0; i < kBlockInputs; ++i)
+        if (in[i]) t[i] = *in[i];
+    const Tensor &m = t[kM];
+    if (!plain(m) || m.dim() != 4 || !m.is_cuda() || m.numel() == 0 || at::autocast::is_autocast_enabled(at::kCUDA)) return std::nullopt;
+    const bool gated = t[kG].defined();
+    const int W = gated ? 4 : 3;
+    if (!t[kQ].defined() || t[kQ].dim() != 2 || !t[kK].defined() || !t[kV].defined() || !t[kO].defined()) return std::nullopt;
+    const int64_t B = m.size(0), S = m.size(1), N = m.size(2), hd = t[kQ].size(0), D = hd / heads, rows = B * S * N;
+    if (hd != heads * D || !head_dim_built(D) || B > INT32_MAX || S > INT32_MAX || N > INT32_MAX || heads > INT32_MAX) return std::nullopt;
+    if (!ln_ok(m, t[kNormMW], t[kNormMB])) return std::nullopt;
+    const std::vector<Tensor> w(t + kQ, t + kQ + W);
+    if (m.size(3) != t[kQ].size(1) || !m.is_contiguous() || !lin_ok(m.view({rows, m.size(3)}), w) || !plain(t[kO]) || t[kO].dim() != 2 ||
+        t[kO].size(1) != hd || t[kO].scalar_type() != m.scalar_type() || t[kO].device() != m.device())
+        return std::nullopt;
+    if (keep && (!plain(*keep) || keep->requires_grad() || keep->dim() != 3 || keep->size(0) != B || keep->size(1) != S || keep->size(2) != N ||
+                 keep->device() != m.device()))
+        return std::nullopt;
+    if (t[kZ].defined() && (t[kZ].scalar_type() != m.scalar_type() || t[kZ].device() != m.device() || t[kZW].size(0) != heads ||
+                            !PairOperands::ok(t[kZ], t[kNormZW], t[kNormZB], t[kZW]) || t[kZ].size(0) != B || t[kZ].size(1) != N || t[kZ].size(2) != N))
+        return std::nullopt;
+    Tensor y, x, stats_m, stats_z, P;
+    SlotAttention::Run r;
+    {
+        at::AutoDispatchBelowADInplaceOrView guard;
+        c10::DeviceGuard on(m.device());
+        for (int i : {kNormMW, kNormMB}) t[i] = t[i].defined() ? t[i].contiguous() : t[i];
+        stats_m = ln_stats(m, rows);
+        x = ln_forward(m, t[kNormMW], t[kNormMB], eps_m, stats_m);
+        P = lin_forward(as_rows(x), w, t[kGBias]);
+        if (!P.defined()) return std::nullopt;
+        P = P.view({B, S, N, W, heads, D});
+        OptTensor mask, bias;
+        if (keep) {
+            const Tensor k = keep->to(at::kFloat).contiguous();
+            mask = at::empty({B, S, 1, 1, N}, k.options());
+            check(evoattn_keep_mask((const float *)k.data_ptr(), (float *)mask->data_ptr(), rows, (float)inf, stream_of(k)), "evoattn_keep_mask");
+        }
+        if (t[kZ].defined()) {
+            for (int i : {kZ, kNormZW, kNormZB, kZW}) t[i] = PairOperands::ready(t[i]);
+            bias = PairOperands(t[kZ], t[kNormZW], t[kNormZB], t[kZW]).forward(eps_z, stats_z);
+        }
+        r = SlotAttention::enqueue(P, mask, bias, gated);
+        const Tensor o = r.ob.view({rows, W * hd}).narrow(1, (gated ? 1 : 0) * hd, hd);
+        y = lin_forward(o, {t[kO]}, t[kOBias]);
+        if (!y.defined()) y = at::linear(o, t[kO], t[kOBias].defined() ? OptTensor(t[kOBias]) : OptTensor());
+        y = y.view({B, S, N, t[kO].size(0)});
+    }
+    bool wanted = false;
+    variable_list inputs;
+    for (int i = 0; i < kBlockInputs; ++i) {
+        inputs.push_back(in[i] ? *in[i] : Tensor());
+        wanted |= SavingNode::wanted(inputs.back());
+    }
+    if (wanted) {
+        std::shared_ptr<BlockNode> node(new BlockNode(), torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(inputs));
+        node->c = r.c;
+        torch::autograd::set_history(y, node);
+        node->saved.reserve(BlockNode::kSaved);
+        for (const Tensor &i : t) node->save(i);
+        for (const Tensor &i : {x, stats_m, P, *r.mask, *r.bias, r.aux, r.ob, stats_z}) node->save(i);
+    }
+    return y;
 }
 
 }  // namespace
@@ -845,4 +1038,5 @@ PYBIND11_MODULE(_host, m) {
     m.def("stacked_projection", &stacked_projection, no_gil, py::arg("x"), py::arg("gate_bias"), py::arg("weights"));
     m.def("layer_norm", &layer_norm, no_gil, py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("eps"));
     m.def("pair_bias", &pair_bias, no_gil, py::arg("z"), py::arg("ln_weight"), py::arg("ln_bias"), py::arg("eps"), py::arg("weight"));
+    m.def("block", &block, no_gil, py::arg("inputs"), py::arg("keep"), py::arg("heads"), py::arg("eps_m"), py::arg("eps_z"), py::arg("inf"));
 }

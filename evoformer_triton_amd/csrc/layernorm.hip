@@ -358,6 +358,10 @@ static int colsum_launch(const void *a, void *out, float *part, int64_t rows, in
     return hip_rc();
 }
 
+__global__ void __launch_bounds__(256) keep_mask_kernel(const float *__restrict__ keep, float *__restrict__ out, int64_t n, float inf) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) out[i] = inf * (keep[i] - 1.0f);
+}
+
 int launch_column_reduce(const float *part, int blocks, int cols, void *out, int dtype, hipStream_t st) {
     const unsigned grid = (cols + kLnRedCols - 1) / kLnRedCols;
     if (dtype == EVO_BF16) ln_reduce_kernel<bf16_t><<<grid, kLnRedCols * kLnRedSlices, 0, st>>>(part, blocks, 1, cols, (bf16_t *)out, (bf16_t *)nullptr);
@@ -407,6 +411,15 @@ int evoattn_layernorm_bwd(const void *dy, const void *x, const void *gamma, cons
         case EVO_F16: return ln_bwd_launch<f16_t>(dy, x, gamma, mean, rstd, dx, dgamma, dbeta, part, rows, cols, st);
         default: return ln_bwd_launch<float>(dy, x, gamma, mean, rstd, dx, dgamma, dbeta, part, rows, cols, st);
     }
+}
+
+int evoattn_keep_mask(const float *keep, float *out, int64_t n, float inf, void *hip_stream) {
+    using namespace evo;
+    if (n < 0 || (n && (!keep || !out))) return EVO_EINVAL;
+    if (n == 0) return EVO_OK;
+    const int64_t want = (n + 255) / 256;
+    keep_mask_kernel<<<(unsigned)(want < 2048 ? want : 2048), 256, 0, (hipStream_t)hip_stream>>>(keep, out, n, inf);
+    return hip_rc();
 }
 
 size_t evoattn_colsum_workspace_bytes(int64_t rows, int32_t cols, int32_t dtype) {

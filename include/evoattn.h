@@ -237,6 +237,9 @@ size_t evoattn_colsum_workspace_bytes(int64_t rows, int32_t cols, int32_t dtype)
 int evoattn_colsum(const void *a, int64_t row_stride, void *out, void *workspace, size_t workspace_bytes, int64_t rows,
                    int32_t cols, int32_t dtype, void *hip_stream);
 
+/* out[i] = inf * (keep[i] - 1), fp32: the additive mask of a keep-mask (1 where a key counts). */
+int evoattn_keep_mask(const float *keep, float *out, int64_t n, float inf, void *hip_stream);
+
 /* The Linear layers of the block around the attention (no counterpart in the reference's operator), 16-bit, on the matrix
  * cores with fp32 sums.  The weight [n, k] may be `nw` (1 to 4) matrices of w_rows rows each, stacked.
  *   fwd  y [rows, n] = x [rows, k] w^T, plus bias on outputs bias_from .. n - 1 (bias may be NULL)
