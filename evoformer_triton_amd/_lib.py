@@ -22,6 +22,7 @@ EVO_FLAG_PER_PROBLEM = 16
 EVO_FLAG_GATE_DOUT_INPLACE = 0x80
 EVO_FLAG_DEBUG_OTHER_WIDTH = 0x100
 EVO_FLAG_DEBUG_NO_KV_RING = 0x200
+EVO_FLAG_FORWARD_ONLY = 0x8000
 EVO_FLAG_DEBUG_FWD_BIAS_TILES = 0x400
 EVO_FLAG_DEBUG_BIAS_TILES = 0x800
 EVO_FLAG_DEBUG_NO_DQ_WIDE = 0x1000

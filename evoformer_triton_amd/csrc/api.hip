@@ -383,8 +383,15 @@ int evoattn_check(const EvoAttnParams *p, int pass) {
     return EVO_OK;
 }
 
+// Whether the forward is the one whose waves split a row's keys (mfma_stream.hip): single sequences without a backward, where
+// one workgroup per 128 queries leaves some of the CUs without any.
+static bool split_fwd_ok(const EvoAttnParams &p) {
+    return p.D >= 32 && p.S == 1 && p.N <= kSplitFwdMaxN && (p.flags & EVO_FLAG_FORWARD_ONLY) && !(p.flags & EVO_FLAG_PER_PROBLEM) && (int64_t)p.B * p.H * ((p.N + 127) / 128) < 256;
+}
+
 size_t evoattn_prep_bytes(const EvoAttnParams *p) {
     if (!p || p->B <= 0 || p->S <= 0 || p->N <= 0 || p->H <= 0) return 0;
+    if (split_fwd_ok(*p) && mfma_ok(*p, EVO_PASS_FWD)) return 0;
     return prep_layout(*p).total;
 }
 
@@ -457,7 +464,7 @@ const char *evoattn_kernels(const EvoAttnParams *p, int pass) {
     if (!p) return "invalid";
     if (f32_ok(*p, pass)) return pass == EVO_PASS_FWD ? "f32_fwd" : p->dbias ? "f32_dq+f32_dbias,f32_dkdv" : "f32_dq,f32_dkdv";
     if (!mfma_ok(*p, pass)) return "generic";
-    if (pass == EVO_PASS_FWD) return fwd_ring_ok(*p) ? "mfma_fwd_ring" : "mfma_fwd";
+    if (pass == EVO_PASS_FWD) return split_fwd_ok(*p) ? "split_fwd" : fwd_ring_ok(*p) ? "mfma_fwd_ring" : "mfma_fwd";
     const bool kvr = kv_ring_ok(*p);
     if (dq_split_ok(*p)) return kvr ? "mfma_dq_wide+mfma_dbias,mfma_dkdv_ring" : "mfma_dq_wide+mfma_dbias,mfma_dkdv";
     if (dq_wide_ok(*p)) return kvr ? "mfma_dq_wide,mfma_dkdv_ring" : "mfma_dq_wide,mfma_dkdv";
@@ -482,6 +489,7 @@ int evoattn_fwd(const EvoAttnParams *p, void *hip_stream) {
     hipStream_t st = (hipStream_t)hip_stream;
     if (f32_ok(*p, EVO_PASS_FWD)) return launch_f32_fwd(*p, st);
     if (!mfma_ok(*p, EVO_PASS_FWD)) return launch_generic_fwd(*p, st);
+    if (split_fwd_ok(*p)) return launch_split_fwd(*p, st);   // (needs no `prep`)
     if ((rc = check_prep(*p))) return rc;
     return fwd_launches(*p, st);
 }

@@ -53,6 +53,18 @@ EVO_ROUTE(dqw)
 EVO_ROUTE(dbias)
 #undef EVO_ROUTE
 
+int launch_split_fwd_d32(const EvoAttnParams &, hipStream_t);
+int launch_split_fwd_d64(const EvoAttnParams &, hipStream_t);
+int launch_split_fwd_d128(const EvoAttnParams &, hipStream_t);
+int launch_split_fwd(const EvoAttnParams &p, hipStream_t st) {
+    switch (p.D) {
+        case 32: return launch_split_fwd_d32(p, st);
+        case 64: return launch_split_fwd_d64(p, st);
+        case 128: return launch_split_fwd_d128(p, st);
+    }
+    return EVO_EUNSUPPORTED;
+}
+
 int mfma_fwdr_max_n(int D) {
     switch (D) {
         case 8: return mfma_fwdr_max_n_d8();

@@ -306,6 +306,8 @@ OptTensor attention(const Tensor &Q, const Tensor &K, const Tensor &V, OptTensor
 
     OptTensor mask_in = mask, bias_in = bias;
     const Tensor mask0 = mask ? *mask : Tensor(), bias0 = bias ? *bias : Tensor(), gate0 = gated ? *gate : Tensor();
+    const bool wanted = SavingNode::wanted(Q, K, V, mask0, bias0, gate0);
+    if (!wanted) p.flags |= EVO_FLAG_FORWARD_ONLY;
     Tensor q, k, v, g, o, aux;
     {
         at::AutoDispatchBelowADInplaceOrView guard;
@@ -330,7 +332,7 @@ OptTensor attention(const Tensor &Q, const Tensor &K, const Tensor &V, OptTensor
         }
         if (evoattn_fwd(&p, stream_of(q)) != EVO_OK) return std::nullopt;
     }
-    if (SavingNode::wanted(Q, K, V, mask0, bias0, gate0)) {
+    if (wanted) {
         auto node = make_node<AttentionNode>(Q, K, V, mask0, bias0, gate0);
         node->c = c;
         node->c.p.gate = nullptr;

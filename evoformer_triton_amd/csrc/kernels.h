@@ -19,6 +19,8 @@ int launch_mask_shift(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 
 int launch_prep(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_fwd(const EvoAttnParams &p, const Extra &e, hipStream_t st);
+constexpr int kSplitFwdMaxN = 4096;   // (its mask row lies in LDS)
+int launch_split_fwd(const EvoAttnParams &p, hipStream_t st);  // the keys of a row split over waves; reads mask and bias as given
 int launch_mfma_fwdr(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int mfma_fwdr_max_n(int D);  // largest N the chunk-of-rows forward takes, 0 for a head dim it is not built for
 int launch_mfma_dq(const EvoAttnParams &p, const Extra &e, hipStream_t st);

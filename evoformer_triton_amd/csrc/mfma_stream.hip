@@ -335,6 +335,231 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3
     }
 }
 
+// ------------------------------------------------------------------ forward of few problems
+
+// A call whose problems leave most of the chip idle is bound by the chain of one wave: in stream_fwd a wave takes 2.3 us per 64
+// keys of its row, one after the other (16 problems of 128 keys at D = 64: 8.3 us, of 512 keys: 22 us).  Here a workgroup's four
+// waves share 32 queries and split the keys, every fourth tile each, and their partial sums meet in LDS.  A wave needs nobody
+// until then: K comes from memory into the operand's registers, V by the load path into LDS of the wave's own, the next
+// tile's on their way while one is computed on, and no barrier.  The mask is read as given (its largest entry by
+// every wave), so the prep kernel has nothing to do for this one, and a call without a backward skips it.  16 problems,
+// D = 64, fp32 bias, prep and forward before / this: 128 keys 10.7 / 6.7 us, 256 15.4 / 8.1, 512 26.6 / 11.6.  It ends where one
+// workgroup per 128 queries has the chip full: 252 of those 30.5 / 29.6 us.
+// BF: 0 no bias, 1 fp32, 2 in the dtype of q; read as given, four at a time where the rows allow it.
+template <int D>
+struct SplitFwd {
+    static constexpr int TILE = 32 * D * 2, V_BYTES = 4 * 2 * TILE, O_BYTES = 4 * D * 32 * 4, BYTES = (V_BYTES > O_BYTES ? V_BYTES : O_BYTES) + 4 * 2 * 32 * 4;
+};
+
+// mask entries (additive form) of keys j0 + 64 i, i < 8, of one row; keys past the end repeat the last.  (Asked for per
+// kind, so that the eight loads are under way together.)
+__device__ __forceinline__ void mask8(const EvoAttnParams &p, int64_t off, int j0, float (&v)[8]) {
+    int64_t at[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) at[i] = off + min(j0 + 64 * i, p.N - 1);
+    if (p.mask_kind == EVO_MASK_BOOL) {
+        uint8_t x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = ((const uint8_t *)p.mask)[at[i]];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = x[i] ? 0.0f : -FLT_MAX;
+    } else if (p.mask_kind == EVO_MASK_F32) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = ((const float *)p.mask)[at[i]];
+    } else {
+        unsigned short x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = ((const unsigned short *)p.mask)[at[i]];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            v[i] = p.mask_kind == EVO_MASK_BF16 ? (float)__builtin_bit_cast(bf16_t, x[i]) : (float)__builtin_bit_cast(f16_t, x[i]);
+    }
+}
+
+template <typename T, int D, int BF>
+__global__ void __launch_bounds__(256, D == 32 ? 3 : D == 64 ? 2 : 1) split_fwd(EvoAttnParams p, bool vec) {
+    typedef StreamGeo<D> G;
+    typedef SplitFwd<D> R;
+    typedef typename Mfma<T>::v8 v8;
+    constexpr int KSD = D / 16, DT = D / 32, PIECES = R::TILE / 1024, RPP = 1024 / G::ROW;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    float *stats = reinterpret_cast<float *>(lds + R::BYTES - 4 * 2 * 32 * 4);   // [wave][m, l][query]
+    float *masks = reinterpret_cast<float *>(lds + R::BYTES);                    // [key], not below the floor
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, g = lane >> 5;
+    const int NT = (p.N + 31) / 32;
+    const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+    const Prob pr = walk_problem(p, lid / NT);
+    const int q0 = (lid % NT) * 32, qrow = min(q0 + li, p.N - 1), sn = (int)p.stride_n;
+    const T *K = (const T *)p.k + pr.base, *V = (const T *)p.v + pr.base;
+    const int valid = ((p.N - 1) * sn + D) * 2;
+    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void *)V, 0, valid, 0x00020000);
+    const int64_t bias_row = (int64_t)(p.bias_stride_b ? pr.b : 0) * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h + (int64_t)qrow * p.bias_stride_row;
+    unsigned char *vbuf = lds + wave * 2 * R::TILE;
+
+    struct Tile {
+        v8 k[KSD];
+        f32x16 bias;
+    };
+    auto fetch = [&](int t, Tile &d) {   // keys 32 t ..; V to the buffer of the parity of t / 4
+        const int k0 = t * 32;
+        unsigned char *dst = vbuf + ((t >> 2) & 1) * R::TILE;
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int r = i * RPP + lane / G::C, c = (lane % G::C) ^ G::x(r);
+            dma16(vrs, dst + i * 1024, min(k0 + r, p.N - 1) * sn * 2 + c * 16);
+        }
+        const T *krow = K + (int64_t)min(k0 + li, p.N - 1) * sn + g * 8;
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) d.k[ks] = ld8(krow + ks * 16);
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+            const int key = k0 + 8 * rr + 4 * g;
+            if (BF == 1 && vec) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>((const float *)p.bias + bias_row + min(key, p.N - 4));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d.bias[4 * rr + i] = v[i];
+            } else if (BF == 2 && vec) {
+                const typename Mfma<T>::v4 v = *reinterpret_cast<const typename Mfma<T>::v4 *>((const T *)p.bias + bias_row + min(key, p.N - 4));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d.bias[4 * rr + i] = (float)v[i];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int kk = min(key + i, p.N - 1);
+                if (BF == 1 && !vec) d.bias[4 * rr + i] = ((const float *)p.bias)[bias_row + kk];
+                if (BF == 2 && !vec) d.bias[4 * rr + i] = (float)((const T *)p.bias)[bias_row + kk];
+            }
+        }
+    };
+    Tile next;
+    if (wave < NT) fetch(wave, next);
+    v8 qf[KSD];
+#pragma unroll
+    for (int ks = 0; ks < KSD; ++ks) qf[ks] = ld8((const T *)p.q + pr.base + (int64_t)qrow * sn + ks * 16 + g * 8);
+    // The mask into LDS (every wave all of it, the same values: no wave waits for another), and its largest entry: in a row
+    // masked throughout the scores are the mask alone, relative to that (prep.hip).
+    float mx = -INFINITY;
+    if (p.mask_kind != EVO_MASK_NONE) {   // uniform
+        const int64_t off = (int64_t)pr.b * p.mask_stride_b + (int64_t)pr.s * p.mask_stride_s;
+        for (int j0 = 0; j0 < NT * 32; j0 += 512) {
+            float v[8];
+            mask8(p, off, j0 + lane, v);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int j = j0 + lane + 64 * i;
+                v[i] = j < p.N ? fmaxf(v[i], kMaskFloor) : kMaskFloor;
+                mx = fmaxf(mx, v[i]);
+                if (j < NT * 32) masks[j] = v[i];
+            }
+        }
+        mx = wave_max(mx);
+    } else {
+        for (int j = lane; j < NT * 32; j += 64) masks[j] = j < p.N ? 0.0f : kMaskFloor;
+    }
+    const bool dead = p.mask_kind != EVO_MASK_NONE && mx < kShiftThreshold;
+    const float c = dead ? 0.0f : p.scale * kLog2e, bmul = dead ? 0.0f : kLog2e, shift = dead ? mx : 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < KSD; ++ks) qf[ks] = dead ? zero8<T>() : scaled8<T>(qf[ks], c);
+
+    float m = -INFINITY, l = 0.0f;
+    f32x16 o[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
+    for (int t = wave; t < NT; t += 4) {
+        const Tile now = next;
+        wait_loads();   // (V of this tile)
+        if (t + 4 < NT) fetch(t + 4, next);
+        f32x16 a;
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+            const f32x4 mk = *reinterpret_cast<const f32x4 *>(masks + 32 * t + 8 * rr + 4 * g);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float mask = 32 * t + 8 * rr + 4 * g + i < p.N ? fmaxf((mk[i] - shift) * kLog2e, kMaskFloor) : kMaskFloor;
+                a[4 * rr + i] = BF ? now.bias[4 * rr + i] * bmul + mask : mask;
+            }
+        }
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) a = Mfma<T>::mma(now.k[ks], qf[ks], a);
+        float x = a[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) x = fmaxf(x, a[r]);
+        const unsigned u = __float_as_uint(x);
+        auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        const float mn = fmaxf(m, fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]))), alpha = fast_exp2(m - mn);
+        m = mn;
+        float s = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            a[r] = fast_exp2(a[r] - m);
+            s += a[r];
+        }
+        l = l * alpha + s;
+        v8 pf[2];
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pf[ts][i] = (T)a[8 * ts + i];
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+        const unsigned char *vt = vbuf + ((t >> 2) & 1) * R::TILE;
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] = Mfma<T>::mma(transposed<T, D>(vt, 0, ts, dt, lane), pf[ts], o[dt]);
+    }
+    l += __shfl_xor(l, 32);
+
+    // the waves' parts: [wave][d][query]
+    __syncthreads();
+    float *part = reinterpret_cast<float *>(lds);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[(wave * D + dt * 32 + crow(r, g)) * 32 + li] = o[dt][r];
+    if (g == 0) {
+        stats[(wave * 2) * 32 + li] = m;
+        stats[(wave * 2 + 1) * 32 + li] = l;
+    }
+    __syncthreads();
+    const int q = threadIdx.x & 31, d0 = (threadIdx.x >> 5) * (D / 8);
+    float w[4], top = -INFINITY, sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) top = fmaxf(top, stats[(i * 2) * 32 + q]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        w[i] = fast_exp2(stats[(i * 2) * 32 + q] - top);
+        sum += w[i] * stats[(i * 2 + 1) * 32 + q];
+    }
+    if (q0 + q >= p.N) return;
+    if (threadIdx.x < 32) p.lse[pr.row0 + q0 + q] = (top + __log2f(sum)) * kLn2;
+    const float inv = 1.0f / sum;
+    const int64_t off = pr.base + (int64_t)(q0 + q) * sn + d0;
+#pragma unroll
+    for (int d = 0; d < D / 8; d += 4) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[i] += w[k] * part[(k * D + d0 + d + i) * 32 + q];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] *= inv;
+        if (p.o) store4<T>((T *)p.o + off + d, v[0], v[1], v[2], v[3]);
+        if (p.gate) {
+            const typename Mfma<T>::v4 gv = *reinterpret_cast<const typename Mfma<T>::v4 *>((const T *)p.gate + off + d);
+            store4<T>((T *)p.o_gated + off + d, v[0] * sigmoidf((float)gv[0]), v[1] * sigmoidf((float)gv[1]), v[2] * sigmoidf((float)gv[2]),
+                      v[3] * sigmoidf((float)gv[3]));
+        }
+    }
+}
+
 // ------------------------------------------------------------------ dQ
 
 // As mfma_dq_wide.hip, whose place it takes at these head dims: where dBias is no sum over S rows, or its sum comes from a
@@ -791,6 +1016,27 @@ static int fwd_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
 
 int EVO_CAT(launch_mfma_fwd_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     return p.dtype == EVO_BF16 ? fwd_launch<bf16_t, EVO_D>(p, e, st) : fwd_launch<f16_t, EVO_D>(p, e, st);
+}
+
+template <typename T, int D>
+static int split_launch(const EvoAttnParams &p, hipStream_t st) {
+    const unsigned grid = (unsigned)((p.N + 31) / 32) * (unsigned)(p.B * p.H * p.S);
+    const int es = p.bias_dtype == EVO_F32 ? 4 : 2;
+    const bool vec = p.N % 4 == 0 && ((uintptr_t)p.bias % (4 * es)) == 0 && p.bias_stride_b % 4 == 0 && p.bias_stride_h % 4 == 0 && p.bias_stride_row % 4 == 0;
+    auto go = [&](auto kern, PerDevice &done) {
+        constexpr int most = SplitFwd<D>::BYTES + kSplitFwdMaxN * 4;
+        if (most > 64 * 1024)
+            if (const int rc = ensure_dynamic_lds((const void *)kern, most, done, nullptr)) return rc;
+        kern<<<grid, 256, SplitFwd<D>::BYTES + (p.N + 31) / 32 * 128, st>>>(p, vec);
+        return hip_rc();
+    };
+    static PerDevice done[3]{};
+    if (p.bias_dtype == EVO_NONE) return go(split_fwd<T, D, 0>, done[0]);
+    return p.bias_dtype == EVO_F32 ? go(split_fwd<T, D, 1>, done[1]) : go(split_fwd<T, D, 2>, done[2]);
+}
+
+int EVO_CAT(launch_split_fwd_d, EVO_D)(const EvoAttnParams &p, hipStream_t st) {
+    return p.dtype == EVO_BF16 ? split_launch<bf16_t, EVO_D>(p, st) : split_launch<f16_t, EVO_D>(p, st);
 }
 
 template <typename T, int D>

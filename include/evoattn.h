@@ -65,6 +65,9 @@ enum {
     /* Measurement aid: run the one-workgroup-per-(b,h,s) forms of the forward and dQ kernels
      * also where the forms that walk over a chunk of S rows apply (same results). */
     EVO_FLAG_PER_PROBLEM   = 16,
+    /* evoattn_fwd (and evoattn_prep_bytes of it): no evoattn_bwd will read this call's `prep`, which then may be left unwritten
+     * and, where evoattn_prep_bytes says so, missing. */
+    EVO_FLAG_FORWARD_ONLY  = 0x8000,
     /* evoattn_bwd with a gate: the gradient of the ungated output, dout * sigmoid(g), overwrites `dout`
      * instead of going to the workspace, which then does not grow by q's extent.  For a caller that owns
      * the memory of `dout` and does not need it afterwards; not together with EVO_FLAG_ONLY_DQ / _ONLY_DKDV. */
@@ -78,7 +81,7 @@ enum {
     EVO_FLAG_DEBUG_NO_DQ_WIDE   = 0x1000, /* dQ: the kernels that split a row's keys over the waves, also without a dBias sum */
     EVO_FLAG_DEBUG_NO_DQ_SPLIT  = 0x2000  /* dQ + dBias in one kernel, also where dQ and the dBias partials come from two */
 };
-#define EVO_FLAG_ALL (1 | 2 | 4 | 8 | 16 | 0x80 | 0x100 | 0x200 | 0x400 | 0x800 | 0x1000 | 0x2000)
+#define EVO_FLAG_ALL (1 | 2 | 4 | 8 | 16 | 0x80 | 0x100 | 0x200 | 0x400 | 0x800 | 0x1000 | 0x2000 | 0x8000)
 
 /* A problem (b, s) whose every key carries a mask value below this is a "dead row"; see lse below.
  * (An fp32 sum of such a mask value and a score of order one is the mask value: half a unit in the
