@@ -478,9 +478,16 @@ static int fwd_launches(const EvoAttnParams &p, hipStream_t st) {
     e.vec_ok = bias_vec_ok(p);
     fill_prep(p, e);
     EVO_SET_TRACE(e);
-    if (const int rc = launch_prep(p, e, st)) return rc;
-    if (fwd_ring_ok(p)) return launch_mfma_fwdr(p, e, st);
-    return launch_mfma_fwd(p, e, st);
+    // Without a backward the copies of the bias that only its kernels read need not be made, nor any where the forward keeps
+    // the caller's rows (S = 128, N = 251, H = 8, gated, fp16: 36.1 -> 34.7 us).
+    const bool ring = fwd_ring_ok(p), alone = (p.flags & EVO_FLAG_FORWARD_ONLY) != 0;
+    if (alone) {
+        e.bk = nullptr;
+        e.bk16 = nullptr;
+        e.bt = nullptr;
+    }
+    if (const int rc = launch_prep(p, e, st, alone && ring && mfma_fwdr_reads_rows(p))) return rc;
+    return ring ? launch_mfma_fwdr(p, e, st) : launch_mfma_fwd(p, e, st);
 }
 
 int evoattn_fwd(const EvoAttnParams *p, void *hip_stream) {

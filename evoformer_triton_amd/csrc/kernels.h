@@ -17,10 +17,14 @@ int launch_dbias_reduce(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_gate_bwd(const EvoAttnParams &p, void *dout_ungated, float *delta, hipStream_t st);  // dO, dgate and delta from the gradient of the gated output
 int launch_mask_shift(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 
-int launch_prep(const EvoAttnParams &p, const Extra &e, hipStream_t st);
+int launch_prep(const EvoAttnParams &p, const Extra &e, hipStream_t st, bool masks_only = false);
 int launch_mfma_fwd(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 constexpr int kSplitFwdMaxN = 4096;   // (its mask row lies in LDS)
 int launch_split_fwd(const EvoAttnParams &p, hipStream_t st);  // the keys of a row split over waves; reads mask and bias as given
+// whether that kernel (where it serves the call) keeps the caller's 16-bit bias rows, else prepared tiles
+inline bool mfma_fwdr_reads_rows(const EvoAttnParams &p) {
+    return p.bias_dtype == p.dtype && !(p.D == 8 && !p.gate) && !(p.flags & EVO_FLAG_DEBUG_FWD_BIAS_TILES);
+}
 int launch_mfma_fwdr(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int mfma_fwdr_max_n(int D);  // largest N the chunk-of-rows forward takes, 0 for a head dim it is not built for
 int launch_mfma_dq(const EvoAttnParams &p, const Extra &e, hipStream_t st);

@@ -601,10 +601,6 @@ static int fwdr_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     return p.stride_h < p.stride_n ? fwdr_launch_g<T, D, BIASK, 2>(p, e, st) : fwdr_launch_g<T, D, BIASK, 1>(p, e, st);
 }
 
-// whether the form with resident fp32 bias tiles keeps them in registers (the dispatch in api.hip sends an
-// fp32 bias here under the same condition)
-static bool fwdr_tiles_fit(const EvoAttnParams &p) { return EVO_D == 8 && !p.gate; }
-
 template <typename T>
 static int fwdr_bias(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     if (p.bias_dtype == EVO_NONE) return fwdr_launch<T, EVO_D, 0>(p, e, st);
@@ -614,8 +610,7 @@ static int fwdr_bias(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     // against 82 us) and a bias in the dtype of q stays resident as the caller's 16-bit rows (64 registers); an
     // fp32 bias is then served by the one-workgroup-per-problem forward (the dispatch sends none here).
     // EVO_FLAG_DEBUG_FWD_BIAS_TILES selects the fp32 tiles wherever the kernel runs, for comparison.
-    const bool tiles = fwdr_tiles_fit(p) || p.bias_dtype != p.dtype || (p.flags & EVO_FLAG_DEBUG_FWD_BIAS_TILES);
-    return tiles ? fwdr_launch<T, EVO_D, 1>(p, e, st) : fwdr_launch<T, EVO_D, 2>(p, e, st);
+    return mfma_fwdr_reads_rows(p) ? fwdr_launch<T, EVO_D, 2>(p, e, st) : fwdr_launch<T, EVO_D, 1>(p, e, st);
 }
 
 // Largest N this kernel takes for the head dim (0: not built for it).

@@ -47,11 +47,11 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
         if (t == n_bias_blocks - 1) {  // the all-zero tile
             if (e.bq16) {
                 *reinterpret_cast<uint2 *>(e.bq16 + e.zero_tile + tid * 4) = make_uint2(0u, 0u);
-                *reinterpret_cast<uint2 *>(e.bk16 + e.zero_tile + tid * 4) = make_uint2(0u, 0u);
+                if (e.bk16) *reinterpret_cast<uint2 *>(e.bk16 + e.zero_tile + tid * 4) = make_uint2(0u, 0u);
             } else {
                 const f32x4 z = {0.f, 0.f, 0.f, 0.f};
                 *reinterpret_cast<f32x4 *>(e.bq + e.zero_tile + tid * 4) = z;
-                *reinterpret_cast<f32x4 *>(e.bk + e.zero_tile + tid * 4) = z;
+                if (e.bk) *reinterpret_cast<f32x4 *>(e.bk + e.zero_tile + tid * 4) = z;
             }
             return;
         }
@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
                 for (int hh = 0; hh < 2; ++hh) {
                     dq[64 * hh] = make_uint4(wq[8 * hh] | ((unsigned)wq[8 * hh + 1] << 16), wq[8 * hh + 2] | ((unsigned)wq[8 * hh + 3] << 16),
                                         wq[8 * hh + 4] | ((unsigned)wq[8 * hh + 5] << 16), wq[8 * hh + 6] | ((unsigned)wq[8 * hh + 7] << 16));
-                    dk[64 * hh] = make_uint4(wk[8 * hh] | ((unsigned)wk[8 * hh + 1] << 16), wk[8 * hh + 2] | ((unsigned)wk[8 * hh + 3] << 16),
+                    if (e.bk16) dk[64 * hh] = make_uint4(wk[8 * hh] | ((unsigned)wk[8 * hh + 1] << 16), wk[8 * hh + 2] | ((unsigned)wk[8 * hh + 3] << 16),
                                         wk[8 * hh + 4] | ((unsigned)wk[8 * hh + 5] << 16), wk[8 * hh + 6] | ((unsigned)wk[8 * hh + 7] << 16));
                 }
             }
@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
                         vk[i] = sm[a][tl * 32 + li];
                     }
                     *reinterpret_cast<f32x4 *>(e.bq + o + 256 * m) = vq;
-                    *reinterpret_cast<f32x4 *>(e.bk + o + 256 * m) = vk;
+                    if (e.bk) *reinterpret_cast<f32x4 *>(e.bk + o + 256 * m) = vk;
                 }
             }
         }
@@ -198,11 +198,11 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
     if (tid == 0) e.dead[row] = dead ? 1 : 0;
 }
 
-int launch_prep(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+int launch_prep(const EvoAttnParams &p, const Extra &e, hipStream_t st, bool masks_only) {
     const unsigned NT = (p.N + 31) / 32;
     // (no bias tiles where the kernels read the caller's tensor)
     const unsigned NS = (NT + kPrepStrip - 1) / kPrepStrip;
-    const unsigned nb = p.bias && !e.bias_direct ? (unsigned)e.bias_batches * p.H * NT * NS + 1u : 0u;
+    const unsigned nb = p.bias && !e.bias_direct && !masks_only ? (unsigned)e.bias_batches * p.H * NT * NS + 1u : 0u;
     const unsigned nm = (unsigned)(p.B * p.S);
     prep_kernel<<<nb + nm, 256, 0, st>>>(p, e, nb);
     hipError_t err = hipGetLastError();
