@@ -458,11 +458,12 @@ __global__ void __launch_bounds__(256, D == 32 ? 3 : D == 64 ? 2 : 1) split_fwd(
         for (int j = lane; j < NT * 32; j += 64) masks[j] = j < p.N ? 0.0f : kMaskFloor;
     }
     const bool dead = p.mask_kind != EVO_MASK_NONE && mx < kShiftThreshold;
-    const float c = dead ? 0.0f : p.scale * kLog2e, bmul = dead ? 0.0f : kLog2e, shift = dead ? mx : 0.0f;
+    const float c = dead ? 0.0f : p.scale * kLog2e, shift = dead ? mx : 0.0f;
 #pragma unroll
     for (int ks = 0; ks < KSD; ++ks) qf[ks] = dead ? zero8<T>() : scaled8<T>(qf[ks], c);
 
-    float m = -INFINITY, l = 0.0f;
+    // (not from -inf: against a tile whose every bias entry is -inf the maximum stays where it starts, and -inf less -inf is no number)
+    float m = kMaskFloor, l = 0.0f;
     f32x16 o[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -479,7 +480,7 @@ __global__ void __launch_bounds__(256, D == 32 ? 3 : D == 64 ? 2 : 1) split_fwd(
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float mask = 32 * t + 8 * rr + 4 * g + i < p.N ? fmaxf((mk[i] - shift) * kLog2e, kMaskFloor) : kMaskFloor;
-                a[4 * rr + i] = BF ? now.bias[4 * rr + i] * bmul + mask : mask;
+                a[4 * rr + i] = BF && !dead ? now.bias[4 * rr + i] * kLog2e + mask : mask;   // (dropped, not times zero: it may be infinite)
             }
         }
 #pragma unroll
@@ -528,7 +529,7 @@ __global__ void __launch_bounds__(256, D == 32 ? 3 : D == 64 ? 2 : 1) split_fwd(
     }
     __syncthreads();
     const int q = threadIdx.x & 31, d0 = (threadIdx.x >> 5) * (D / 8);
-    float w[4], top = -INFINITY, sum = 0.0f;
+    float w[4], top = kMaskFloor, sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) top = fmaxf(top, stats[(i * 2) * 32 + q]);
 #pragma unroll

@@ -1,0 +1,65 @@
+"""Bias entries of -inf or of the type's lowest value (what a program writes to keep two chains apart): whole key tiles of
+them, in kept and in dropped rows, through each kernel that reads a bias, against eager in fp32."""
+import pytest
+import torch
+
+from oracle import eager
+
+pytestmark = pytest.mark.gpu
+
+# A result is a sum of products rounded to 16 bits on its way: the tolerance of the other tests against eager in fp32.
+REL = 1.5e-2
+
+
+def _closed(kind, B, H, N, value, g):
+    """A bias whose entries `kind` names are closed; every query keeps a key."""
+    b = torch.randn((B, 1, H, N, N), generator=g) * 0.5
+    if kind == "chains":
+        b[..., : N // 2, N // 2:] = value
+        b[..., N // 2:, : N // 2] = value
+    elif kind == "first":                      # the first tiles of a row, of half of the queries
+        b[..., N // 2:, : min(64, N - 1)] = value
+    elif kind == "last":                       # the last key (a tile of one where N = 32 n + 1)
+        b[..., N - 1] = value
+    return b
+
+
+def _check(dev, shape, kind, bias_dt, dt, lowest, mask, layout, grad):
+    import evoformer_triton_amd.evoformer as E
+    B, S, N, H, D = shape
+    g = torch.Generator().manual_seed(41)
+    Q, K, V, dO = ((torch.randn(shape, generator=g) * 0.7).to(dt) for _ in range(4))
+    bdt = dt if bias_dt == "q" else torch.float32
+    b = _closed(kind, B, H, N, torch.finfo(bdt).min if lowest else -float("inf"), g).to(bdt)
+    m = None
+    if mask == "dead":                         # a row with every key dropped: uniform over the keys, whatever the bias says
+        m = torch.ones((B, S, 1, 1, N), dtype=torch.bool)
+        m[:, S - 1] = False
+    # (the oracle's own bias closed by a finite value: the same probabilities, and gradients that its autograd forms)
+    want = eager.attention_fwd_bwd(Q, K, V, m, b.float().clamp_min(-1e30), dO, layout=layout, compute_dtype=torch.float32)
+    q, k, v, bb = (t.to(dev).requires_grad_(grad) for t in (Q, K, V, b))
+    o = E.evoformer_attention(q, k, v, None if m is None else m.to(dev), bb, layout=layout)
+    got = {"O": o}
+    if grad:
+        o.backward(dO.to(dev))
+        got.update(dQ=q.grad, dK=k.grad, dV=v.grad, dBias=bb.grad)
+    for name, t in got.items():
+        d = t.detach().float().cpu() - want[name]
+        assert torch.isfinite(d).all(), name
+        assert d.norm() <= REL * want[name].norm() + 1e-4 * d.numel() ** 0.5, (name, (d.norm() / want[name].norm()).item())
+
+
+SPLIT = [  # single sequences without a backward: each wave has every fourth tile of 32 keys
+    ((1, 1, 33, 2, 32), "last", "f", torch.bfloat16, False, None, "reference"),
+    ((1, 1, 65, 3, 64), "last", "q", torch.float16, False, None, "ds4sci"),
+    ((2, 1, 97, 2, 128), "last", "q", torch.bfloat16, True, None, "reference"),
+    ((1, 1, 250, 4, 64), "chains", "f", torch.bfloat16, False, None, "reference"),
+    ((1, 1, 256, 4, 32), "first", "q", torch.bfloat16, False, "dead", "reference"),
+    ((1, 1, 130, 2, 128), "chains", "f", torch.float16, False, "dead", "reference"),
+    ((1, 1, 128, 16, 64), "chains", "f", torch.bfloat16, True, "dead", "reference"),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_forward_that_splits_the_keys(gpu_device, case):
+    _check(gpu_device, *case, grad=False)
