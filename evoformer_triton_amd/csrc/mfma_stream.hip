@@ -39,6 +39,7 @@ struct StreamGeo {
 };
 
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void wait_loads_and_lds() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void wait_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, unsigned char *dst, int off) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16, off, 0, 0, 0);
@@ -471,7 +472,9 @@ __global__ void __launch_bounds__(256, D == 32 ? 3 : D == 64 ? 2 : 1) split_fwd(
         for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
     for (int t = wave; t < NT; t += 4) {
         const Tile now = next;
-        wait_loads();   // (V of this tile)
+        // V of this tile has landed; and the reads of the tile before have left the buffer that the next fetch writes (nothing else
+        // orders a read of LDS before the load path's write to it: the products that use the reads may come after the fetch)
+        wait_loads_and_lds();
         if (t + 4 < NT) fetch(t + 4, next);
         f32x16 a;
 #pragma unroll
