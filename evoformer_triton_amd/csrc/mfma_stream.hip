@@ -231,7 +231,8 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3
             for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, a[t][r]);
         const unsigned u = __float_as_uint(mloc);
         auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-        const float cand = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) + used;
+        // (not below the floor of masked keys: the scores of a step are -inf where the bias is, and -inf less -inf is no number)
+        const float cand = fmaxf(fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) + used, kMaskFloor);
         const bool grow = first || cand > m + 8.0f;   // (moved only when it grows by more than 2^8)
         if (__any(grow || m != used)) {
             const float mn = grow ? cand : m;

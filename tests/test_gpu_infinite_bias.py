@@ -63,3 +63,19 @@ SPLIT = [  # single sequences without a backward: each wave has every fourth til
 @pytest.mark.parametrize("case", SPLIT, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
 def test_forward_that_splits_the_keys(gpu_device, case):
     _check(gpu_device, *case, grad=False)
+
+
+STREAM = [  # rows that stream through LDS: the first step has 32 keys (head dim 32: 64)
+    ((1, 6, 96, 2, 64), "chains", "q", torch.bfloat16, False, None, "reference"),
+    ((1, 6, 130, 2, 128), "first", "f", torch.float16, False, None, "ds4sci"),
+    ((1, 5, 65, 1, 64), "first", "f", torch.bfloat16, True, "dead", "reference"),
+    ((2, 1, 200, 4, 128), "chains", "q", torch.bfloat16, True, None, "reference"),
+    ((1, 6, 130, 2, 32), "chains", "f", torch.bfloat16, False, None, "reference"),
+    ((1, 9, 300, 2, 32), "first", "q", torch.float16, True, None, "ds4sci"),
+    ((1, 2, 1100, 1, 64), "last", "q", torch.bfloat16, False, None, "reference"),
+]
+
+
+@pytest.mark.parametrize("case", STREAM, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_kernels_whose_rows_stream(gpu_device, case):
+    _check(gpu_device, *case, grad=True)
