@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(64) gen_fwd(EvoAttnParams p) {
     for (int d = 0; d < D; ++d) acc[d] = 0.0f;
     const float shift = row_shift(p, pr.b, pr.s);
     const int64_t brow = (int64_t)pr.b * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h + (int64_t)rowc * p.bias_stride_row;
-    float m = -INFINITY, l = 0.0f;
+    float m = -FLT_MAX, l = 0.0f;   // (a score of -inf less a maximum of -inf is no number)
     for (int j = 0; j < p.N; ++j) {
         const T *kr = K + (int64_t)j * p.stride_n, *vr = V + (int64_t)j * p.stride_n;
         float qk = 0.0f;

@@ -127,7 +127,9 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_fwd(EvoAttnPara
                                     : dead  ? e.bq16 + e.zero_tile + lane * 8
                                             : e.bq16 + ((((int64_t)bb * p.H + pr.h) * NT + qt) * NT) * 1024 + lane * 8;
 
-    float m = LAZY ? 0.0f : -INFINITY, mf = 0.0f, l = 0.0f;
+    // (never below the floor of masked keys: against a step whose every bias entry is -inf the difference to a maximum of -inf
+    // would be no number)
+    float m = LAZY ? 0.0f : kMaskFloor, mf = 0.0f, l = 0.0f;
     f32x16 oacc[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -222,7 +224,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_fwd(EvoAttnPara
             auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
             mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
         }
-        const float cand = mloc + used;
+        const float cand = fmaxf(mloc + used, kMaskFloor);
         // move m only when the maximum grows by more than 2^TAU (always at the first step)
         const bool grow = first || cand > m + TAU;
         if (__any(grow || m != used)) {

@@ -407,7 +407,7 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
                     auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
                     mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
                 }
-                const float cand = mloc + used;
+                const float cand = fmaxf(mloc + used, kMaskFloor);   // (see mfma_fwd.hip)
                 // move m only when the maximum grows by more than 2^TAU (always at the first step)
                 const bool grow = step == 0 || cand > m + TAU;
                 if (__any(grow || m != used)) {

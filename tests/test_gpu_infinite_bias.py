@@ -79,3 +79,21 @@ STREAM = [  # rows that stream through LDS: the first step has 32 keys (head dim
 @pytest.mark.parametrize("case", STREAM, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
 def test_kernels_whose_rows_stream(gpu_device, case):
     _check(gpu_device, *case, grad=True)
+
+
+ONE_STEP = [  # kernels whose first step has 64 keys, and the plain ones, which go key by key
+    ((1, 6, 130, 2, 8), "first", "f", torch.bfloat16, False, None, "reference"),
+    ((1, 6, 96, 2, 16), "first", "q", torch.float16, False, None, "ds4sci"),
+    ((1, 5, 300, 2, 16), "chains", "f", torch.bfloat16, True, None, "reference"),
+    ((2, 1, 300, 4, 8), "chains", "q", torch.bfloat16, False, None, "reference"),
+    ((1, 40, 200, 2, 8), "first", "f", torch.bfloat16, False, None, "reference"),       # fp32 tiles resident
+]
+
+
+@pytest.mark.parametrize("plain", [False, True], ids=["matrix_core", "plain"])
+@pytest.mark.parametrize("case", ONE_STEP, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_kernels_with_a_step_of_64_keys_and_plain_ones(gpu_device, case, plain, monkeypatch):
+    import evoformer_triton_amd.evoformer as E
+    from evoformer_triton_amd import _lib
+    monkeypatch.setattr(E, "FLAGS", _lib.EVO_FLAG_FORCE_GENERIC if plain else 0)
+    _check(gpu_device, *case, grad=True)
