@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_fwd(EvoAttnPara
     // caller's tensor
     const bool bdirect = HAS_BIAS && e.bias_direct;
     const bool bf32 = p.bias_dtype == EVO_F32;
-    const char *brow = (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h +
+    const char *brow = dead ? dead_bias(p, e, pr.b, pr.s) : (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h +
                                                (int64_t)qrow * p.bias_stride_row) * (bf32 ? 4 : 2);
     const float bmul = dead ? 0.0f : kLog2e;
     const unsigned short *btile16 = !TILE16 ? nullptr

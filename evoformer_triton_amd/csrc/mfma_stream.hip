@@ -104,9 +104,9 @@ struct BiasStream {
         const int bb = e.bias_batches > 1 ? pr.b : 0;
         if (BT == 3) {
             f32 = p.bias_dtype == EVO_F32;
-            row_stride = (unsigned)p.bias_stride_row;
+            row_stride = dead ? 0u : (unsigned)p.bias_stride_row;
             col = (unsigned)own_row;
-            mat = (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h + (COLS ? 0 : (int64_t)own_row * p.bias_stride_row)) * (f32 ? 4 : 2);
+            mat = dead ? dead_bias(p, e, pr.b, pr.s) : (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h + (COLS ? 0 : (int64_t)own_row * p.bias_stride_row)) * (f32 ? 4 : 2);
         } else {
             const int64_t first = (((int64_t)bb * p.H + pr.h) * NT * NT + (COLS ? own_tile : own_tile * NT)) * 1024;
             step = dead ? 0 : COLS ? (int64_t)NT * 1024 : 1024;

@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
         const int li = lane & 31, g = lane >> 5, tl = tid >> 6;
         const int64_t tile0 = (((int64_t)bb * p.H + h) * NT + qt) * NT + kt0;
         if (e.bq16) {
-            // the entries as given (the bias has the dtype of q: 16 bits, exact)
+            // the entries as given (the bias has the dtype of q: 16 bits, exact; -inf as the lowest finite value)
             constexpr int PITCH = kPrepCols + 8;                       // entries; rows 16 bytes further apart than long
             unsigned short(*sm)[PITCH] = reinterpret_cast<unsigned short(*)[PITCH]>(strip);
             const unsigned short *src = (const unsigned short *)p.bias + base;
@@ -86,6 +86,8 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
                                        w[4] | ((unsigned)w[5] << 16), w[6] | ((unsigned)w[7] << 16));
                     }
                 }
+                if (p.dtype == EVO_F16) v = make_uint4(finite_pair<f16_t>(v.x), finite_pair<f16_t>(v.y), finite_pair<f16_t>(v.z), finite_pair<f16_t>(v.w));
+                else v = make_uint4(finite_pair<bf16_t>(v.x), finite_pair<bf16_t>(v.y), finite_pair<bf16_t>(v.z), finite_pair<bf16_t>(v.w));
                 *reinterpret_cast<uint4 *>(&sm[r][c]) = v;
             }
             __syncthreads();

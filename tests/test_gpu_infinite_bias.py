@@ -97,3 +97,33 @@ def test_kernels_with_a_step_of_64_keys_and_plain_ones(gpu_device, case, plain, 
     from evoformer_triton_amd import _lib
     monkeypatch.setattr(E, "FLAGS", _lib.EVO_FLAG_FORCE_GENERIC if plain else 0)
     _check(gpu_device, *case, grad=True)
+
+
+TIMES_ZERO = [  # entries that a kernel multiplies by zero: the identity product of a resident bias, rows with every key dropped
+    ((1, 40, 256, 2, 32), "chains", "q", torch.bfloat16, False, "dead", "reference"),
+    ((1, 40, 200, 2, 16), "last", "q", torch.float16, False, None, "ds4sci"),
+    ((1, 40, 250, 1, 8), "chains", "q", torch.bfloat16, True, "dead", "reference"),        # rows that pass through LDS
+    ((1, 6, 130, 2, 64), "first", "q", torch.bfloat16, False, "dead", "reference"),
+    ((1, 2, 256, 2, 32), "chains", "f", torch.bfloat16, False, "dead", "reference"),       # the caller's rows
+    ((2, 1, 200, 2, 16), "chains", "q", torch.bfloat16, False, "dead", "ds4sci"),
+    ((1, 64, 200, 2, 64), "chains", "q", torch.bfloat16, False, "dead", "reference"),      # dBias from a kernel of its own
+    ((1, 64, 544, 1, 32), "chains", "q", torch.float16, False, "dead", "reference"),
+    ((1, 24, 384, 2, 8), "chains", "q", torch.bfloat16, False, "dead", "reference"),
+]
+
+
+@pytest.mark.parametrize("grad", [False, True], ids=["forward", "step"])
+@pytest.mark.parametrize("case", TIMES_ZERO, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_entries_that_meet_a_factor_of_zero(gpu_device, case, grad):
+    _check(gpu_device, *case, grad=grad)
+
+
+def test_a_gated_forward_with_a_resident_bias(gpu_device):
+    import evoformer_triton_amd.evoformer as E
+    g = torch.Generator().manual_seed(43)
+    B, S, N, H, D = shape = (1, 40, 250, 2, 32)
+    Q, K, V, G = ((torch.randn(shape, generator=g) * 0.7).to(torch.bfloat16) for _ in range(4))
+    b = _closed("chains", B, H, N, -float("inf"), g).to(torch.bfloat16)
+    want = eager.attention_fwd_bwd(Q, K, V, None, b.float().clamp_min(-1e30), torch.zeros_like(Q), compute_dtype=torch.float32, gate=G)["Og"]
+    d = E.evoformer_attention(*(t.to(gpu_device) for t in (Q, K, V)), None, b.to(gpu_device), gate=G.to(gpu_device)).float().cpu() - want
+    assert torch.isfinite(d).all() and d.norm() <= REL * want.norm()
