@@ -103,7 +103,8 @@ class _Projections(torch.autograd.Function):
 
 class _Linear(torch.autograd.Function):
     """x W^T + b with the weight gradient summed over slices of the rows (see _row_slices); forward and
-    input gradient are the library's GEMMs as torch.nn.functional.linear calls them.  What the tracer sees."""
+    input gradient are the library's GEMMs as torch.nn.functional.linear calls them.  What the compiler's tracer sees, and
+    what a call reaches that the C++ node does not stand for (under vmap, func.grad and the like, which refuse it)."""
 
     @staticmethod
     def forward(ctx, x, weight, bias):
@@ -129,9 +130,9 @@ class _Linear(torch.autograd.Function):
 
 
 def _linear(layer: nn.Linear, x: torch.Tensor, dx_place: Optional[torch.Tensor] = None) -> torch.Tensor:
-    if torch.compiler.is_compiling():
-        return _Linear.apply(x, layer.weight, layer.bias)
-    return _lib.host().linear(x, layer.weight, layer.bias, dx_place)      # (the same in C++)
+    # (the same in C++)
+    y = None if torch.compiler.is_compiling() else _lib.host().linear(x, layer.weight, layer.bias, dx_place)
+    return _Linear.apply(x, layer.weight, layer.bias) if y is None else y
 
 
 class _StackedProjection:
@@ -143,7 +144,13 @@ class _StackedProjection:
 
     @staticmethod
     def apply(x, gate_bias, *weights):
-        return _lib.host().stacked_projection(x, gate_bias, weights)
+        y = _lib.host().stacked_projection(x, gate_bias, weights)
+        if y is not None:
+            return y
+        w = torch.cat(weights, 0)
+        if gate_bias is not None:
+            gate_bias = torch.cat([gate_bias.new_zeros(w.shape[0] - gate_bias.shape[0]), gate_bias])
+        return _Linear.apply(x, w, gate_bias)
 
 
 class _LayerNorm:

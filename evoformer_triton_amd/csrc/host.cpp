@@ -616,8 +616,9 @@ struct LinearNode : SavingNode {
 };
 
 // x W^T + b with the weight gradient summed over slices of the rows; `dx_place` (shaped like x, rows may lie apart): where
-// the input gradient is to be written.
-Tensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, const OptTensor &dx_place) {
+// the input gradient is to be written.  None under a mode or for tensors that a hand-made node does not stand for.
+OptTensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, const OptTensor &dx_place) {
+    if (!plain_modes() || !plain(x) || !plain(weight) || (bias && bias->defined() && !plain(*bias))) return std::nullopt;
     Tensor y;
     {
         at::AutoDispatchBelowADInplaceOrView guard;
@@ -679,9 +680,13 @@ struct StackedNode : SavingNode {
 };
 
 // Several projections of one input as one GEMM with their weights stacked; `gate_bias` is added on the last layer's columns.
-Tensor stacked_projection(const Tensor &x, const OptTensor &gate_bias, const std::vector<Tensor> &weights) {
+// None as above.
+OptTensor stacked_projection(const Tensor &x, const OptTensor &gate_bias, const std::vector<Tensor> &weights) {
     Tensor y;
     const Tensor gb = gate_bias ? *gate_bias : Tensor();
+    bool taken = plain_modes() && plain(x) && (!gb.defined() || plain(gb));
+    for (const Tensor &t : weights) taken = taken && plain(t);
+    if (!taken) return std::nullopt;
     {
         at::AutoDispatchBelowADInplaceOrView guard;
         y = lin_forward(as_rows(x), weights, gb);
