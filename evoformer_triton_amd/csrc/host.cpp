@@ -50,14 +50,18 @@ int evo_dtype(at::ScalarType t) {
 
 bool head_dim_built(int64_t D) { return D == 8 || D == 16 || D == 32 || D == 64 || D == 128; }
 
-// An ordinary tensor with memory of its own kind: no subclass or mode with a dispatch in Python, no functorch wrapper
-// and no lazily negated or conjugated view, whose data pointer would not be what it stands for.
+// Whether `t` carries a tangent of forward-mode differentiation.  No node here has a formula for it, and launches drop it without a
+// word, which counts as a tangent of zero.
+bool dual(const Tensor &t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
+
+// An ordinary tensor with memory of its own kind: no subclass or mode with a dispatch in Python, no functorch wrapper,
+// no tangent and no lazily negated or conjugated view, whose data pointer would not be what it stands for.
 bool plain(const Tensor &t) {
     static const auto special = c10::DispatchKeySet({
         c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::FuncTorchBatched,
         c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate,
         c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
-    return t.layout() == at::kStrided && !t.key_set().has_any(special);
+    return t.layout() == at::kStrided && !t.key_set().has_any(special) && !dual(t);
 }
 
 bool plain_modes() {
@@ -486,6 +490,8 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
 };
 
 variable_list slot_attention(const Tensor &P, const OptTensor &mask, const OptTensor &bias, bool gated) {
+    TORCH_CHECK_NOT_IMPLEMENTED(!dual(P) && !(mask && dual(*mask)) && !(bias && dual(*bias)),
+                                "slot_attention has no formula for forward mode differentiation");
     TORCH_CHECK_VALUE(plain(P) && P.is_cuda() && P.dim() == 6 && P.numel() > 0 && P.is_contiguous() && P.size(3) >= (gated ? 4 : 3) &&
                           (P.scalar_type() == at::kBFloat16 || P.scalar_type() == at::kHalf) && head_dim_built(P.size(5)),
                       "P must be a contiguous 16-bit [B,S,N,W,H,D] tensor with W >= 3 (4 with a gate) and a head dim the library is built for");
@@ -971,7 +977,9 @@ OptTensor block(const std::vector<OptTensor> &in, const OptTensor &keep, int64_t
     for (int i = 0; i < kBlockInputs; ++i)
         if (in[i]) t[i] = *in[i];
     const Tensor &m = t[kM];
-    if (!plain(m) || m.dim() != 4 || !m.is_cuda() || m.numel() == 0 || at::autocast::is_autocast_enabled(at::kCUDA)) return std::nullopt;
+    for (const Tensor &i : t)
+        if (i.defined() && !plain(i)) return std::nullopt;
+    if (m.dim() != 4 || !m.is_cuda() || m.numel() == 0 || at::autocast::is_autocast_enabled(at::kCUDA)) return std::nullopt;
     const bool gated = t[kG].defined();
     const int W = gated ? 4 : 3;
     if (!t[kQ].defined() || t[kQ].dim() != 2 || !t[kK].defined() || !t[kV].defined() || !t[kO].defined()) return std::nullopt;

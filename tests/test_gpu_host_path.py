@@ -69,3 +69,47 @@ def test_what_the_native_path_does_not_take(gpu_device):
         E.EvoformerAttention.apply(p, p, p, None, torch.zeros(1, 1, 3, 32, 32, device=gpu_device))
     with pytest.raises(RuntimeError, match="same device"):
         E.EvoformerAttention.apply(p, p, p, torch.zeros(1, 2, 1, 1, 32), None)
+
+
+def _gpu_block(dev):
+    from evoformer_triton_amd.block import GatedAttentionBlock
+    torch.manual_seed(4)
+    blk = GatedAttentionBlock(64, 32, 4, c_z=64).to(dev).to(torch.bfloat16)
+    m = torch.randn(1, 3, 40, 64, device=dev).to(torch.bfloat16)
+    z = torch.randn(1, 40, 40, 64, device=dev).to(torch.bfloat16)
+    return blk, m, z
+
+
+def _attention_operands(dev):
+    g = torch.Generator().manual_seed(5)
+    q = [torch.randn((1, 3, 40, 4, 32), generator=g).to(torch.bfloat16).to(dev) for _ in range(4)]
+    return q, torch.randn((1, 3, 1, 1, 40), generator=g).to(dev), torch.randn((1, 1, 4, 40, 40), generator=g).to(torch.bfloat16).to(dev)
+
+
+@pytest.mark.parametrize("which", ["q", "v", "mask", "bias", "gate"])
+def test_a_forward_mode_tangent_is_refused_by_the_attention(gpu_device, which):
+    import evoformer_triton_amd.evoformer as E
+    from torch.autograd import forward_ad
+    (q, k, v, gate), mask, bias = _attention_operands(gpu_device)
+    args = {"q": q, "k": k, "v": v, "mask": mask, "bias": bias, "gate": gate}
+    with forward_ad.dual_level():
+        args[which] = forward_ad.make_dual(args[which], torch.ones_like(args[which]))
+        with pytest.raises(NotImplementedError, match="jvp|forward mode"):
+            E.evoformer_attention(args["q"], args["k"], args["v"], args["mask"], args["bias"], gate=args["gate"] if which == "gate" else None)
+
+
+def test_a_forward_mode_tangent_is_refused_by_the_block_and_its_slots(gpu_device):
+    import evoformer_triton_amd.evoformer as E
+    from torch.autograd import forward_ad
+    blk, m, z = _gpu_block(gpu_device)
+    dual = lambda t: forward_ad.make_dual(t.detach(), torch.ones_like(t))
+    with forward_ad.dual_level():
+        for args in ((dual(m), z), (m, dual(z))):
+            with pytest.raises(NotImplementedError, match="jvp|forward mode"):
+                blk(*args)
+        for name in ("linear_q.weight", "linear_g.bias", "linear_o.weight", "linear_o.bias", "linear_z.weight"):
+            with pytest.raises(NotImplementedError, match="jvp|forward mode"):
+                torch.func.functional_call(blk, {name: dual(blk.get_parameter(name))}, (m, z))
+        P = torch.randn((1, 3, 40, 3, 2, 32), device=gpu_device).to(torch.bfloat16)
+        with pytest.raises(NotImplementedError, match="forward mode"):
+            E.slot_attention(dual(P))

@@ -40,3 +40,25 @@ def test_a_dispatch_mode_sees_the_layers_and_changes_nothing(name):
     with Recorder():
         got = call(x)
     assert torch.equal(got, want) and any("mm" in f for f in seen)
+
+
+@pytest.mark.parametrize("name", ["linear", "stacked"])
+def test_a_forward_mode_tangent_is_refused_not_dropped(name):
+    from torch.autograd import forward_ad
+    call, x = _calls()[name], torch.randn(3, 5, 16)
+    with forward_ad.dual_level():
+        with pytest.raises(NotImplementedError, match="jvp|forward mode"):
+            call(forward_ad.make_dual(x, torch.ones_like(x)))
+
+
+def test_a_forward_mode_tangent_of_a_parameter_is_refused():
+    from torch.autograd import forward_ad
+    x = torch.randn(3, 5, 16)
+    with forward_ad.dual_level():
+        for part in ("weight", "bias"):
+            layer = nn.Linear(16, 8)
+            p = getattr(layer, part).detach()
+            delattr(layer, part)
+            setattr(layer, part, forward_ad.make_dual(p, torch.ones_like(p)))
+            with pytest.raises(NotImplementedError, match="jvp|forward mode"):
+                block._linear(layer, x)
