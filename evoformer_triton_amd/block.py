@@ -242,7 +242,7 @@ class GatedAttentionBlock(nn.Module):
     def _slots_ok(self, m: torch.Tensor) -> bool:
         """Whether Q, K, V and the gate can come from one GEMM and reach the kernels as slots of its result."""
         if not m.is_cuda or m.dtype not in (torch.bfloat16, torch.float16) or m.numel() == 0 or torch.compiler.is_compiling() \
-                or self.c_hidden not in _HEAD_DIMS:
+                or torch.jit.is_tracing() or self.c_hidden not in _HEAD_DIMS:
             return False
         mods = self._modules
         layers = [mods["linear_q"], mods["linear_k"], mods["linear_v"], mods["linear_o"]] + ([mods["linear_g"]] if mods.get("linear_g") is not None else [])

@@ -34,6 +34,7 @@ using torch::autograd::AutogradContext;
 using torch::autograd::Node;
 using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
+using c10::impl::tls_local_dispatch_key_set;
 
 void check(int rc, const char *where) {
     TORCH_CHECK(rc == EVO_OK, where, " failed: ", evoattn_strerror(rc), " (code ", rc, ")");
@@ -64,9 +65,11 @@ bool plain(const Tensor &t) {
     return t.layout() == at::kStrided && !t.key_set().has_any(special) && !dual(t);
 }
 
+// No mode that has to see the call itself: a dispatch mode in Python, functorch, or torch.jit's tracer, which records the operators
+// called here but none of the launches.
 bool plain_modes() {
-    const auto tls = c10::impl::tls_local_dispatch_key_set();
-    return !tls.included_.has(c10::DispatchKey::Python) && !tls.included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+    static const auto modes = c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::Tracer});
+    return !tls_local_dispatch_key_set().included_.has_any(modes);
 }
 
 hipStream_t stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }

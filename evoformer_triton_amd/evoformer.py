@@ -607,6 +607,10 @@ class _SlotAttention:
 
     @staticmethod
     def apply(P, res_mask, pair_bias, gated):
+        if torch.jit.is_tracing():     # (torch.jit's tracer records autograd.Functions in Python, not the C++ one)
+            q, k, v, *g = P.unbind(3)[:4 if gated else 3]
+            out = evoformer_attention(q, k, v, res_mask, pair_bias, layout="ds4sci", gate=g[0] if gated else None)
+            return out, torch.empty_like(out)
         return _lib.host().slot_attention(P, res_mask, pair_bias, bool(gated))
 
 

@@ -7,11 +7,11 @@ from torch import nn
 from evoformer_triton_amd import block
 
 
-def _calls():
+def _calls(requires_grad=True):
     g = torch.Generator().manual_seed(8)
-    layer = nn.Linear(16, 8)
-    ws = [torch.randn((8, 16), generator=g, requires_grad=True) for _ in range(4)]
-    bg = torch.randn((8,), generator=g, requires_grad=True)
+    layer = nn.Linear(16, 8).requires_grad_(requires_grad)
+    ws = [torch.randn((8, 16), generator=g, requires_grad=requires_grad) for _ in range(4)]
+    bg = torch.randn((8,), generator=g, requires_grad=requires_grad)
     return {"linear": lambda x: block._linear(layer, x), "stacked": lambda x: block._StackedProjection.apply(x, bg, *ws)}
 
 
@@ -62,3 +62,11 @@ def test_a_forward_mode_tangent_of_a_parameter_is_refused():
             setattr(layer, part, forward_ad.make_dual(p, torch.ones_like(p)))
             with pytest.raises(NotImplementedError, match="jvp|forward mode"):
                 block._linear(layer, x)
+
+
+@pytest.mark.parametrize("name", ["linear", "stacked"])
+def test_a_traced_layer_computes_on_replay(name):
+    call = _calls(requires_grad=False)[name]     # (the tracer takes what a call closes over as constants)
+    traced = torch.jit.trace(call, (torch.randn(3, 5, 16),), check_trace=False)
+    x = torch.randn(3, 5, 16)
+    assert torch.equal(traced(x), call(x)) and "_Linear" in str(traced.inlined_graph)
