@@ -30,6 +30,7 @@ import torch
 from torch import nn
 
 from . import _lib
+from . import evoformer as _evoformer
 from .evoformer import _DTYPES, _HEAD_DIMS, _SlotAttention, _alloc_bytes, _on_device, _ptr, _stream, evoformer_attention
 
 
@@ -264,7 +265,8 @@ class GatedAttentionBlock(nn.Module):
                 inputs.append(own["weight"])
             else:
                 inputs += (own["weight"], own["bias"])
-        return _lib.host().block(inputs, mask, self.no_heads, mods["layer_norm_m"].eps, mods["layer_norm_z"].eps if with_z else 0.0, self.inf)
+        return _lib.host().block(inputs, mask, self.no_heads, mods["layer_norm_m"].eps, mods["layer_norm_z"].eps if with_z else 0.0, self.inf,
+                                 _evoformer.FLAGS)
 
     def forward(self, m: torch.Tensor, z: Optional[torch.Tensor] = None, mask: Optional[torch.Tensor] = None):
         B, S, N, _ = m.shape

@@ -376,7 +376,7 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
         Tensor ob, aux;
         OptTensor mask, bias;
     };
-    static Run enqueue(const Tensor &P, const OptTensor &mask, const OptTensor &bias, bool gated) {
+    static Run enqueue(const Tensor &P, const OptTensor &mask, const OptTensor &bias, bool gated, int64_t flags) {
         Run r;
         Call &c = r.c;
         EvoAttnParams &p = c.p;
@@ -387,6 +387,7 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
         p.D = (int32_t)P.size(5);
         p.dtype = evo_dtype(P.scalar_type());
         p.dbias_dtype = EVO_F32;
+        p.flags = (int32_t)flags;
         p.scale = (float)(1.0 / std::sqrt((double)p.D));
         strides(p, P);
         c.gated = gated;
@@ -441,8 +442,8 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
         return DP;
     }
 
-    static variable_list forward(AutogradContext *ctx, const Tensor &P, OptTensor mask, OptTensor bias, bool gated) {
-        const Run r = enqueue(P, mask, bias, gated);
+    static variable_list forward(AutogradContext *ctx, const Tensor &P, OptTensor mask, OptTensor bias, bool gated, int64_t flags) {
+        const Run r = enqueue(P, mask, bias, gated, flags);
         const Call &c = r.c;
         const Tensor &ob = r.ob, &aux = r.aux;
         Tensor out = ob.select(3, gated ? 1 : 0);
@@ -460,7 +461,7 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
 
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const bool rec = at::GradMode::is_enabled();
-        variable_list res(4);
+        variable_list res(5);
         {
             at::AutoDispatchBelowADInplaceOrView guard;
             const auto saved = ctx->get_saved_variables();
@@ -492,13 +493,13 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
     }
 };
 
-variable_list slot_attention(const Tensor &P, const OptTensor &mask, const OptTensor &bias, bool gated) {
+variable_list slot_attention(const Tensor &P, const OptTensor &mask, const OptTensor &bias, bool gated, int64_t flags) {
     TORCH_CHECK_NOT_IMPLEMENTED(!dual(P) && !(mask && dual(*mask)) && !(bias && dual(*bias)),
                                 "slot_attention has no formula for forward mode differentiation");
     TORCH_CHECK_VALUE(plain(P) && P.is_cuda() && P.dim() == 6 && P.numel() > 0 && P.is_contiguous() && P.size(3) >= (gated ? 4 : 3) &&
                           (P.scalar_type() == at::kBFloat16 || P.scalar_type() == at::kHalf) && head_dim_built(P.size(5)),
                       "P must be a contiguous 16-bit [B,S,N,W,H,D] tensor with W >= 3 (4 with a gate) and a head dim the library is built for");
-    return SlotAttention::apply(P, mask, bias, gated);
+    return SlotAttention::apply(P, mask, bias, gated, flags);
 }
 
 // ------------------------------------------------------------------ the layers of the block around the attention
@@ -974,7 +975,7 @@ struct BlockNode : SavingNode {
 
 // The block around the attention, in.size() == kBlockInputs (those that a block does not have undefined); `keep` [B,S,N], 1 where a
 // key counts.  None where some part of it does not take the call.
-OptTensor block(const std::vector<OptTensor> &in, const OptTensor &keep, int64_t heads, double eps_m, double eps_z, double inf) {
+OptTensor block(const std::vector<OptTensor> &in, const OptTensor &keep, int64_t heads, double eps_m, double eps_z, double inf, int64_t flags) {
     Tensor t[kBlockInputs];
     TORCH_CHECK(in.size() == kBlockInputs, "block: wrong number of inputs");
     for (int i = 0; i < kBlockInputs; ++i)
@@ -1020,7 +1021,7 @@ OptTensor block(const std::vector<OptTensor> &in, const OptTensor &keep, int64_t
             for (int i : {kZ, kNormZW, kNormZB, kZW}) t[i] = PairOperands::ready(t[i]);
             bias = PairOperands(t[kZ], t[kNormZW], t[kNormZB], t[kZW]).forward(eps_z, stats_z);
         }
-        r = SlotAttention::enqueue(P, mask, bias, gated);
+        r = SlotAttention::enqueue(P, mask, bias, gated, flags);
         const Tensor o = r.ob.view({rows, W * hd}).narrow(1, (gated ? 1 : 0) * hd, hd);
         y = lin_forward(o, {t[kO]}, t[kOBias]);
         if (!y.defined()) y = at::linear(o, t[kO], t[kOBias].defined() ? OptTensor(t[kOBias]) : OptTensor());
@@ -1051,10 +1052,11 @@ PYBIND11_MODULE(_host, m) {
     const py::call_guard<py::gil_scoped_release> no_gil;
     m.def("attention", &attention, no_gil, py::arg("Q"), py::arg("K"), py::arg("V"), py::arg("res_mask"), py::arg("pair_bias"), py::arg("gate"),
           py::arg("per_head"), py::arg("flags"));
-    m.def("slot_attention", &slot_attention, no_gil, py::arg("P"), py::arg("res_mask"), py::arg("pair_bias"), py::arg("gated"));
+    m.def("slot_attention", &slot_attention, no_gil, py::arg("P"), py::arg("res_mask"), py::arg("pair_bias"), py::arg("gated"), py::arg("flags"));
     m.def("linear", &linear, no_gil, py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("dx_place"));
     m.def("stacked_projection", &stacked_projection, no_gil, py::arg("x"), py::arg("gate_bias"), py::arg("weights"));
     m.def("layer_norm", &layer_norm, no_gil, py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("eps"));
     m.def("pair_bias", &pair_bias, no_gil, py::arg("z"), py::arg("ln_weight"), py::arg("ln_bias"), py::arg("eps"), py::arg("weight"));
-    m.def("block", &block, no_gil, py::arg("inputs"), py::arg("keep"), py::arg("heads"), py::arg("eps_m"), py::arg("eps_z"), py::arg("inf"));
+    m.def("block", &block, no_gil, py::arg("inputs"), py::arg("keep"), py::arg("heads"), py::arg("eps_m"), py::arg("eps_z"), py::arg("inf"),
+          py::arg("flags"));
 }

@@ -611,7 +611,7 @@ class _SlotAttention:
             q, k, v, *g = P.unbind(3)[:4 if gated else 3]
             out = evoformer_attention(q, k, v, res_mask, pair_bias, layout="ds4sci", gate=g[0] if gated else None)
             return out, torch.empty_like(out)
-        return _lib.host().slot_attention(P, res_mask, pair_bias, bool(gated))
+        return _lib.host().slot_attention(P, res_mask, pair_bias, bool(gated), FLAGS)
 
 
 def slot_attention(P, res_mask=None, pair_bias=None, gated: bool = False):

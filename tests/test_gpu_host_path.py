@@ -138,3 +138,26 @@ def test_traced_calls_compute_on_replay(gpu_device):
         # (the block and its slots go another way under the tracer: their results differ by roundings to bf16)
         assert torch.isfinite(got).all() and (got - want).norm() <= 1e-2 * want.norm(), name
         assert "^" in str(traced.graph) or "^" in str(traced.inlined_graph), name
+
+
+def test_the_flags_reach_the_slots_and_the_block(gpu_device, monkeypatch):
+    """`FLAGS` selects kernels for every call: with the plain fp32-arithmetic kernels the results differ by roundings."""
+    import evoformer_triton_amd.evoformer as E
+    from evoformer_triton_amd import _lib
+    (q, k, v, gate), mask, bias = _attention_operands(gpu_device)
+    P = torch.stack([q, k, v, gate], 3).contiguous()
+    blk, m, z = _gpu_block(gpu_device)
+
+    def run():
+        p, mm = P.detach().requires_grad_(), m.detach().requires_grad_()
+        out, _ = E.slot_attention(p, mask, bias, gated=True)
+        y = blk(mm, z)
+        return [out, *torch.autograd.grad(out, p, torch.ones_like(out)), y, *torch.autograd.grad(y, mm, torch.ones_like(y))]
+
+    got = run()
+    monkeypatch.setattr(E, "FLAGS", _lib.EVO_FLAG_FORCE_GENERIC)
+    want = run()
+    for a, b in zip(got, want):
+        assert not torch.equal(a, b) and (a.float() - b.float()).norm() <= 2e-2 * b.float().norm()
+    ref = E.evoformer_attention(q, k, v, mask, bias, layout="ds4sci", gate=gate)
+    assert torch.equal(want[0], ref)
