@@ -550,6 +550,27 @@ bool lin_ok(const Tensor &a, const std::vector<Tensor> &w) {
     const int64_t rows = w[0].size(0), n = rows * (int64_t)w.size(), k = w[0].size(1);
     return n <= INT32_MAX && k <= INT32_MAX && rows % 64 == 0 && evoattn_linear_dw_workspace_bytes(a.size(0), (int32_t)n, (int32_t)k, evo_dtype(dt)) != 0;
 }
+// Where the library's kernels take over.  They run a large product in half to three quarters of the time of linear.hip's (which waits
+// for memory once per 64 of the contraction), and cost 18 us of host time and, with several weights, 6 us for a copy of them
+// (forward: 20 with the padded bias).  linear.hip takes 2.7 us for a round of 512 workgroups and 1.2 for each of its stages; up to 90 us
+// by this count the two are level or what the library saves is less than what it costs.  bf16, rows, n, k: own / library, us:
+//   y    8192, 1024, 1024 22 / 22; 32 768, 1024, 256 30 / 30; 98 304, 1024, 256 84 / 77; 8192, 4096, 1024 83 / 56; beyond: 131 072, 1024, 256
+//        163 / 107; 16 384, 3072, 768 100 / 68; 32 768, 2048, 2048 300 / 191; 131 072, 4096, 4096 5044 / 2878
+//   dx   32 768, 1024, 256 25 / 23; 98 304, 1024, 256 71 / 54; 32 768, 1024, 1024 87 / 65; beyond: 16 384, 3072, 768 108 / 68; 32 768, 2048,
+//        2048 342 / 216
+// (Whole block, 98 304 rows of 256: 1036 us with linear.hip throughout, 1080 with the library for y and dx.)
+bool lin_rows_pay(int64_t rows, int64_t outs, int64_t depth) {
+    const int64_t tiles = ((rows + 127) / 128) * ((outs + 127) / 128), rounds = (tiles + 511) / 512, stages = (depth + 63) / 64;
+    return (double)rounds * (2.7 + 1.2 * (double)stages) <= 90.0;
+}
+// dW and the column sums, of which the library's way takes 42 us of host time: level at 64 stages in all rounds of 512 workgroups.  32 768,
+// 1024, 256 38 / 51; 131 072, 1024, 256 124 / 131; 32 768, 1024, 1024 99 / 94; beyond: 32 768, 768, 768 99 / 70; 65 536, 1024, 1024 213 / 171;
+// 8192, 4096, 4096 367 / 245; and where a slice's gradient in fp32 is itself large: 1024, 4096, 1024 29 / 44, but 1024, 4096, 4096 72 / 53.
+bool lin_weight_pays(int64_t rows, int64_t n, int64_t k, size_t workspace) {
+    const int64_t slices = (int64_t)(workspace / ((size_t)(n * k + n) * sizeof(float))), wgs = ((n + 127) / 128) * ((k + 127) / 128) * slices;
+    return n * k <= (int64_t)1 << 22 && (wgs + 511) / 512 * ((rows + slices * 64 - 1) / (slices * 64)) <= 64;
+}
+
 struct WeightPtrs {
     const void *p[4] = {};
     explicit WeightPtrs(const std::vector<Tensor> &w) {
@@ -561,6 +582,7 @@ struct WeightPtrs {
 Tensor lin_forward(const Tensor &a, const std::vector<Tensor> &w, const Tensor &bias) {
     if (at::autocast::is_autocast_enabled(at::kCUDA) || !lin_ok(a, w) || a.size(1) != w[0].size(1)) return Tensor();
     const int64_t n = w[0].size(0) * (int64_t)w.size();
+    if (!lin_rows_pay(a.size(0), n, a.size(1))) return Tensor();
     const int64_t from = bias.defined() ? n - bias.numel() : 0;
     if (bias.defined() && (!plain(bias) || bias.dim() != 1 || bias.scalar_type() != a.scalar_type() || bias.device() != a.device() || !bias.is_contiguous() ||
                            from < 0 || from % 16 || (uintptr_t)bias.data_ptr() % 16))
@@ -576,7 +598,7 @@ Tensor lin_forward(const Tensor &a, const std::vector<Tensor> &w, const Tensor &
 // dy w into `dx`, whose rows may lie apart; false where the kernels do not take it
 bool lin_input_grad(const Tensor &dy, const std::vector<Tensor> &w, const Tensor &dx) {
     if (!lin_ok(dy, w) || !lin_rows_ok(dx, dy.scalar_type()) || dy.size(1) != w[0].size(0) * (int64_t)w.size() || dx.size(0) != dy.size(0) ||
-        dx.size(1) != w[0].size(1) || dx.device() != dy.device())
+        dx.size(1) != w[0].size(1) || dx.device() != dy.device() || !lin_rows_pay(dy.size(0), dx.size(1), dy.size(1)))
         return false;
     c10::DeviceGuard on(dy.device());
     check(evoattn_linear_dx(dy.data_ptr(), dy.stride(0), WeightPtrs(w).p, (int32_t)w.size(), (int32_t)w[0].size(0), dx.data_ptr(), dx.stride(0), dy.size(0),
@@ -592,7 +614,7 @@ std::pair<Tensor, Tensor> lin_weight_grad(const Tensor &dy, const Tensor &x, boo
     if ((dt == at::kBFloat16 || dt == at::kHalf) && plain_modes() && lin_rows_ok(dy, dt) && lin_rows_ok(x, dt) && x.device() == dy.device() &&
         n <= INT32_MAX && k <= INT32_MAX)
         bytes = evoattn_linear_dw_workspace_bytes(rows, (int32_t)n, (int32_t)k, evo_dtype(dt));
-    if (!bytes) return {weight_grad(dy, x), sums ? bias_grad(dy) : Tensor()};
+    if (!bytes || !lin_weight_pays(rows, n, k, bytes)) return {weight_grad(dy, x), sums ? bias_grad(dy) : Tensor()};
     c10::DeviceGuard on(dy.device());
     Tensor out = at::empty({n * k + (sums ? n : 0)}, dy.options()), ws = scratch(bytes, dy);
     check(evoattn_linear_dw(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), out.data_ptr(), sums, ws.data_ptr(), (size_t)ws.numel(), rows, (int32_t)n,
@@ -689,6 +711,16 @@ struct StackedNode : SavingNode {
     }
 };
 
+// x [rows, k] times the stacked weights, `gb` on the last columns
+Tensor stacked_forward(const Tensor &x, const std::vector<Tensor> &weights, const Tensor &gb) {
+    const Tensor y = lin_forward(x, weights, gb);
+    if (y.defined()) return y;
+    const Tensor w = at::cat(weights, 0);
+    OptTensor bias;
+    if (gb.defined()) bias = at::constant_pad_nd(gb, {w.size(0) - gb.size(0), 0});
+    return at::linear(x, w, bias);
+}
+
 // Several projections of one input as one GEMM with their weights stacked; `gate_bias` is added on the last layer's columns.
 // None as above.
 OptTensor stacked_projection(const Tensor &x, const OptTensor &gate_bias, const std::vector<Tensor> &weights) {
@@ -699,17 +731,10 @@ OptTensor stacked_projection(const Tensor &x, const OptTensor &gate_bias, const 
     if (!taken) return std::nullopt;
     {
         at::AutoDispatchBelowADInplaceOrView guard;
-        y = lin_forward(as_rows(x), weights, gb);
-        if (y.defined()) {
-            auto shape = x.sizes().vec();
-            shape.back() = y.size(1);
-            y = y.view(shape);
-        } else {
-            const Tensor w = at::cat(weights, 0);
-            OptTensor bias;
-            if (gb.defined()) bias = at::constant_pad_nd(gb, {w.size(0) - gb.size(0), 0});
-            y = at::linear(x, w, bias);
-        }
+        y = stacked_forward(as_rows(x), weights, gb);
+        auto shape = x.sizes().vec();
+        shape.back() = y.size(1);
+        y = y.view(shape);
     }
     bool needed = SavingNode::wanted(x, gb);
     for (const auto &t : weights) needed |= SavingNode::wanted(t);
@@ -1008,9 +1033,7 @@ OptTensor block(const std::vector<OptTensor> &in, const OptTensor &keep, int64_t
         for (int i : {kNormMW, kNormMB}) t[i] = t[i].defined() ? t[i].contiguous() : t[i];
         stats_m = ln_stats(m, rows);
         x = ln_forward(m, t[kNormMW], t[kNormMB], eps_m, stats_m);
-        P = lin_forward(as_rows(x), w, t[kGBias]);
-        if (!P.defined()) return std::nullopt;
-        P = P.view({B, S, N, W, heads, D});
+        P = stacked_forward(as_rows(x), w, t[kGBias]).view({B, S, N, W, heads, D});
         OptTensor mask, bias;
         if (keep) {
             const Tensor k = keep->to(at::kFloat).contiguous();

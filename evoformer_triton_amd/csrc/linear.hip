@@ -14,8 +14,10 @@
 // while one is computed on: 64 KB, two workgroups per CU.  A 16-byte chunk of a staged row is stored at chunk ^ x(row)
 // (mfma_stream.hip), so that plain reads of 32 rows and transposing reads both touch all banks evenly.  Output tiles are formed
 // transposed (outputs along the accumulator's registers), with the 32 outputs of a tile dealt so that a lane ends up with 16
-// consecutive ones of a row: 32 bytes to store.  The contraction runs in ascending order, which makes y and dx equal to the
-// library's to the bit.
+// consecutive ones of a row: 32 bytes to store.  The contraction runs in ascending order, with one
+// rounding of the fp32 sum.
+//
+// Large products are the library's business: host.cpp has the lines and both sides.
 #include "common.h"
 #include "bwd_common.h"
 #include "kernels.h"
