@@ -406,12 +406,15 @@ const char *evoattn_path(const EvoAttnParams *p, int pass) {
 }
 
 // Whether a kernel that walks over a chunk of S rows, one workgroup per CU with the head's bias resident, is ahead of one
-// whose workgroups take single problems and stream (head dim 32): it gains a quarter to a sixth per row of 225 to 256 keys
-// and pays `start` rows' worth per round and the rows that do not fill its last round; shorter rows leave waves of its eight
-// idle.  (Forward, H = 8: S = 512, N = 256 103 against 120 us; S = 300, N = 248 67 / 75; N = 216 65 / 66; S = 200,
-// N = 200, H = 4 32 / 30.  dK/dV: S = 512, N = 256 133 / 140; S = 300, N = 248 77 / 81; N = 216 67 / 66; S = 200,
-// N = 200, H = 4 35 / 31.)  Rows of exactly 256 keys keep it throughout: there the two are level from a few S rows per
-// workgroup on.
+// whose workgroups take single problems and stream (head dim 32): it gains a quarter to a fifth per row of 225 to 256 keys (both
+// take the same time for all of these) and pays `start` rows' worth per round and the rows that do not fill its last round; shorter
+// rows leave waves of its eight idle.  This kernel / the streaming one, us:
+//   forward  N = 256, H = 8, S = 16 13.9 / 10.7; 64 19.8 / 18.6; 128 29.3 / 29.3; 192 38.9 / 39.0; 256 46.9 / 49.6; 512 88 / 101; H = 4, S = 256
+//            29.5 / 29.1, 512 46.7 / 49.4; N = 248, S = 300, H = 8 67 / 75; N = 216 65 / 66
+//   dK/dV    N = 256, H = 8, S = 16 18.2 / 11.4; 64 26.9 / 23.3; 96 33.2 / 30.3; 128 39.0 / 40.8; 192 50.4 / 55.7; 512 130 / 155; N = 232,
+//            S = 128 34.4 / 39.1 (left to the other one by this count)
+// Rows of exactly 256 keys keep it throughout, a length at which callers of the C ABI (and the tests of capture and of the library's own
+// allocations) count on these kernels; below some 100 S rows at 8 heads that costs 1 to 7 us.
 static bool ring_pays(const EvoAttnParams &p, double start, double per_row) {
     if (p.N == 256) return true;
     if (p.N <= 224) return false;
