@@ -93,12 +93,16 @@ __global__ void __launch_bounds__(256) mfma_dq(EvoAttnParams p, Extra e) {
     const char *brow = (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)h * p.bias_stride_h +
                                                (int64_t)qrow * p.bias_stride_row) * (bf32 ? 4 : 2);
     // key tile kt of this wave's query rows, in log2 units (zero for a row with every key masked)
-    auto load_btile = [&](int kt, int s, bool dead_row, f32x16 &dst) {
+    auto load_btile = [&](int kt, bool dead_row, f32x16 &dst) {
         if (bdirect) {   // uniform
-            const float mul = dead_row ? 0.0f : kLog2e;
-            const char *row = dead_row ? dead_bias(p, e, b, s) : brow;
-            if (bf32) bias_tile_rows<T, true>(row, kt * 32, p.N, g, mul, dst);
-            else bias_tile_rows<T, false>(row, kt * 32, p.N, g, mul, dst);
+            if (dead_row) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dst[r] = 0.0f;
+            } else if (bf32) {
+                bias_tile_rows<T, true>(brow, kt * 32, p.N, g, kLog2e, dst);
+            } else {
+                bias_tile_rows<T, false>(brow, kt * 32, p.N, g, kLog2e, dst);
+            }
             return;
         }
         if (e.bq16) {   // uniform: a bias in the dtype of q is prepared as given, 16 bits per entry
@@ -113,7 +117,7 @@ __global__ void __launch_bounds__(256) mfma_dq(EvoAttnParams p, Extra e) {
     f32x16 bres[NRES];
     if (BIAS_RESIDENT) {
 #pragma unroll
-        for (int j = 0; j < NRES; ++j) load_btile(min(wave + 4 * j, NT - 1), 0, false, bres[j]);
+        for (int j = 0; j < NRES; ++j) load_btile(min(wave + 4 * j, NT - 1), false, bres[j]);
     }
 
     const uint2 one3 = ones3<T>();
@@ -208,7 +212,7 @@ __global__ void __launch_bounds__(256) mfma_dq(EvoAttnParams p, Extra e) {
                             for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
                         }
                     } else {
-                        load_btile(kt, s, dead, acc);
+                        load_btile(kt, dead, acc);
                     }
                 }
 #pragma unroll
@@ -411,8 +415,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_dkdv(EvoAttnPar
     // the caller's tensor
     const bool bdirect = HAS_BIAS && e.bias_direct;
     const bool bf32 = p.bias_dtype == EVO_F32;
-    const char *bmat = dead ? dead_bias(p, e, pr.b, pr.s) : (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h) * (bf32 ? 4 : 2);
-    const unsigned brow_stride = dead ? 0u : (unsigned)p.bias_stride_row;
+    const char *bmat = (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h) * (bf32 ? 4 : 2);
     const float bmul = dead ? 0.0f : kLog2e;
     const unsigned short *btile16 = !TILE16 ? nullptr
                                     : dead  ? e.bk16 + e.zero_tile + lane * 8
@@ -430,8 +433,10 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_dkdv(EvoAttnPar
         if constexpr (TILE16) {
             load_tile16(btile16 + (int64_t)min(qt, NT - 1) * bstep, dst);
         } else if (HAS_BIAS && bdirect) {   // uniform
-            if (bf32) bias_tile_cols<T, true>(bmat, keyc, min(qt, NT - 1) * 32, p.N, brow_stride, g, bmul, dst);
-            else bias_tile_cols<T, false>(bmat, keyc, min(qt, NT - 1) * 32, p.N, brow_stride, g, bmul, dst);
+            const char *mat = dead ? dead_bias(p, e, pr.b, pr.s) : bmat;
+            const unsigned stride = dead ? 0u : (unsigned)p.bias_stride_row;
+            if (bf32) bias_tile_cols<T, true>(mat, keyc, min(qt, NT - 1) * 32, p.N, stride, g, bmul, dst);
+            else bias_tile_cols<T, false>(mat, keyc, min(qt, NT - 1) * 32, p.N, stride, g, bmul, dst);
         } else if (HAS_BIAS) {
             const float *src = btile + (int64_t)min(qt, NT - 1) * bstep;
             load_tile32(src, dst);

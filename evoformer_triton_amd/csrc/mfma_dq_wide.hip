@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_dq_wide(EvoAttn
     const float *ztile = e.bq + e.zero_tile + lane * 4;
     const bool bdirect = HAS_BIAS && e.bias_direct;
     const bool bf32 = p.bias_dtype == EVO_F32;
-    const char *brow = dead ? dead_bias(p, e, pr.b, pr.s) : (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h +
+    const char *brow = (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h +
                                                (int64_t)qrow * p.bias_stride_row) * (bf32 ? 4 : 2);
     const unsigned short *btile16 = !TILE16 ? nullptr
                                     : dead  ? e.bq16 + e.zero_tile + lane * 8
@@ -98,8 +98,9 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_dq_wide(EvoAttn
         }
         if (bdirect) {   // uniform
             const float mul = dead ? 0.0f : kLog2e;
-            if (bf32) bias_tile_rows<T, true>(brow, kt * 32, p.N, g, mul, dst);
-            else bias_tile_rows<T, false>(brow, kt * 32, p.N, g, mul, dst);
+            const char *row = dead ? dead_bias(p, e, pr.b, pr.s) : brow;
+            if (bf32) bias_tile_rows<T, true>(row, kt * 32, p.N, g, mul, dst);
+            else bias_tile_rows<T, false>(row, kt * 32, p.N, g, mul, dst);
             return;
         }
         const float *src = dead ? ztile : btile0 + (int64_t)kt * 1024;

@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_fwd(EvoAttnPara
     // caller's tensor
     const bool bdirect = HAS_BIAS && e.bias_direct;
     const bool bf32 = p.bias_dtype == EVO_F32;
-    const char *brow = dead ? dead_bias(p, e, pr.b, pr.s) : (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h +
+    const char *brow = (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h +
                                                (int64_t)qrow * p.bias_stride_row) * (bf32 ? 4 : 2);
     const float bmul = dead ? 0.0f : kLog2e;
     const unsigned short *btile16 = !TILE16 ? nullptr
@@ -142,8 +142,9 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) mfma_fwd(EvoAttnPara
         if constexpr (TILE16) {
             load_tile16(btile16 + (int64_t)min(kt, NT - 1) * bstep, dst);
         } else if (HAS_BIAS && bdirect) {   // uniform
-            if (bf32) bias_tile_rows<T, true>(brow, min(kt, NT - 1) * 32, p.N, g, bmul, dst);
-            else bias_tile_rows<T, false>(brow, min(kt, NT - 1) * 32, p.N, g, bmul, dst);
+            const char *row = dead ? dead_bias(p, e, pr.b, pr.s) : brow;
+            if (bf32) bias_tile_rows<T, true>(row, min(kt, NT - 1) * 32, p.N, g, bmul, dst);
+            else bias_tile_rows<T, false>(row, min(kt, NT - 1) * 32, p.N, g, bmul, dst);
         } else if (HAS_BIAS) {
             const float *src = btile + (int64_t)min(kt, NT - 1) * bstep;
             load_tile32(src, dst);
