@@ -52,8 +52,8 @@ def _units():
         units.append((f"mfma_fwdr_d{d}", "mfma_fwd_ring.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
         units.append((f"mfma_dqr_d{d}", "mfma_dq_ring.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
         units.append((f"mfma_kvr_d{d}", "mfma_dkdv_ring.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
-    # head dim 128: the one-workgroup-per-problem kernels (the chunk-of-rows kernels and the
-    # dBias kernel keep more per wave than 256 registers hold at that width)
+    # head dim 128: the kernels whose rows stream through LDS and the one-workgroup-per-problem dQ (the chunk-of-rows kernels
+    # keep more per wave than 256 registers hold at that width)
     units.append(("mfma_stream_d128", "mfma_stream.hip", ["-DEVO_D=128", *VGPR_FORM]))
     units.append(("mfma_bwd_d128", "mfma_bwd.hip", ["-DEVO_D=128", *VGPR_FORM]))
     return units

@@ -164,12 +164,12 @@ static bool dq_wide_grid_ok(const EvoAttnParams &p) {
 // blocks of 256 keys with one query tile), or dQ from the kernel whose waves own their query rows for all keys
 // and the dBias partials from a kernel of their own that forms dS a second time.  The pair is taken where
 // the one kernel has no form (beyond 768 keys; head dim 64 beyond 128 keys; head dim 8 beyond 512) and, between
-// 513 and 768 keys, where the row leaves the one kernel's last 256-key block mostly empty.  Whole backward,
-// bf16, H = 4, head dim 32, one kernel / the pair: N = 320 (S = 128) 92 / 110 us; N = 352, 448, 480 (S = 256)
-// 177 / 190, 259 / 274, 277 / 291 us; N = 576, 704, 736 (S = 256) 459 / 436, 633 / 623, 660 / 654 us; N = 640
-// (B = 2, S = 256) 1.06 / 0.99 ms; head dim 16, H = 8, S = 512: N = 576 1.51 / 1.46 ms, N = 640 1.72 / 1.63 ms,
-// N = 704 2.01 / 2.06 ms.  At head dim 128 the one kernel is the one-workgroup-per-problem form, one workgroup per CU without
-// a prefetch: dQ and dBias, H = 4, N = 512, S = 64 245 / 172 us, N = 201, S = 32 58 / 38 us.
+// 513 and 768 keys, where the row leaves the one kernel's last 256-key block mostly empty.  dQ with dBias, bf16, one kernel / the
+// pair (at head dim 32 stream_dq and mfma_dbias), us: H = 4, head dim 32: N = 320 (S = 128) 40 / 58; N = 352, 448, 480, 512
+// (S = 256) 79 / 104, 146 / 161, 155 / 169, 158 / 178; N = 576, 704, 736, 768 267 / 250, 363 / 358, 367 / 374, 378 / 390; N = 640
+// (B = 2) 650 / 565; S = N = 768 1119 / 1156; head dim 16, H = 8, S = 512: N = 576, 640, 704 881 / 838, 1003 / 915, 1145 / 1196.
+// At head dim 128 the one kernel is the one-workgroup-per-problem form, one workgroup per CU without a prefetch: H = 4, N = 512,
+// S = 64 241 / 152, N = 201, S = 32 54 / 35.
 // EVO_FLAG_DEBUG_NO_DQ_SPLIT selects the one kernel, for comparison.
 static bool dq_split_ok(const EvoAttnParams &p) {
     if (p.D == 128 && p.N > 2048) return false;   // (rows that long keep the plain kernels at that head dim)
@@ -178,15 +178,11 @@ static bool dq_split_ok(const EvoAttnParams &p) {
     const bool full_blocks = rem == 0 || rem >= (p.D == 32 ? 224 : 192);
     const bool ring = dq_ring_ok(p);
     if (full_blocks && ring) return false;
-    // Fewest S rows: the second kernel's start-up has to pay.  Against the one kernel over a chunk of rows
-    // (N = 768, D = 32: ahead from 8 rows on); where that kernel has no form, against the one-workgroup-per-problem
-    // dQ kernel, which the pair beats from 8 rows on (bf16, dQ + dBias, us, S = 8 / 16 / 32 / 52: D = 8, H = 8, N = 768
-    // 50 / 71 / 102 / 146 against 47 / 92 / 159 / 228; D = 16, N = 1024, S = 8 / 16 / 32: 53 / 84 / 152 against
-    // 63 / 99 / 175; D = 64, H = 4, N = 1024, S = 16 / 32 / 59: 99 / 194 / 327 against 152 / 277 / 599; N = 300,
-    // S = 16 / 32: 32 / 41 against 30 / 47), and from 1024 keys on from 2 rows (whole step, us, the pair against
-    // that kernel: D = 32, H = 8, N = 1024, S = 2 / 3 / 4 / 5 / 7 108 / 113 / 114 / 149 / 159 against 110 / 131 / 150 /
-    // 185 / 215; N = 2048, S = 4 / 7 331 / 600 against 444 / 826; D = 8, S = 7 472 against 730; D = 64, B = 4, H = 32,
-    // N = 1024, S = 4 1.89 against 2.33 ms; at N = 640..768 with S = 5, 6 the one kernel stays ahead, 76 / 103
+    // Fewest S rows: the second kernel's start-up has to pay.  Where the one kernel over a chunk of rows has no form, against the
+    // one-workgroup-per-problem dQ kernel (dQ with dBias, us, that kernel / the pair): D = 8, H = 8, N = 768, S = 8 / 16 / 32 46 / 50,
+    // 92 / 70, 158 / 102; D = 64, H = 4, N = 1024, S = 8 / 16 / 32 89 / 56, 152 / 78, 274 / 152; N = 300, S = 16 / 32 29 / 26, 47 / 33;
+    // N = 130, S = 64 32 / 27; and from 1024 keys on from 2 rows: D = 32, H = 8, N = 1024, S = 2 / 4 / 7 35 / 38, 65 / 42, 100 / 53;
+    // N = 2048, S = 4 / 7 215 / 114, 362 / 175 (at N = 640..768 with S = 5, 6 the one kernel stays ahead, whole step 76 / 103
     // against 88 / 111).  Beyond 2048 keys that kernel has no form either.
     const int min_s = p.D == 128 ? 2 : p.N >= 1024 ? 2 : !ring ? (p.D == 64 ? 16 : 8) : p.D == 32 && p.N > 512 ? 8 : 64;
     if (!p.dbias || p.S < min_s || p.N <= min_n || (p.flags & EVO_FLAG_DEBUG_NO_DQ_SPLIT) || bias_direct(p) || !dq_wide_grid_ok(p)) return false;

@@ -7,10 +7,10 @@
 // 11 sum of slices, 16 + 6 LayerNorm backward, each a launch or two with an array of z's size in between, the products
 // at 18 us of host time each; here 9.5 forward, 17.5 + 6 backward.
 //
-// Results are those of the separate steps to the bit: the normalised row is rounded to 16 bits before the product and the
-// gradient of the normalised row after it, the LayerNorm sums are in layernorm.hip's order, and the matrix instruction adds
-// in the order of the library's.  (It matters: the gradient of the LayerNorm's bias is zero but for those roundings, since
-// a constant added to a query's bias changes no probability.)
+// The rounding is that of the separate steps: the normalised row to 16 bits before the product, the gradient of the
+// normalised row after it, and the LayerNorm sums in layernorm.hip's order; the matrix instruction adds in the order of the
+// library's kernels seen at these shapes.  (It matters for comparisons: the gradient of the LayerNorm's bias is zero but for
+// those roundings, since a constant added to a query's bias changes no probability.)
 //
 // A wave owns 32 rows (pairs) at a time.  LayerNorm steps work as in layernorm.hip: C / 8 lanes per row, 16 bytes each.  The
 // products are v_mfma_f32_16x16x32 with the heads as one side (lane l, q = l / 16: operands row l % 16, contraction
@@ -66,7 +66,7 @@ struct PairBiasFwd {
     float eps;
 };
 
-// SPLIT: every 32 channels of a product are summed apart and the sums added, as the library does for so few rows.
+// SPLIT: every 32 channels of a product are summed apart and the sums added, as the library was seen to do for so few rows (of 128 channels).
 template <typename T, int C, bool SPLIT>
 __global__ void __launch_bounds__(kPbWaves * 64) pair_bias_fwd(PairBiasFwd<T> p) {
     typedef typename Mfma<T>::v8 v8;
@@ -333,7 +333,7 @@ static int pb_fwd(const PairBiasFwd<T> &p, int cols, hipStream_t st) {
         else if (cols == 128) pair_bias_fwd<T, 128, SPLIT><<<grid, kPbWaves * 64, 0, st>>>(p);
         else pair_bias_fwd<T, 256, SPLIT><<<grid, kPbWaves * 64, 0, st>>>(p);
     };
-    if (p.rows <= 7424) go(std::true_type());   // (29 x 256: measured on the library's results for rows of 128)
+    if (p.rows <= 7424) go(std::true_type());   // (29 x 256: seen in the library's results for rows of 128; it changes roundings, not the time)
     else go(std::false_type());
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? EVO_OK : EVO_EHIP - (int)err;

@@ -74,7 +74,8 @@ enum {
     EVO_FLAG_GATE_DOUT_INPLACE = 0x80,
     /* Debug switches for A/B comparisons of kernel forms (same results, other kernels); a
      * production caller leaves them clear.  All other bits of `flags` must be zero. */
-    EVO_FLAG_DEBUG_OTHER_WIDTH  = 0x100,  /* one-workgroup-per-problem kernels: the other of their two workgroup widths (4 / 8 waves) */
+    EVO_FLAG_DEBUG_OTHER_WIDTH  = 0x100,  /* one-workgroup-per-problem kernels that come in two workgroup widths (4 / 8 waves),
+                                             the other one: head dims 8 and 16, dK/dV also 32 */
     EVO_FLAG_DEBUG_NO_KV_RING   = 0x200,  /* dK/dV: the one-workgroup-per-problem kernel instead of the chunk-of-rows one */
     EVO_FLAG_DEBUG_FWD_BIAS_TILES = 0x400, /* chunk-of-rows forward: prepared bias tiles as C operands instead of the caller's 16-bit rows */
     EVO_FLAG_DEBUG_BIAS_TILES   = 0x800,  /* S <= 4: prepare the bias tiles instead of reading the caller's bias */
@@ -209,7 +210,9 @@ int evoattn_bwd(const EvoAttnParams *p, void *hip_stream);
 const char *evoattn_path(const EvoAttnParams *p, int pass);
 
 /* Names of the main kernels that pass would launch, comma separated (e.g. "mfma_fwd_ring",
- * "mfma_dq_ring,mfma_dkdv", "mfma_dq_wide,mfma_dkdv", "f32_dq+f32_dbias,f32_dkdv", "generic"); for reports and profiles. */
+ * "mfma_dq_ring,mfma_dkdv", "mfma_dq_wide,mfma_dkdv", "f32_dq+f32_dbias,f32_dkdv", "generic"); for reports and profiles.
+ * One name stands for a place in the routes, whichever head dim: from 32 on mfma_fwd is the kernel stream_fwd in a profile,
+ * mfma_dq_wide stream_dq and the four-wave mfma_dkdv stream_dkdv, from 64 on mfma_dbias is stream_dbias. */
 const char *evoattn_kernels(const EvoAttnParams *p, int pass);
 
 /* ---- LayerNorm of the block around the attention -------------------------------------------
