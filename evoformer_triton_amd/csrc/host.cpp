@@ -552,18 +552,19 @@ bool lin_ok(const Tensor &a, const std::vector<Tensor> &w) {
 }
 // Where the library's kernels take over.  They run a large product in half to three quarters of the time of linear.hip's (which waits
 // for memory once per 64 of the contraction), and cost 18 us of host time and, with several weights, 6 us for a copy of them
-// (forward: 20 with the padded bias).  linear.hip takes 2.7 us for a round of 512 workgroups and 1.2 for each of its stages; up to 90 us
-// by this count the two are level or what the library saves is less than what it costs.  bf16, rows, n, k: own / library, us:
-//   y    8192, 1024, 1024 22 / 22; 32 768, 1024, 256 30 / 30; 98 304, 1024, 256 84 / 77; 8192, 4096, 1024 83 / 56; beyond: 131 072, 1024, 256
-//        163 / 107; 16 384, 3072, 768 100 / 68; 32 768, 2048, 2048 300 / 191; 131 072, 4096, 4096 5044 / 2878
-//   dx   32 768, 1024, 256 25 / 23; 98 304, 1024, 256 71 / 54; 32 768, 1024, 1024 87 / 65; beyond: 16 384, 3072, 768 108 / 68; 32 768, 2048,
-//        2048 342 / 216
-// (Whole block, 98 304 rows of 256: 1036 us with linear.hip throughout, 1080 with the library for y and dx.)
+// (forward: 20 with the padded bias).  linear.hip takes 1.2 us for each stage of 64 of each round of 512 workgroups; up to 64 of these the
+// two are level, or what the library saves is less than what it costs.  bf16, back to back, rows, n, k (stages in all rounds): own / library, us:
+//   y    8192, 1024, 1024 (16) 22 / 22; 32 768, 1024, 256 (16) 30 / 30; 98 304, 1024, 256 (48) 84 / 77; 8192, 4096, 1024 (64) 83 / 56;
+//        beyond: 16 384, 3072, 768 (72) 100 / 68; 32 768, 2048, 2048 300 / 191; 131 072, 4096, 4096 5044 / 2878
+//   dx   32 768, 1024, 256 (16) 25 / 23; 98 304, 1024, 256 (48) 71 / 54; 2048, 4096, 1024 (64) 65 / 33; beyond: 16 384, 3072, 768 (96)
+//        108 / 68; 32 768, 2048, 2048 342 / 216
+// Whole block steps, linear.hip throughout / the library beyond, us: 131 072 rows of 256 (64 for y) 1102 / 1137; 32 768 of 512, n = 2048 (64)
+// 793 / 808; 32 768 of 768, n = 1536 (72) 866 / 797; 65 536 of 512, n = 2048 (128) 1490 / 1430; 16 384 of 1024, n = 4096 (128) 1115 / 1014.
 bool lin_rows_pay(int64_t rows, int64_t outs, int64_t depth) {
-    const int64_t tiles = ((rows + 127) / 128) * ((outs + 127) / 128), rounds = (tiles + 511) / 512, stages = (depth + 63) / 64;
-    return (double)rounds * (2.7 + 1.2 * (double)stages) <= 90.0;
+    const int64_t tiles = ((rows + 127) / 128) * ((outs + 127) / 128);
+    return (tiles + 511) / 512 * ((depth + 63) / 64) <= 64;
 }
-// dW and the column sums, of which the library's way takes 42 us of host time: level at 64 stages in all rounds of 512 workgroups.  32 768,
+// dW and the column sums, of which the library's way takes 42 us of host time: level at 64 of its stages.  32 768,
 // 1024, 256 38 / 51; 131 072, 1024, 256 124 / 131; 32 768, 1024, 1024 99 / 94; beyond: 32 768, 768, 768 99 / 70; 65 536, 1024, 1024 213 / 171;
 // 8192, 4096, 4096 367 / 245; and where a slice's gradient in fp32 is itself large: 1024, 4096, 1024 29 / 44, but 1024, 4096, 4096 72 / 53.
 bool lin_weight_pays(int64_t rows, int64_t n, int64_t k, size_t workspace) {
