@@ -3,17 +3,17 @@
 The reference stops at the attention itself and returns O ungated (evoformer.py:735); in an
 Evoformer block the steps around it are a LayerNorm, the Q/K/V and gate projections, the
 pair-bias projection from the pair representation, sigmoid(gate) * O and the output
-projection.  This module does those with the library GEMMs (torch.nn.functional.linear is
-hipBLASLt on ROCm; the weight gradients are summed over slices of the rows, which as single
-GEMMs would leave most of the chip idle) and this package's LayerNorm kernels, and lays the
-results out so that the attention kernels read them as they fall:
+projection.  This module does those with this package's LayerNorm and Linear kernels (csrc/linear.hip;
+fp32, large products and sizes that it does not take through the library's GEMMs, the weight
+gradients summed over slices of the rows, which as single GEMMs would leave most of the chip
+idle), and lays the results out so that the attention kernels read them as they fall:
 
   * in 16-bit on the GPU Q, K, V and the gate come out of one GEMM with the four weights stacked,
     as [B,S,N,4*H*D]; viewed as [B,S,N,4,H,D] each is a slot that the kernels take by its strides
     (per-head rows, a token's 4*H*D elements from the next token's): no permute, no copy, and the
     gradients come back in the same arrangement, so the projection's backward is one GEMM for the
     input and one for the weights (`evoformer._SlotAttention`);
-  * elsewhere (fp32, under the tracer, head dims that need padding) they come out of the four
+  * elsewhere (fp32, under a tracer, head dims that need padding) they come out of the four
     Linear layers as [B,S,N,H*D], which viewed as [B,S,N,H,D] is the per-head ("ds4sci") layout;
   * the gate is applied in the forward kernel's epilogue and its gradient comes from the
     backward (`evoformer_attention(..., gate=g)`), so sigmoid(g) * O never makes a round trip
@@ -171,8 +171,8 @@ def _layer_norm(layer: nn.LayerNorm, x: torch.Tensor) -> torch.Tensor:
 
 
 def _pair_bias(norm: nn.LayerNorm, layer: nn.Linear, z: torch.Tensor) -> Optional[torch.Tensor]:
-    """Linear(LayerNorm(z)) permuted to [B,1,H,N,N] in one pass over z (csrc/pair_bias.hip), with the results of the separate
-    steps.  None where that kernel does not take the call."""
+    """Linear(LayerNorm(z)) permuted to [B,1,H,N,N] in one pass over z (csrc/pair_bias.hip), rounded where the separate steps
+    round.  None where that kernel does not take the call."""
     if torch.compiler.is_compiling() or layer.bias is not None or z.dim() != 4:
         return None
     return _lib.host().pair_bias(z, norm.weight, norm.bias, norm.eps, layer.weight)
