@@ -89,6 +89,23 @@ struct Call {
     bool gated;
 };
 
+// A mask and a bias of the right shapes and dtypes into the parameter block: their addresses and strides.
+void point_at(EvoAttnParams &p, Tensor &mask, Tensor &bias) {
+    if (mask.defined()) {
+        if (mask.stride(4) != 1) mask = mask.contiguous();
+        p.mask_stride_b = mask.size(0) == p.B && p.B > 1 ? mask.stride(0) : 0;
+        p.mask_stride_s = mask.size(1) == p.S && p.S > 1 ? mask.stride(1) : 0;
+        p.mask = mask.data_ptr();
+    }
+    if (bias.defined()) {
+        if (bias.stride(4) != 1 || bias.stride(3) < p.N) bias = bias.contiguous();
+        p.bias_stride_b = bias.size(0) == p.B && p.B > 1 ? bias.stride(0) : 0;
+        p.bias_stride_h = bias.stride(2);
+        p.bias_stride_row = bias.stride(3);
+        p.bias = bias.data_ptr();
+    }
+}
+
 // The mask and the bias as the kernels read them; false where they do not fit the shape of Q.
 bool operands(Call &c, const Tensor &q, OptTensor &mask, OptTensor &bias) {
     EvoAttnParams &p = c.p;
@@ -113,10 +130,6 @@ bool operands(Call &c, const Tensor &q, OptTensor &mask, OptTensor &bias) {
                 p.mask_kind = m.is_floating_point() ? EVO_MASK_F32 : EVO_MASK_BOOL;
                 m = m.is_floating_point() ? m.to(at::kFloat) : m.ne(0);
         }
-        if (m.stride(4) != 1) m = m.contiguous();
-        p.mask_stride_b = m.size(0) == p.B && p.B > 1 ? m.stride(0) : 0;
-        p.mask_stride_s = m.size(1) == p.S && p.S > 1 ? m.stride(1) : 0;
-        p.mask = m.data_ptr();
         mask = m;
     } else {
         mask = Tensor();
@@ -129,16 +142,12 @@ bool operands(Call &c, const Tensor &q, OptTensor &mask, OptTensor &bias) {
         c.bias_b = sz[0];
         c.bias_dtype = b.scalar_type();
         if (b.scalar_type() != at::kFloat && b.scalar_type() != q.scalar_type()) b = b.to(at::kFloat);
-        if (b.stride(4) != 1 || b.stride(3) < p.N) b = b.contiguous();
         p.bias_dtype = evo_dtype(b.scalar_type());
-        p.bias_stride_b = b.size(0) == p.B && p.B > 1 ? b.stride(0) : 0;
-        p.bias_stride_h = b.stride(2);
-        p.bias_stride_row = b.stride(3);
-        p.bias = b.data_ptr();
         bias = b;
     } else {
         bias = Tensor();
     }
+    point_at(p, *mask, *bias);
     return true;
 }
 
@@ -170,9 +179,21 @@ Tensor finish_dmask(Tensor d, const Call &c) {
 }
 
 // The backward's scratch and results beside dQ, dK, dV: allocates dBias, dMask and the workspace, sets their
-// pointers in `p`, and enqueues the backward.
-void enqueue_backward(EvoAttnParams &p, const Tensor &like, const Tensor &bias, bool want_dbias, bool want_dmask, Tensor &dbias,
+// pointers in `p`, and enqueues the backward.  `p` holds the mask and the bias as the forward read them, `mask` and `bias` are
+// what was saved of them: hooks on saved tensors may hand back copies, laid out otherwise, for which the forward's prepared
+// operands are made anew (their form depends on strides and alignment).
+void enqueue_backward(EvoAttnParams &p, const Tensor &like, Tensor mask, Tensor bias, bool want_dbias, bool want_dmask, Tensor &dbias,
                       Tensor &dmask) {
+    const EvoAttnParams fwd = p;
+    point_at(p, mask, bias);
+    const bool same = p.mask == fwd.mask && p.bias == fwd.bias && p.mask_stride_b == fwd.mask_stride_b && p.mask_stride_s == fwd.mask_stride_s &&
+                      p.bias_stride_b == fwd.bias_stride_b && p.bias_stride_h == fwd.bias_stride_h && p.bias_stride_row == fwd.bias_stride_row;
+    Tensor prep;
+    if (!same) {
+        prep = scratch(evoattn_prep_bytes(&p), like);
+        p.prep = prep.data_ptr();
+        p.prep_bytes = (size_t)prep.numel();
+    }
     if (want_dbias) {
         dbias = at::empty({p.B, p.H, p.N, p.N}, bias.options());
         p.dbias = dbias.data_ptr();
@@ -185,7 +206,7 @@ void enqueue_backward(EvoAttnParams &p, const Tensor &like, const Tensor &bias, 
     Tensor ws = scratch(evoattn_bwd_workspace_bytes(&p), like);
     p.workspace = ws.data_ptr();
     p.workspace_bytes = (size_t)ws.numel();
-    p.flags |= EVO_FLAG_PREP_VALID;   // same bias and mask as the forward
+    if (same) p.flags |= EVO_FLAG_PREP_VALID;
     check(evoattn_bwd(&p, stream_of(like)), "evoattn_bwd");
 }
 
@@ -241,9 +262,10 @@ struct AttentionNode : SavingNode {
         variable_list out(6);
         {
             at::AutoDispatchBelowADInplaceOrView guard;
-            const Tensor q = saved[0].unpack(), k = saved[1].unpack(), v = saved[2].unpack(), mask = saved[3].unpack(),
-                         bias = saved[4].unpack(), aux = saved[5].unpack(), o = saved[6].unpack(shared_from_this());
-            const Tensor gate = c.gated ? saved[7].unpack() : Tensor();
+            const Tensor q = saved[0].unpack().contiguous(), k = saved[1].unpack().contiguous(), v = saved[2].unpack().contiguous(),
+                         mask = saved[3].unpack(), bias = saved[4].unpack(), aux = saved[5].unpack(),
+                         o = saved[6].unpack(shared_from_this()).contiguous();
+            const Tensor gate = c.gated ? saved[7].unpack().contiguous() : Tensor();
             c10::DeviceGuard on(q.device());
             Tensor dO = grads[0].defined() ? grads[0].contiguous() : at::zeros_like(q);
             if (dO.scalar_type() != q.scalar_type()) dO = dO.to(q.scalar_type());
@@ -252,8 +274,6 @@ struct AttentionNode : SavingNode {
             p.q = q.data_ptr();
             p.k = k.data_ptr();
             p.v = v.data_ptr();
-            p.mask = mask.defined() ? mask.data_ptr() : nullptr;
-            p.bias = bias.defined() ? bias.data_ptr() : nullptr;
             p.dout = dO.data_ptr();
             Tensor dbias, dmask;
             for (int i = 0; i < 3; ++i) out[i] = at::empty_like(q);
@@ -271,7 +291,7 @@ struct AttentionNode : SavingNode {
             }
             const bool want_dmask = mask.defined() && mask.is_floating_point() && task_should_compute_output(3);
             const bool want_dbias = bias.defined() && task_should_compute_output(4);
-            enqueue_backward(p, q, bias, want_dbias, want_dmask, dbias, dmask);
+            enqueue_backward(p, q, mask, bias, want_dbias, want_dmask, dbias, dmask);
             if (want_dbias) out[4] = finish_dbias(dbias, c);
             if (want_dmask) out[3] = finish_dmask(dmask, c);
         }
@@ -423,8 +443,6 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
         p.q = slot(P, p, 0);
         p.k = slot(P, p, 1);
         p.v = slot(P, p, 2);
-        p.mask = mask.defined() ? mask.data_ptr() : nullptr;
-        p.bias = bias.defined() ? bias.data_ptr() : nullptr;
         p.dout = dout;
         p.dq = slot(DP, p, 0);
         p.dk = slot(DP, p, 1);
@@ -438,7 +456,7 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
         } else {
             p.o = out;
         }
-        enqueue_backward(p, P, bias, want_dbias, want_dmask, dbias, dmask);
+        enqueue_backward(p, P, mask, bias, want_dbias, want_dmask, dbias, dmask);
         return DP;
     }
 
@@ -465,7 +483,7 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
         {
             at::AutoDispatchBelowADInplaceOrView guard;
             const auto saved = ctx->get_saved_variables();
-            const Tensor &P = saved[0], &mask = saved[1], &bias = saved[2], &aux = saved[3], &out = saved[4];
+            const Tensor P = saved[0].contiguous(), &mask = saved[1], &bias = saved[2], &aux = saved[3];
             Call c;
             const std::string bytes = ctx->saved_data["call"].toStringRef();
             memcpy(&c, bytes.data(), sizeof c);
@@ -473,6 +491,12 @@ struct SlotAttention : torch::autograd::Function<SlotAttention> {
             if (!grads[0].defined()) {   // the output took no part in what is differentiated
                 res[0] = at::zeros_like(P);
                 return res;
+            }
+            // (a hook on saved tensors may hand back a copy whose rows do not lie as slots do)
+            Tensor out = saved[4];
+            if (!out.strides().equals(slot2.strides())) {
+                const Tensor ob = at::empty_like(P);
+                out = ob.select(3, 0).copy_(out);
             }
             const Tensor &dout = grads[0];
             bool in_place = dout.data_ptr() == slot2.data_ptr() && dout.scalar_type() == slot2.scalar_type() && dout.sizes().equals(slot2.sizes());
@@ -802,7 +826,7 @@ struct LayerNormNode : SavingNode {
         if (!grads[0].defined()) return out;
         {
             at::AutoDispatchBelowADInplaceOrView guard;
-            const Tensor x = saved[0].unpack(), w = saved[1].unpack(), stats = saved[2].unpack();
+            const Tensor x = saved[0].unpack().contiguous(), w = saved[1].unpack(), stats = saved[2].unpack();
             ln_backward(grads[0].contiguous(), x, w, stats, task_should_compute_output(0), w.defined() && task_should_compute_output(1),
                         has_bias && task_should_compute_output(2), out[0], out[1], out[2]);
         }
@@ -899,7 +923,7 @@ struct PairBiasNode : SavingNode {
         if (!grads[0].defined()) return out;
         {
             at::AutoDispatchBelowADInplaceOrView guard;
-            const PairOperands o(saved[0].unpack(), saved[1].unpack(), saved[2].unpack(), saved[3].unpack());
+            const PairOperands o(PairOperands::ready(saved[0].unpack()), saved[1].unpack(), saved[2].unpack(), PairOperands::ready(saved[3].unpack()));
             const bool lw = task_should_compute_output(1), lb = task_should_compute_output(2), w = task_should_compute_output(3);
             Tensor dparams;
             o.backward(grads[0].contiguous(), saved[4].unpack(), task_should_compute_output(0), lw || lb || w, out[0], dparams);
@@ -952,6 +976,7 @@ struct BlockNode : SavingNode {
             at::AutoDispatchBelowADInplaceOrView guard;
             Tensor t[kSaved];
             for (int i = 0; i < kSaved; ++i) t[i] = saved[i].unpack();
+            for (int i : {(int)kM, (int)kX, (int)kP, (int)kOut}) t[i] = t[i].contiguous();   // (after a hook on saved tensors)
             bool want[kBlockInputs], inner = false;
             for (int i = 0; i < kBlockInputs; ++i) {
                 want[i] = t[i].defined() && task_should_compute_output(i);

@@ -236,8 +236,12 @@ def _forward(ctx, Q, K, V, res_mask, pair_bias, layout):
     Qc, Kc, Vc, mask, bias, O, lse, prep, mask_meta, bias_meta = _fwd_impl(Q, K, V, res_mask, pair_bias, layout)
     ctx.save_for_backward(Qc, Kc, Vc, mask, bias, O, lse, prep)  # :729
     ctx.layout, ctx.through_ops = layout, False
-    ctx.mask_meta, ctx.bias_meta = mask_meta, bias_meta
+    ctx.mask_meta, ctx.bias_meta, ctx.seen = mask_meta, bias_meta, _addresses(mask, bias)
     return O
+
+
+def _addresses(mask, bias):
+    return (0 if mask is None else mask.data_ptr(), 0 if bias is None else bias.data_ptr())
 
 
 def _bwd_impl(dO, Q, K, V, mask, bias, O, lse, prep, layout, mask_meta, bias_meta, need_dmask, need_dbias,
@@ -245,11 +249,19 @@ def _bwd_impl(dO, Q, K, V, mask, bias, O, lse, prep, layout, mask_meta, bias_met
     """Allocate the gradients and the workspace and enqueue the backward; `mask` and `bias`
     are the tensors the forward's kernels saw.  With `gate`, `O` is the gated output sigmoid(gate) * O
     and dO its gradient.  Returns (dQ, dK, dV, dmask, dbias) with the last two in the shape and dtype
-    of the caller's tensors, or None."""
+    of the caller's tensors, or None.  Hooks on saved tensors may have handed back copies, laid out otherwise: strides
+    are read anew, and the forward's prepared operands serve only the strides they were made for."""
     lib = _lib.load()
     B, S, N, H, D = Q.shape
     mask_kind, mstr, mask_orig = mask_meta
     bias_dt, bstr, bias_orig = bias_meta
+    Q, K, V, O = Q.contiguous(), K.contiguous(), V.contiguous(), O.contiguous()
+    gate = None if gate is None else gate.contiguous()
+    if Q.numel():
+        fwd_strides = mstr, bstr
+        mask, mask_kind, mstr = _prep_mask(mask, B, S, N, Q.device)
+        bias, bias_dt, bstr = _prep_bias(bias, B, H, N, Q.dtype, Q.device)
+        prep_valid = prep_valid and (mstr, bstr) == fwd_strides
     if Q.numel() == 0:          # empty problem: empty gradients, zeros for the bias and a floating mask
         dmask = dbias = None
         if need_dbias and bias is not None:
@@ -310,7 +322,7 @@ def _backward(ctx, dO, need_dmask, need_dbias):
         return dQ, dK, dV, (dmask if want_dmask else None), (dbias if need_dbias and pair_bias is not None else None)
     Q, K, V, mask, bias, O, lse, prep = ctx.saved_tensors
     return _bwd_impl(dO, Q, K, V, mask, bias, O, lse, prep, ctx.layout, ctx.mask_meta, ctx.bias_meta,
-                     need_dmask, need_dbias)
+                     need_dmask, need_dbias, prep_valid=_addresses(mask, bias) == ctx.seen)
 
 
 # ---- the same two calls as registered operators (torch.ops.evoattn.fwd / .bwd) ------------------
@@ -330,8 +342,7 @@ def _op_fwd(Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor, res_mask: Optiona
 
 
 def _seen(mask, bias):
-    return torch.tensor([0 if mask is None else mask.data_ptr(), 0 if bias is None else bias.data_ptr()],
-                        dtype=torch.int64)
+    return torch.tensor(_addresses(mask, bias), dtype=torch.int64)
 
 
 @_op_fwd.register_fake
@@ -547,7 +558,7 @@ class _GatedAttention(torch.autograd.Function):
         Qc, Kc, Vc, mask, bias, O, lse, prep, mask_meta, bias_meta, Og = _fwd_impl(Q, K, V, res_mask, pair_bias, layout,
                                                                                  gate=gate)
         ctx.save_for_backward(Qc, Kc, Vc, mask, bias, O, lse, prep, gate.contiguous())
-        ctx.layout, ctx.mask_meta, ctx.bias_meta, ctx.through_ops = layout, mask_meta, bias_meta, False
+        ctx.layout, ctx.mask_meta, ctx.bias_meta, ctx.through_ops, ctx.seen = layout, mask_meta, bias_meta, False, _addresses(mask, bias)
         return Og
 
     @staticmethod
@@ -562,7 +573,8 @@ class _GatedAttention(torch.autograd.Function):
             return dQ, dK, dV, (dmask if want_dmask else None), (dbias if need_dbias and pair_bias is not None else None), dgate, None
         Q, K, V, mask, bias, O, lse, prep, gate = ctx.saved_tensors
         dQ, dK, dV, dmask, dbias, dgate = _bwd_impl(dOg, Q, K, V, mask, bias, O, lse, prep, ctx.layout, ctx.mask_meta,
-                                                    ctx.bias_meta, ctx.needs_input_grad[3], ctx.needs_input_grad[4], gate=gate)
+                                                    ctx.bias_meta, ctx.needs_input_grad[3], ctx.needs_input_grad[4],
+                                                    prep_valid=_addresses(mask, bias) == ctx.seen, gate=gate)
         return dQ, dK, dV, dmask, dbias, dgate, None
 
 
