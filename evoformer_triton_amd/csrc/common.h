@@ -338,6 +338,20 @@ __device__ __forceinline__ unsigned finite_pair(unsigned w) {
     constexpr unsigned neg_inf = std::is_same<T, f16_t>::value ? 0xfc00u : 0xff80u;
     return w - ((w & 0xffffu) == neg_inf ? 1u : 0u) - ((w >> 16) == neg_inf ? 0x10000u : 0u);
 }
+// Whether a running unsigned maximum of pairs (`pair_max`) leaves room for -inf among them: only -inf and negative NaNs lie that high.
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u16x2_t pair_max(u16x2_t top, unsigned pair) { return __builtin_elementwise_max(top, __builtin_bit_cast(u16x2_t, pair)); }
+template <typename T>
+__device__ __forceinline__ bool maybe_neg_inf(u16x2_t top) {
+    constexpr unsigned neg_inf = std::is_same<T, f16_t>::value ? 0xfc00u : 0xff80u;
+    return top[0] >= neg_inf || top[1] >= neg_inf;
+}
+template <typename T>
+__device__ __forceinline__ uint4 finite8(uint4 v) {
+    if (maybe_neg_inf<T>(pair_max(pair_max(pair_max(pair_max(u16x2_t{0, 0}, v.x), v.y), v.z), v.w)))
+        v = make_uint4(finite_pair<T>(v.x), finite_pair<T>(v.y), finite_pair<T>(v.z), finite_pair<T>(v.w));
+    return v;
+}
 
 // A 32x32 bias tile in accumulator order, times `mul`, straight from the caller's tensor (for
 // problems whose bias is used too few times to pay for the prepared fp32 tiles): `row` points

@@ -198,32 +198,6 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
         }
     }
 
-    if (BIASK == 2) {
-        // -inf becomes the lowest finite value (finite_pair).  Looked for first, with one packed maximum per two entries: as
-        // unsigned numbers only -inf and negative NaNs lie that high.
-        typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-        constexpr unsigned kNegInf = std::is_same<T, f16_t>::value ? 0xfc00u : 0xff80u;
-        u16x2 top = {0, 0};
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const u32x4 w = __builtin_bit_cast(u32x4, bres[j]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned pair = w[i];   // (a vector's element itself cannot be bit-cast: that gives the first one)
-                top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, pair));
-            }
-        }
-        if (__any(top[0] >= kNegInf || top[1] >= kNegInf)) {
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                u32x4 w = __builtin_bit_cast(u32x4, bres[j]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) w[i] = finite_pair<T>(w[i]);
-                bres[j] = __builtin_bit_cast(v8, w);
-            }
-        }
-    }
-
     const int s_begin = c * e.chunk, s_end = min(p.S, s_begin + e.chunk);
     const int nrows = s_end - s_begin;
     if (nrows <= 0) return;   // uniform over the workgroup
@@ -308,6 +282,26 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
 
     fetch(0);
     fetch_q(0, qraw);
+    if (BIASK == 2) {
+        // -inf becomes the lowest finite value (finite_pair), looked for first with one packed maximum per two entries.  (Here, with
+        // the first row's loads on their way: ahead of them it cost a short forward 0.3 us.)
+        u16x2_t top = {0, 0};
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const u32x4 w = __builtin_bit_cast(u32x4, bres[j]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) top = pair_max(top, w[i]);
+        }
+        if (__any(maybe_neg_inf<T>(top))) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                u32x4 w = __builtin_bit_cast(u32x4, bres[j]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] = finite_pair<T>(w[i]);
+                bres[j] = __builtin_bit_cast(v8, w);
+            }
+        }
+    }
     stash(0);
 
     for (int t = 0; t < nrows; ++t) {

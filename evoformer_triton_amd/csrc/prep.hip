@@ -86,9 +86,7 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
                                        w[4] | ((unsigned)w[5] << 16), w[6] | ((unsigned)w[7] << 16));
                     }
                 }
-                if (p.dtype == EVO_F16) v = make_uint4(finite_pair<f16_t>(v.x), finite_pair<f16_t>(v.y), finite_pair<f16_t>(v.z), finite_pair<f16_t>(v.w));
-                else v = make_uint4(finite_pair<bf16_t>(v.x), finite_pair<bf16_t>(v.y), finite_pair<bf16_t>(v.z), finite_pair<bf16_t>(v.w));
-                *reinterpret_cast<uint4 *>(&sm[r][c]) = v;
+                *reinterpret_cast<uint4 *>(&sm[r][c]) = p.dtype == EVO_F16 ? finite8<f16_t>(v) : finite8<bf16_t>(v);
             }
             __syncthreads();
             if (tl < ntile) {
