@@ -39,10 +39,22 @@ struct StreamGeo {
 };
 
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// all but the youngest N of the wave's loads and stores (they end in the order they were issued)
+template <int N>
+__device__ __forceinline__ void wait_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void wait_loads_and_lds() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void wait_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// 16 bytes per lane from memory into LDS, lane after lane from `dst` (uniform) on.  As an instruction the compiler does not know:
+// it takes every read of LDS after one that it knows as depending on it and waits for all loads of the wave first, also where
+// the read is of the other buffer, so that no stage was ever on its way while another was computed on.  The kernels wait
+// themselves (`wait_loads`), before the barrier that opens the buffer.  What the compiler counts without these loads only
+// makes its own waits longer: where a wave waits for a bias tile, nothing younger than that tile should be under way.
+// (With the caller's fp32 rows kept unscaled until they are used, and dBias stored without a wait: B = 4, S = 1, N = 1024, H = 32, D = 64, step 691 ->
+// 611 us; three waves per SIMD had hidden most of it elsewhere: S = N = 768, H = 4, D = 32 2311 -> 2284; S = 200, N = 640, H = 5, D = 64 1006 -> 987.)
+// (s_nop: five states between a vector instruction's write of a scalar register and its use as an address.)
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, unsigned char *dst, int off) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16, off, 0, 0, 0);
+    const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)dst;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(base), "v"(off), "s"(rs));
 }
 
 // Rows r0 .. r0 + ROWS - 1 of two arrays that share their strides, into LDS at `dst` and `dst` + ROWS rows: this wave's share
@@ -84,10 +96,14 @@ __device__ __forceinline__ typename Mfma<T>::v8 transposed(const unsigned char *
 }
 
 // The bias tiles of one wave: its 32 rows (or, COLS, its 32 columns) against the tiles of the other side.
-// BT: 1 prepared fp32 tiles (times log2 e), 2 prepared 16-bit tiles as given, 3 the caller's rows (few S rows).
+// BT: 1 prepared fp32 tiles (times log2 e), 2 prepared 16-bit tiles as given; the caller's rows (few S rows), 3 in fp32, 4 in the
+// dtype of q.  A tile is kept as it comes from memory: whatever is done to it (`value`) would wait for it.
+struct Rows16 {   // entry r, the 16 bits as given, in the low half of w[r] (columns) or two to a register (rows)
+    unsigned w[16];
+};
 template <typename T, int BT, bool COLS>
 struct BiasStream {
-    typedef typename std::conditional<BT == 2, Tile16, f32x16>::type Tile;
+    typedef typename std::conditional<BT == 2, Tile16, typename std::conditional<BT == 4, Rows16, f32x16>::type>::type Tile;
     const float *t32;
     const unsigned short *t16;
     const char *mat;
@@ -95,18 +111,16 @@ struct BiasStream {
     unsigned col, row_stride;
     float mul;
     int NT, N, g;
-    bool f32;
     __device__ __forceinline__ BiasStream(const EvoAttnParams &p, const Extra &e, const Prob &pr, int own_tile, int own_row, bool dead, int lane) {
         NT = (p.N + 31) / 32;
         N = p.N;
         g = lane >> 5;
         mul = dead ? 0.0f : kLog2e;
         const int bb = e.bias_batches > 1 ? pr.b : 0;
-        if (BT == 3) {
-            f32 = p.bias_dtype == EVO_F32;
+        if (BT >= 3) {
             row_stride = dead ? 0u : (unsigned)p.bias_stride_row;
             col = (unsigned)own_row;
-            mat = dead ? dead_bias(p, e, pr.b, pr.s) : (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h + (COLS ? 0 : (int64_t)own_row * p.bias_stride_row)) * (f32 ? 4 : 2);
+            mat = dead ? dead_bias(p, e, pr.b, pr.s) : (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h + (COLS ? 0 : (int64_t)own_row * p.bias_stride_row)) * (BT == 3 ? 4 : 2);
         } else {
             const int64_t first = (((int64_t)bb * p.H + pr.h) * NT * NT + (COLS ? own_tile : own_tile * NT)) * 1024;
             step = dead ? 0 : COLS ? (int64_t)NT * 1024 : 1024;
@@ -119,13 +133,28 @@ struct BiasStream {
         t = min(t, NT - 1);
         if constexpr (BT == 1) load_tile32(t32 + t * step, dst);
         if constexpr (BT == 2) load_tile16(t16 + t * step, dst);
-        if constexpr (BT == 3) {
-            if (COLS) {
-                if (f32) bias_tile_cols<T, true>(mat, col, t * 32, N, row_stride, g, mul, dst);
-                else bias_tile_cols<T, false>(mat, col, t * 32, N, row_stride, g, mul, dst);
-            } else {
-                if (f32) bias_tile_rows<T, true>(mat, t * 32, N, g, mul, dst);
-                else bias_tile_rows<T, false>(mat, t * 32, N, g, mul, dst);
+        // (rows: groups past column n repeat the last whole group, columns: rows past n - 1 the last one; as bias_tile_rows and _cols)
+        if constexpr (BT >= 3 && COLS) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const unsigned o = (unsigned)min(t * 32 + crow(r, g), N - 1) * row_stride + col;
+                if constexpr (BT == 3) dst[r] = ((const float *)mat)[o];
+                else dst.w[r] = ((const unsigned short *)mat)[o];
+            }
+        }
+        if constexpr (BT >= 3 && !COLS) {
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+                const int c = min(t * 32 + 8 * rr + 4 * g, N - 4);
+                if constexpr (BT == 3) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>((const float *)mat + c);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) dst[4 * rr + i] = v[i];
+                } else {
+                    const uint2 v = *reinterpret_cast<const uint2 *>((const unsigned short *)mat + c);
+                    dst.w[2 * rr] = v.x;
+                    dst.w[2 * rr + 1] = v.y;
+                }
             }
         }
     }
@@ -135,9 +164,30 @@ struct BiasStream {
             f32x16 v;
             unpack_tile16<T>(t, mul, v);
             return v;
+        } else if constexpr (BT == 3) {
+            f32x16 v;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = t[r] * mul;
+            return v;
+        } else if constexpr (BT == 4) {
+            f32x16 v;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float lo, hi;
+                if (COLS) unpack2<T>(t.w[r], lo, hi);
+                else unpack2<T>(t.w[r >> 1], lo, hi);
+                v[r] = (COLS || r % 2 == 0 ? lo : hi) * mul;
+            }
+            return v;
         } else {
             return t;
         }
+    }
+    // `value`, formed here: the wait for the tile stands before whatever the wave asks for next
+    __device__ __forceinline__ f32x16 take(const Tile &t) const {
+        f32x16 v = value(t);
+        asm volatile("" : "+v"(v));
+        return v;
     }
 };
 template <typename T, bool COLS>
@@ -151,6 +201,7 @@ struct BiasStream<T, 0, COLS> {
         for (int r = 0; r < 16; ++r) z[r] = 0.0f;
         return z;
     }
+    __device__ __forceinline__ f32x16 take(const Tile &t) const { return value(t); }
 };
 
 // ------------------------------------------------------------------ forward
@@ -273,14 +324,17 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3
             for (int i = 0; i < 8; ++i) pf[ts][i] = (T)a[ts / 2][8 * (ts & 1) + i];
         return s;
     };
-    // ST tiles, from tile kt and row kb of the stage on
-    auto step = [&](const unsigned char *buf, int kt, int kb) {
+    // ST tiles, from tile kt and row kb of the stage on; `between`: what is asked for once their bias has arrived
+    auto step = [&](const unsigned char *buf, int kt, int kb, auto between) {
         const float used = mf;
-        f32x16 a[ST];
+        f32x16 a[ST], init[ST];
 #pragma unroll
-        for (int t = 0; t < ST; ++t) score(buf, kb + 32 * t, bias.value(ct[t]), a[t]);
+        for (int t = 0; t < ST; ++t) init[t] = bias.take(ct[t]);
+        between();
 #pragma unroll
         for (int t = 0; t < ST; ++t) bias.load(kt + ST + t, ct[t]);
+#pragma unroll
+        for (int t = 0; t < ST; ++t) score(buf, kb + 32 * t, init[t], a[t]);
         const bool lazy = kt != 0 && !__any(m != used);
         if (!lazy) settle(kt == 0, a, used);
         v8 pf[2 * ST];
@@ -307,11 +361,13 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3
     wait_loads();
     wait_lds_barrier();
     for (int s = 0; s < nst; ++s) {
-        if (s + 1 < nst) fetch(s + 1);
+        auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
         if (active) {
             const unsigned char *buf = lds[s & 1];
-            step(buf, 2 * s, 0);
-            if (ST == 1 && 2 * s + 1 < NT) step(buf, 2 * s + 1, 32);
+            step(buf, 2 * s, 0, next);
+            if (ST == 1 && 2 * s + 1 < NT) step(buf, 2 * s + 1, 32, [] {});
+        } else {
+            next();
         }
         if (s + 1 < nst) {
             wait_loads();
@@ -638,8 +694,11 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 ? 3 : 2) stream_dq(
 #pragma unroll
         for (int r = 0; r < 16; ++r) dq[dt][r] = 0.0f;
 
-    auto tile = [&](const unsigned char *buf, int kt, int kb) {
-        f32x16 a = bias.value(ct), dp;
+    auto tile = [&](const unsigned char *buf, int kt, int kb, auto between) {
+        f32x16 a = bias.take(ct), dp;
+        between();
+        if (WRITE_DS) asm volatile("" ::: "memory");   // (this stage's stores are younger than what `between` asked for)
+        bias.load(kt + 1, ct);
 #pragma unroll
         for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
 #pragma unroll
@@ -650,7 +709,6 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 ? 3 : 2) stream_dq(
         }
         a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (kb + li) * 16), qf[KSD], a);
         dp = Mfma<T>::mma(vaug, gf[KSD], dp);
-        bias.load(kt + 1, ct);
 #pragma unroll
         for (int r = 0; r < 16; ++r) a[r] = fast_exp2(a[r]) * dp[r];
         if (WRITE_DS && q0 + li < p.N) {
@@ -690,14 +748,19 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 ? 3 : 2) stream_dq(
     wait_loads();
     wait_lds_barrier();
     for (int s = 0; s < nst; ++s) {
-        if (s + 1 < nst) fetch(s + 1);
+        auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
         if (active) {
             const unsigned char *buf = lds[s & 1];
-            tile(buf, 2 * s, 0);
-            if (2 * s + 1 < NT) tile(buf, 2 * s + 1, 32);
+            tile(buf, 2 * s, 0, next);
+            if (2 * s + 1 < NT) tile(buf, 2 * s + 1, 32, [] {});
+        } else {
+            next();
         }
         if (s + 1 < nst) {
-            wait_loads();
+            // A stage before the last has two whole tiles: a wave that has queries stored at least eight pieces of dBias after it had asked
+            // for the next stage, and need not wait for them.
+            if (WRITE_DS && active) wait_loads_but<8>();
+            else wait_loads();
             wait_lds_barrier();
         }
     }
@@ -799,8 +862,10 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
         for (int r = 0; r < 16; ++r) dk[dt][r] = dv[dt][r] = 0.0f;
     float dm = 0.0f;
 
-    auto tile = [&](const unsigned char *buf, int qt, int qb) {
-        f32x16 a = bias.value(ct), dp;
+    auto tile = [&](const unsigned char *buf, int qt, int qb, auto between) {
+        f32x16 a = bias.take(ct), dp;
+        between();
+        if (D < 128) bias.load(qt + 1, ct);
 #pragma unroll
         for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
 #pragma unroll
@@ -814,7 +879,7 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
         }
         a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_AQ + (qb + li) * 16), kaug, a);
         dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_AG + (qb + li) * 16), vaug, dp);
-        bias.load(qt + 1, ct);
+        if (D == 128) bias.load(qt + 1, ct);   // (no registers for it any sooner)
         v8 pf[2], ds[2];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -844,11 +909,13 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
     const int nst = (p.N + ROWS - 1) / ROWS;
     finish(0);
     for (int s = 0; s < nst; ++s) {
-        if (s + 1 < nst) fetch(s + 1);
+        auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
         if (active) {
             const unsigned char *buf = lds + (s & 1) * R::STAGE;
-            tile(buf, s * (ROWS / 32), 0);
-            if (ROWS == 64 && 2 * s + 1 < NT) tile(buf, 2 * s + 1, 32);
+            tile(buf, s * (ROWS / 32), 0, next);
+            if (ROWS == 64 && 2 * s + 1 < NT) tile(buf, 2 * s + 1, 32, [] {});
+        } else {
+            next();
         }
         if (s + 1 < nst) finish(s + 1);
     }
@@ -1013,7 +1080,8 @@ template <typename T, int D>
 static int fwd_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const unsigned grid = (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H * p.S);
     if (p.bias_dtype == EVO_NONE) stream_fwd<T, D, 0><<<grid, 256, 0, st>>>(p, e);
-    else if (e.bias_direct) stream_fwd<T, D, 3><<<grid, 256, 0, st>>>(p, e);
+    else if (e.bias_direct && p.bias_dtype == EVO_F32) stream_fwd<T, D, 3><<<grid, 256, 0, st>>>(p, e);
+    else if (e.bias_direct) stream_fwd<T, D, 4><<<grid, 256, 0, st>>>(p, e);
     else if (e.bq16) stream_fwd<T, D, 2><<<grid, 256, 0, st>>>(p, e);
     else stream_fwd<T, D, 1><<<grid, 256, 0, st>>>(p, e);
     return hip_rc();
@@ -1047,13 +1115,15 @@ int EVO_CAT(launch_split_fwd_d, EVO_D)(const EvoAttnParams &p, hipStream_t st) {
 template <typename T, int D>
 static int dq_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const unsigned grid = (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H * p.S);
-    const bool direct = e.bias_direct, t16 = e.bq16 != nullptr;
+    const bool f32_rows = e.bias_direct && p.bias_dtype == EVO_F32, t16_rows = e.bias_direct && !f32_rows, t16 = e.bq16 != nullptr;
     if (p.dbias && p.S != 1) return EVO_EUNSUPPORTED;   // (a sum over S rows is the other kernels' business)
     if (p.bias_dtype == EVO_NONE) stream_dq<T, D, 0, false><<<grid, 256, 0, st>>>(p, e);
-    else if (!p.dbias && direct) stream_dq<T, D, 3, false><<<grid, 256, 0, st>>>(p, e);
+    else if (!p.dbias && f32_rows) stream_dq<T, D, 3, false><<<grid, 256, 0, st>>>(p, e);
+    else if (!p.dbias && t16_rows) stream_dq<T, D, 4, false><<<grid, 256, 0, st>>>(p, e);
     else if (!p.dbias && t16) stream_dq<T, D, 2, false><<<grid, 256, 0, st>>>(p, e);
     else if (!p.dbias) stream_dq<T, D, 1, false><<<grid, 256, 0, st>>>(p, e);
-    else if (direct) stream_dq<T, D, 3, true><<<grid, 256, 0, st>>>(p, e);
+    else if (f32_rows) stream_dq<T, D, 3, true><<<grid, 256, 0, st>>>(p, e);
+    else if (t16_rows) stream_dq<T, D, 4, true><<<grid, 256, 0, st>>>(p, e);
     else if (t16) stream_dq<T, D, 2, true><<<grid, 256, 0, st>>>(p, e);
     else stream_dq<T, D, 1, true><<<grid, 256, 0, st>>>(p, e);
     return hip_rc();
@@ -1079,7 +1149,7 @@ static int dkdv_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
 template <typename T, int D, int NW>
 static int dkdv_bias(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     if (p.bias_dtype == EVO_NONE) return dkdv_launch<T, D, 0, NW>(p, e, st);
-    if (e.bias_direct) return dkdv_launch<T, D, 3, NW>(p, e, st);
+    if (e.bias_direct) return p.bias_dtype == EVO_F32 ? dkdv_launch<T, D, 3, NW>(p, e, st) : dkdv_launch<T, D, 4, NW>(p, e, st);
     return e.bk16 ? dkdv_launch<T, D, 2, NW>(p, e, st) : dkdv_launch<T, D, 1, NW>(p, e, st);
 }
 
