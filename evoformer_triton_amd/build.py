@@ -44,10 +44,9 @@ def _units():
         if d <= 16:
             units.append((f"mfma_fwd_d{d}", "mfma_fwd.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
             units.append((f"mfma_dqw_d{d}", "mfma_dq_wide.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
+            units.append((f"mfma_dbias_d{d}", "mfma_dbias.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
         else:
             units.append((f"mfma_stream_d{d}", "mfma_stream.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
-        if d <= 32:
-            units.append((f"mfma_dbias_d{d}", "mfma_dbias.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
         units.append((f"mfma_bwd_d{d}", "mfma_bwd.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
         units.append((f"mfma_fwdr_d{d}", "mfma_fwd_ring.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
         units.append((f"mfma_dqr_d{d}", "mfma_dq_ring.hip", [f"-DEVO_D={d}", *VGPR_FORM]))

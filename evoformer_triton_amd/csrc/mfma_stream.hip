@@ -1,4 +1,4 @@
-// Forward, dQ, dK/dV and dBias for head dims 32 (without dBias), 64 and 128: one workgroup per block of rows of a problem
+// Forward, dQ, dK/dV and dBias for head dims 32, 64 and 128: one workgroup per block of rows of a problem
 // (b, h, s), the other side's rows streamed through LDS.  Compiled once per head dim (-DEVO_D=32|64|128).
 //
 // The arithmetic is that of the one-workgroup-per-problem kernels for smaller head dims (mfma_fwd.hip, mfma_bwd.hip,
@@ -937,15 +937,22 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
 
 // ------------------------------------------------------------------ dBias partials
 
-// What mfma_dbias.hip is for the smaller head dims: dS a second time, summed over a chunk of S rows in registers.  A
-// workgroup has 128 queries x 64 keys of one (b, h), a wave 32 queries x 2 key tiles.  Keys (K, V, mask columns) are shared and
-// double-buffered in LDS; a wave's own rows of Q and dO come into LDS of its own, which it reads into registers at the
+// What mfma_dbias.hip is for the smallest head dims: dS a second time, summed over a chunk of S rows in registers.  A
+// workgroup has 128 queries x 64 keys (head dim 32: 128) of one (b, h), a wave 32 queries x all of the block's key tiles.  Keys (K, V, mask
+// columns) are shared and double-buffered in LDS; a wave's own rows of Q and dO come into LDS of its own, which it reads into registers at the
 // top of a row and refills at once, so they need no second buffer and no barrier.
+// Bound by the vector unit's issue together with the matrix core (two waves per SIMD), so what can be said once is: the bias of a wave's tiles
+// stays in registers in fp32, log2 units, the first operand C of a tile's chain where it lies (as 16-bit pairs it was unpacked and multiplied
+// per tile and row, 32 instructions of 131); -delta, one value per lane, is the C of the other chain, in place of a matrix step of
+// its own; array bases advance by the scalar unit and a lane's offsets are formed once.  dBias of S = N = 768, H = 4, D = 32 (mfma_dbias.hip
+// before) 595 -> 491 us, of S = 200, N = 640, H = 5, D = 64 with an fp32 bias 238 -> 193; S = 64, N = 512, H = 4, D = 128 78 -> 74.
+// Two tiles per wave and three waves per SIMD at head dim 32: 596; -delta in a matrix step: 516.
 template <int D>
 struct DbStream {
-    static constexpr int KB = 64, QB = 128, BLK = KB * D * 2;
+    static constexpr int TPW = D == 32 ? 4 : 2, KB = TPW * 32, QB = 128, BLK = KB * D * 2;   // key tiles per wave; keys, queries per workgroup
     static constexpr int OFF_V = BLK, OFF_A = 2 * BLK, KEYS = OFF_A + KB * 16;
     static constexpr int OFF_Q = 2 * KEYS, WAVE = 2 * 32 * D * 2, BYTES = OFF_Q + 4 * WAVE;
+    static constexpr int KP = BLK / 4096, QP = 32 * D * 2 / 1024, RPP = 1024 / (D * 2);   // pieces of 1 KB per wave: of an array of keys, of one of queries; rows of one
 };
 
 template <typename T, int D, bool BF32>
@@ -963,54 +970,78 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
     const unsigned bh = (lid / (nkb * nqb)) % (unsigned)(p.B * p.H);
     const int c = lid / (nkb * nqb) / (unsigned)(p.B * p.H), b = bh / p.H, h = bh % p.H;
     const int q0 = qbi * R::QB + wave * 32, k0 = kbi * R::KB, qrow = min(q0 + li, p.N - 1);
-    const bool active = q0 < p.N, two = k0 + 32 < p.N;   // wave-uniform; a second key tile exists
+    const bool active = q0 < p.N;                    // wave-uniform
+    const int tiles = min(R::TPW, NT - k0 / 32);     // of the block's keys that exist
     const int sn2 = (int)p.stride_n * 2, valid = (p.N - 1) * sn2 + D * 2, np256 = (p.N + 255) / 256 * 256;
     const float cs = p.scale * kLog2e;
-    const uint2 one3 = ones3<T>(), zero3 = {0u, 0u};
-    const v8 vaug = aug8<T>(one3, zero3);
+    const uint2 one3 = ones3<T>();
 
-    // the bias of the wave's two tiles, resident: 16-bit pairs as given or fp32 in log2 units
     const int bb = e.bias_batches > 1 ? b : 0;
-    Tile16 b16[2];
-    f32x16 b32[BF32 ? 2 : 1], sum[2];
+    f32x16 bias[R::TPW], sum[R::TPW];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < R::TPW; ++j) {
         const int64_t o = ((((int64_t)bb * p.H + h) * NT + min(q0 >> 5, NT - 1)) * NT + min(k0 / 32 + j, NT - 1)) * 1024;
-        if constexpr (BF32) load_tile32(e.bq + o + lane * 4, b32[j]);
-        else load_tile16(e.bq16 + o + lane * 8, b16[j]);
+        if constexpr (BF32) {
+            load_tile32(e.bq + o + lane * 4, bias[j]);
+        } else {
+            Tile16 t;
+            load_tile16(e.bq16 + o + lane * 8, t);
+            unpack_tile16<T>(t, kLog2e, bias[j]);
+        }
 #pragma unroll
         for (int r = 0; r < 16; ++r) sum[j][r] = 0.0f;
     }
     const int s_begin = c * e.chunk, s_end = min(p.S, s_begin + e.chunk);
     if (s_begin >= s_end) return;   // uniform over the workgroup
 
+    // offsets of this lane's 16 bytes of a piece of keys and of queries (rows past the end repeat the last one), from row 0 of the problem on
+    int koff[R::KP], qoff[R::QP];
+#pragma unroll
+    for (int i = 0; i < R::KP; ++i) {
+        const int r = (wave + 4 * i) * R::RPP + lane / G::C;
+        koff[i] = min(k0 + r, p.N - 1) * sn2 + (((lane % G::C) ^ G::x(r)) << 4);
+    }
+#pragma unroll
+    for (int i = 0; i < R::QP; ++i) {
+        const int r = i * R::RPP + lane / G::C;
+        qoff[i] = min(q0 + r, p.N - 1) * sn2 + (((lane % G::C) ^ G::x(r)) << 4);
+    }
+    const int64_t base0 = (int64_t)b * p.stride_b + (int64_t)h * p.stride_h;
+    auto rows = [&](const void *x, int s) { return __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)x + base0 + (int64_t)s * p.stride_s), 0, valid, 0x00020000); };
     unsigned char *const own = lds + R::OFF_Q + wave * R::WAVE;
     float lse_n = 0.0f, delta_n = 0.0f;
     auto fetch_keys = [&](int s) {
-        const Prob pr = decode_problem(p, bh * (unsigned)p.S + s);
-        const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.k + pr.base), 0, valid, 0x00020000);
-        const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.v + pr.base), 0, valid, 0x00020000);
-        const __amdgpu_buffer_rsrc_t mrs = __builtin_amdgcn_make_buffer_rsrc((void *)(e.m2a + ((int64_t)b * p.S + s) * np256), 0, np256 * 16, 0x00020000);
+        const __amdgpu_buffer_rsrc_t krs = rows(p.k, s), vrs = rows(p.v, s);
         unsigned char *dst = lds + ((s - s_begin) & 1) * R::KEYS;
-        dma_rows<D, R::KB, 4>(krs, vrs, dst, k0, p.N, sn2, wave, lane);
-        if (wave == 0) dma16(mrs, dst + R::OFF_A, (k0 + lane) * 16);
+#pragma unroll
+        for (int i = 0; i < R::KP; ++i) {
+            dma16(krs, dst + (wave + 4 * i) * 1024, koff[i]);
+            dma16(vrs, dst + R::OFF_V + (wave + 4 * i) * 1024, koff[i]);
+        }
+        if (wave < R::KB / 64) {
+            const __amdgpu_buffer_rsrc_t mrs = __builtin_amdgcn_make_buffer_rsrc((void *)(e.m2a + ((int64_t)b * p.S + s) * np256 + k0), 0, R::KB * 16, 0x00020000);
+            dma16(mrs, dst + R::OFF_A + wave * 1024, (wave * 64 + lane) * 16);
+        }
     };
     auto fetch_queries = [&](int s) {
-        const Prob pr = decode_problem(p, bh * (unsigned)p.S + s);
-        const __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.q + pr.base), 0, valid, 0x00020000);
-        const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.dout + pr.base), 0, valid, 0x00020000);
-        dma_rows<D, 32, 1>(qrs, grs, own, q0, p.N, sn2, 0, lane);
-        lse_n = p.lse[pr.row0 + qrow];
-        delta_n = e.delta[pr.row0 + qrow];
+        const __amdgpu_buffer_rsrc_t qrs = rows(p.q, s), grs = rows(p.dout, s);
+#pragma unroll
+        for (int i = 0; i < R::QP; ++i) {
+            dma16(qrs, own + i * 1024, qoff[i]);
+            dma16(grs, own + 32 * G::ROW + i * 1024, qoff[i]);
+        }
+        const int64_t row0 = ((int64_t)bh * p.S + s) * p.N;
+        lse_n = (p.lse + row0)[(unsigned)qrow];
+        delta_n = (e.delta + row0)[(unsigned)qrow];
     };
     fetch_keys(s_begin);
     fetch_queries(s_begin);
     for (int s = s_begin; s < s_end; ++s) {
-        const bool dead = e.dead[b * p.S + s] != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
+        const bool dead = uniform_load(e.dead + b * p.S + s) != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
         wait_loads();
         wait_lds_barrier();
         if (s + 1 < s_end) fetch_keys(s + 1);   // (everybody has left that buffer: it held row s - 1)
-        v8 qf[KS], gf[KS];
+        v8 qf[KS], gf[KSD];
 #pragma unroll
         for (int ks = 0; ks < KSD; ++ks) {
             const int o = G::at(li, 2 * ks + g);
@@ -1018,46 +1049,49 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
             gf[ks] = *reinterpret_cast<const v8 *>(own + 32 * G::ROW + o);
         }
         qf[KSD] = g == 0 ? aug8<T>(one3, pack_split3<T>(-lse_n * kLog2e)) : zero8<T>();
-        gf[KSD] = g == 0 ? aug8<T>(pack_split3<T>(-delta_n), zero3) : zero8<T>();
+        f32x16 nd;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) nd[r] = -delta_n;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (s + 1 < s_end) fetch_queries(s + 1);
 #pragma unroll
-        for (int ks = 0; ks < KSD; ++ks) qf[ks] = dead ? zero8<T>() : scaled8<T>(qf[ks], cs);
+        for (int ks = 0; ks < KSD; ++ks) qf[ks] = scaled8<T>(qf[ks], dead ? 0.0f : cs);
         if (!active || kill) continue;
         const unsigned char *buf = lds + ((s - s_begin) & 1) * R::KEYS;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            if (j == 1 && !two) break;   // uniform
-            f32x16 a, dp;
-            if constexpr (BF32) {
+        for (int j = 0; j < R::TPW; ++j) {
+            // uniform.  Head dim 128, a wave per SIMD: both tiles together, also where the second's keys do not exist (masked, and
+            // not stored): 78 -> 74 us; at head dim 64 that is slower, 193 -> 205.
+            if (D == 128 || j < tiles) {
+                f32x16 a, dp;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) a[r] = dead ? 0.0f : b32[j][r];   // (uniform)
-            } else {
+                for (int ks = 0; ks < KSD; ++ks) {
+                    const int o = G::at(32 * j + li, 2 * ks + g);
+                    const v8 k = *reinterpret_cast<const v8 *>(buf + o);
+                    if (ks) {
+                        a = Mfma<T>::mma(k, qf[ks], a);                                                        // log2 P^T
+                    } else if (__builtin_expect(!dead, 1)) {
+                        a = Mfma<T>::mma(k, qf[0], bias[j]);
+                    } else {   // (a row with every key masked takes no bias)
+                        f32x16 z;
 #pragma unroll
-                for (int i = 0; i < 2; ++i)   // (unpacked anew for each row: expanded once the tiles would take twice the registers)
+                        for (int r = 0; r < 16; ++r) z[r] = 0.0f;
+                        a = Mfma<T>::mma(k, qf[0], z);
+                    }
+                    dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_V + o), gf[ks], ks ? dp : nd);         // dP^T - delta
+                }
+                a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (32 * j + li) * 16), qf[KSD], a);
 #pragma unroll
-                    for (int w = 0; w < 4; ++w) asm volatile("" : "+v"(b16[j].w[i][w]));
-                unpack_tile16<T>(b16[j], dead ? 0.0f : kLog2e, a);
+                for (int r = 0; r < 16; ++r) sum[j][r] += fast_exp2(a[r]) * dp[r];
             }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
-#pragma unroll
-            for (int ks = 0; ks < KSD; ++ks) {
-                const int o = G::at(32 * j + li, 2 * ks + g);
-                a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + o), qf[ks], a);                  // log2 P^T
-                dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_V + o), gf[ks], dp);     // dP^T - delta
-            }
-            a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (32 * j + li) * 16), qf[KSD], a);
-            dp = Mfma<T>::mma(vaug, gf[KSD], dp);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sum[j][r] += fast_exp2(a[r]) * dp[r];
+            if (D < 128) __builtin_amdgcn_sched_barrier(0);   // (the next tile's operands would take the registers)
         }
     }
     // the partial of this chunk: lane = query li, registers 4 rr .. 4 rr + 3 = keys 8 rr + 4 g ..
     if (active && q0 + li < p.N) {
         float *part = e.dbias_part + ((((int64_t)c * p.B + b) * p.H + h) * p.N + (q0 + li)) * p.N;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < R::TPW; ++j)
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
                 const int kg = k0 + 32 * j + 8 * rr + 4 * g;
@@ -1170,7 +1204,6 @@ int EVO_CAT(launch_mfma_dkdv_d, EVO_D)(const EvoAttnParams &p, const Extra &e, h
     return p.dtype == EVO_BF16 ? dkdv_waves<bf16_t, EVO_D>(p, e, st) : dkdv_waves<f16_t, EVO_D>(p, e, st);
 }
 
-#if EVO_D >= 64
 template <typename T, int D, bool BF32>
 static int dbias_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     typedef DbStream<D> R;
@@ -1187,6 +1220,5 @@ int EVO_CAT(launch_mfma_dbias_d, EVO_D)(const EvoAttnParams &p, const Extra &e, 
     if (p.dtype == EVO_BF16) return f ? dbias_launch<bf16_t, EVO_D, true>(p, e, st) : dbias_launch<bf16_t, EVO_D, false>(p, e, st);
     return f ? dbias_launch<f16_t, EVO_D, true>(p, e, st) : dbias_launch<f16_t, EVO_D, false>(p, e, st);
 }
-#endif
 
 }  // namespace evo
