@@ -39,7 +39,7 @@ VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form", "-fno-honor-nans"]
 def _units():
     units = [("api", "api.hip", []), ("generic", "generic.hip", []), ("dispatch", "dispatch.hip", []),
              ("prep", "prep.hip", []), ("layernorm", "layernorm.hip", []), ("pair_bias", "pair_bias.hip", VGPR_FORM[:2]),
-             ("linear", "linear.hip", VGPR_FORM[:2]), ("f32", "f32.hip", VGPR_FORM[:2])]
+             ("linear", "linear.hip", VGPR_FORM[:2]), ("f32", "f32.hip", VGPR_FORM[:2]), ("mfma_bwd_fused", "mfma_bwd_fused.hip", VGPR_FORM)]
     for d in HEAD_DIMS:
         if d <= 16:
             units.append((f"mfma_fwd_d{d}", "mfma_fwd.hip", [f"-DEVO_D={d}", *VGPR_FORM]))

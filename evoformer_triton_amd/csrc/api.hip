@@ -189,6 +189,30 @@ static bool dq_split_ok(const EvoAttnParams &p) {
     return p.bias_dtype == p.dtype || p.bias_dtype == EVO_F32;   // (the dBias kernel keeps 16-bit pairs or fp32 tiles)
 }
 
+// dQ, dK and dV from one kernel (head dim 32), dBias, where it is wanted, from the kernel that forms dS for it alone.  The scores and dS, which
+// two kernels would form, are formed once, or with dBias twice instead of three times.  Backward, bf16, us, the kernels otherwise / this way:
+//   no dBias     H = 8: N = 96, S = 256 40 / 34; N = 128, S = 48, 256 14 / 11, 54 / 43; N = 256, S = 48, 128, 256 36 / 25, 68 / 50, 116 / 94; N = 384,
+//                S = 256 263 / 196; N = 768, S = 192 668 / 495; N = 2048, S = 192 4305 / 3528
+//   with dBias   N = 256 stays with the kernels over a chunk of rows, whose dBias comes with dQ: S = 128 78 / 83; S = 512, N = 300 489 / 482, N = 320,
+//                H = 4 149 / 152; N = 340, S = 160 168 / 159; N = 384, S = 256 313 / 292; N = 400, S = 128 232 / 186; N = 512, S = 192 431 / 353;
+//                N = S = 768, H = 4 1793 / 1497; N = 1024, S = 192 1649 / 1280
+// A problem is one workgroup's, two at a time on each of 256 CUs, so what counts beside is how full its last half round is.  H = 8, S = 48
+// (three quarters), 56, 64 (full), 65 (two thirds), 75: N = 512 81 / 70, 92 / 73, 101 / 78, 114 / 109, 121 / 109; N = 2048 1091 / 963, 1265 /
+// 1066, 1448 / 1156, 1494 / 1568, 1701 / 1582; with dBias N = 512 109 / 111, 126 / 119, 139 / 127, 152 / 162, 165 / 165; N = 1024 410 / 364,
+// 471 / 392, 531 / 438, 561 / 549, 633 / 580.  From 321 to 384 keys, where the gain is least, only whole rounds of at least 1024 problems.
+static bool fused_ok(const EvoAttnParams &p) {
+    constexpr int apart = EVO_FLAG_PER_PROBLEM | EVO_FLAG_ONLY_DQ | EVO_FLAG_ONLY_DKDV | EVO_FLAG_DEBUG_NO_KV_RING | EVO_FLAG_DEBUG_NO_DQ_WIDE |
+                          EVO_FLAG_DEBUG_NO_DQ_SPLIT | EVO_FLAG_DEBUG_OTHER_WIDTH;
+    if ((p.flags & apart) || (p.dtype != EVO_BF16 && p.dtype != EVO_F16) || p.D != 32 || p.gate || p.dmask || bias_direct(p)) return false;
+    if (p.N < 96 || p.N > 2048) return false;
+    const int64_t problems = (int64_t)p.B * p.H * p.S;
+    const double full = (double)problems / (double)((problems + 255) / 256 * 256);
+    if (problems < 384) return false;
+    if (!p.dbias) return full >= 0.7;
+    if (p.S < 8 || p.N <= 320) return false;
+    return p.N <= 384 ? problems >= 1024 && full >= 0.95 : full >= (p.N > 768 ? 0.75 : 0.85);
+}
+
 static bool dq_wide_ok(const EvoAttnParams &p) {
     return dq_wide_grid_ok(p) && (!p.dbias || p.S == 1 || dq_split_ok(p));
 }
@@ -212,7 +236,7 @@ static void chunking(const EvoAttnParams &p, int *n_chunks, int *chunk) {
         *n_chunks = (p.S + *chunk - 1) / *chunk;
         return;
     }
-    if (dq_split_ok(p)) {
+    if (fused_ok(p) || dq_split_ok(p)) {
         // the dBias kernel: one workgroup per block of 128 queries x 128 keys (64 from head dim 64 on), (b, h) and chunk, two
         // (head dim 128: one) workgroups per CU (256 CUs) at a time; among the chunk counts that give one to four rounds
         // the one that leaves the fewest slots idle in the last round (near ties: the fewest chunks)
@@ -305,7 +329,7 @@ static int check_prep(const EvoAttnParams &p) {
 }
 
 struct WsLayout {
-    size_t delta, shift, dmask_part, dbias_part, dout_ungated, total;
+    size_t delta, shift, dmask_part, dbias_part, dout_ungated, dq_part, total;
     int n_chunks, chunk;
 };
 
@@ -321,6 +345,8 @@ static WsLayout ws_layout(const EvoAttnParams &p) {
     if (p.dbias && !dq_writes_dbias(p)) off += align_up((size_t)w.n_chunks * p.B * p.H * p.N * p.N * 4);
     w.dout_ungated = off;
     if (p.gate && !(p.flags & EVO_FLAG_GATE_DOUT_INPLACE)) off += align_up((size_t)q_span(p) * (size_t)elem_size(p.dtype));
+    w.dq_part = off;
+    if (fused_ok(p) && p.N > mfma_fused_tiles(p.N) * 64) off += align_up((size_t)kFusedWgs * p.N * p.D * 4);
     w.total = off;
     return w;
 }
@@ -393,7 +419,14 @@ size_t evoattn_prep_bytes(const EvoAttnParams *p) {
 
 size_t evoattn_bwd_workspace_bytes(const EvoAttnParams *p) {
     if (!p || p->B <= 0 || p->S <= 0 || p->N <= 0 || p->H <= 0) return 0;
-    return ws_layout(*p).total;
+    size_t bytes = ws_layout(*p).total;
+    if (fused_ok(*p)) {   // (a caller that times the phases of this call alone, by its flags, gets other kernels)
+        EvoAttnParams q = *p;
+        q.flags |= EVO_FLAG_ONLY_DQ;
+        const size_t apart = ws_layout(q).total;
+        if (apart > bytes) bytes = apart;
+    }
+    return bytes;
 }
 
 const char *evoattn_path(const EvoAttnParams *p, int pass) {
@@ -464,6 +497,7 @@ const char *evoattn_kernels(const EvoAttnParams *p, int pass) {
     if (f32_ok(*p, pass)) return pass == EVO_PASS_FWD ? "f32_fwd" : p->dbias ? "f32_dq+f32_dbias,f32_dkdv" : "f32_dq,f32_dkdv";
     if (!mfma_ok(*p, pass)) return "generic";
     if (pass == EVO_PASS_FWD) return split_fwd_ok(*p) ? "split_fwd" : fwd_ring_ok(*p) ? "mfma_fwd_ring" : "mfma_fwd";
+    if (fused_ok(*p)) return p->dbias ? "mfma_bwd_fused+mfma_dbias" : "mfma_bwd_fused";
     const bool kvr = kv_ring_ok(*p);
     if (dq_split_ok(*p)) return kvr ? "mfma_dq_wide+mfma_dbias,mfma_dkdv_ring" : "mfma_dq_wide+mfma_dbias,mfma_dkdv";
     if (dq_wide_ok(*p)) return kvr ? "mfma_dq_wide,mfma_dkdv_ring" : "mfma_dq_wide,mfma_dkdv";
@@ -570,12 +604,19 @@ int evoattn_bwd(const EvoAttnParams *p0, void *hip_stream) {
     e.shift = (float *)(ws + w.shift);
     e.dmask_part = (float *)(ws + w.dmask_part);
     e.dbias_part = (float *)(ws + w.dbias_part);
+    e.dq_part = (float *)(ws + w.dq_part);
     if (f32_ok(*p, EVO_PASS_BWD)) return launch_f32_bwd(*p, e, st);
     if (!mfma_ok(*p, EVO_PASS_BWD)) return launch_generic_bwd(*p, e, st);
     if ((rc = check_prep(*p))) return rc;
     fill_prep(*p, e);
     EVO_SET_TRACE(e);
     if (!(p->flags & EVO_FLAG_PREP_VALID) && (rc = launch_prep(*p, e, st))) return rc;
+    if (!p0->gate && fused_ok(*p)) {
+        if ((rc = launch_mfma_fused(*p, e, st))) return rc;   // (writes delta as well)
+        if (!p->dbias) return EVO_OK;
+        if ((rc = launch_mfma_dbias(*p, e, st))) return rc;
+        return launch_dbias_reduce(*p, e, st);
+    }
     if (p->flags & EVO_FLAG_ONLY_DQ) return launch_dq(*p, e, st);
     const bool kvring = kv_ring_ok(*p);
     // that kernel sums the dBias partials on its way in (they lie 16-byte aligned for it)

@@ -51,6 +51,7 @@ struct Extra {
     float *shift;      // [B][S] per-row mask shift (plain kernels)
     float *dbias_part; // [n_chunks][B][H][N][N]
     float *dmask_part; // [B][H][S][N]
+    float *dq_part;    // [workgroup][N][D] partial dQ of the kernel that forms dQ, dK and dV at once (several blocks of keys)
     // prepared operands of the matrix-core kernels (written by the prep kernel)
     float *bq;         // bias * log2(e) in accumulator-tile order, lane = query  [Bb][H][NT][NT][64][16]
     float *bk;         // same, lane = key
