@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3
     constexpr int NW = 4, KSD = D / 16, KS = KSD + 1, DT = D / 32;
     constexpr int ST = D == 32 ? 2 : 1;
     // ST: key tiles per step.  Wider heads leave no registers for a second tile of scores.  Two tiles
-    // add up exactly as in mfma_fwd.hip, so that a D = 32 row's result does not depend on which of the two forms it.
+    // add up exactly as in mfma_fwd.hip.
     // (Three waves per SIMD: S = N = 384, H = 4 97 us; at four the second tile spills, 124 us; mfma_fwd.hip's form 124 us.)
     typedef typename Mfma<T>::v8 v8;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[2][R::BYTES];
@@ -392,6 +392,243 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3
         }
     }
 }
+
+#if EVO_D == 32
+// ------------------------------------------------------------------ forward, two S rows at a time
+
+// stream_fwd for head dim 32 where the vector unit's issue is the bound (0.86 of the time, 101 instructions per tile, 32 of them to unpack and
+// scale 16 bit bias entries): a workgroup takes the same 128 queries of two S rows, which have the same bias, so a tile of it is
+// unpacked once and is the first C of both rows' chains.  After the first two tiles a step takes one key tile of
+// both rows instead of two of one: the scores of two tiles are what the registers of three waves per SIMD hold, and two rows keep the units
+// as busy.  (The probabilities are stream_fwd's, their sums are added in another order.  Gated calls keep stream_fwd: the bias of a block's pair norm
+// has a gradient that is zero but for the rounding of O.)
+// us, stream_fwd / this: H = 4, S = N = 768 501 / 455, 512 168 / 153, 384 81 / 75; H = 8, S = 128, N = 384 53.7 / 50.6; S = 300, N = 224 54.5 / 51.1; with
+// an fp32 bias S = N = 768, H = 4 536 / 486.
+template <typename T, int BT>
+__global__ void __launch_bounds__(256, 3) stream_fwd_pair(EvoAttnParams p, Extra e) {
+    constexpr int D = 32, NW = 4, KSD = D / 16, KS = KSD + 1;
+    typedef StreamGeo<D> G;
+    typedef FwdStream<D> R;
+    typedef typename Mfma<T>::v8 v8;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2][2][R::BYTES];   // stage parity, S row
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, g = lane >> 5;
+    const int NT = (p.N + 31) / 32, nqb = (p.N + 127) / 128;
+    const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+    unsigned pid;   // of the pair's first row
+    {
+        // (pairs in the order in which walk_problem takes problems)
+        const unsigned t = lid / nqb, S2 = (unsigned)(p.S + 1) / 2, H = (unsigned)p.H;
+        const bool heads_first = p.stride_h < p.stride_n && p.N <= 512;
+        const unsigned bh = heads_first ? t / H / S2 * H + t % H : t / S2, i = heads_first ? t / H % S2 : t % S2;
+        pid = bh * (unsigned)p.S + 2 * i;
+    }
+    const Prob pr = decode_problem(p, pid);
+    const int n = pr.s + 1 < p.S ? 2 : 1;   // rows of this pair (uniform)
+    const int q0 = (lid % nqb) * 128 + wave * 32, qrow = min(q0 + li, p.N - 1);
+    const bool active = q0 < p.N;   // wave-uniform
+    const int sn2 = (int)p.stride_n * 2, valid = (p.N - 1) * sn2 + D * 2, np256 = (p.N + 255) / 256 * 256;
+    bool dead[2];
+    int64_t base[2];
+    __amdgpu_buffer_rsrc_t krs[2], vrs[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int s = j < n ? pr.s + j : pr.s;
+        dead[j] = uniform_load(e.dead + pr.b * p.S + s) != 0;
+        base[j] = pr.base + (int64_t)(s - pr.s) * p.stride_s;
+        krs[j] = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.k + base[j]), 0, valid, 0x00020000);
+        vrs[j] = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.v + base[j]), 0, valid, 0x00020000);
+    }
+    const int sm = pr.s + (wave < n ? wave : 0);   // the first two waves fetch a row's mask each
+    const __amdgpu_buffer_rsrc_t mrs = __builtin_amdgcn_make_buffer_rsrc((void *)(e.m2a + ((int64_t)pr.b * p.S + sm) * np256), 0, np256 * 16, 0x00020000);
+    auto fetch = [&](int stage) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            if (j < n) dma_rows<D, R::ROWS, NW>(krs[j], vrs[j], lds[stage & 1][j], stage * R::ROWS, p.N, sn2, wave, lane);
+        if (wave < n) dma16(mrs, lds[stage & 1][wave] + R::OFF_A, (stage * R::ROWS + lane) * 16);
+    };
+    fetch(0);
+
+    const float c = p.scale * kLog2e;
+    v8 qf[2][KS];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const T *Q = (const T *)p.q + base[j] + (int64_t)qrow * p.stride_n;
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) qf[j][ks] = dead[j] ? zero8<T>() : scaled8<T>(ld8(Q + ks * 16 + g * 8), c);
+        qf[j][KSD] = zero8<T>();
+        if (g == 0) qf[j][KSD][0] = qf[j][KSD][1] = qf[j][KSD][2] = (T)1.0f;
+    }
+    const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, false, lane);
+    typename BiasStream<T, BT, false>::Tile ct, c1;
+    bias.load(0, ct);
+    bias.load(1, c1);
+
+    float m[2] = {0.0f, 0.0f}, mf[2] = {0.0f, 0.0f}, l[2] = {0.0f, 0.0f};   // as in stream_fwd
+    f32x16 o[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[0][r] = o[1][r] = 0.0f;
+
+    auto score = [&](int j, bool plain, const unsigned char *buf, int kb, const f32x16 &init, f32x16 &a) {
+        const v8 k0 = *reinterpret_cast<const v8 *>(buf + G::at(kb + li, g));
+        if (plain || !dead[j]) {
+            a = Mfma<T>::mma(k0, qf[j][0], init);
+        } else {   // (a row with every key masked takes no bias)
+            f32x16 z;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z[r] = 0.0f;
+            a = Mfma<T>::mma(k0, qf[j][0], z);
+        }
+#pragma unroll
+        for (int ks = 1; ks < KSD; ++ks) a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + G::at(kb + li, 2 * ks + g)), qf[j][ks], a);
+        a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (kb + li) * 16), qf[j][KSD], a);   // (zero in the step's upper half)
+    };
+    // (`a`: the one or two tiles of a step)
+    auto settle = [&](int j, bool first, auto &a, float used) {
+        constexpr int ST = sizeof(a) / sizeof(f32x16);
+        float mloc = a[0][0];
+#pragma unroll
+        for (int t = 0; t < ST; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, a[t][r]);
+        const unsigned u = __float_as_uint(mloc);
+        auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        const float cand = fmaxf(fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) + used, kMaskFloor);
+        const bool grow = first || cand > m[j] + 8.0f;
+        if (__any(grow || m[j] != used)) {
+            const float mn = grow ? cand : m[j];
+            if (!first) {
+                const float alpha = fast_exp2(m[j] - mn);
+                l[j] *= alpha;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
+            }
+            m[j] = mn;
+            const float dsub = mn - used;
+#pragma unroll
+            for (int t = 0; t < ST; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) a[t][r] -= dsub;
+            mf[j] = fabsf(mn) <= 1024.0f ? mn : 0.0f;
+            const v8 qa = aug8<T>(ones3<T>(), pack_split3<T>(-mf[j]));
+            if (g == 0) qf[j][KSD] = qa;
+        }
+    };
+    auto probs = [&](f32x16 &a, v8 (&pf)[2]) {
+        float s = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            a[r] = fast_exp2(a[r]);
+            s += a[r];
+        }
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pf[ts][i] = (T)a[8 * ts + i];
+        return s;
+    };
+    auto add = [&](int j, const unsigned char *buf, int kb, const v8 (&pf)[2]) {
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts) o[j] = Mfma<T>::mma(transposed<T, D>(buf + R::OFF_V, kb, ts, 0, lane), pf[ts], o[j]);
+    };
+    // The first two tiles, row after row, each row relative to its maximum over both, as in stream_fwd (its probabilities
+    // are then that kernel's to the bit); `between`: what is asked for once the bias has arrived
+    auto first = [&](const unsigned char *buf, auto rows, auto plain, auto between) {
+        constexpr int ROWS = decltype(rows)::value;
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j) {
+            f32x16 a[2];
+            v8 pf[2];
+            {
+                const f32x16 i0 = bias.take(ct), i1 = bias.take(c1);
+                if (j == 0) between();
+                score(j, plain, buf + j * R::BYTES, 0, i0, a[0]);
+                score(j, plain, buf + j * R::BYTES, 32, i1, a[1]);
+            }
+            settle(j, true, a, 0.0f);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                l[j] += probs(a[t], pf);
+                add(j, buf + j * R::BYTES, 32 * t, pf);
+            }
+            __builtin_amdgcn_sched_barrier(0);   // (both rows' tiles at once would not fit the registers)
+        }
+        bias.load(2, ct);
+    };
+    // a key tile of all (one or both) rows: kt, from row kb of the stage on
+    auto step = [&](const unsigned char *buf, int kt, int kb, auto rows, auto plain, auto between) {
+        constexpr int ROWS = decltype(rows)::value;
+        const f32x16 init = bias.take(ct);
+        between();
+        bias.load(kt + 1, ct);
+        f32x16 a[ROWS][1];
+        float used[ROWS], s[ROWS];
+        v8 pf[ROWS][2];
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j) {
+            used[j] = mf[j];
+            score(j, plain, buf + j * R::BYTES, kb, init, a[j][0]);
+        }
+        const bool lazy = !__any(m[0] != mf[0] || m[ROWS - 1] != mf[ROWS - 1]);
+        if (!lazy)
+#pragma unroll
+            for (int j = 0; j < ROWS; ++j) settle(j, false, a[j], used[j]);
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j) s[j] = probs(a[j][0], pf[j]);
+        if (__builtin_expect(lazy && __any(!(s[0] <= 8192.0f) || !(s[ROWS - 1] <= 8192.0f)), 0)) {   // some score stands far above m: once more, the long way
+            typename BiasStream<T, BT, false>::Tile again;
+            bias.load(kt, again);
+#pragma unroll
+            for (int j = 0; j < ROWS; ++j) {
+                score(j, plain, buf + j * R::BYTES, kb, bias.value(again), a[j][0]);
+                settle(j, false, a[j], used[j]);
+                s[j] = probs(a[j][0], pf[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j) {
+            l[j] += s[j];
+            add(j, buf + j * R::BYTES, kb, pf[j]);
+        }
+    };
+
+    const int nst = (p.N + R::ROWS - 1) / R::ROWS;
+    wait_loads();
+    wait_lds_barrier();
+    auto walk = [&](auto rows, auto plain) {
+        if (active) first(lds[0][0], rows, plain, [&] { fetch(1); });
+        else fetch(1);
+        for (int s = 1; s < nst; ++s) {   // (at least two stages)
+            wait_loads();
+            wait_lds_barrier();
+            auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
+            if (active) {
+                const unsigned char *buf = lds[s & 1][0];
+                step(buf, 2 * s, 0, rows, plain, next);
+                if (2 * s + 1 < NT) step(buf, 2 * s + 1, 32, rows, plain, [] {});
+            } else {
+                next();
+            }
+        }
+    };
+    // (fp32 tiles: another copy of the loop spills 350 registers)
+    if (BT == 2 && n == 2 && !dead[0] && !dead[1]) walk(std::integral_constant<int, 2>(), std::integral_constant<bool, BT == 2>());
+    else if (n == 2) walk(std::integral_constant<int, 2>(), std::false_type());
+    else walk(std::integral_constant<int, 1>(), std::false_type());
+
+    if (!active) return;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        if (j >= n) break;   // uniform
+        const float sum = l[j] + __shfl_xor(l[j], 32);
+        if (q0 + li < p.N) {
+            if (g == 0) p.lse[pr.row0 + (int64_t)j * p.N + q0 + li] = (m[j] + __log2f(sum)) * kLn2;
+            store_row_tile<T>((T *)p.o + base[j] + (int64_t)(q0 + li) * p.stride_n, 0, D, o[j], 1.0f / sum, g);
+        }
+    }
+}
+
+#endif
 
 // ------------------------------------------------------------------ forward of few problems
 
@@ -1110,9 +1347,26 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
 
 // ------------------------------------------------------------------ launchers
 
+#if EVO_D == 32
+// Two rounds of the three workgroups that a CU holds, or the last one is too empty for a workgroup that takes twice as long (stream_fwd / pairs, us, H = 8: N = 384,
+// S = 48, 64, 96, 128 26.7 / 27.8, 30.3 / 29.6, 40.4 / 41.2, 50.4 / 47.2; N = 300, S = 96, 128 34.5 / 35.5, 42.3 / 39.9); up to 192 keys what a
+// workgroup costs beside its tiles decides (N = 128, S = 200 20.4 / 22.8; N = 192 32.9 / 33.9; N = 224 39.8 / 37.2).
+static bool fwd_pair_ok(const EvoAttnParams &p, const Extra &e, int64_t pairs) {
+    return p.N > 192 && pairs >= 2 * 768 && p.bias_dtype != EVO_NONE && !e.bias_direct && !p.gate && !(p.flags & EVO_FLAG_PER_PROBLEM);
+}
+#endif
+
 template <typename T, int D>
 static int fwd_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const unsigned grid = (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H * p.S);
+#if EVO_D == 32
+    const int64_t pairs = (int64_t)((p.N + 127) / 128) * p.B * p.H * ((p.S + 1) / 2);
+    if (fwd_pair_ok(p, e, pairs)) {
+        if (e.bq16) stream_fwd_pair<T, 2><<<(unsigned)pairs, 256, 0, st>>>(p, e);
+        else stream_fwd_pair<T, 1><<<(unsigned)pairs, 256, 0, st>>>(p, e);
+        return hip_rc();
+    }
+#endif
     if (p.bias_dtype == EVO_NONE) stream_fwd<T, D, 0><<<grid, 256, 0, st>>>(p, e);
     else if (e.bias_direct && p.bias_dtype == EVO_F32) stream_fwd<T, D, 3><<<grid, 256, 0, st>>>(p, e);
     else if (e.bias_direct) stream_fwd<T, D, 4><<<grid, 256, 0, st>>>(p, e);
