@@ -189,7 +189,7 @@ static bool dq_split_ok(const EvoAttnParams &p) {
     return p.bias_dtype == p.dtype || p.bias_dtype == EVO_F32;   // (the dBias kernel keeps 16-bit pairs or fp32 tiles)
 }
 
-// dQ, dK and dV from one kernel (head dim 32), dBias, where it is wanted, from the kernel that forms dS for it alone.  The scores and dS, which
+// dQ, dK and dV from one kernel (head dims 32 and 8), dBias, where it is wanted, from the kernel that forms dS for it alone.  The scores and dS, which
 // two kernels would form, are formed once, or with dBias twice instead of three times.  Backward, bf16, us, the kernels otherwise / this way:
 //   no dBias     H = 8: N = 96, S = 256 40 / 34; N = 128, S = 48, 256 14 / 11, 54 / 43; N = 256, S = 48, 128, 256 36 / 25, 68 / 50, 116 / 94; N = 384,
 //                S = 256 263 / 196; N = 768, S = 192 668 / 495; N = 2048, S = 192 4305 / 3528
@@ -200,13 +200,20 @@ static bool dq_split_ok(const EvoAttnParams &p) {
 // (three quarters), 56, 64 (full), 65 (two thirds), 75: N = 512 81 / 70, 92 / 73, 101 / 78, 114 / 109, 121 / 109; N = 2048 1091 / 963, 1265 /
 // 1066, 1448 / 1156, 1494 / 1568, 1701 / 1582; with dBias N = 512 109 / 111, 126 / 119, 139 / 127, 152 / 162, 165 / 165; N = 1024 410 / 364,
 // 471 / 392, 531 / 438, 561 / 549, 633 / 580.  From 321 to 384 keys, where the gain is least, only whole rounds of at least 1024 problems.
+// Head dim 8, H = 8 (up to 384 keys are one block there):
+//   no dBias     S = 32, 128, 1024: N = 64 9 / 7, 11 / 11, 58 / 62 (left out); N = 96 10 / 7, 14 / 13, 74 / 71; N = 192 14 / 10, 32 / 23, 215 / 152; N = 384
+//                27 / 20, 84 / 54, 663 / 400; N = 1024 135 / 120, 503 / 352, 4190 / 2896; S = 65 N = 256 28 / 25, N = 1024 275 / 249
+//   with dBias   N = 192, S = 128, 1024 48 / 53, 289 / 283 (left out); N = 300, S = 64, 65, 96, 256 56 / 56, 58 / 65, 74 / 73, 166 / 156; N = 384
+//                66 / 66, 69 / 79, 91 / 87, 206 / 185, S = 1024 774 / 706; N = 512, S = 64, 256 99 / 98, 329 / 321; from 513 keys on the pair of kernels for dQ
+//                stands against it: N = 768, S = 32, 65, 256 160 / 150, 279 / 251, 886 / 683; N = 1024, S = 32, 1024 212 / 199, 6352 / 4888
 static bool fused_ok(const EvoAttnParams &p) {
     constexpr int apart = EVO_FLAG_PER_PROBLEM | EVO_FLAG_ONLY_DQ | EVO_FLAG_ONLY_DKDV | EVO_FLAG_DEBUG_NO_KV_RING | EVO_FLAG_DEBUG_NO_DQ_WIDE |
                           EVO_FLAG_DEBUG_NO_DQ_SPLIT | EVO_FLAG_DEBUG_OTHER_WIDTH;
-    if ((p.flags & apart) || (p.dtype != EVO_BF16 && p.dtype != EVO_F16) || p.D != 32 || p.gate || p.dmask || bias_direct(p)) return false;
+    if ((p.flags & apart) || (p.dtype != EVO_BF16 && p.dtype != EVO_F16) || (p.D != 32 && p.D != 8) || p.gate || p.dmask || bias_direct(p)) return false;
     if (p.N < 96 || p.N > 2048) return false;
     const int64_t problems = (int64_t)p.B * p.H * p.S;
     const double full = (double)problems / (double)((problems + 255) / 256 * 256);
+    if (p.D == 8) return problems >= 256 && (!p.dbias || (p.S >= 8 && (p.N > 512 || (p.N >= 288 && problems >= 768 && full >= 0.9))));
     if (problems < 384) return false;
     if (!p.dbias) return full >= 0.7;
     if (p.S < 8 || p.N <= 320) return false;
@@ -346,7 +353,7 @@ static WsLayout ws_layout(const EvoAttnParams &p) {
     w.dout_ungated = off;
     if (p.gate && !(p.flags & EVO_FLAG_GATE_DOUT_INPLACE)) off += align_up((size_t)q_span(p) * (size_t)elem_size(p.dtype));
     w.dq_part = off;
-    if (fused_ok(p) && p.N > mfma_fused_tiles(p.N) * 64) off += align_up((size_t)kFusedWgs * p.N * p.D * 4);
+    if (fused_ok(p) && p.N > (p.D == 8 ? mfma_fused8_tiles(p.N) : mfma_fused_tiles(p.N)) * 64) off += align_up((size_t)(p.D == 8 ? kFusedWgs8 : kFusedWgs) * p.N * p.D * 4);
     w.total = off;
     return w;
 }
@@ -612,7 +619,7 @@ int evoattn_bwd(const EvoAttnParams *p0, void *hip_stream) {
     EVO_SET_TRACE(e);
     if (!(p->flags & EVO_FLAG_PREP_VALID) && (rc = launch_prep(*p, e, st))) return rc;
     if (!p0->gate && fused_ok(*p)) {
-        if ((rc = launch_mfma_fused(*p, e, st))) return rc;   // (writes delta as well)
+        if ((rc = p->D == 8 ? launch_mfma_fused8(*p, e, st) : launch_mfma_fused(*p, e, st))) return rc;   // (writes delta as well)
         if (!p->dbias) return EVO_OK;
         if ((rc = launch_mfma_dbias(*p, e, st))) return rc;
         return launch_dbias_reduce(*p, e, st);

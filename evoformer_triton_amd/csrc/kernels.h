@@ -37,13 +37,19 @@ inline bool mfma_dqr_gate_ok(int D, int N) { return D == 32 && N <= 256; }
 int mfma_dqr_qrows(int D, int N);  // query rows per workgroup of the double-buffered dQ kernel (64 or 32), 0 where it is not built for such rows
 int launch_mfma_dkdv(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_dqw(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // dQ where no dBias is asked for
-// dQ, dK and dV at once: workgroups where several share the problems among them (a scratch for dQ each), key tiles of 16 per wave
-constexpr int kFusedWgs = 512;
+// dQ, dK and dV at once (head dims 32, 8): workgroups where several share the problems among them (a scratch for dQ each), key tiles of 16 per wave
+constexpr int kFusedWgs = 512, kFusedWgs8 = 768;   // head dims 32, 8
 inline int mfma_fused_tiles(int N) {
     if (N <= 128) return 2;
     const int blocks = (N + 255) / 256;   // fewest blocks of at most 256 keys, as narrow as they can be
     return (N + blocks * 64 - 1) / (blocks * 64);
 }
+inline int mfma_fused8_tiles(int N) {
+    if (N <= 128) return 2;
+    const int blocks = (N + 383) / 384;   // (of at most 384 keys)
+    return (N + blocks * 64 - 1) / (blocks * 64);
+}
+int launch_mfma_fused8(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_fused(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_dbias(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // dBias partials alone (reads delta)
 int launch_column_reduce(const float *part, int blocks, int cols, void *out, int dtype, hipStream_t st);  // out[c] = sum of part[.][c], fixed order

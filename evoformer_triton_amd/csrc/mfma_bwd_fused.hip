@@ -14,20 +14,10 @@
 // vector and 12 matrix instructions.  S = N = 768, H = 4 without dBias 1292 -> 992 us (dQ and dK/dV kernels before), S = N = 384 180 -> 143,
 // N = 256, S = 512, H = 8 281 -> 209.  Two tiles per wave and three waves per SIMD spill (1650); the next block's keys and first stage fetched
 // during this one's last: more scalar registers than there are, 1035; head dim 64, of 32-query stages, 960 against the two kernels' 560.
-#include "bwd_common.h"
+#include "fused_common.h"
 #include "kernels.h"
 
 namespace evo {
-
-typedef short s16x4f __attribute__((ext_vector_type(4)));
-
-template <typename T> struct Mfma16;
-template <> struct Mfma16<bf16_t> {
-    static __device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
-};
-template <> struct Mfma16<f16_t> {
-    static __device__ __forceinline__ f32x4 mma(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-};
 
 // KT: key tiles of 16 per wave
 template <int KT>
@@ -49,34 +39,6 @@ struct Fused {
     static __device__ __forceinline__ int atk(int r, int c) { return r * ROW + ((c ^ xk(r)) << 4); }
     static __device__ __forceinline__ int ate(int r, int c) { return r * 64 + ((c ^ xk(r)) << 4); }
 };
-
-// all but the youngest N of the wave's loads and stores (they end in the order they were issued)
-template <int N>
-__device__ __forceinline__ void fused_wait_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-__device__ __forceinline__ void fused_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-// 16 bytes per lane, from the lane's offset and a uniform one, into LDS from `dst` on; past the end of the array zeros.  (As an instruction that
-// the compiler does not know: see dma16 in mfma_stream.hip.)
-__device__ __forceinline__ void fused_dma(__amdgpu_buffer_rsrc_t rs, unsigned char *dst, int off, int from) {
-    const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)dst;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" : : "s"(base), "v"(off), "s"(rs), "s"(from));
-}
-// A lane's offset past the end of any array here.  (What decides is the lane's offset: a uniform one past the end is taken from the array's size
-// before the two are compared, so it stays inside.)
-constexpr unsigned kFusedPast = 0x7ff00000;
-typedef unsigned u32x2f __attribute__((ext_vector_type(2)));
-typedef unsigned u32x4f __attribute__((ext_vector_type(4)));
-// d of the lane `o` (1, 2 or 4) apart in a group of eight, by the vector unit's own paths (o is a constant where this is used)
-__device__ __forceinline__ float fused_xor(float d, int o) {
-    const int i = __float_as_int(d);
-    if (o == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0xB1, 0xf, 0xf, true));   // lanes 1 0 3 2 of each four
-    if (o == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0x4E, 0xf, 0xf, true));   // 2 3 0 1
-    return __shfl_xor(d, o);
-}
-// four rows at this lane's address' column of each of the 16 lanes' group
-template <typename T>
-__device__ __forceinline__ typename Mfma<T>::v4 fused_tr(const unsigned char *at) {
-    return __builtin_bit_cast(typename Mfma<T>::v4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4f __attribute__((address_space(3))) *)at));
-}
 
 template <typename T, int KT, int BT>
 __global__ void __launch_bounds__(256, 2) bwd_fused(EvoAttnParams p, Extra e, unsigned problems, int nb) {

@@ -1,5 +1,5 @@
 // dBias partials for rows of more than 256 keys, as a kernel of its own.
-// Compiled once per head dim (-DEVO_D=8|16; from 32 on: mfma_stream.hip).
+// Compiled once per head dim (-DEVO_D=16; 8: mfma_stream8.hip, from 32 on: mfma_stream.hip).
 //
 // dBias[b][h] is the sum over the S rows of dS = P * (dP - delta) (reference: the atomic add of
 // every dS tile, evoformer.py:458).  Summing it inside the dQ kernel ties every wave of that

@@ -1,4 +1,4 @@
-"""dBias from the kernel of its own whose bias stays resident (csrc/mfma_stream.hip, stream_dbias) at the edges of its blocks of queries and
+"""dBias from the kernel of its own whose bias stays resident (csrc/mfma_stream.hip, stream_dbias; csrc/mfma_stream8.hip) at the edges of its blocks of queries and
 keys and of its chunks of S rows, against eager in fp32."""
 import ctypes
 
@@ -14,6 +14,9 @@ CASES = [  # B, S, N, H, D, mask, bias dtype, dtype
     (2, 9, 545, 1, 32, "bool", "f32", torch.float16),           # a last block of 33 keys: one tile and one key; two batches
     (1, 67, 640, 1, 32, "dead_added", "q", torch.float16),      # whole blocks; a last chunk that is shorter
     (1, 8, 1120, 1, 32, None, "f32", torch.bfloat16),           # chunks of one row
+    (1, 9, 513, 2, 8, "dead", "q", torch.bfloat16),
+    (2, 8, 609, 1, 8, "bool", "f32", torch.float16),
+    (1, 67, 640, 1, 8, "dead_added", "q", torch.bfloat16),
     (1, 16, 129, 2, 64, "dead", "f32", torch.bfloat16),
     (2, 17, 161, 1, 64, "dead_added", "q", torch.float16),
     (1, 5, 129, 16, 128, "dead", "q", torch.bfloat16),

@@ -1,4 +1,4 @@
-"""dQ, dK and dV from one kernel (csrc/mfma_bwd_fused.hip) at the edges of its tiles, groups, stages and blocks of keys, against eager
+"""dQ, dK and dV from one kernel (csrc/mfma_bwd_fused.hip, mfma_bwd_fused8.hip) at the edges of its tiles, groups, stages and blocks of keys, against eager
 in fp32."""
 import ctypes
 
@@ -9,24 +9,33 @@ from oracle import eager
 
 pytestmark = pytest.mark.gpu
 
-CASES = [  # B, S, N, H, mask, bias, layout, dtype, dBias
-    (1, 48, 96, 8, "bool", "q", "reference", torch.bfloat16, False),
-    (2, 48, 127, 4, "soft", "f32", "ds4sci", torch.float16, False),
-    (1, 64, 128, 6, "dead", "q", "reference", torch.bfloat16, False),
-    (1, 96, 129, 4, "dead", "f32", "reference", torch.bfloat16, False),     # a group of one query; three tiles of keys per wave
-    (1, 192, 192, 2, None, None, "ds4sci", torch.bfloat16, False),
-    (2, 96, 193, 2, "bool", "q", "reference", torch.float16, False),
-    (1, 128, 251, 3, "soft", "q", "ds4sci", torch.bfloat16, False),
-    (1, 96, 256, 4, "jump", "q", "reference", torch.bfloat16, False),
-    (1, 96, 256, 4, "dead", "q", "ds4sci", torch.float16, False),
-    (2, 96, 250, 2, "dead_added", "f32", "reference", torch.bfloat16, False),
-    (1, 200, 257, 2, "dead", "q", "reference", torch.bfloat16, False),      # a second block of keys, a last one of one key
-    (1, 768, 264, 1, "bool", "f32", "ds4sci", torch.float16, False),        # more problems than workgroups
-    (1, 193, 384, 2, "dead_added", "q", "reference", torch.bfloat16, False),
-    (1, 128, 516, 3, "soft", "q", "reference", torch.bfloat16, False),      # three blocks
-    (1, 1024, 321, 1, "dead", "q", "reference", torch.bfloat16, True),
-    (2, 224, 385, 1, "dead_added", "f32", "ds4sci", torch.float16, True),
-    (1, 224, 516, 2, "bool", "q", "reference", torch.bfloat16, True),
+CASES = [  # B, S, N, H, D, mask, bias, layout, dtype, dBias
+    (1, 48, 96, 8, 32, "bool", "q", "reference", torch.bfloat16, False),
+    (2, 48, 127, 4, 32, "soft", "f32", "ds4sci", torch.float16, False),
+    (1, 64, 128, 6, 32, "dead", "q", "reference", torch.bfloat16, False),
+    (1, 96, 129, 4, 32, "dead", "f32", "reference", torch.bfloat16, False),     # a group of one query; three tiles of keys per wave
+    (1, 192, 192, 2, 32, None, None, "ds4sci", torch.bfloat16, False),
+    (2, 96, 193, 2, 32, "bool", "q", "reference", torch.float16, False),
+    (1, 128, 251, 3, 32, "soft", "q", "ds4sci", torch.bfloat16, False),
+    (1, 96, 256, 4, 32, "jump", "q", "reference", torch.bfloat16, False),
+    (1, 96, 256, 4, 32, "dead", "q", "ds4sci", torch.float16, False),
+    (2, 96, 250, 2, 32, "dead_added", "f32", "reference", torch.bfloat16, False),
+    (1, 200, 257, 2, 32, "dead", "q", "reference", torch.bfloat16, False),      # a second block of keys, a last one of one key
+    (1, 768, 264, 1, 32, "bool", "f32", "ds4sci", torch.float16, False),        # more problems than workgroups
+    (1, 193, 384, 2, 32, "dead_added", "q", "reference", torch.bfloat16, False),
+    (1, 128, 516, 3, 32, "soft", "q", "reference", torch.bfloat16, False),      # three blocks
+    (1, 1024, 321, 1, 32, "dead", "q", "reference", torch.bfloat16, True),
+    (2, 224, 385, 1, 32, "dead_added", "f32", "ds4sci", torch.float16, True),
+    (1, 224, 516, 2, 32, "bool", "q", "reference", torch.bfloat16, True),
+    (1, 96, 96, 8, 8, "bool", "q", "reference", torch.bfloat16, False),
+    (2, 48, 129, 4, 8, "dead", "f32", "ds4sci", torch.float16, False),         # a last group of one query, a last tile of one key
+    (1, 128, 193, 4, 8, "jump", "q", "reference", torch.bfloat16, False),
+    (1, 300, 257, 2, 8, "dead_added", "q", "ds4sci", torch.bfloat16, False),
+    (1, 96, 384, 8, 8, "dead", "q", "reference", torch.bfloat16, True),        # the widest block
+    (1, 256, 385, 3, 8, "soft", "q", "reference", torch.float16, True),        # two blocks of keys
+    (1, 128, 300, 6, 8, None, "f32", "ds4sci", torch.bfloat16, True),
+    (1, 600, 1000, 1, 8, "dead", None, "reference", torch.bfloat16, False),    # three blocks, keys past the padded mask; more problems than workgroups
+    (1, 256, 545, 1, 8, "dead_added", "q", "reference", torch.bfloat16, True),
 ]
 
 
@@ -34,8 +43,7 @@ CASES = [  # B, S, N, H, mask, bias, layout, dtype, dBias
 def test_fused_backward_matches_eager(gpu_device, case):
     import evoformer_triton_amd.evoformer as E
     from evoformer_triton_amd import _lib
-    B, S, N, H, mask, bias, layout, dt, dbias = case
-    D = 32
+    B, S, N, H, D, mask, bias, layout, dt, dbias = case
     g = torch.Generator().manual_seed(29)
     Q, K, V, dO = ((torch.randn((B, S, N, H, D), generator=g) * 0.7).to(dt) for _ in range(4))
     keep = torch.rand((B, S, 1, 1, N), generator=g) < 0.85
