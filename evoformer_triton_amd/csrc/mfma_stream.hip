@@ -1001,7 +1001,7 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
 // stays in registers in fp32, log2 units, the first operand C of a tile's chain where it lies (as 16-bit pairs it was unpacked and multiplied
 // per tile and row, 32 instructions of 131); -delta, one value per lane, is the C of the other chain, in place of a matrix step of
 // its own; array bases advance by the scalar unit and a lane's offsets are formed once.  dBias of S = N = 768, H = 4, D = 32 (mfma_dbias.hip
-// before) 595 -> 491 us, of S = 200, N = 640, H = 5, D = 64 with an fp32 bias 238 -> 193; S = 64, N = 512, H = 4, D = 128 78 -> 74.
+// before) 595 -> 455 us, of S = 200, N = 640, H = 5, D = 64 with an fp32 bias 238 -> 193; S = 64, N = 512, H = 4, D = 128 78 -> 65.
 // Two tiles per wave and three waves per SIMD at head dim 32: 596; -delta in a matrix step: 516.
 template <int D>
 struct DbStream {
@@ -1066,6 +1066,7 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
     auto rows = [&](const void *x, int s) { return __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)x + base0 + (int64_t)s * p.stride_s), 0, valid, 0x00020000); };
     unsigned char *const own = lds + R::OFF_Q + wave * R::WAVE;
     float lse_n = 0.0f, delta_n = 0.0f;
+    int dead_n = 0;
     auto fetch_keys = [&](int s) {
         const __amdgpu_buffer_rsrc_t krs = rows(p.k, s), vrs = rows(p.v, s);
         unsigned char *dst = lds + ((s - s_begin) & 1) * R::KEYS;
@@ -1089,12 +1090,15 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
         const int64_t row0 = ((int64_t)bh * p.S + s) * p.N;
         lse_n = (p.lse + row0)[(unsigned)qrow];
         delta_n = (e.delta + row0)[(unsigned)qrow];
+        // (With the rest: as a scalar load it is waited for at the top of each row.  S = N = 768, H = 4, D = 32 495 -> 455 us, S = 64, N = 512, H = 4, D = 128
+        // 71 -> 65; at head dim 64 203 / 209.)
+        if (D != 64) dead_n = e.dead[b * p.S + s];
     };
     fetch_keys(s_begin);
     fetch_queries(s_begin);
     for (int s = s_begin; s < s_end; ++s) {
-        const bool dead = uniform_load(e.dead + b * p.S + s) != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
         wait_loads();
+        const bool dead = (D != 64 ? __builtin_amdgcn_readfirstlane(dead_n) : uniform_load(e.dead + b * p.S + s)) != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
         wait_lds_barrier();
         if (s + 1 < s_end) fetch_keys(s + 1);   // (everybody has left that buffer: it held row s - 1)
         v8 qf[KS], gf[KSD];
