@@ -460,8 +460,21 @@ static bool ring_pays(const EvoAttnParams &p, double start, double per_row) {
     return per_row * rounds * (rows + start) * 256.0 < (double)bh * p.S;
 }
 
+// Head dim 8 with a bias, no gate: two S rows per workgroup.  With the bias in the dtype of q it is ahead of the kernel over a chunk of rows
+// (129..256 keys) from few rows on (H = 8, S = 8 / 64 / 1000, that one / this, us: N = 160 10.5 / 9.9, 14.0 / 12.3, 102 / 86; N = 256 11.9 / 11.5,
+// 16.1 / 15.0, 125 / 116; with an fp32 bias N = 192, S = 128 20.4 / 24.6: left to it); of the one-workgroup-per-problem forward where the
+// pairs fill two rounds of the three workgroups that a CU holds, for long rows one (H = 8: N = 96, S = 200, 400 15.3 / 14.8, 23.9 / 21.1; N = 384, S = 32, 96,
+// 128 17.0 / 19.2, 34.0 / 34.5, 41.9 / 39.3; N = 768, S = 16, 32 30.1 / 33.5, 44.7 / 42.3).
+static bool fwd_pairs8_ok(const EvoAttnParams &p) {
+    if (p.D != 8 || !p.bias || p.gate || p.S < 2 || p.N <= 32 || bias_direct(p) || (p.flags & (EVO_FLAG_PER_PROBLEM | EVO_FLAG_DEBUG_FWD_BIAS_TILES))) return false;
+    const int64_t pairs = (int64_t)((p.N + 127) / 128) * p.B * p.H * ((p.S + 1) / 2);
+    if (p.N > 128 && p.N <= 256) return p.bias_dtype == p.dtype && pairs >= 64;
+    return pairs >= (p.N >= 512 ? 768 : 1536);
+}
+
 // rows of 129..256 keys: a workgroup per chunk of S rows with the head's bias resident
 static bool fwd_ring_ok(const EvoAttnParams &p) {
+    if (fwd_pairs8_ok(p)) return false;
     if ((p.flags & EVO_FLAG_PER_PROBLEM) || bias_direct(p) || p.N <= 128 || p.N > mfma_fwdr_max_n(p.D)) return false;
     // (a gated call keeps it at every length: the bias of a block's pair norm has a gradient that is zero but for
     // the rounding of O, and the two kernels round P against different maxima)
@@ -527,7 +540,7 @@ static int fwd_launches(const EvoAttnParams &p, hipStream_t st) {
         e.bt = nullptr;
     }
     if (const int rc = launch_prep(p, e, st, alone && ring && mfma_fwdr_reads_rows(p))) return rc;
-    return ring ? launch_mfma_fwdr(p, e, st) : launch_mfma_fwd(p, e, st);
+    return fwd_pairs8_ok(p) ? launch_stream_fwd8(p, e, st) : ring ? launch_mfma_fwdr(p, e, st) : launch_mfma_fwd(p, e, st);
 }
 
 int evoattn_fwd(const EvoAttnParams *p, void *hip_stream) {

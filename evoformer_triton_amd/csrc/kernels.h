@@ -49,6 +49,7 @@ inline int mfma_fused8_tiles(int N) {
     const int blocks = (N + 383) / 384;   // (of at most 384 keys)
     return (N + blocks * 64 - 1) / (blocks * 64);
 }
+int launch_stream_fwd8(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // forward with a bias, head dim 8: two S rows per workgroup
 int launch_mfma_fused8(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_fused(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_dbias(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // dBias partials alone (reads delta)

@@ -1,4 +1,4 @@
-"""The forward that takes two S rows at a time (csrc/mfma_stream.hip, stream_fwd_pair) at the edges of its stages, tiles and pairs, against eager in fp32
+"""The forward that takes two S rows at a time (csrc/mfma_stream.hip, stream_fwd_pair; csrc/mfma_stream8.hip, stream_fwd8) at the edges of its stages, tiles and pairs, against eager in fp32
 and against the kernel that takes one row."""
 import ctypes
 
@@ -9,13 +9,19 @@ from oracle import eager
 
 pytestmark = pytest.mark.gpu
 
-CASES = [  # B, S, N, H, mask, bias, layout, dtype
-    (1, 193, 193, 8, "dead", "q", "reference", torch.bfloat16),          # a last pair of one row; a last tile of one key
-    (2, 97, 224, 8, "dead_added", "f32", "reference", torch.float16),    # the same in two batches, each with a bias of its own
-    (1, 256, 257, 4, "bool", "q", "ds4sci", torch.bfloat16),           # a last query block and a last stage of one
-    (1, 258, 300, 4, "jump", "q", "reference", torch.float16),           # scores that outgrow the first tile's maximum
-    (3, 171, 288, 2, "dead", "f32", "ds4sci", torch.bfloat16),
-    (1, 300, 513, 3, None, "q", "reference", torch.bfloat16),
+CASES = [  # B, S, N, H, D, mask, bias, layout, dtype
+    (1, 193, 193, 8, 32, "dead", "q", "reference", torch.bfloat16),          # a last pair of one row; a last tile of one key
+    (2, 97, 224, 8, 32, "dead_added", "f32", "reference", torch.float16),    # the same in two batches, each with a bias of its own
+    (1, 256, 257, 4, 32, "bool", "q", "ds4sci", torch.bfloat16),           # a last query block and a last stage of one
+    (1, 258, 300, 4, 32, "jump", "q", "reference", torch.float16),           # scores that outgrow the first tile's maximum
+    (3, 171, 288, 2, 32, "dead", "f32", "ds4sci", torch.bfloat16),
+    (1, 300, 513, 3, 32, None, "q", "reference", torch.bfloat16),
+    (1, 17, 130, 4, 8, "dead", "q", "reference", torch.bfloat16),      # a last pair of one row; a second stage and block of two
+    (2, 16, 256, 2, 8, "dead_added", "q", "ds4sci", torch.float16),
+    (1, 21, 193, 4, 8, "jump", "q", "reference", torch.float16),
+    (3, 257, 33, 4, 8, "dead", "f32", "reference", torch.bfloat16),    # two tiles, the second of one key
+    (1, 257, 300, 4, 8, "bool", "f32", "ds4sci", torch.bfloat16),
+    (1, 129, 513, 3, 8, None, "q", "reference", torch.bfloat16),       # a last stage of one key
 ]
 
 
@@ -23,8 +29,7 @@ CASES = [  # B, S, N, H, mask, bias, layout, dtype
 def test_forward_pairs_match_eager(gpu_device, case):
     import evoformer_triton_amd.evoformer as E
     from evoformer_triton_amd import _lib
-    B, S, N, H, mask, bias, layout, dt = case
-    D = 32
+    B, S, N, H, D, mask, bias, layout, dt = case
     g = torch.Generator().manual_seed(37)
     q, k, v = ((torch.randn((B, S, N, H, D), generator=g) * 0.7).to(dt).to(gpu_device) for _ in range(3))
     keep = torch.rand((B, S, 1, 1, N), generator=g) < 0.85
@@ -50,7 +55,8 @@ def test_forward_pairs_match_eager(gpu_device, case):
         p.flags |= flags
         prep = torch.empty(lib.evoattn_prep_bytes(ctypes.byref(p)), dtype=torch.uint8, device=q.device)
         p.prep, p.prep_bytes = prep.data_ptr(), prep.numel()
-        assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == b"mfma_fwd"
+        if name == "pairs":
+            assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == b"mfma_fwd"
         assert lib.evoattn_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
         got[name] = (o.float(), lse)
     # the scaled Q, the probabilities and O are each rounded by at most 2^-9 of their size, and the scores' error that comes of the first moves the
