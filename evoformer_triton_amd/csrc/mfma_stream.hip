@@ -31,7 +31,7 @@ struct FwdStream {
 };
 
 template <typename T, int D, int BT>
-__global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3 : 2) stream_fwd(EvoAttnParams p, Extra e) {
+__global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && BT < 3 ? 3 : 2) stream_fwd(EvoAttnParams p, Extra e) {
     typedef StreamGeo<D> G;
     typedef FwdStream<D> R;
     constexpr int NW = 4, KSD = D / 16, KS = KSD + 1, DT = D / 32;
@@ -73,9 +73,13 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3
         if (g == 0) qf[KSD][0] = qf[KSD][1] = qf[KSD][2] = (T)1.0f;
     }
     const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, dead, lane);
-    typename BiasStream<T, BT, false>::Tile ct[ST];
+    // AHEAD: tiles whose bias is asked for together, and ahead of a step.  Where few S rows leave the caller's bias rows as the traffic (head dim 64) it is
+    // both tiles of a stage, 256 bytes of a row at a time, which memory serves better than 128, at two waves per SIMD: B = 4, S = 1, N = 1024, H = 32,
+    // fp32 164 -> 148 us.  (Prepared tiles lie whole: S = 200, N = 640, H = 5, fp32 190 / 204.)
+    constexpr int AHEAD = D == 64 && BT >= 3 ? 2 : ST;
+    typename BiasStream<T, BT, false>::Tile ct[AHEAD];
 #pragma unroll
-    for (int t = 0; t < ST; ++t) bias.load(t, ct[t]);
+    for (int t = 0; t < AHEAD; ++t) bias.load(t, ct[t]);
 
     // m: the maximum the probabilities are relative to; mf: what the mask step subtracts inside the product (m, or 0 while
     // m is unknown or too large for three 16-bit columns): after the first step the scores arrive relative to m, and
@@ -143,15 +147,18 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3
             for (int i = 0; i < 8; ++i) pf[ts][i] = (T)a[ts / 2][8 * (ts & 1) + i];
         return s;
     };
-    // ST tiles, from tile kt and row kb of the stage on; `between`: what is asked for once their bias has arrived
-    auto step = [&](const unsigned char *buf, int kt, int kb, auto between) {
-        const float used = mf;
-        f32x16 a[ST], init[ST];
+    // AHEAD tiles' bias, from tile kt on, and the next ones asked for; `between`: what is asked for once these have arrived
+    auto biases = [&](int kt, f32x16 (&init)[AHEAD], auto between) {
 #pragma unroll
-        for (int t = 0; t < ST; ++t) init[t] = bias.take(ct[t]);
+        for (int t = 0; t < AHEAD; ++t) init[t] = bias.take(ct[t]);
         between();
 #pragma unroll
-        for (int t = 0; t < ST; ++t) bias.load(kt + ST + t, ct[t]);
+        for (int t = 0; t < AHEAD; ++t) bias.load(kt + AHEAD + t, ct[t]);
+    };
+    // ST tiles, from tile kt and row kb of the stage on
+    auto step = [&](const unsigned char *buf, int kt, int kb, const f32x16 *init) {
+        const float used = mf;
+        f32x16 a[ST];
 #pragma unroll
         for (int t = 0; t < ST; ++t) score(buf, kb + 32 * t, init[t], a[t]);
         const bool lazy = kt != 0 && !__any(m != used);
@@ -183,8 +190,13 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 ? 3
         auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
         if (active) {
             const unsigned char *buf = lds[s & 1];
-            step(buf, 2 * s, 0, next);
-            if (ST == 1 && 2 * s + 1 < NT) step(buf, 2 * s + 1, 32, [] {});
+            f32x16 init[AHEAD];
+            biases(2 * s, init, next);
+            step(buf, 2 * s, 0, init);
+            if (ST == 1 && 2 * s + 1 < NT) {
+                if (AHEAD == 1) biases(2 * s + 1, init, [] {});
+                step(buf, 2 * s + 1, 32, init + AHEAD - 1);
+            }
         } else {
             next();
         }
@@ -682,7 +694,7 @@ __global__ void __launch_bounds__(256, D == 32 ? 3 : D == 64 ? 2 : 1) split_fwd(
 // As mfma_dq_wide.hip, whose place it takes at these head dims: where dBias is no sum over S rows, or its sum comes from a
 // kernel of its own.  A wave has 32 queries for all keys; with WRITE_DS (S = 1) dBias is dS and goes out as it is formed.
 template <typename T, int D, int BT, bool WRITE_DS>
-__global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 ? 3 : 2) stream_dq(EvoAttnParams p, Extra e) {
+__global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 && BT < 3 ? 3 : 2) stream_dq(EvoAttnParams p, Extra e) {
     typedef StreamGeo<D> G;
     typedef FwdStream<D> R;
     constexpr int NW = 4, KSD = D / 16, KS = KSD + 1, DT = D / 32;
@@ -737,8 +749,12 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 ? 3 : 2) stream_dq(
     }
     const v8 vaug = aug8<T>(ones3<T>(), {0u, 0u});
     const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, dead, lane);
-    typename BiasStream<T, BT, false>::Tile ct;
+    // PAIR: the caller's rows of a stage's two tiles are asked for together, and its dBias is stored together: 256 bytes of a row at a time (see
+    // stream_fwd; B = 4, S = 1, N = 1024, H = 32, fp32 312 -> 285 us).  (Loads and stores that bypass the caches: 348, 731: pieces of a line meet there.)
+    constexpr bool PAIR = D == 64 && BT >= 3;
+    typename BiasStream<T, BT, false>::Tile ct, c1;
     bias.load(0, ct);
+    if (PAIR) bias.load(1, c1);
 
     // S = 1: this lane's row of dBias[b][h]
     const int64_t dsrow = (((int64_t)pr.b * p.H + pr.h) * p.N + qrow) * p.N;
@@ -750,11 +766,8 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 ? 3 : 2) stream_dq(
 #pragma unroll
         for (int r = 0; r < 16; ++r) dq[dt][r] = 0.0f;
 
-    auto tile = [&](const unsigned char *buf, int kt, int kb, auto between) {
-        f32x16 a = bias.take(ct), dp;
-        between();
-        if (WRITE_DS) asm volatile("" ::: "memory");   // (this stage's stores are younger than what `between` asked for)
-        bias.load(kt + 1, ct);
+    auto tile = [&](const unsigned char *buf, int kb, f32x16 a, auto leave) {   // `leave` takes dS
+        f32x16 dp;
 #pragma unroll
         for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
 #pragma unroll
@@ -767,28 +780,7 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 ? 3 : 2) stream_dq(
         dp = Mfma<T>::mma(vaug, gf[KSD], dp);
 #pragma unroll
         for (int r = 0; r < 16; ++r) a[r] = fast_exp2(a[r]) * dp[r];
-        if (WRITE_DS && q0 + li < p.N) {
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                const int kg = kt * 32 + 8 * rr + 4 * g;   // registers 4 rr .. 4 rr + 3 hold keys kg .. kg + 3
-                if (ds_vec && kg + 4 <= p.N) {
-                    if (ds_f32) {
-                        f32x4 v;
-                        v[0] = a[4 * rr]; v[1] = a[4 * rr + 1]; v[2] = a[4 * rr + 2]; v[3] = a[4 * rr + 3];
-                        *reinterpret_cast<f32x4 *>((float *)p.dbias + dsrow + kg) = v;
-                    } else {
-                        store4<T>((T *)p.dbias + dsrow + kg, a[4 * rr], a[4 * rr + 1], a[4 * rr + 2], a[4 * rr + 3]);
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (kg + i < p.N) {
-                            if (ds_f32) ((float *)p.dbias)[dsrow + kg + i] = a[4 * rr + i];
-                            else ((T *)p.dbias)[dsrow + kg + i] = (T)a[4 * rr + i];
-                        }
-                }
-            }
-        }
+        leave(a);
         v8 ds[2];
 #pragma unroll
         for (int ts = 0; ts < 2; ++ts)
@@ -799,16 +791,66 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 ? 3 : 2) stream_dq(
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) dq[dt] = Mfma<T>::mma(transposed<T, D>(buf, kb, ts, dt, lane), ds[ts], dq[dt]);
     };
+    auto write = [&](int kt, const f32x16 &a) {
+        if (!WRITE_DS || q0 + li >= p.N) return;
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+            const int kg = kt * 32 + 8 * rr + 4 * g;   // registers 4 rr .. 4 rr + 3 hold keys kg .. kg + 3
+            if (ds_vec && kg + 4 <= p.N) {
+                if (ds_f32) {
+                    f32x4 v;
+                    v[0] = a[4 * rr]; v[1] = a[4 * rr + 1]; v[2] = a[4 * rr + 2]; v[3] = a[4 * rr + 3];
+                    *reinterpret_cast<f32x4 *>((float *)p.dbias + dsrow + kg) = v;
+                } else {
+                    store4<T>((T *)p.dbias + dsrow + kg, a[4 * rr], a[4 * rr + 1], a[4 * rr + 2], a[4 * rr + 3]);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (kg + i < p.N) {
+                        if (ds_f32) ((float *)p.dbias)[dsrow + kg + i] = a[4 * rr + i];
+                        else ((T *)p.dbias)[dsrow + kg + i] = (T)a[4 * rr + i];
+                    }
+            }
+        }
+    };
 
     const int nst = (p.N + R::ROWS - 1) / R::ROWS;
     wait_loads();
     wait_lds_barrier();
     for (int s = 0; s < nst; ++s) {
-        auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
+        auto next = [&] {
+            if (s + 1 < nst) fetch(s + 1);
+            if (WRITE_DS) asm volatile("" ::: "memory");   // (this stage's stores are younger than what is asked for here)
+        };
         if (active) {
             const unsigned char *buf = lds[s & 1];
-            tile(buf, 2 * s, 0, next);
-            if (2 * s + 1 < NT) tile(buf, 2 * s + 1, 32, [] {});
+            const f32x16 b0 = bias.take(ct);
+            if constexpr (PAIR) {
+                const f32x16 b1 = bias.take(c1);
+                next();
+                bias.load(2 * s + 2, ct);
+                bias.load(2 * s + 3, c1);
+                f32x16 d0;
+                tile(buf, 0, b0, [&](const f32x16 &d) { d0 = d; });
+                if (2 * s + 1 < NT) {
+                    tile(buf, 32, b1, [&](const f32x16 &d) {
+                        write(2 * s, d0);
+                        write(2 * s + 1, d);
+                    });
+                } else {
+                    write(2 * s, d0);
+                }
+            } else {
+                next();
+                bias.load(2 * s + 1, ct);
+                tile(buf, 0, b0, [&](const f32x16 &d) { write(2 * s, d); });
+                if (2 * s + 1 < NT) {
+                    const f32x16 b1 = bias.take(ct);
+                    bias.load(2 * s + 2, ct);
+                    tile(buf, 32, b1, [&](const f32x16 &d) { write(2 * s + 1, d); });
+                }
+            }
         } else {
             next();
         }
