@@ -230,6 +230,17 @@ static bool dq_wide_ok(const EvoAttnParams &p) {
 static bool long_rows_bwd_ok(const EvoAttnParams &p) { return dq_wide_ok(p); }
 static bool dq_writes_dbias(const EvoAttnParams &p) { return p.dbias && p.S == 1 && dq_wide_ok(p); }
 
+// One S row, its bias read from the caller's tensor, head dim 64: dQ (which writes dBias) and dK/dV from one launch.  512 workgroups are on the chip
+// at a time: where each kernel has just one full round of them nothing is left to fill, and two kinds of different length end less
+// evenly.  H = 32, fp32 bias, forward and backward, us, two launches / one: B = 4, N = 384 (384 workgroups of each) 95 / 90, B = 2, N = 768 (384) 175 / 169,
+// 896 (448) 224 / 221, 1024 (512) 292 / 297, B = 4, N = 512 (512) 133 / 138, 640 (640) 270 / 242, 768 347 / 324, 896 473 / 424, 1024 (1024) 582 / 525.
+static bool bwd_one_ok(const EvoAttnParams &p) {
+    constexpr int apart = EVO_FLAG_PER_PROBLEM | EVO_FLAG_ONLY_DQ | EVO_FLAG_ONLY_DKDV | EVO_FLAG_DEBUG_NO_DQ_WIDE;
+    const int64_t wgs = (int64_t)((p.N + 127) / 128) * p.B * p.H;
+    if (wgs > 448 && wgs <= 512) return false;
+    return p.D == 64 && p.S == 1 && !(p.flags & apart) && !p.gate && !p.dmask && bias_direct(p) && dq_writes_dbias(p);
+}
+
 // S is split into chunks; one workgroup of the dQ kernel sums dS over one chunk and
 // writes one partial dBias tile.  Enough chunks to fill the chip, no more.  The kernel that
 // walks over its chunk with one workgroup per CU (256 CUs) runs in rounds of 256 workgroups:
@@ -520,6 +531,7 @@ const char *evoattn_kernels(const EvoAttnParams *p, int pass) {
     if (fused_ok(*p)) return p->dbias ? "mfma_bwd_fused+mfma_dbias" : "mfma_bwd_fused";
     const bool kvr = kv_ring_ok(*p);
     if (dq_split_ok(*p)) return kvr ? "mfma_dq_wide+mfma_dbias,mfma_dkdv_ring" : "mfma_dq_wide+mfma_dbias,mfma_dkdv";
+    // (one launch of both where bwd_one_ok says so)
     if (dq_wide_ok(*p)) return kvr ? "mfma_dq_wide,mfma_dkdv_ring" : "mfma_dq_wide,mfma_dkdv";
     if (kvr) return dq_ring_ok(*p) ? "mfma_dq_ring,mfma_dkdv_ring" : "mfma_dq,mfma_dkdv_ring";
     return dq_ring_ok(*p) ? "mfma_dq_ring,mfma_dkdv" : "mfma_dq,mfma_dkdv";
@@ -637,6 +649,7 @@ int evoattn_bwd(const EvoAttnParams *p0, void *hip_stream) {
         if ((rc = launch_mfma_dbias(*p, e, st))) return rc;
         return launch_dbias_reduce(*p, e, st);
     }
+    if (!p0->gate && bwd_one_ok(*p)) return launch_stream_bwd_one_d64(*p, e, st);
     if (p->flags & EVO_FLAG_ONLY_DQ) return launch_dq(*p, e, st);
     const bool kvring = kv_ring_ok(*p);
     // that kernel sums the dBias partials on its way in (they lie 16-byte aligned for it)

@@ -52,6 +52,7 @@ inline int mfma_fused8_tiles(int N) {
 int launch_stream_fwd8(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // forward with a bias, head dim 8: two S rows per workgroup
 int launch_mfma_fused8(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_fused(const EvoAttnParams &p, const Extra &e, hipStream_t st);
+int launch_stream_bwd_one_d64(const EvoAttnParams &p, const Extra &e, hipStream_t st);   // dQ, dK, dV and dBias of one S row (mfma_stream.hip)
 int launch_mfma_dbias(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // dBias partials alone (reads delta)
 int launch_column_reduce(const float *part, int blocks, int cols, void *out, int dtype, hipStream_t st);  // out[c] = sum of part[.][c], fixed order
 

@@ -693,19 +693,18 @@ __global__ void __launch_bounds__(256, D == 32 ? 3 : D == 64 ? 2 : 1) split_fwd(
 
 // As mfma_dq_wide.hip, whose place it takes at these head dims: where dBias is no sum over S rows, or its sum comes from a
 // kernel of its own.  A wave has 32 queries for all keys; with WRITE_DS (S = 1) dBias is dS and goes out as it is formed.
+// Block `block` of 128 queries of problem `problem`, in `lds` of 2 R::BYTES.
 template <typename T, int D, int BT, bool WRITE_DS>
-__global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 && BT < 3 ? 3 : 2) stream_dq(EvoAttnParams p, Extra e) {
+__device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, unsigned char *lds, unsigned problem, int block) {
     typedef StreamGeo<D> G;
     typedef FwdStream<D> R;
     constexpr int NW = 4, KSD = D / 16, KS = KSD + 1, DT = D / 32;
     typedef typename Mfma<T>::v8 v8;
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[2][R::BYTES];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, g = lane >> 5;
-    const int NT = (p.N + 31) / 32, nqb = (p.N + 127) / 128;
-    const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
-    const Prob pr = walk_problem(p, lid / nqb);
-    const int q0 = (lid % nqb) * 128 + wave * 32, qrow = min(q0 + li, p.N - 1);
+    const int NT = (p.N + 31) / 32;
+    const Prob pr = walk_problem(p, problem);
+    const int q0 = block * 128 + wave * 32, qrow = min(q0 + li, p.N - 1);
     const bool active = q0 < p.N;
     const bool dead = e.dead[pr.b * p.S + pr.s] != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
     const int sn2 = (int)p.stride_n * 2, valid = (p.N - 1) * sn2 + D * 2;
@@ -715,7 +714,7 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 && BT < 3 ? 3 : 2) 
     const __amdgpu_buffer_rsrc_t mrs =
         __builtin_amdgcn_make_buffer_rsrc((void *)(e.m2a + ((int64_t)pr.b * p.S + pr.s) * np256), 0, np256 * 16, 0x00020000);
     auto fetch = [&](int stage) {
-        unsigned char *dst = lds[stage & 1];
+        unsigned char *dst = lds + (stage & 1) * R::BYTES;
         dma_rows<D, R::ROWS, NW>(krs, vrs, dst, stage * R::ROWS, p.N, sn2, wave, lane);
         if (wave == 0) dma16(mrs, dst + R::OFF_A, (stage * R::ROWS + lane) * 16);
     };
@@ -824,7 +823,7 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 && BT < 3 ? 3 : 2) 
             if (WRITE_DS) asm volatile("" ::: "memory");   // (this stage's stores are younger than what is asked for here)
         };
         if (active) {
-            const unsigned char *buf = lds[s & 1];
+            const unsigned char *buf = lds + (s & 1) * R::BYTES;
             const f32x16 b0 = bias.take(ct);
             if constexpr (PAIR) {
                 const f32x16 b1 = bias.take(c1);
@@ -869,6 +868,13 @@ __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 && BT < 3 ? 3 : 2) 
     }
 }
 
+template <typename T, int D, int BT, bool WRITE_DS>
+__global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 && BT < 3 ? 3 : 2) stream_dq(EvoAttnParams p, Extra e) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * FwdStream<D>::BYTES];
+    const unsigned nqb = (p.N + 127) / 128, lid = xcd_remap(blockIdx.x, gridDim.x);
+    dq_rows<T, D, BT, WRITE_DS>(p, e, lds, lid / nqb, lid % nqb);
+}
+
 // ------------------------------------------------------------------ dK and dV
 
 // A wave has 32 keys, the queries stream by.  The score product wants Q scaled and rounded, dK wants it as given: a wave
@@ -882,19 +888,20 @@ struct KvStream {
     static constexpr int OFF_K = 2 * STAGE, BYTES = OFF_K + (K_LDS ? NW * 32 * D * 2 : 0);
 };
 
-template <typename T, int D, int BT, int NW>
-__global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnParams p, Extra e) {
+// Block `block` of NW * 32 keys of problem `problem`.  OWN_DELTA: delta = <dO, O> is formed here, by four threads per row of a stage; else read.
+template <typename T, int D, int BT, int NW, bool OWN_DELTA>
+__device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e, unsigned char *lds, unsigned problem, int block) {
     typedef StreamGeo<D> G;
     typedef KvStream<D, NW> R;
     constexpr int KSD = D / 16, DT = D / 32, ROWS = R::ROWS;
+    constexpr int TPR = OWN_DELTA ? 4 : 1, OC = G::C / TPR;   // threads per row of a stage, chunks of O of each
+    static_assert(!OWN_DELTA || (NW == 4 && D == 64), "every thread has a quarter of a row of its wave's two pieces of eight");
     typedef typename Mfma<T>::v8 v8;
-    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, g = lane >> 5;
-    const int NT = (p.N + 31) / 32, nkb = (p.N + NW * 32 - 1) / (NW * 32);
-    const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
-    const Prob pr = walk_problem(p, lid / nkb);
-    const int key0 = (lid % nkb) * NW * 32 + wave * 32, key = key0 + li, keyc = min(key, p.N - 1);
+    const int NT = (p.N + 31) / 32;
+    const Prob pr = walk_problem(p, problem);
+    const int key0 = block * NW * 32 + wave * 32, key = key0 + li, keyc = min(key, p.N - 1);
     const bool active = key0 < p.N;
     const bool dead = e.dead[pr.b * p.S + pr.s] != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
     const bool want_dm = e.dmask_part != nullptr && p.dmask != nullptr;
@@ -904,11 +911,18 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
     const __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.q + pr.base), 0, valid, 0x00020000);
     const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.dout + pr.base), 0, valid, 0x00020000);
 
-    float nl = 0.0f, nd = 0.0f;   // -LSE log2(e) and -delta of a row of the stage on its way (threads 0 .. ROWS - 1)
+    // this thread's row of a stage (OWN_DELTA: of those that its wave fetches)
+    const int myrow = OWN_DELTA ? wave * 8 + (lane >> 2 & 7) + (lane >> 5) * 32 : (int)threadIdx.x;
+    float nl = 0.0f, nd = 0.0f;   // -LSE log2(e) and -delta of that row of the stage on its way (myrow < ROWS)
+    v8 orow[OWN_DELTA ? OC : 1];  // (or this thread's part of O)
     auto fetch = [&](int stage) {
         dma_rows<D, ROWS, NW>(qrs, grs, lds + (stage & 1) * R::STAGE, stage * ROWS, p.N, sn2, wave, lane);
-        const int q = stage * ROWS + (int)threadIdx.x;
-        if (threadIdx.x < ROWS) {   // rows at and beyond N: probability zero
+        const int q = stage * ROWS + myrow;
+        if constexpr (OWN_DELTA) {
+#pragma unroll
+            for (int i = 0; i < OC; ++i) orow[i] = ld8((const T *)p.o + pr.base + (int64_t)min(q, p.N - 1) * p.stride_n + (threadIdx.x % TPR * OC + i) * 8);
+            nl = q < p.N ? -p.lse[pr.row0 + q] * kLog2e : kMaskFloor;
+        } else if (myrow < ROWS) {   // rows at and beyond N: probability zero
             nl = q < p.N ? -p.lse[pr.row0 + q] * kLog2e : kMaskFloor;
             nd = q < p.N ? -e.delta[pr.row0 + q] : 0.0f;
         }
@@ -924,9 +938,19 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
             const v8 a = *reinterpret_cast<const v8 *>(buf + m * 1024 + lane * 16);
             *reinterpret_cast<v8 *>(buf + R::OFF_QS + m * 1024 + lane * 16) = scaled8<T>(a, cs);
         }
-        if (threadIdx.x < ROWS) {
-            *reinterpret_cast<v8 *>(buf + R::OFF_AQ + threadIdx.x * 16) = aug8<T>(one3, pack_split3<T>(nl));
-            *reinterpret_cast<v8 *>(buf + R::OFF_AG + threadIdx.x * 16) = aug8<T>(pack_split3<T>(nd), zero3);
+        bool mine = myrow < ROWS;
+        if constexpr (OWN_DELTA) {
+            float d = 0.0f;
+#pragma unroll
+            for (int i = 0; i < OC; ++i) d = dot8<T>(*reinterpret_cast<const v8 *>(buf + R::OFF_G + G::at(myrow, threadIdx.x % TPR * OC + i)), orow[i], d);
+            d += __shfl_xor(d, 1);
+            d += __shfl_xor(d, 2);
+            nd = -d;
+            mine = threadIdx.x % TPR == 0;
+        }
+        if (mine) {
+            *reinterpret_cast<v8 *>(buf + R::OFF_AQ + myrow * 16) = aug8<T>(one3, pack_split3<T>(nl));
+            *reinterpret_cast<v8 *>(buf + R::OFF_AG + myrow * 16) = aug8<T>(pack_split3<T>(nd), zero3);
         }
         wait_lds_barrier();
     };
@@ -1031,6 +1055,30 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
             store_row_tile<T>(dV, dt * 32, D, dv[dt], 1.0f, g);
         }
     }
+}
+
+template <typename T, int D, int BT, int NW>
+__global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnParams p, Extra e) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const unsigned nkb = (p.N + NW * 32 - 1) / (NW * 32), lid = xcd_remap(blockIdx.x, gridDim.x);
+    dkdv_rows<T, D, BT, NW, false>(p, e, lds, lid / nkb, lid % nkb);
+}
+
+// ------------------------------------------------------------------ dQ, dK, dV and dBias of one S row
+
+// With one S row the traffic is the bias, which both kernels read, and dBias, and few problems do not fill the chip with either kernel.
+// Here the workgroups of both are one launch, those of a problem next to each other on one XCD: what one has read of the bias the other finds in
+// the memory-side cache, the one that waits for memory shares the chip with the one that computes, and a last round is
+// one instead of two.  dK/dV forms delta for itself.  The last problems come first: what the forward has left in the caches.
+// H = 32, fp32 bias, dQ and dK/dV one after the other / this, us: B = 1, N = 128 19.6 / 11.2, 256 28.7 / 16.8, 512 51 / 29, 1024 101 / 90; B = 3, N = 724
+// 220 / 176; B = 4, N = 1024 424 / 387 (4.7 TB/s past L2; problems in order 388, and the next call's forward 161 instead of 144;
+// sweeps turned so that both kinds meet in the same tile at the same time: no change); H = 8, B = 1, N = 2048 176 / 93.
+template <typename T, int BT>
+__global__ void __launch_bounds__(256, 2) stream_bwd_one(EvoAttnParams p, Extra e) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const unsigned nb = (p.N + 127) / 128, lid = gridDim.x - 1 - xcd_remap(blockIdx.x, gridDim.x), problem = lid / (2 * nb), r = lid % (2 * nb);
+    if (r >= nb) dkdv_rows<T, 64, BT, 4, true>(p, e, lds, problem, r - nb);
+    else dq_rows<T, 64, BT, true>(p, e, lds, problem, r);
 }
 
 // ------------------------------------------------------------------ dBias partials
@@ -1314,6 +1362,20 @@ static int dkdv_waves(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     }
     return dkdv_bias<T, D, 4>(p, e, st);
 }
+
+#if EVO_D == 64
+int launch_stream_bwd_one_d64(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    const unsigned grid = 2 * (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H);
+    auto go = [&](auto kern) {
+        constexpr int lds = KvStream<64, 4>::BYTES;
+        static_assert(lds >= 2 * FwdStream<64>::BYTES && lds <= 64 * 1024, "the larger of the two");
+        kern<<<grid, 256, lds, st>>>(p, e);
+        return hip_rc();
+    };
+    if (p.dtype == EVO_BF16) return p.bias_dtype == EVO_F32 ? go(stream_bwd_one<bf16_t, 3>) : go(stream_bwd_one<bf16_t, 4>);
+    return p.bias_dtype == EVO_F32 ? go(stream_bwd_one<f16_t, 3>) : go(stream_bwd_one<f16_t, 4>);
+}
+#endif
 
 #if EVO_D == 32   // (mfma_bwd.hip chooses between its kernel of eight waves and this one)
 int launch_stream_dkdv_d32(const EvoAttnParams &p, const Extra &e, hipStream_t st) {

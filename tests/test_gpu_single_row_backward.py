@@ -1,0 +1,48 @@
+"""The backward of one S row at head dim 64, dQ with dBias and dK/dV in one launch (csrc/mfma_stream.hip), at the edges of its blocks of 128 queries and
+keys, stages of 64 rows and tiles of 32, against eager in fp32."""
+import pytest
+import torch
+
+from oracle import eager
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # B, N, H, mask, bias, layout, dtype
+    (32, 4, 1, "bool", "f32", "reference", torch.bfloat16),      # the smallest: one block of each kind per problem, four rows of it
+    (16, 64, 2, "dead", "f32", "ds4sci", torch.float16),         # one whole stage
+    (11, 68, 3, "soft", "q", "reference", torch.bfloat16),       # a second stage of four rows
+    (2, 128, 16, "dead_added", "f32", "reference", torch.bfloat16),
+    (4, 132, 5, "dead", "f32", "reference", torch.bfloat16),     # a second block of four rows
+    (2, 256, 8, "dead", "q", "ds4sci", torch.float16),
+    (3, 292, 4, "bool", "f32", "ds4sci", torch.bfloat16),        # an odd number of tiles
+    (1, 516, 8, None, "f32", "reference", torch.float16),
+    (2, 1000, 3, "dead_added", "q", "reference", torch.bfloat16),
+    (3, 724, 32, "bool", "f32", "reference", torch.bfloat16),    # more workgroups than the chip takes at a time
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_single_row_backward_matches_eager(gpu_device, case):
+    import evoformer_triton_amd.evoformer as E
+    B, N, H, mask, bias, layout, dt = case
+    g = torch.Generator().manual_seed(31)
+    Q, K, V, dO = ((torch.randn((B, 1, N, H, 64), generator=g) * 0.7).to(dt) for _ in range(4))
+    keep = torch.rand((B, 1, 1, 1, N), generator=g) < 0.85
+    keep[..., 0] = True
+    if mask in ("dead", "dead_added"):
+        keep[1] = False
+    m = {None: None, "bool": keep, "dead": keep, "dead_added": torch.where(keep, 0.0, -1e9), "soft": torch.randn((B, 1, 1, 1, N), generator=g)}[mask]
+    b = (torch.randn((B, 1, H, N, N), generator=g) * 0.5).to(torch.float32 if bias == "f32" else dt)
+    xs = [None if t is None else t.to(gpu_device) for t in (Q, K, V, m, b, dO)]
+    ref = eager.attention_fwd_bwd(*xs, layout=layout, compute_dtype=torch.float32, s_chunk=16)
+    q, k, v = (t.detach().clone().requires_grad_() for t in xs[:3])
+    bb = xs[4].detach().clone().requires_grad_()
+    o = E.evoformer_attention(q, k, v, xs[3], bb, layout=layout)
+    o.backward(xs[5])
+    # P, dS, the scaled Q, O (in delta) and the results are each rounded by at most 2^-9 of their size, and the errors of the probabilities that
+    # come of the scaled Q are of that order too: 5 * 2^-9, as relative 2-norms
+    for name, t in {"O": o, "dQ": q.grad, "dK": k.grad, "dV": v.grad, "dBias": bb.grad}.items():
+        want = ref[name].float()
+        d = t.detach().float() - want
+        assert torch.isfinite(d).all(), name
+        assert d.norm() <= 1e-2 * want.norm(), (name, (d.norm() / want.norm()).item())
