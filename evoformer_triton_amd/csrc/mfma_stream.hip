@@ -889,7 +889,8 @@ struct KvStream {
 };
 
 // Block `block` of NW * 32 keys of problem `problem`.  OWN_DELTA: delta = <dO, O> is formed here, by four threads per row of a stage; else read.
-template <typename T, int D, int BT, int NW, bool OWN_DELTA>
+// DM: the row sums of dS that a mask's gradient is summed from are wanted (head dim 64; the other head dims ask at run time).
+template <typename T, int D, int BT, int NW, bool OWN_DELTA, bool DM>
 __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e, unsigned char *lds, unsigned problem, int block) {
     typedef StreamGeo<D> G;
     typedef KvStream<D, NW> R;
@@ -904,7 +905,7 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
     const int key0 = block * NW * 32 + wave * 32, key = key0 + li, keyc = min(key, p.N - 1);
     const bool active = key0 < p.N;
     const bool dead = e.dead[pr.b * p.S + pr.s] != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
-    const bool want_dm = e.dmask_part != nullptr && p.dmask != nullptr;
+    const bool want_dm = DM || (D != 64 && e.dmask_part != nullptr && p.dmask != nullptr);
     const float cs = p.scale * kLog2e;
     const uint2 one3 = ones3<T>(), zero3 = {0u, 0u};
     const int sn2 = (int)p.stride_n * 2, valid = (p.N - 1) * sn2 + D * 2;
@@ -972,8 +973,14 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
         vaug = g == 0 && !kill ? aug8<T>(one3, zero3) : zero8<T>();    // ones x -delta
     }
     const BiasStream<T, BT, true> bias(p, e, pr, min(key0 >> 5, NT - 1), keyc, dead, lane);
-    typename BiasStream<T, BT, true>::Tile ct;
+    // TWO: the bias of a stage's two tiles is asked for when the stage before begins, which its end waits for anyway, and nothing in a tile is waited
+    // for or branched on.  S = 200, N = 640, H = 5, fp32 bias 331 -> 321 us; B = 4, S = 1, N = 1024, H = 32 with dQ 387 -> 378.  (Head dim 32 spills with
+    // a second tile under way.  Every read of LDS four or six matrix instructions ahead of its use, by groups of the scheduler: 320; two waves
+    // per SIMD hide these already.)
+    constexpr bool TWO = D == 64;
+    typename BiasStream<T, BT, true>::Tile ct, c1;
     bias.load(0, ct);
+    if (TWO) bias.load(1, c1);
     // (the dBias partials of the kernels before this one, summed on the way in where the caller asks for it)
     if (e.dbias_chunks > 0) sum_dbias_partials<NW * 64>(p, e, threadIdx.x);
 
@@ -984,10 +991,8 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
         for (int r = 0; r < 16; ++r) dk[dt][r] = dv[dt][r] = 0.0f;
     float dm = 0.0f;
 
-    auto tile = [&](const unsigned char *buf, int qt, int qb, auto between) {
-        f32x16 a = bias.take(ct), dp;
-        between();
-        if (D < 128) bias.load(qt + 1, ct);
+    auto tile = [&](const unsigned char *buf, int qb, auto begin, auto behind) {   // `begin`: the bias, and what is asked for once it is there
+        f32x16 a = begin(), dp;
 #pragma unroll
         for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
 #pragma unroll
@@ -1001,7 +1006,7 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
         }
         a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_AQ + (qb + li) * 16), kaug, a);
         dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_AG + (qb + li) * 16), vaug, dp);
-        if (D == 128) bias.load(qt + 1, ct);   // (no registers for it any sooner)
+        behind();
         v8 pf[2], ds[2];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -1034,8 +1039,26 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
         auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
         if (active) {
             const unsigned char *buf = lds + (s & 1) * R::STAGE;
-            tile(buf, s * (ROWS / 32), 0, next);
-            if (ROWS == 64 && 2 * s + 1 < NT) tile(buf, 2 * s + 1, 32, [] {});
+            const int qt = s * (ROWS / 32);
+            if constexpr (TWO) {
+                const f32x16 b0 = bias.take(ct), b1 = bias.take(c1);
+                next();
+                bias.load(qt + 2, ct);
+                bias.load(qt + 3, c1);
+                tile(buf, 0, [&] { return b0; }, [] {});
+                if (qt + 1 < NT) tile(buf, 32, [&] { return b1; }, [] {});
+            } else {
+                auto one = [&](int t, int qb, auto then) {
+                    tile(buf, qb, [&] {
+                        const f32x16 b = bias.take(ct);
+                        then();
+                        if (D < 128) bias.load(t + 1, ct);
+                        return b;
+                    }, [&] { if (D == 128) bias.load(t + 1, ct); });   // (no registers for it any sooner)
+                };
+                one(qt, 0, next);
+                if (ROWS == 64 && qt + 1 < NT) one(qt + 1, 32, [] {});
+            }
         } else {
             next();
         }
@@ -1057,11 +1080,11 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
     }
 }
 
-template <typename T, int D, int BT, int NW>
+template <typename T, int D, int BT, int NW, bool DM>
 __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnParams p, Extra e) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const unsigned nkb = (p.N + NW * 32 - 1) / (NW * 32), lid = xcd_remap(blockIdx.x, gridDim.x);
-    dkdv_rows<T, D, BT, NW, false>(p, e, lds, lid / nkb, lid % nkb);
+    dkdv_rows<T, D, BT, NW, false, DM>(p, e, lds, lid / nkb, lid % nkb);
 }
 
 // ------------------------------------------------------------------ dQ, dK, dV and dBias of one S row
@@ -1071,13 +1094,13 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
 // the memory-side cache, the one that waits for memory shares the chip with the one that computes, and a last round is
 // one instead of two.  dK/dV forms delta for itself.  The last problems come first: what the forward has left in the caches.
 // H = 32, fp32 bias, dQ and dK/dV one after the other / this, us: B = 1, N = 128 19.6 / 11.2, 256 28.7 / 16.8, 512 51 / 29, 1024 101 / 90; B = 3, N = 724
-// 220 / 176; B = 4, N = 1024 424 / 387 (4.7 TB/s past L2; problems in order 388, and the next call's forward 161 instead of 144;
+// 220 / 171; B = 4, N = 1024 424 / 378 (4.8 TB/s past L2; problems in order the next call's forward takes 161 instead of 144;
 // sweeps turned so that both kinds meet in the same tile at the same time: no change); H = 8, B = 1, N = 2048 176 / 93.
 template <typename T, int BT>
 __global__ void __launch_bounds__(256, 2) stream_bwd_one(EvoAttnParams p, Extra e) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const unsigned nb = (p.N + 127) / 128, lid = gridDim.x - 1 - xcd_remap(blockIdx.x, gridDim.x), problem = lid / (2 * nb), r = lid % (2 * nb);
-    if (r >= nb) dkdv_rows<T, 64, BT, 4, true>(p, e, lds, problem, r - nb);
+    if (r >= nb) dkdv_rows<T, 64, BT, 4, true, false>(p, e, lds, problem, r - nb);
     else dq_rows<T, 64, BT, true>(p, e, lds, problem, r);
 }
 
@@ -1338,7 +1361,10 @@ template <typename T, int D, int BT, int NW>
 static int dkdv_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const unsigned grid = (unsigned)((p.N + NW * 32 - 1) / (NW * 32)) * (unsigned)(p.B * p.H * p.S);
     constexpr int lds = KvStream<D, NW>::BYTES;
-    auto kern = stream_dkdv<T, D, BT, NW>;
+    auto kern = stream_dkdv<T, D, BT, NW, false>;
+    if constexpr (D == 64) {
+        if (p.dmask) kern = stream_dkdv<T, D, BT, NW, true>;
+    }
     if constexpr (lds > 64 * 1024) {
         static PerDevice done{};
         if (const int rc = ensure_dynamic_lds((const void *)kern, lds, done, nullptr)) return rc;
