@@ -125,7 +125,18 @@ static int bias_vec_ok(const EvoAttnParams &p) {
 // used one; each kernel then reads 2 or 4 bytes per entry and S row.  With very few S rows per (batch, head) - the reference's own speed benchmark has one -
 // the one-workgroup-per-problem kernels read the caller's tensor instead, which needs rows that
 // allow 16-byte (fp32) or 8-byte loads.  EVO_FLAG_DEBUG_BIAS_TILES keeps the tiles, for comparison.
+//
+// One S row of an fp32 bias whose rows start or end within a group of four (any length that is no multiple of 4): the kernels for head
+// dim 64 read these in place too, and the tiles, which nobody then needs, are most of such a call.  Forward and backward, us, H = 32, tiles / in place: B = 1, N = 251
+// 55 / 36, 517 101 / 78, 1023 284 / 158; B = 2, N = 771 357 / 216; B = 4, N = 517 362 / 211, 1023 1116 / 633 (N = 1024: 525).
+// Fewer than 32 workgroups keep the tiles: their backward is another kernel's.
+static bool bias_ragged(const EvoAttnParams &p) {
+    if (!p.bias || p.S != 1 || p.D != 64 || p.bias_dtype != EVO_F32 || p.dtype == EVO_F32 || (p.flags & EVO_FLAG_DEBUG_BIAS_TILES)) return false;
+    if ((p.N % 4 == 0 && bias_vec_ok(p)) || p.N < 4 || (int64_t)p.N * p.bias_stride_row >= ((int64_t)1 << 31)) return false;
+    return (int64_t)((p.N + 127) / 128) * p.B * p.H >= 32;
+}
 static bool bias_direct(const EvoAttnParams &p) {
+    if (bias_ragged(p)) return true;
     if (!p.bias || p.S > 4 || (p.flags & EVO_FLAG_DEBUG_BIAS_TILES) || p.N % 4) return false;
     // The 16-bit tiles of a bias in the dtype of q are cheap to prepare (2 + 4 bytes of traffic per entry at
     // streaming rate) and pay from the first S row on where the score work per entry is small: they are taken
@@ -156,6 +167,7 @@ static bool dq_ring_ok(const EvoAttnParams &p) {
 // kernels that split a row's keys over the waves finish sooner (N = 300, 6 workgroups: 10.4 us
 // against 8.2 us).  EVO_FLAG_DEBUG_NO_DQ_WIDE selects the other kernels, for comparison.
 static bool dq_wide_grid_ok(const EvoAttnParams &p) {
+    if (bias_ragged(p)) return true;   // (the other dQ kernels read such rows as tiles, which are not made)
     return !(p.flags & (EVO_FLAG_PER_PROBLEM | EVO_FLAG_DEBUG_NO_DQ_WIDE)) && (int64_t)((p.N + 127) / 128) * p.B * p.H * p.S >= 32;
 }
 

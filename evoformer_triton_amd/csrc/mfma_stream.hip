@@ -795,11 +795,11 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
             const int kg = kt * 32 + 8 * rr + 4 * g;   // registers 4 rr .. 4 rr + 3 hold keys kg .. kg + 3
-            if (ds_vec && kg + 4 <= p.N) {
+            if ((ds_vec || ds_f32) && kg + 4 <= p.N) {   // (16 bytes in fp32 wherever they start)
                 if (ds_f32) {
                     f32x4 v;
                     v[0] = a[4 * rr]; v[1] = a[4 * rr + 1]; v[2] = a[4 * rr + 2]; v[3] = a[4 * rr + 3];
-                    *reinterpret_cast<f32x4 *>((float *)p.dbias + dsrow + kg) = v;
+                    *reinterpret_cast<f32x4_at4 *>((float *)p.dbias + dsrow + kg) = v;
                 } else {
                     store4<T>((T *)p.dbias + dsrow + kg, a[4 * rr], a[4 * rr + 1], a[4 * rr + 2], a[4 * rr + 3]);
                 }
@@ -1100,7 +1100,7 @@ template <typename T, int BT>
 __global__ void __launch_bounds__(256, 2) stream_bwd_one(EvoAttnParams p, Extra e) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const unsigned nb = (p.N + 127) / 128, lid = gridDim.x - 1 - xcd_remap(blockIdx.x, gridDim.x), problem = lid / (2 * nb), r = lid % (2 * nb);
-    if (r >= nb) dkdv_rows<T, 64, BT, 4, true, false>(p, e, lds, problem, r - nb);
+    if (r >= nb) dkdv_rows<T, 64, BT == 5 ? 3 : BT, 4, true, false>(p, e, lds, problem, r - nb);
     else dq_rows<T, 64, BT, true>(p, e, lds, problem, r);
 }
 
@@ -1292,6 +1292,9 @@ static bool fwd_pair_ok(const EvoAttnParams &p, const Extra &e, int64_t pairs) {
 }
 #endif
 
+// the caller's bias rows start or end within a group of four (fp32, head dim 64: bias_ragged in api.hip)
+static bool ragged_rows(const EvoAttnParams &p, const Extra &e) { return p.N % 4 != 0 || !e.vec_ok; }
+
 template <typename T, int D>
 static int fwd_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const unsigned grid = (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H * p.S);
@@ -1304,6 +1307,7 @@ static int fwd_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     }
 #endif
     if (p.bias_dtype == EVO_NONE) stream_fwd<T, D, 0><<<grid, 256, 0, st>>>(p, e);
+    else if (e.bias_direct && p.bias_dtype == EVO_F32 && ragged_rows(p, e)) stream_fwd<T, D, D == 64 ? 5 : 3><<<grid, 256, 0, st>>>(p, e);
     else if (e.bias_direct && p.bias_dtype == EVO_F32) stream_fwd<T, D, 3><<<grid, 256, 0, st>>>(p, e);
     else if (e.bias_direct) stream_fwd<T, D, 4><<<grid, 256, 0, st>>>(p, e);
     else if (e.bq16) stream_fwd<T, D, 2><<<grid, 256, 0, st>>>(p, e);
@@ -1342,10 +1346,12 @@ static int dq_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const bool f32_rows = e.bias_direct && p.bias_dtype == EVO_F32, t16_rows = e.bias_direct && !f32_rows, t16 = e.bq16 != nullptr;
     if (p.dbias && p.S != 1) return EVO_EUNSUPPORTED;   // (a sum over S rows is the other kernels' business)
     if (p.bias_dtype == EVO_NONE) stream_dq<T, D, 0, false><<<grid, 256, 0, st>>>(p, e);
+    else if (!p.dbias && f32_rows && ragged_rows(p, e)) stream_dq<T, D, D == 64 ? 5 : 3, false><<<grid, 256, 0, st>>>(p, e);
     else if (!p.dbias && f32_rows) stream_dq<T, D, 3, false><<<grid, 256, 0, st>>>(p, e);
     else if (!p.dbias && t16_rows) stream_dq<T, D, 4, false><<<grid, 256, 0, st>>>(p, e);
     else if (!p.dbias && t16) stream_dq<T, D, 2, false><<<grid, 256, 0, st>>>(p, e);
     else if (!p.dbias) stream_dq<T, D, 1, false><<<grid, 256, 0, st>>>(p, e);
+    else if (f32_rows && ragged_rows(p, e)) stream_dq<T, D, D == 64 ? 5 : 3, true><<<grid, 256, 0, st>>>(p, e);
     else if (f32_rows) stream_dq<T, D, 3, true><<<grid, 256, 0, st>>>(p, e);
     else if (t16_rows) stream_dq<T, D, 4, true><<<grid, 256, 0, st>>>(p, e);
     else if (t16) stream_dq<T, D, 2, true><<<grid, 256, 0, st>>>(p, e);
@@ -1398,8 +1404,8 @@ int launch_stream_bwd_one_d64(const EvoAttnParams &p, const Extra &e, hipStream_
         kern<<<grid, 256, lds, st>>>(p, e);
         return hip_rc();
     };
-    if (p.dtype == EVO_BF16) return p.bias_dtype == EVO_F32 ? go(stream_bwd_one<bf16_t, 3>) : go(stream_bwd_one<bf16_t, 4>);
-    return p.bias_dtype == EVO_F32 ? go(stream_bwd_one<f16_t, 3>) : go(stream_bwd_one<f16_t, 4>);
+    if (p.dtype == EVO_BF16) return p.bias_dtype == EVO_F32 ? ragged_rows(p, e) ? go(stream_bwd_one<bf16_t, 5>) : go(stream_bwd_one<bf16_t, 3>) : go(stream_bwd_one<bf16_t, 4>);
+    return p.bias_dtype == EVO_F32 ? ragged_rows(p, e) ? go(stream_bwd_one<f16_t, 5>) : go(stream_bwd_one<f16_t, 3>) : go(stream_bwd_one<f16_t, 4>);
 }
 #endif
 

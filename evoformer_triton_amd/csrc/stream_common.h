@@ -79,7 +79,8 @@ __device__ __forceinline__ typename Mfma<T>::v8 transposed(const unsigned char *
 
 // The bias tiles of one wave: its 32 rows (or, COLS, its 32 columns) against the tiles of the other side.
 // BT: 1 prepared fp32 tiles (times log2 e), 2 prepared 16-bit tiles as given; the caller's rows (few S rows), 3 in fp32, 4 in the
-// dtype of q.  A tile is kept as it comes from memory: whatever is done to it (`value`) would wait for it.
+// dtype of q, 5 in fp32 where rows start anywhere and end within a group of four.  A tile is kept as it comes from memory: whatever is done to it (`value`) would wait for it.
+typedef f32x4 f32x4_at4 __attribute__((aligned(4)));   // (the load path takes 16 bytes at any multiple of four)
 struct Rows16 {   // entry r, the 16 bits as given, in the low half of w[r] (columns) or two to a register (rows)
     unsigned w[16];
 };
@@ -102,7 +103,7 @@ struct BiasStream {
         if (BT >= 3) {
             row_stride = dead ? 0u : (unsigned)p.bias_stride_row;
             col = (unsigned)own_row;
-            mat = dead ? dead_bias(p, e, pr.b, pr.s) : (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h + (COLS ? 0 : (int64_t)own_row * p.bias_stride_row)) * (BT == 3 ? 4 : 2);
+            mat = dead ? dead_bias(p, e, pr.b, pr.s) : (const char *)p.bias + ((int64_t)bb * p.bias_stride_b + (int64_t)pr.h * p.bias_stride_h + (COLS ? 0 : (int64_t)own_row * p.bias_stride_row)) * (BT == 4 ? 2 : 4);
         } else {
             const int64_t first = (((int64_t)bb * p.H + pr.h) * NT * NT + (COLS ? own_tile : own_tile * NT)) * 1024;
             step = dead ? 0 : COLS ? (int64_t)NT * 1024 : 1024;
@@ -120,16 +121,23 @@ struct BiasStream {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const unsigned o = (unsigned)min(t * 32 + crow(r, g), N - 1) * row_stride + col;
-                if constexpr (BT == 3) dst[r] = ((const float *)mat)[o];
+                if constexpr (BT != 4) dst[r] = ((const float *)mat)[o];
                 else dst.w[r] = ((const unsigned short *)mat)[o];
             }
+        }
+        if (BT == 5 && !COLS && t * 32 + 32 > N) {   // (uniform: the last tile, entry by entry)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if constexpr (BT == 5) dst[r] = ((const float *)mat)[min(t * 32 + crow(r, g), N - 1)];
+            }
+            return;
         }
         if constexpr (BT >= 3 && !COLS) {
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
                 const int c = min(t * 32 + 8 * rr + 4 * g, N - 4);
-                if constexpr (BT == 3) {
-                    const f32x4 v = *reinterpret_cast<const f32x4 *>((const float *)mat + c);
+                if constexpr (BT != 4) {
+                    const f32x4 v = BT == 5 ? *reinterpret_cast<const f32x4_at4 *>((const float *)mat + c) : *reinterpret_cast<const f32x4 *>((const float *)mat + c);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) dst[4 * rr + i] = v[i];
                 } else {
@@ -146,7 +154,7 @@ struct BiasStream {
             f32x16 v;
             unpack_tile16<T>(t, mul, v);
             return v;
-        } else if constexpr (BT == 3) {
+        } else if constexpr (BT == 3 || BT == 5) {
             f32x16 v;
 #pragma unroll
             for (int r = 0; r < 16; ++r) v[r] = t[r] * mul;

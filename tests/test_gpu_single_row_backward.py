@@ -17,6 +17,13 @@ CASES = [  # B, N, H, mask, bias, layout, dtype
     (3, 292, 4, "bool", "f32", "ds4sci", torch.bfloat16),        # an odd number of tiles
     (1, 516, 8, None, "f32", "reference", torch.float16),
     (2, 1000, 3, "dead_added", "q", "reference", torch.bfloat16),
+    (32, 5, 1, "dead", "f32", "reference", torch.bfloat16),      # rows that end within a group of four: one entry of it,
+    (16, 31, 2, "bool", "f32", "ds4sci", torch.float16),         # three in a tile's last group,
+    (8, 33, 4, "soft", "f32", "reference", torch.bfloat16),      # a tile of one key,
+    (3, 250, 8, "dead_added", "f32", "reference", torch.bfloat16),
+    (2, 517, 5, "dead", "f32", "ds4sci", torch.bfloat16),
+    (4, 1023, 17, "bool", "f32", "reference", torch.float16),    # 544 workgroups of each kind
+    (4, 1023, 16, "bool", "f32", "reference", torch.bfloat16),   # 512: two launches
     (3, 724, 32, "bool", "f32", "reference", torch.bfloat16),    # more workgroups than the chip takes at a time
 ]
 
