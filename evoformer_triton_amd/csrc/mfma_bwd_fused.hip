@@ -89,11 +89,13 @@ __global__ void __launch_bounds__(256, 2) bwd_fused(EvoAttnParams p, Extra e, un
             const int key0 = kb * R::KB + wave * KT * 16;
             v8 orow;
             float lse;
-            auto fetch = [&](int stage, int parity) {   // (rows past the end: zeros)
+            auto fetch = [&](int stage, int parity, bool ask) {   // (rows past the end: zeros)
                 unsigned char *dst = lds + parity * R::STAGE + wave * 1024;
                 const int from = stage * R::QR * sn2;
-                fused_dma(qrs, dst, doff, from);
-                fused_dma(grs, dst + R::OFF_G, doff, from);
+                if (ask) {
+                    fused_dma(qrs, dst, doff, from);
+                    fused_dma(grs, dst + R::OFF_G, doff, from);
+                }
                 orow = __builtin_bit_cast(v8, __builtin_amdgcn_raw_buffer_load_b128(ors, doff, from, 0));
                 lse = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(lrs, drow * 4, stage * R::QR * 4, 0));
             };
@@ -118,7 +120,7 @@ __global__ void __launch_bounds__(256, 2) bwd_fused(EvoAttnParams p, Extra e, un
                 const int m = wave * (R::KBYTES / 4096) + i, r = m * R::RPP + lane / R::C, ch = (lane % R::C) ^ R::xk(r);
                 fused_dma(krs, keys + m * 1024, r * sn2 + ch * 16, kb * R::KB * sn2);
             }
-            fetch(0, 0);
+            fetch(0, 0, true);
             v8 kf[KT], vf[KT];
             v8 mk[KT];   // the keys' columns of the step that adds mask and -LSE: in its first eight, of lanes 0 to 15, alone
 #pragma unroll
@@ -213,12 +215,12 @@ __global__ void __launch_bounds__(256, 2) bwd_fused(EvoAttnParams p, Extra e, un
 #pragma unroll
                 for (int u = 0; u < 2 * GPS; ++u) {
                     const int n = n0 + u, s1 = min(n / GPS + 1, nst - 1), gb = u % GPS * 32, parity = u / GPS;
-                    const bool first = u % GPS == 0, last = u % GPS == GPS - 1 || n + 1 >= NT;   // group of its stage
+                    const bool first = u % GPS == 0, last = u % GPS == GPS - 1, more = n / GPS + 1 < nst;   // group of its stage; a stage follows (this one is whole)
                     if (n < NT) {
                     const unsigned char *buf = lds + parity * R::STAGE;
                     unsigned char *const exb = ex + (u & 1) * R::EX, *const exq = ex + ((u & 1) ^ 1) * R::EX;
                     dq_store(n - 2);
-                    if (first) fetch(s1, parity ^ 1);   // (after the last stage: that one once more, for nobody)
+                    if (first) fetch(s1, parity ^ 1, more);
                     dq_begin(n - 1);
                     asm volatile("" ::: "memory");   // (the bias asked for below is younger: `finish` counts on it)
 
@@ -247,7 +249,8 @@ __global__ void __launch_bounds__(256, 2) bwd_fused(EvoAttnParams p, Extra e, un
                         }
 #pragma unroll
                     for (int kt = 0; kt < KT; ++kt) {
-                        if (kt == KT - 1 && last)   // (since then this wave has asked for the bias of the tiles between, a load or, in fp32, two for each)
+                        // since `fetch`, GPS - 1 groups before, this wave has asked for the bias of the tiles between, a load or, in fp32, two for each
+                        if (kt == KT - 1 && last && more)
                             finish(s1, parity ^ 1, std::integral_constant<int, (BT == 0 ? 0 : BT == 1 ? 2 : 1) * (KT * GPS - 1)>());
                         f32x4 a[2], dp[2];
                         if (BT == 2) {

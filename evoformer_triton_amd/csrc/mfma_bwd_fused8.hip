@@ -92,9 +92,9 @@ __global__ void __launch_bounds__(256, KT == 2 ? 3 : 2) bwd_fused8(EvoAttnParams
             const int key0 = kb * R::KB + wave * KT * 16;
             v8 orow;
             float lse;
-            auto fetch = [&](int stage, int parity) {   // (rows past the end: zeros)
+            auto fetch = [&](int stage, int parity, bool ask) {   // (rows past the end: zeros)
                 const int from = stage * R::QR * sn2;
-                fused_dma(frs, lds + parity * R::STAGE + (has_q ? 0 : R::OFF_G) + (wave & 1) * 1024, doff, from);
+                if (ask) fused_dma(frs, lds + parity * R::STAGE + (has_q ? 0 : R::OFF_G) + (wave & 1) * 1024, doff, from);
                 orow = __builtin_bit_cast(v8, __builtin_amdgcn_raw_buffer_load_b128(ors, ooff, from, 0));
                 lse = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(lrs, loff, stage * R::QR * 4, 0));
             };
@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(256, KT == 2 ? 3 : 2) bwd_fused8(EvoAttnParams
             };
             // the block's keys in LDS
             for (int i = wave; i < KT; i += R::NW) fused_dma(krs, ex + i * 1024, (i * 64 + lane) * sn2, kb * R::KB * sn2);
-            fetch(0, 0);
+            fetch(0, 0, true);
             v8 kv[KT];
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt) {
@@ -209,12 +209,12 @@ __global__ void __launch_bounds__(256, KT == 2 ? 3 : 2) bwd_fused8(EvoAttnParams
 #pragma unroll
                 for (int u = 0; u < 2 * GPS; ++u) {
                     const int n = n0 + u, s1 = min(n / GPS + 1, nst - 1), gb = u % GPS * 32, parity = u / GPS;
-                    const bool first = u % GPS == 0, last = u % GPS == GPS - 1 || n + 1 >= NT;   // group of its stage
+                    const bool first = u % GPS == 0, last = u % GPS == GPS - 1, more = n / GPS + 1 < nst;   // group of its stage; a stage follows (this one is whole)
                     if (n < NT) {   // uniform
                         const unsigned char *buf = lds + parity * R::STAGE;
                         unsigned char *const exb = ex + (u & 1) * R::EX, *const exq = ex + ((u & 1) ^ 1) * R::EX;
                         dq_store(n - 2, (u & 1) ^ 1);
-                        if (first) fetch(s1, parity ^ 1);   // (after the last stage: that one once more, for nobody)
+                        if (first) fetch(s1, parity ^ 1, more);
                         dq_begin(n - 1);
                         asm volatile("" ::: "memory");   // (the bias asked for below is younger: `finish` counts on it)
 
@@ -237,7 +237,8 @@ __global__ void __launch_bounds__(256, KT == 2 ? 3 : 2) bwd_fused8(EvoAttnParams
                         }
 #pragma unroll
                         for (int kt = 0; kt < KT; ++kt) {
-                            if (kt == KT - 1 && last)   // (since then this wave has asked for the bias of the tiles between, a load or, in fp32, two for each)
+                            // since `fetch`, GPS - 1 groups before, this wave has asked for the bias of the tiles between, a load or, in fp32, two for each
+                            if (kt == KT - 1 && last && more)
                                 finish(s1, parity ^ 1, std::integral_constant<int, (BT == 0 ? 0 : BT == 1 ? 2 : 1) * (KT * GPS - 1)>());
                             f32x4 a[2], dp[2];
                             if (BT == 2) {

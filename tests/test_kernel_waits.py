@@ -44,3 +44,80 @@ def test_a_split_forwards_fetch_follows_the_reads_of_its_buffer(head_dim, tmp_pa
                 assert waited, (name, line)
                 seen += 1
     assert seen >= 6      # two dtypes, three kinds of bias
+
+
+VMEM = re.compile(r"(buffer|global|flat|scratch)_(load|store|atomic)")
+
+
+def _blocks(lines):
+    """Basic blocks as (instructions, successors): by label, with whether an instruction was written by hand."""
+    blocks, name, hand = {"entry": []}, "entry", False
+    order = ["entry"]
+    for line in lines:
+        label = re.match(r"(\.LBB\w+):", line)
+        s = line.strip()
+        if label:
+            name = label.group(1)
+            blocks[name] = []
+            order.append(name)
+        elif s.startswith(";"):
+            hand = "#ASMSTART" in s or (hand and "#ASMEND" not in s)
+        elif s and not s.startswith("."):
+            blocks[name].append((s.split(";")[0].strip(), hand))
+            if s.startswith(("s_cbranch", "s_branch", "s_endpgm")):   # (what follows a branch is a block of its own)
+                name = f"{order[-1]}+"
+                blocks[name] = []
+                order.append(name)
+    following = {}
+    for i, b in enumerate(order):
+        end = blocks[b][-1][0] if blocks[b] else ""
+        following[b] = []
+        if end.startswith(("s_cbranch", "s_branch")):
+            following[b].append(end.split()[1])
+        if not end.startswith(("s_branch", "s_endpgm")) and i + 1 < len(order):
+            following[b].append(order[i + 1])
+    return blocks, following
+
+
+def _after(instructions, younger, check=None):
+    """`younger`: the fewest memory instructions that may have been issued since the last load into LDS that may be under way; None where none is."""
+    for s, hand in instructions:
+        wait = re.match(r"s_waitcnt\b.*vmcnt\((\d+)\)", s)
+        if wait:
+            if younger is not None and int(wait.group(1)) <= younger:
+                younger = None
+            if hand and check is not None:
+                check(s, younger)
+        elif VMEM.match(s):
+            younger = 0 if s.endswith(" lds") else younger if younger is None else min(younger + 1, 64)
+    return younger
+
+
+@pytest.mark.parametrize("source", ["mfma_bwd_fused.hip", "mfma_bwd_fused8.hip"])
+def test_a_stage_is_there_when_it_is_prepared(source, tmp_path):
+    """The kernels that form dQ, dK and dV at once wait for all but so many of the youngest loads before they read what they had loaded into LDS: on every way
+    through the kernel at least as many have been issued since."""
+    text = _assembly(source, [], tmp_path)
+    seen = 0
+    for name, lines in _functions(text, "bwd_fused"):
+        blocks, following = _blocks(lines)
+        into = {"entry": None}
+        todo = ["entry"]
+        while todo:
+            b = todo.pop()
+            out = _after(blocks[b], into[b])
+            for f in following[b]:
+                new = out if f not in into else into[f] if out is None else out if into[f] is None else min(out, into[f])
+                if f not in into or new != into[f]:
+                    into[f] = new
+                    todo.append(f)
+
+        def check(s, younger):
+            nonlocal seen
+            seen += 1
+            assert younger is None, (name, s, younger)
+
+        for b in blocks:
+            if b in into:
+                _after(blocks[b], into[b], check)
+    assert seen >= 36     # two dtypes, three kinds of bias, three widths or more, the first stage and the others
