@@ -223,6 +223,7 @@ static bool fused_ok(const EvoAttnParams &p) {
                           EVO_FLAG_DEBUG_NO_DQ_SPLIT | EVO_FLAG_DEBUG_OTHER_WIDTH;
     if ((p.flags & apart) || (p.dtype != EVO_BF16 && p.dtype != EVO_F16) || (p.D != 32 && p.D != 8) || p.gate || p.dmask || bias_direct(p)) return false;
     if (p.N < 96 || p.N > 2048) return false;
+    if (p.dbias && !p.bias) return false;   // (the dBias kernel keeps bias tiles; dBias without a bias, the sum of dS alone, comes with dQ)
     const int64_t problems = (int64_t)p.B * p.H * p.S;
     const double full = (double)problems / (double)((problems + 255) / 256 * 256);
     if (p.D == 8) return problems >= 256 && (!p.dbias || (p.S >= 8 && (p.N > 512 || (p.N >= 288 && problems >= 768 && full >= 0.9))));

@@ -151,6 +151,22 @@ def test_path_selection(lib):
     assert lib.evoattn_path(ctypes.byref(p), 1) == b"mfma"
 
 
+@pytest.mark.parametrize("shape", [(1, 384, 384, 4, 32), (1, 192, 705, 4, 32), (1, 64, 2048, 8, 32), (1, 1024, 384, 8, 8), (1, 256, 600, 8, 8)])
+def test_dbias_without_a_bias_comes_with_dq(lib, shape):
+    """The kernel that sums dBias by itself keeps the bias' tiles: without a bias there are none, and the dQ kernels sum dS."""
+    p = good(*shape)
+    assert b"+mfma_dbias" in lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD)
+    p.bias, p.bias_dtype = None, _lib.EVO_NONE
+    need = lib.evoattn_bwd_workspace_bytes(ctypes.byref(p))
+    p.workspace_bytes = need
+    assert lib.evoattn_check(ctypes.byref(p), _lib.EVO_PASS_BWD) == 0
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD).split(b",")[0] in (b"mfma_dq_ring", b"mfma_dq")
+    B, S, N, H, D = shape
+    assert need >= B * H * S * N * 4 + B * H * N * N * 4           # delta, at least one dBias partial
+    p.dbias = None
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD) == b"mfma_bwd_fused"
+
+
 def test_error_strings(lib):
     assert _lib.strerror(0) == "ok"
     assert "workspace" in _lib.strerror(_lib.EVO_EWORKSPACE)
