@@ -234,7 +234,8 @@ static bool fused_ok(const EvoAttnParams &p) {
 }
 
 static bool dq_wide_ok(const EvoAttnParams &p) {
-    return dq_wide_grid_ok(p) && (!p.dbias || p.S == 1 || dq_split_ok(p));
+    // (without a bias that kernel has no form that writes dS)
+    return dq_wide_grid_ok(p) && (!p.dbias || (p.S == 1 && p.bias) || dq_split_ok(p));
 }
 // Rows of more than 2048 keys: the dQ kernels that keep the dBias sums of a wave's key tiles in
 // registers have no form that long (16 tiles per wave would be the whole register file).  The

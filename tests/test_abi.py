@@ -167,6 +167,20 @@ def test_dbias_without_a_bias_comes_with_dq(lib, shape):
     assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD) == b"mfma_bwd_fused"
 
 
+@pytest.mark.parametrize("D", [8, 16, 32, 64, 128])
+def test_dbias_of_one_row_without_a_bias(lib, D):
+    """One S row: the dQ kernel that writes dBias as it goes does so beside a bias; without one the partial sums are kept."""
+    p = good(4, 1, 512, 8, D)
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD).startswith(b"mfma_dq_wide")
+    with_bias = lib.evoattn_bwd_workspace_bytes(ctypes.byref(p))
+    p.bias, p.bias_dtype = None, _lib.EVO_NONE
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD).split(b",")[0] in (b"mfma_dq_ring", b"mfma_dq")
+    assert lib.evoattn_bwd_workspace_bytes(ctypes.byref(p)) >= with_bias + 4 * 8 * 512 * 512 * 4
+    p.N = 4096                                                             # (no such sums that long)
+    p.stride_b, p.stride_h, p.stride_s = 4096 * 8 * D, 4096 * D, 4096 * D
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD) == b"generic"
+
+
 def test_error_strings(lib):
     assert _lib.strerror(0) == "ok"
     assert "workspace" in _lib.strerror(_lib.EVO_EWORKSPACE)

@@ -14,6 +14,12 @@ CASES = [  # B, S, N, H, D, layout, dtype; with a bias dQ, dK and dV would come 
     (1, 256, 1030, 2, 32, "reference", torch.bfloat16),
     (1, 96, 384, 8, 8, "reference", torch.bfloat16),
     (2, 64, 600, 2, 8, "ds4sci", torch.float16),
+    (8, 1, 130, 4, 8, "reference", torch.bfloat16),          # one S row, where dBias is dS itself
+    (4, 1, 300, 8, 16, "ds4sci", torch.float16),
+    (2, 1, 512, 8, 32, "reference", torch.bfloat16),
+    (4, 1, 257, 8, 64, "ds4sci", torch.bfloat16),
+    (2, 1, 512, 4, 128, "reference", torch.float16),
+    (1, 1, 2100, 2, 32, "reference", torch.bfloat16),
 ]
 
 
@@ -44,7 +50,7 @@ def test_dbias_without_a_bias(gpu_device, case):
     ws = torch.empty(lib.evoattn_bwd_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8, device=q.device)
     p.prep, p.prep_bytes, p.workspace, p.workspace_bytes = prep.data_ptr(), prep.numel(), ws.data_ptr(), ws.numel()
     names = lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD)
-    assert b"fused" not in names and b"mfma_dbias" not in names, names
+    assert all(x not in names for x in (b"fused", b"mfma_dbias", b"mfma_dq_wide")), names
     assert lib.evoattn_fwd(ctypes.byref(p), st) == 0
     assert lib.evoattn_bwd(ctypes.byref(p), st) == 0
     # P, dS, the scaled Q, O (in delta) and the results are each rounded by at most 2^-9 of their size, and the errors of the probabilities that
