@@ -377,8 +377,12 @@ static WsLayout ws_layout(const EvoAttnParams &p) {
     if (p.dbias && !dq_writes_dbias(p)) off += align_up((size_t)w.n_chunks * p.B * p.H * p.N * p.N * 4);
     w.dout_ungated = off;
     if (p.gate && !(p.flags & EVO_FLAG_GATE_DOUT_INPLACE)) off += align_up((size_t)q_span(p) * (size_t)elem_size(p.dtype));
-    w.dq_part = off;
-    if (fused_ok(p) && p.N > (p.D == 8 ? mfma_fused8_tiles(p.N) : mfma_fused_tiles(p.N)) * 64) off += align_up((size_t)(p.D == 8 ? kFusedWgs8 : kFusedWgs) * p.N * p.D * 4);
+    // dQ of the blocks of keys before, in the place of the dBias partials: those are written when dQ is done (and there is no gate)
+    w.dq_part = w.dbias_part;
+    if (fused_ok(p) && mfma_fused_blocks(p) > 1) {
+        const size_t end = w.dq_part + align_up((size_t)mfma_fused_wgs(p) * p.N * p.D * 4);
+        if (end > off) off = end;
+    }
     w.total = off;
     return w;
 }

@@ -37,8 +37,7 @@ inline bool mfma_dqr_gate_ok(int D, int N) { return D == 32 && N <= 256; }
 int mfma_dqr_qrows(int D, int N);  // query rows per workgroup of the double-buffered dQ kernel (64 or 32), 0 where it is not built for such rows
 int launch_mfma_dkdv(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_dqw(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // dQ where no dBias is asked for
-// dQ, dK and dV at once (head dims 32, 8): workgroups where several share the problems among them (a scratch for dQ each), key tiles of 16 per wave
-constexpr int kFusedWgs = 512, kFusedWgs8 = 768;   // head dims 32, 8
+// dQ, dK and dV at once (head dims 32, 8): key tiles of 16 per wave
 inline int mfma_fused_tiles(int N) {
     if (N <= 128) return 2;
     const int blocks = (N + 255) / 256;   // fewest blocks of at most 256 keys, as narrow as they can be
@@ -48,6 +47,16 @@ inline int mfma_fused8_tiles(int N) {
     if (N <= 128) return 2;
     const int blocks = (N + 383) / 384;   // (of at most 384 keys)
     return (N + blocks * 64 - 1) / (blocks * 64);
+}
+inline int mfma_fused_blocks(const EvoAttnParams &p) {   // blocks of keys, one after the other
+    const int keys = 64 * (p.D == 8 ? mfma_fused8_tiles(p.N) : mfma_fused_tiles(p.N));
+    return (p.N + keys - 1) / keys;
+}
+// Workgroups.  With several blocks each has a scratch of a problem's dQ (N x D fp32) in the workspace and at most as many as are resident at a time,
+// two on each CU, share the problems.
+inline int64_t mfma_fused_wgs(const EvoAttnParams &p) {
+    const int64_t problems = (int64_t)p.B * p.H * p.S;
+    return mfma_fused_blocks(p) > 1 && problems > 512 ? 512 : problems;
 }
 int launch_stream_fwd8(const EvoAttnParams &p, const Extra &e, hipStream_t st);  // forward with a bias, head dim 8: two S rows per workgroup
 int launch_mfma_fused8(const EvoAttnParams &p, const Extra &e, hipStream_t st);

@@ -312,13 +312,11 @@ __global__ void __launch_bounds__(256, KT == 2 ? 3 : 2) bwd_fused8(EvoAttnParams
 template <typename T, int KT>
 static int fused8_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     typedef Fused8<KT> R;
-    const int64_t problems = (int64_t)p.B * p.H * p.S;
-    const int nb = (p.N + R::KB - 1) / R::KB;
-    const int wgs = KT == 2 ? kFusedWgs8 : kFusedWgs;   // as many as are resident
-    const unsigned grid = (unsigned)(nb > 1 && problems > wgs ? wgs : problems);
+    const unsigned grid = (unsigned)mfma_fused_wgs(p), problems = (unsigned)((int64_t)p.B * p.H * p.S);
+    const int nb = mfma_fused_blocks(p);
     auto go = [&](auto kern, PerDevice &done) {
         if (const int rc = ensure_dynamic_lds((const void *)kern, R::BYTES, done, nullptr)) return rc;
-        kern<<<grid, 256, R::BYTES, st>>>(p, e, (unsigned)problems, nb);
+        kern<<<grid, 256, R::BYTES, st>>>(p, e, problems, nb);
         return hip_rc();
     };
     static PerDevice done[3]{};

@@ -181,6 +181,22 @@ def test_dbias_of_one_row_without_a_bias(lib, D):
     assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD) == b"generic"
 
 
+@pytest.mark.parametrize("shape,wgs", [((1, 384, 384, 4, 32), 512), ((1, 96, 2048, 4, 32), 384), ((1, 32, 1024, 8, 8), 256), ((1, 1024, 400, 8, 8), 512), ((1, 1024, 384, 8, 8), 0)])
+def test_dq_scratch_is_that_of_the_workgroups_that_run(lib, shape, wgs):
+    """Several blocks of keys: a problem's dQ in fp32 for every workgroup, of which at most 512 run; with dBias in the place of its partial sums."""
+    B, S, N, H, D = shape
+    up = lambda n: (n + 255) // 256 * 256
+    p = good(*shape)
+    with_dbias = lib.evoattn_bwd_workspace_bytes(ctypes.byref(p))
+    p.flags = _lib.EVO_FLAG_ONLY_DQ                                          # the dQ kernel of its own: no scratch
+    partials = lib.evoattn_bwd_workspace_bytes(ctypes.byref(p))
+    p.flags, p.dbias = 0, None
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD) == b"mfma_bwd_fused"
+    plain = up(B * H * S * N * 4) + up(B * S * 4)
+    assert lib.evoattn_bwd_workspace_bytes(ctypes.byref(p)) == plain + up(wgs * N * D * 4)
+    assert with_dbias <= max(partials, plain + up(wgs * N * D * 4), plain + up(4 * 512 * 128 * 128 * 4))   # (as many partials as four rounds of workgroups have blocks)
+
+
 def test_error_strings(lib):
     assert _lib.strerror(0) == "ok"
     assert "workspace" in _lib.strerror(_lib.EVO_EWORKSPACE)
