@@ -218,6 +218,21 @@ static bool dq_split_ok(const EvoAttnParams &p) {
 //   with dBias   N = 192, S = 128, 1024 48 / 53, 289 / 283 (left out); N = 300, S = 64, 65, 96, 256 56 / 56, 58 / 65, 74 / 73, 166 / 156; N = 384
 //                66 / 66, 69 / 79, 91 / 87, 206 / 185, S = 1024 774 / 706; N = 512, S = 64, 256 99 / 98, 329 / 321; from 513 keys on the pair of kernels for dQ
 //                stands against it: N = 768, S = 32, 65, 256 160 / 150, 279 / 251, 886 / 683; N = 1024, S = 32, 1024 212 / 199, 6352 / 4888
+//
+// Over sizes drawn at random (some 5000 backwards, heads times batches from 1 to 128) some calls were slower than with the other kernels, and are
+// left to them:
+//   Rows of several blocks (from 513 keys on, head dim 8 385 without dBias) are also padded to whole blocks, up to 1.3 times, and share 512 workgroups. `fused_share`
+//   is the part of the rounds' slots, a last half round at .62, that works on keys that exist.  Median and most of this way / otherwise where it is just
+//   below the lines here, and just above: head dim 32 without dBias 1.03, 1.22 and .93, 1.06 up to 768 keys, 1.01, 1.16 and .94, 1.07 up to 1024, 1.01, 1.07 and .90, 1.03
+//   beyond; with it .97, 1.06 and .96, .99; head dim 8 .96, 1.06 and .91, 1.04 up to 768 keys, 1.05, 1.17 and .91, 1.03 beyond.  (H = 8, S = 73, N = 784, head dim 32 246 / 298 us.)
+//   With dBias and up to 384 keys, where the other way is one kernel whose dBias comes with dQ, few S rows per head leave this one's second kernel with partial sums of a row or
+//   two each: up to 64 rows 1.06, 1.58 (B = 2, S = 24, N = 377, H = 16, D = 8 109 / 172), from 65 on .93, 1.06.  One head alone at head dim 8 1.05, 1.09;
+//   an fp32 bias of one or two heads at head dim 32 1.03, 1.05.
+static double fused_share(const EvoAttnParams &p) {
+    const int64_t problems = (int64_t)p.B * p.H * p.S, rest = problems % 512;
+    const double rounds = (double)(problems / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.62 : 1.0);
+    return (double)problems / 512.0 / rounds * p.N / (mfma_fused_blocks(p) * mfma_fused_keys(p));
+}
 static bool fused_ok(const EvoAttnParams &p) {
     constexpr int apart = EVO_FLAG_PER_PROBLEM | EVO_FLAG_ONLY_DQ | EVO_FLAG_ONLY_DKDV | EVO_FLAG_DEBUG_NO_KV_RING | EVO_FLAG_DEBUG_NO_DQ_WIDE |
                           EVO_FLAG_DEBUG_NO_DQ_SPLIT | EVO_FLAG_DEBUG_OTHER_WIDTH;
@@ -226,11 +241,19 @@ static bool fused_ok(const EvoAttnParams &p) {
     if (p.dbias && !p.bias) return false;   // (the dBias kernel keeps bias tiles; dBias without a bias, the sum of dS alone, comes with dQ)
     const int64_t problems = (int64_t)p.B * p.H * p.S;
     const double full = (double)problems / (double)((problems + 255) / 256 * 256);
-    if (p.D == 8) return problems >= 256 && (!p.dbias || (p.S >= 8 && (p.N > 512 || (p.N >= 288 && problems >= 768 && full >= 0.9))));
+    const double share = fused_share(p);
+    const int heads = p.B * p.H;
+    if (p.D == 8) {
+        if (problems < 256) return false;
+        if (p.N > (p.dbias ? 512 : 384)) return (!p.dbias || p.S >= 8) && share >= (p.N > 768 ? 0.54 : 0.48);
+        if (!p.dbias) return true;
+        return p.N >= 288 && problems >= 768 && full >= 0.9 && (p.N > 384 ? p.S >= 8 : p.S > 64 && heads > 1);
+    }
     if (problems < 384) return false;
-    if (!p.dbias) return full >= 0.7;
+    if (!p.dbias) return p.N <= 512 ? full >= 0.7 : share >= (p.N <= 768 ? 0.66 : p.N <= 1024 ? 0.7 : 0.75);
     if (p.S < 8 || p.N <= 320) return false;
-    return p.N <= 384 ? problems >= 1024 && full >= 0.95 : full >= (p.N > 768 ? 0.75 : 0.85);
+    if (p.N <= 384) return problems >= 1024 && full >= 0.95 && p.S > 64 && (p.bias_dtype == p.dtype || heads > 2);
+    return full >= (p.N > 768 ? 0.75 : 0.85) && share >= 0.58;
 }
 
 static bool dq_wide_ok(const EvoAttnParams &p) {

@@ -48,10 +48,8 @@ inline int mfma_fused8_tiles(int N) {
     const int blocks = (N + 383) / 384;   // (of at most 384 keys)
     return (N + blocks * 64 - 1) / (blocks * 64);
 }
-inline int mfma_fused_blocks(const EvoAttnParams &p) {   // blocks of keys, one after the other
-    const int keys = 64 * (p.D == 8 ? mfma_fused8_tiles(p.N) : mfma_fused_tiles(p.N));
-    return (p.N + keys - 1) / keys;
-}
+inline int mfma_fused_keys(const EvoAttnParams &p) { return 64 * (p.D == 8 ? mfma_fused8_tiles(p.N) : mfma_fused_tiles(p.N)); }   // of a block
+inline int mfma_fused_blocks(const EvoAttnParams &p) { return (p.N + mfma_fused_keys(p) - 1) / mfma_fused_keys(p); }   // one after the other
 // Workgroups.  With several blocks each has a scratch of a problem's dQ (N x D fp32) in the workspace and at most as many as are resident at a time,
 // two on each CU, share the problems.
 inline int64_t mfma_fused_wgs(const EvoAttnParams &p) {

@@ -365,3 +365,23 @@ def test_layernorm_entry_points_validate_on_the_host(lib):
     assert lib.evoattn_colsum(a, 12, a, a, 1 << 30, 4, 12, _lib.EVO_BF16, None) == _lib.EVO_EALIGN
     assert lib.evoattn_colsum(a, 32, a, a, 1 << 30, 4, 64, _lib.EVO_BF16, None) == _lib.EVO_EINVAL       # rows overlap
     assert lib.evoattn_colsum(a, 68, a, a, 1 << 30, 4, 64, _lib.EVO_BF16, None) == _lib.EVO_EALIGN
+
+
+@pytest.mark.parametrize("shape,dbias,fused", [
+    ((1, 73, 784, 8, 32), False, False), ((1, 96, 784, 8, 32), False, True),     # 784 keys are four blocks of 256, 584 problems a round and a bit
+    ((1, 68, 602, 8, 32), False, False), ((1, 64, 602, 8, 32), False, True),
+    ((2, 35, 1182, 8, 32), False, False), ((1, 64, 2048, 8, 32), False, True),
+    ((1, 145, 824, 4, 32), True, False), ((1, 192, 824, 4, 32), True, True),
+    ((4, 8, 384, 32, 32), True, False), ((1, 128, 384, 8, 32), True, True),      # partial sums of few S rows
+    ((2, 24, 377, 16, 8), True, False), ((1, 96, 377, 8, 8), True, True),
+    ((1, 958, 336, 1, 8), True, False), ((1, 480, 336, 2, 8), True, True),       # one head alone
+    ((2, 18, 824, 8, 8), False, False), ((2, 16, 824, 8, 8), False, True),
+    ((1, 137, 864, 2, 8), True, False), ((1, 256, 864, 2, 8), True, True),
+])
+def test_backward_of_padded_rows_and_few_rows(lib, shape, dbias, fused):
+    """The kernel of dQ, dK and dV leaves calls alone whose keys, padded to whole blocks, or problems fill its rounds badly, and dBias of few S rows per head."""
+    p = good(*shape)
+    p.bias_dtype = p.dtype
+    if not dbias:
+        p.dbias = None
+    assert (b"mfma_bwd_fused" in lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD)) == fused
