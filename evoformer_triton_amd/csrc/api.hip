@@ -519,7 +519,7 @@ static bool ring_pays(const EvoAttnParams &p, double start, double per_row) {
 // 128 17.0 / 19.2, 34.0 / 34.5, 41.9 / 39.3; N = 768, S = 16, 32 30.1 / 33.5, 44.7 / 42.3).
 static bool fwd_pairs8_ok(const EvoAttnParams &p) {
     if (p.D != 8 || !p.bias || p.gate || p.S < 2 || p.N <= 32 || bias_direct(p) || (p.flags & (EVO_FLAG_PER_PROBLEM | EVO_FLAG_DEBUG_FWD_BIAS_TILES))) return false;
-    const int64_t pairs = (int64_t)((p.N + 127) / 128) * p.B * p.H * ((p.S + 1) / 2);
+    const int64_t pairs = mfma_fwd_pairs(p);
     if (p.N > 128 && p.N <= 256) return p.bias_dtype == p.dtype && pairs >= 64;
     return pairs >= (p.N >= 512 ? 768 : 1536);
 }
@@ -568,11 +568,15 @@ const char *evoattn_kernels(const EvoAttnParams *p, int pass) {
     if (!p) return "invalid";
     if (f32_ok(*p, pass)) return pass == EVO_PASS_FWD ? "f32_fwd" : p->dbias ? "f32_dq+f32_dbias,f32_dkdv" : "f32_dq,f32_dkdv";
     if (!mfma_ok(*p, pass)) return "generic";
-    if (pass == EVO_PASS_FWD) return split_fwd_ok(*p) ? "split_fwd" : fwd_ring_ok(*p) ? "mfma_fwd_ring" : "mfma_fwd";
+    if (pass == EVO_PASS_FWD) {
+        if (split_fwd_ok(*p)) return "split_fwd";
+        if (fwd_ring_ok(*p)) return "mfma_fwd_ring";
+        return fwd_pairs8_ok(*p) || mfma_fwd_pair_ok(*p, bias_direct(*p)) ? "mfma_fwd_pair" : "mfma_fwd";
+    }
     if (fused_ok(*p)) return p->dbias ? "mfma_bwd_fused+mfma_dbias" : "mfma_bwd_fused";
     const bool kvr = kv_ring_ok(*p);
     if (dq_split_ok(*p)) return kvr ? "mfma_dq_wide+mfma_dbias,mfma_dkdv_ring" : "mfma_dq_wide+mfma_dbias,mfma_dkdv";
-    // (one launch of both where bwd_one_ok says so)
+    if (bwd_one_ok(*p)) return "mfma_dq_wide,mfma_dkdv(one launch)";
     if (dq_wide_ok(*p)) return kvr ? "mfma_dq_wide,mfma_dkdv_ring" : "mfma_dq_wide,mfma_dkdv";
     if (kvr) return dq_ring_ok(*p) ? "mfma_dq_ring,mfma_dkdv_ring" : "mfma_dq,mfma_dkdv_ring";
     return dq_ring_ok(*p) ? "mfma_dq_ring,mfma_dkdv" : "mfma_dq,mfma_dkdv";

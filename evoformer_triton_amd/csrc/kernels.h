@@ -25,6 +25,14 @@ int launch_split_fwd(const EvoAttnParams &p, hipStream_t st);  // the keys of a 
 inline bool mfma_fwdr_reads_rows(const EvoAttnParams &p) {
     return p.bias_dtype == p.dtype && !(p.D == 8 && !p.gate) && !(p.flags & EVO_FLAG_DEBUG_FWD_BIAS_TILES);
 }
+// Workgroups of the forwards that take two S rows (stream_fwd_pair, stream_fwd8), and whether launch_mfma_fwd takes that of head dim 32: two
+// rounds of the three workgroups that a CU holds, or the last one is too empty for a workgroup that takes twice as long (stream_fwd / pairs, us, H = 8: N = 384,
+// S = 48, 64, 96, 128 26.7 / 27.8, 30.3 / 29.6, 40.4 / 41.2, 50.4 / 47.2; N = 300, S = 96, 128 34.5 / 35.5, 42.3 / 39.9); up to 192 keys what a
+// workgroup costs beside its tiles decides (N = 128, S = 200 20.4 / 22.8; N = 192 32.9 / 33.9; N = 224 39.8 / 37.2).
+inline int64_t mfma_fwd_pairs(const EvoAttnParams &p) { return (int64_t)((p.N + 127) / 128) * p.B * p.H * ((p.S + 1) / 2); }
+inline bool mfma_fwd_pair_ok(const EvoAttnParams &p, bool bias_direct) {
+    return p.D == 32 && p.N > 192 && mfma_fwd_pairs(p) >= 2 * 768 && p.bias_dtype != EVO_NONE && !bias_direct && !p.gate && !(p.flags & EVO_FLAG_PER_PROBLEM);
+}
 int launch_mfma_fwdr(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int mfma_fwdr_max_n(int D);  // largest N the chunk-of-rows forward takes, 0 for a head dim it is not built for
 int launch_mfma_dq(const EvoAttnParams &p, const Extra &e, hipStream_t st);

@@ -1283,15 +1283,6 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
 
 // ------------------------------------------------------------------ launchers
 
-#if EVO_D == 32
-// Two rounds of the three workgroups that a CU holds, or the last one is too empty for a workgroup that takes twice as long (stream_fwd / pairs, us, H = 8: N = 384,
-// S = 48, 64, 96, 128 26.7 / 27.8, 30.3 / 29.6, 40.4 / 41.2, 50.4 / 47.2; N = 300, S = 96, 128 34.5 / 35.5, 42.3 / 39.9); up to 192 keys what a
-// workgroup costs beside its tiles decides (N = 128, S = 200 20.4 / 22.8; N = 192 32.9 / 33.9; N = 224 39.8 / 37.2).
-static bool fwd_pair_ok(const EvoAttnParams &p, const Extra &e, int64_t pairs) {
-    return p.N > 192 && pairs >= 2 * 768 && p.bias_dtype != EVO_NONE && !e.bias_direct && !p.gate && !(p.flags & EVO_FLAG_PER_PROBLEM);
-}
-#endif
-
 // the caller's bias rows start or end within a group of four (fp32, head dim 64: bias_ragged in api.hip)
 static bool ragged_rows(const EvoAttnParams &p, const Extra &e) { return p.N % 4 != 0 || !e.vec_ok; }
 
@@ -1299,10 +1290,10 @@ template <typename T, int D>
 static int fwd_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const unsigned grid = (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H * p.S);
 #if EVO_D == 32
-    const int64_t pairs = (int64_t)((p.N + 127) / 128) * p.B * p.H * ((p.S + 1) / 2);
-    if (fwd_pair_ok(p, e, pairs)) {
-        if (e.bq16) stream_fwd_pair<T, 2><<<(unsigned)pairs, 256, 0, st>>>(p, e);
-        else stream_fwd_pair<T, 1><<<(unsigned)pairs, 256, 0, st>>>(p, e);
+    if (mfma_fwd_pair_ok(p, e.bias_direct)) {
+        const unsigned pairs = (unsigned)mfma_fwd_pairs(p);
+        if (e.bq16) stream_fwd_pair<T, 2><<<pairs, 256, 0, st>>>(p, e);
+        else stream_fwd_pair<T, 1><<<pairs, 256, 0, st>>>(p, e);
         return hip_rc();
     }
 #endif

@@ -212,7 +212,9 @@ const char *evoattn_path(const EvoAttnParams *p, int pass);
 /* Names of the main kernels that pass would launch, comma separated (e.g. "mfma_fwd_ring",
  * "mfma_dq_ring,mfma_dkdv", "mfma_dq_wide,mfma_dkdv", "f32_dq+f32_dbias,f32_dkdv", "generic"); for reports and profiles.
  * One name stands for a place in the routes, whichever head dim: from 32 on mfma_fwd is the kernel stream_fwd in a profile,
- * mfma_dq_wide stream_dq and the four-wave mfma_dkdv stream_dkdv, and mfma_dbias stream_dbias. */
+ * mfma_dq_wide stream_dq and the four-wave mfma_dkdv stream_dkdv; mfma_dbias is stream_dbias (head dim 8: stream_dbias8, 16:
+ * mfma_dbias); mfma_fwd_pair, the forward that takes two S rows, stream_fwd_pair (head dim 8: stream_fwd8); mfma_bwd_fused bwd_fused
+ * (head dim 8: bwd_fused8); "mfma_dq_wide,mfma_dkdv(one launch)" is stream_bwd_one.  The names depend on the flags. */
 const char *evoattn_kernels(const EvoAttnParams *p, int pass);
 
 /* ---- LayerNorm of the block around the attention -------------------------------------------

@@ -385,3 +385,17 @@ def test_backward_of_padded_rows_and_few_rows(lib, shape, dbias, fused):
     if not dbias:
         p.dbias = None
     assert (b"mfma_bwd_fused" in lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD)) == fused
+
+
+@pytest.mark.parametrize("shape,bias,fwd,bwd", [
+    ((1, 384, 384, 4, 32), "q", b"mfma_fwd_pair", b"mfma_bwd_fused+mfma_dbias"), ((1, 100, 384, 4, 32), "q", b"mfma_fwd", b"mfma_dq_ring,mfma_dkdv"),
+    ((1, 1024, 384, 8, 8), "q", b"mfma_fwd_pair", b"mfma_bwd_fused+mfma_dbias"), ((1, 64, 200, 4, 8), "f32", b"mfma_fwd_ring", b"mfma_dq_ring,mfma_dkdv"),
+    ((4, 1, 1024, 32, 64), "f32", b"mfma_fwd", b"mfma_dq_wide,mfma_dkdv(one launch)"), ((4, 1, 1023, 16, 64), "f32", b"mfma_fwd", b"mfma_dq_wide,mfma_dkdv"),
+])
+def test_kernel_names_tell_the_forms_apart(lib, shape, bias, fwd, bwd):
+    p = good(*shape)
+    p.bias_dtype = p.dtype if bias == "q" else _lib.EVO_F32
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == fwd
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD) == bwd
+    p.flags = _lib.EVO_FLAG_PER_PROBLEM
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == b"mfma_fwd"

@@ -55,8 +55,8 @@ def test_forward_pairs_match_eager(gpu_device, case):
         p.flags |= flags
         prep = torch.empty(lib.evoattn_prep_bytes(ctypes.byref(p)), dtype=torch.uint8, device=q.device)
         p.prep, p.prep_bytes = prep.data_ptr(), prep.numel()
-        if name == "pairs":
-            assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == b"mfma_fwd"
+        kernel = lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD)
+        assert (kernel == b"mfma_fwd_pair") == (name == "pairs"), kernel
         assert lib.evoattn_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
         got[name] = (o.float(), lse)
     # the scaled Q, the probabilities and O are each rounded by at most 2^-9 of their size, and the scores' error that comes of the first moves the

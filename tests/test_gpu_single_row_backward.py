@@ -1,5 +1,7 @@
 """The backward of one S row at head dim 64, dQ with dBias and dK/dV in one launch (csrc/mfma_stream.hip), at the edges of its blocks of 128 queries and
 keys, stages of 64 rows and tiles of 32, against eager in fp32."""
+import ctypes
+
 import pytest
 import torch
 
@@ -31,6 +33,7 @@ CASES = [  # B, N, H, mask, bias, layout, dtype
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
 def test_single_row_backward_matches_eager(gpu_device, case):
     import evoformer_triton_amd.evoformer as E
+    from evoformer_triton_amd import _lib
     B, N, H, mask, bias, layout, dt = case
     g = torch.Generator().manual_seed(31)
     Q, K, V, dO = ((torch.randn((B, 1, N, H, 64), generator=g) * 0.7).to(dt) for _ in range(4))
@@ -44,6 +47,12 @@ def test_single_row_backward_matches_eager(gpu_device, case):
     ref = eager.attention_fwd_bwd(*xs, layout=layout, compute_dtype=torch.float32, s_chunk=16)
     q, k, v = (t.detach().clone().requires_grad_() for t in xs[:3])
     bb = xs[4].detach().clone().requires_grad_()
+    mz, mk, mstr = E._prep_mask(xs[3], B, 1, N, q.device)
+    bz, bdt, bstr = E._prep_bias(xs[4], B, H, N, dt, q.device)
+    p = E._params(q, k, v, mz, mk, mstr, bz, bdt, bstr, q, bz, layout)
+    p.dout = p.dq = p.dk = p.dv = p.dbias = p.q
+    kernels = _lib.load().evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD)
+    assert kernels == b"mfma_dq_wide,mfma_dkdv" + (b"" if (B, N, H) == (4, 1023, 16) else b"(one launch)"), kernels   # (that one: a full round of each kernel)
     o = E.evoformer_attention(q, k, v, xs[3], bb, layout=layout)
     o.backward(xs[5])
     # P, dS, the scaled Q, O (in delta) and the results are each rounded by at most 2^-9 of their size, and the errors of the probabilities that
