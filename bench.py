@@ -49,6 +49,25 @@ def measured_traffic(config, kernel):
         return None, None
 
 
+def backward_phases(lib, p):
+    """[(phase, flags beside PREP_VALID, kernels)] of the backward that `p` describes: its dQ and dK/dV kernels one at a time, or, where the call
+    does not launch these two (asked for alone it would be other kernels), the whole backward."""
+    from evoformer_triton_amd import _lib
+
+    def kernels(flags):
+        p.flags = flags
+        return lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD).decode()
+
+    whole, alone = kernels(0), kernels(_lib.EVO_FLAG_ONLY_DQ)
+    same = whole == alone == kernels(_lib.EVO_FLAG_ONLY_DKDV)
+    p.flags = 0
+    if not same:
+        return [("bwd", 0, whole)]
+    names = whole.split(",")
+    k_dq, k_dkdv = (names[0] + " (dQ)", names[0] + " (dK/dV)") if len(names) == 1 else names
+    return [("bwd_dq", _lib.EVO_FLAG_ONLY_DQ, k_dq), ("bwd_dkdv", _lib.EVO_FLAG_ONLY_DKDV, k_dkdv)]
+
+
 def parse():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -422,15 +441,14 @@ def main():
         assert rc == 0, _lib.strerror(rc)
 
     V = _lib.EVO_FLAG_PREP_VALID
-    phases = {
-        "fwd": (lambda: call(lib.evoattn_fwd, 0), f_fwd),
-        "bwd_dq": (lambda: call(lib.evoattn_bwd, V | _lib.EVO_FLAG_ONLY_DQ), f_bwd / 2),
-        "bwd_dkdv": (lambda: call(lib.evoattn_bwd, V | _lib.EVO_FLAG_ONLY_DKDV), f_bwd / 2),
-    }
+    bwd = backward_phases(lib, p)
+    phases = {"fwd": (lambda: call(lib.evoattn_fwd, 0), f_fwd)}
+    for name, flags, _ in bwd:
+        phases[name] = (lambda flags=flags: call(lib.evoattn_bwd, V | flags), f_bwd / len(bwd))
     call(lib.evoattn_fwd, 0)
     call(lib.evoattn_bwd, V)
     n_k = max(10, args.steps)
-    # The three phases in the order of a step (forward, dQ, dK/dV), an event between every two
+    # The phases in the order of a step (forward, dQ, dK/dV or the whole backward), an event between every two
     # calls on the stream they are launched on: a kernel is timed in the state the one before
     # it leaves the chip in, not back to back with itself (the kernels that run one workgroup
     # per CU measure 8-15 % faster that way).
@@ -452,9 +470,7 @@ def main():
     achieved = phases[dom][1] / t_phase[dom] / 1e12
     p.flags = 0
     k_fwd = lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD).decode()
-    k_bwd = lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD).decode().split(",")
-    k_dq, k_dkdv = (k_bwd[0] + " (dQ)", k_bwd[0] + " (dK/dV)") if len(k_bwd) == 1 else k_bwd
-    kernel_names = {"fwd": "prep_kernel+" + k_fwd, "bwd_dq": k_dq, "bwd_dkdv": k_dkdv}
+    kernel_names = {"fwd": "prep_kernel+" + k_fwd, **{name: kernels for name, _, kernels in bwd}}
     if args.copy_calibration:
         src = torch.empty(256 << 20, dtype=torch.uint8, device=dev)
         dst = torch.empty_like(src)
@@ -469,7 +485,8 @@ def main():
     t_b, l_b = qc.numel() * esz, lse.numel() * 4
     phase_bytes = {"fwd": 4 * t_b + l_b + b_b,                  # Q,K,V -> O, LSE
                    "bwd_dq": 6 * t_b + 2 * l_b + 2 * b_b,       # Q,K,V,dO,O,LSE -> dQ, delta, dBias
-                   "bwd_dkdv": 6 * t_b + 2 * l_b + b_b}         # Q,K,V,dO,LSE,delta -> dK,dV
+                   "bwd_dkdv": 6 * t_b + 2 * l_b + b_b,         # Q,K,V,dO,LSE,delta -> dK,dV
+                   "bwd": 8 * t_b + l_b + 2 * b_b}              # Q,K,V,dO,O,LSE -> dQ,dK,dV,dBias
     hbm_gbs = phase_bytes[dom] / t_phase[dom] / 1e9
     traffic, traffic_commit = measured_traffic(args.config, kernel_names[dom].split(" ")[0]) if bias is not None else (None, None)
     out = {
@@ -496,8 +513,8 @@ def main():
         "c_abi_tflops": f_full / t_abi / 1e12,
         "kernel_ms": {kernel_names[n]: t * 1e3 for n, t in t_phase.items()},
         "peak_mem_bytes_beyond_inputs": int(peak_extra),
-        "kernel_ms_note": "each phase is timed between two HIP events inside a step (forward, dQ, dK/dV in that order), so the "
-                          "three figures include the gaps between the launches and can sum to more than ms_per_step, which is "
+        "kernel_ms_note": "each phase is timed between two HIP events inside a step (forward, then dQ and dK/dV or the backward as a whole), so the "
+                          "figures include the gaps between the launches and can sum to more than ms_per_step, which is "
                           "wall time over back-to-back steps",
         "roofline": {"bound": "mfma", "kernel": kernel_names[dom], "achieved": achieved, "peak": MFMA_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": achieved / MFMA_PEAK_TFLOPS,

@@ -399,3 +399,20 @@ def test_kernel_names_tell_the_forms_apart(lib, shape, bias, fwd, bwd):
     assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD) == bwd
     p.flags = _lib.EVO_FLAG_PER_PROBLEM
     assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == b"mfma_fwd"
+
+
+@pytest.mark.parametrize("shape,phases", [((1, 512, 256, 8, 32), 2), ((1, 384, 384, 4, 32), 1), ((1, 768, 768, 4, 32), 1), ((1, 1024, 384, 8, 8), 1),
+                                          ((1, 200, 640, 5, 64), 2), ((4, 1, 1024, 32, 64), 1), ((1, 64, 512, 4, 128), 2)])
+def test_the_benchmark_names_the_kernels_that_it_times(lib, shape, phases):
+    """A phase's time is that of the kernels that the call with its flags launches, and the step launches the same ones."""
+    import bench
+    p = good(*shape)
+    if shape[1] == 1:
+        p.bias_dtype = _lib.EVO_F32
+    got = bench.backward_phases(lib, p)
+    assert p.flags == 0 and len(got) == phases
+    for _, flags, kernels in got:
+        p.flags = flags
+        assert kernels in lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD).decode()
+    p.flags = 0
+    assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD).decode() == ",".join(kernels for _, _, kernels in got)
