@@ -517,11 +517,17 @@ static bool ring_pays(const EvoAttnParams &p, double start, double per_row) {
 // 16.1 / 15.0, 125 / 116; with an fp32 bias N = 192, S = 128 20.4 / 24.6: left to it); of the one-workgroup-per-problem forward where the
 // pairs fill two rounds of the three workgroups that a CU holds, for long rows one (H = 8: N = 96, S = 200, 400 15.3 / 14.8, 23.9 / 21.1; N = 384, S = 32, 96,
 // 128 17.0 / 19.2, 34.0 / 34.5, 41.9 / 39.3; N = 768, S = 16, 32 30.1 / 33.5, 44.7 / 42.3).
+// Left out again after some 2900 forwards of sizes drawn at random (this / that, median and most): an fp32 bias up to 64 keys .96, 1.16 (S = 197, N = 64, 16 heads times batches
+// 18.7 / 21.6), and from 97 to 128 of more than 8 heads times batches .96, 1.14; rows of 512 keys and more that overflow one round by little with the bias in the dtype of q
+// 1.01, 1.10 (800 pairs: S = 9, B = 2, N = 576, H = 16 45.1 / 49.6), and of three S rows, whose second pair is half empty, 1.05, 1.07.
 static bool fwd_pairs8_ok(const EvoAttnParams &p) {
     if (p.D != 8 || !p.bias || p.gate || p.S < 2 || p.N <= 32 || bias_direct(p) || (p.flags & (EVO_FLAG_PER_PROBLEM | EVO_FLAG_DEBUG_FWD_BIAS_TILES))) return false;
     const int64_t pairs = mfma_fwd_pairs(p);
-    if (p.N > 128 && p.N <= 256) return p.bias_dtype == p.dtype && pairs >= 64;
-    return pairs >= (p.N >= 512 ? 768 : 1536);
+    const bool own = p.bias_dtype == p.dtype;
+    if (p.N > 128 && p.N <= 256) return own && pairs >= 64;
+    if (p.N >= 512) return p.S != 3 && pairs >= (own ? 900 : 768);
+    if (!own && (p.N <= 64 || (p.N > 96 && p.N <= 128 && (int64_t)p.B * p.H > 8))) return false;
+    return pairs >= 1536;
 }
 
 // rows of 129..256 keys: a workgroup per chunk of S rows with the head's bias resident

@@ -416,3 +416,16 @@ def test_the_benchmark_names_the_kernels_that_it_times(lib, shape, phases):
         assert kernels in lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD).decode()
     p.flags = 0
     assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD).decode() == ",".join(kernels for _, _, kernels in got)
+
+
+@pytest.mark.parametrize("shape,bias,pairs", [
+    ((1, 197, 64, 16, 8), "f32", False), ((1, 197, 64, 16, 8), "q", True), ((1, 197, 65, 16, 8), "f32", True),
+    ((1, 323, 128, 16, 8), "f32", False), ((1, 323, 96, 16, 8), "f32", True), ((1, 400, 128, 8, 8), "f32", True),
+    ((2, 9, 576, 16, 8), "q", False), ((2, 9, 576, 16, 8), "f32", True), ((2, 12, 576, 16, 8), "q", True),
+    ((4, 3, 823, 16, 8), "q", False), ((4, 5, 823, 16, 8), "q", True),
+])
+def test_forward_of_two_rows_where_it_pays(lib, shape, bias, pairs):
+    p = good(*shape)
+    p.bias_dtype = p.dtype if bias == "q" else _lib.EVO_F32
+    p.flags = _lib.EVO_FLAG_DEBUG_BIAS_TILES if shape[1] <= 4 else 0
+    assert (lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == b"mfma_fwd_pair") == pairs

@@ -19,9 +19,11 @@ CASES = [  # B, S, N, H, D, mask, bias, layout, dtype
     (1, 17, 130, 4, 8, "dead", "q", "reference", torch.bfloat16),      # a last pair of one row; a second stage and block of two
     (2, 16, 256, 2, 8, "dead_added", "q", "ds4sci", torch.float16),
     (1, 21, 193, 4, 8, "jump", "q", "reference", torch.float16),
-    (3, 257, 33, 4, 8, "dead", "f32", "reference", torch.bfloat16),    # two tiles, the second of one key
+    (3, 257, 33, 4, 8, "dead", "q", "reference", torch.bfloat16),      # two tiles, the second of one key
+    (1, 401, 65, 8, 8, "jump", "f32", "reference", torch.bfloat16),    # three
+    (2, 401, 97, 4, 8, "dead_added", "f32", "ds4sci", torch.float16),  # four, one stage
     (1, 257, 300, 4, 8, "bool", "f32", "ds4sci", torch.bfloat16),
-    (1, 129, 513, 3, 8, None, "q", "reference", torch.bfloat16),       # a last stage of one key
+    (1, 145, 513, 3, 8, None, "q", "reference", torch.bfloat16),       # a last stage of one key
 ]
 
 
