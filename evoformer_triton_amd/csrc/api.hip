@@ -129,7 +129,8 @@ static int bias_vec_ok(const EvoAttnParams &p) {
 // One S row of an fp32 bias whose rows start or end within a group of four (any length that is no multiple of 4): the kernels for head
 // dim 64 read these in place too, and the tiles, which nobody then needs, are most of such a call.  Forward and backward, us, H = 32, tiles / in place: B = 1, N = 251
 // 55 / 36, 517 101 / 78, 1023 284 / 158; B = 2, N = 771 357 / 216; B = 4, N = 517 362 / 211, 1023 1116 / 633 (N = 1024: 525).
-// Fewer than 32 workgroups keep the tiles: their backward is another kernel's.
+// Fewer than 32 workgroups keep the tiles: their backward is another kernel's.  (The forward, which decides, does not know whether dBias will be wanted: without it, and with a
+// gate, such a backward is one launch as well, see bwd_one_ok.)
 static bool bias_ragged(const EvoAttnParams &p) {
     if (!p.bias || p.S != 1 || p.D != 64 || p.bias_dtype != EVO_F32 || p.dtype == EVO_F32 || (p.flags & EVO_FLAG_DEBUG_BIAS_TILES)) return false;
     if ((p.N % 4 == 0 && bias_vec_ok(p)) || p.N < 4 || (int64_t)p.N * p.bias_stride_row >= ((int64_t)1 << 31)) return false;
@@ -271,11 +272,15 @@ static bool dq_writes_dbias(const EvoAttnParams &p) { return p.dbias && p.S == 1
 // at a time: where each kernel has just one full round of them nothing is left to fill, and two kinds of different length end less
 // evenly.  H = 32, fp32 bias, forward and backward, us, two launches / one: B = 4, N = 384 (384 workgroups of each) 95 / 90, B = 2, N = 768 (384) 175 / 169,
 // 896 (448) 224 / 221, 1024 (512) 292 / 297, B = 4, N = 512 (512) 133 / 138, 640 (640) 270 / 242, 768 347 / 324, 896 473 / 424, 1024 (1024) 582 / 525.
+// Rows that start or end within a group of four are one launch also without dBias and with a gate.  Forward and backward over some 2700 random sizes against the
+// prepared tiles that such rows had before, median and most: two launches 32 workgroups 1.19, 1.29, 64 1.06, 1.22 (with a gate 1.11, 1.25 and 1.06,
+// 1.18), one launch .84, .96 and .82, .92 (.89, .98 and .89, .96); B = 1, N = 129, H = 16 without dBias 28.0 (tiles) / 36.0 (two) / 25 us.
 static bool bwd_one_ok(const EvoAttnParams &p) {
     constexpr int apart = EVO_FLAG_PER_PROBLEM | EVO_FLAG_ONLY_DQ | EVO_FLAG_ONLY_DKDV | EVO_FLAG_DEBUG_NO_DQ_WIDE;
     const int64_t wgs = (int64_t)((p.N + 127) / 128) * p.B * p.H;
     if (wgs > 448 && wgs <= 512) return false;
-    return p.D == 64 && p.S == 1 && !(p.flags & apart) && !p.gate && !p.dmask && bias_direct(p) && dq_writes_dbias(p);
+    if (p.D != 64 || p.S != 1 || (p.flags & apart) || p.dmask || !bias_direct(p)) return false;
+    return bias_ragged(p) ? dq_wide_ok(p) : !p.gate && dq_writes_dbias(p);
 }
 
 // S is split into chunks; one workgroup of the dQ kernel sums dS over one chunk and
@@ -700,7 +705,7 @@ int evoattn_bwd(const EvoAttnParams *p0, void *hip_stream) {
         if ((rc = launch_mfma_dbias(*p, e, st))) return rc;
         return launch_dbias_reduce(*p, e, st);
     }
-    if (!p0->gate && bwd_one_ok(*p)) return launch_stream_bwd_one_d64(*p, e, st);
+    if (bwd_one_ok(*p0)) return launch_stream_bwd_one_d64(*p, e, st);
     if (p->flags & EVO_FLAG_ONLY_DQ) return launch_dq(*p, e, st);
     const bool kvring = kv_ring_ok(*p);
     // that kernel sums the dBias partials on its way in (they lie 16-byte aligned for it)

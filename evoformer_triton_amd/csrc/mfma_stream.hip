@@ -1096,12 +1096,14 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
 // H = 32, fp32 bias, dQ and dK/dV one after the other / this, us: B = 1, N = 128 19.6 / 11.2, 256 28.7 / 16.8, 512 51 / 29, 1024 101 / 90; B = 3, N = 724
 // 220 / 171; B = 4, N = 1024 424 / 378 (4.8 TB/s past L2; problems in order the next call's forward takes 161 instead of 144;
 // sweeps turned so that both kinds meet in the same tile at the same time: no change); H = 8, B = 1, N = 2048 176 / 93.
-template <typename T, int BT>
+// Also without dBias (WRITE_DS) and with delta from the gate's pass (GIVEN), for rows that start or end within a group of four: as two launches, whose bias is read
+// entry by entry, these lost to the prepared tiles where there are few workgroups.
+template <typename T, int BT, bool WRITE_DS, bool GIVEN>
 __global__ void __launch_bounds__(256, 2) stream_bwd_one(EvoAttnParams p, Extra e) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const unsigned nb = (p.N + 127) / 128, lid = gridDim.x - 1 - xcd_remap(blockIdx.x, gridDim.x), problem = lid / (2 * nb), r = lid % (2 * nb);
-    if (r >= nb) dkdv_rows<T, 64, BT == 5 ? 3 : BT, 4, true, false>(p, e, lds, problem, r - nb);
-    else dq_rows<T, 64, BT, true>(p, e, lds, problem, r);
+    if (r >= nb) dkdv_rows<T, 64, BT == 5 ? 3 : BT, 4, !GIVEN, false>(p, e, lds, problem, r - nb);
+    else dq_rows<T, 64, BT, WRITE_DS>(p, e, lds, problem, r);
 }
 
 // ------------------------------------------------------------------ dBias partials
@@ -1387,7 +1389,8 @@ static int dkdv_waves(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
 }
 
 #if EVO_D == 64
-int launch_stream_bwd_one_d64(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+template <typename T>
+static int bwd_one_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const unsigned grid = 2 * (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H);
     auto go = [&](auto kern) {
         constexpr int lds = KvStream<64, 4>::BYTES;
@@ -1395,8 +1398,13 @@ int launch_stream_bwd_one_d64(const EvoAttnParams &p, const Extra &e, hipStream_
         kern<<<grid, 256, lds, st>>>(p, e);
         return hip_rc();
     };
-    if (p.dtype == EVO_BF16) return p.bias_dtype == EVO_F32 ? ragged_rows(p, e) ? go(stream_bwd_one<bf16_t, 5>) : go(stream_bwd_one<bf16_t, 3>) : go(stream_bwd_one<bf16_t, 4>);
-    return p.bias_dtype == EVO_F32 ? ragged_rows(p, e) ? go(stream_bwd_one<f16_t, 5>) : go(stream_bwd_one<f16_t, 3>) : go(stream_bwd_one<f16_t, 4>);
+    if (p.bias_dtype != EVO_F32) return go(stream_bwd_one<T, 4, true, false>);
+    if (!ragged_rows(p, e)) return go(stream_bwd_one<T, 3, true, false>);
+    if (e.delta_given) return p.dbias ? go(stream_bwd_one<T, 5, true, true>) : go(stream_bwd_one<T, 5, false, true>);
+    return p.dbias ? go(stream_bwd_one<T, 5, true, false>) : go(stream_bwd_one<T, 5, false, false>);
+}
+int launch_stream_bwd_one_d64(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    return p.dtype == EVO_BF16 ? bwd_one_launch<bf16_t>(p, e, st) : bwd_one_launch<f16_t>(p, e, st);
 }
 #endif
 
