@@ -274,7 +274,7 @@ static bool dq_writes_dbias(const EvoAttnParams &p) { return p.dbias && p.S == 1
 // 896 (448) 224 / 221, 1024 (512) 292 / 297, B = 4, N = 512 (512) 133 / 138, 640 (640) 270 / 242, 768 347 / 324, 896 473 / 424, 1024 (1024) 582 / 525.
 // Rows that start or end within a group of four are one launch also without dBias and with a gate.  Forward and backward over some 2700 random sizes against the
 // prepared tiles that such rows had before, median and most: two launches 32 workgroups 1.19, 1.29, 64 1.06, 1.22 (with a gate 1.11, 1.25 and 1.06,
-// 1.18), one launch .84, .96 and .82, .92 (.89, .98 and .89, .96); B = 1, N = 129, H = 16 without dBias 28.0 (tiles) / 36.0 (two) / 25 us.
+// 1.18), one launch .84, .96 and .82, .92 (.89, .98 and .89, .96); B = 1, N = 129, H = 16 without dBias 28.0 (tiles) / 36.0 (two) / 26.3 us.
 static bool bwd_one_ok(const EvoAttnParams &p) {
     constexpr int apart = EVO_FLAG_PER_PROBLEM | EVO_FLAG_ONLY_DQ | EVO_FLAG_ONLY_DKDV | EVO_FLAG_DEBUG_NO_DQ_WIDE;
     const int64_t wgs = (int64_t)((p.N + 127) / 128) * p.B * p.H;

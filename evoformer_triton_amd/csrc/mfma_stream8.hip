@@ -135,9 +135,12 @@ __global__ void __launch_bounds__(256, 3) stream_fwd8(EvoAttnParams p, Extra e) 
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // rows of an operand: keys 16 (c / 8) + 8 t + c % 8 of the tile; transposed ones: the keys of this lane's eight entries, columns 8 .. 15: 0 .. 7 again
+    // rows of an operand: keys 16 (c / 8) + 8 t + c % 8 of the tile; transposed ones: the keys of this lane's eight entries, columns 0 .. 7 of V and, from 8 on,
+    // twice the second half of the mask's chunk, 1 1 0 0: row 8 of O^T is the sum of the probabilities as they are rounded, by which O is divided.  (Divided
+    // by the sum of the unrounded ones O is 4 % further from 64 bits: S = 64, N = 256 2.24e-3 against 2.17e-3.  LSE keeps that sum, and O with an fp32 bias, where
+    // the forwards that served these calls before divide by it too and the other reads cost 2 %: columns 0 .. 7 again.)
     const int ka = (j == 1 ? 2 * R::ARR : 0) + (24 * (c >> 3) + (c & 7)) * 16, kstep = c < 8 ? 128 : -128;
-    const int va = R::ARR + (24 * (j >> 1) + 4 * (j & 1) + (c >> 2)) * 16 + (c & 1) * 8, vstep = j < 2 ? 128 : -128;
+    const int va = (BT == 2 && (c & 2) ? 2 * R::ARR + 8 : R::ARR + (c & 1) * 8) + (24 * (j >> 1) + 4 * (j & 1) + (c >> 2)) * 16, vstep = j < 2 ? 128 : -128;
     auto score = [&](const unsigned char *buf, int kb, int row, bool plain, const Init &init, f32x4 (&a)[2][2]) __attribute__((always_inline)) {   // both halves of the queries
         const unsigned char *x = buf + row * R::ROW + ka + kb * 16;
 #pragma unroll
@@ -315,10 +318,10 @@ __global__ void __launch_bounds__(256, 3) stream_fwd8(EvoAttnParams p, Extra e) 
         float sum = __uint_as_float(x[0]) + __uint_as_float(x[1]);
         x = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
         sum = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+        const float inv = 1.0f / (BT == 2 ? __shfl(o[i][0], 32 + c) : sum);
         const int q = q0 + 16 * (i & 1) + c;
         if (q < N) {
             if (j == 0) p.lse[pr.row0 + (int64_t)(i / 2) * N + q] = (m[i] + __log2f(sum)) * kLn2;
-            const float inv = 1.0f / sum;
             if (j < 2) store4<T>((T *)p.o + pr.base + (int64_t)(i / 2) * p.stride_s + (int64_t)q * p.stride_n + 4 * j, o[i][0] * inv, o[i][1] * inv, o[i][2] * inv, o[i][3] * inv);
         }
     }

@@ -70,3 +70,32 @@ def test_forward_pairs_match_eager(gpu_device, case):
     # the two kernels form the same scores and differ in the order of fp32 sums alone (N + 2 rounding steps of 2^-24 at most)
     a, c = got["pairs"][1], got["one"][1]
     assert ((a - c).abs() <= (N + 2) * 2.0 ** -24 * (1.0 + c.abs())).all()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N", [130, 160, 256])
+def test_no_further_from_64_bits_than_the_kernel_over_a_chunk_of_rows(gpu_device, N, dt):
+    """Head dim 8, 129 to 256 keys: O is divided by the sum of the probabilities as they are rounded, as that kernel does."""
+    import evoformer_triton_amd.evoformer as E
+    from evoformer_triton_amd import _lib
+    B, S, H, D = 1, 64, 4, 8
+    g = torch.Generator(device=gpu_device).manual_seed(5)
+    q, k, v = (torch.randn((B, S, N, H, D), device=gpu_device, generator=g).to(dt) for _ in range(3))
+    b = torch.randn((B, 1, H, N, N), device=gpu_device, generator=g).to(dt)
+    heads = [t.double().permute(0, 3, 1, 2, 4).contiguous() for t in (q, k, v)]
+    p64 = torch.softmax(torch.matmul(heads[0], heads[1].transpose(-1, -2).contiguous()) * D ** -0.5 + b.double().permute(0, 2, 1, 3, 4), -1)
+    want = torch.matmul(p64, heads[2])
+    lib = _lib.load()
+    bz, bdt, bstr = E._prep_bias(b, B, H, N, dt, gpu_device)
+    err = {}
+    for name, flags in ((b"mfma_fwd_pair", 0), (b"mfma_fwd_ring", _lib.EVO_FLAG_DEBUG_FWD_BIAS_TILES)):
+        o, lse = torch.empty_like(q), torch.empty((B, H, S, N), device=gpu_device)
+        p = E._params(q, k, v, None, _lib.EVO_MASK_NONE, (0, 0), bz, bdt, bstr, o, lse, "ds4sci")
+        p.flags |= flags
+        prep = torch.empty(lib.evoattn_prep_bytes(ctypes.byref(p)), dtype=torch.uint8, device=gpu_device)
+        p.prep, p.prep_bytes = prep.data_ptr(), prep.numel()
+        assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == name
+        assert lib.evoattn_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        err[name] = ((o.double().permute(0, 3, 1, 2, 4) - want).norm() / want.norm()).item()
+    # some 65000 independent roundings each: the two norms are known to well under 1 %
+    assert err[b"mfma_fwd_pair"] <= 1.01 * err[b"mfma_fwd_ring"], err
