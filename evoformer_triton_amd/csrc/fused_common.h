@@ -20,10 +20,10 @@ template <int N>
 __device__ __forceinline__ void fused_wait_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void fused_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 // 16 bytes per lane, from the lane's offset and a uniform one, into LDS from `dst` on; past the end of the array zeros.  (As an instruction that
-// the compiler does not know: see dma16 in mfma_stream.hip.)
+// the compiler does not know: see dma16 in stream_common.h.)
 __device__ __forceinline__ void fused_dma(__amdgpu_buffer_rsrc_t rs, unsigned char *dst, int off, int from) {
     const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)dst;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" : : "s"(base), "v"(off), "s"(rs), "s"(from));
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" : : "s"(base), "v"(off), "s"(rs), "s"(from) : "m0", "memory");
 }
 // A lane's offset past the end of any array here.  (What decides is the lane's offset: a uniform one past the end is taken from the array's size
 // before the two are compared, so it stays inside.)

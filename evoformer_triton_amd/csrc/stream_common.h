@@ -33,10 +33,11 @@ __device__ __forceinline__ void wait_lds_barrier() { asm volatile("s_waitcnt lgk
 // makes its own waits longer: where a wave waits for a bias tile, nothing younger than that tile should be under way.
 // (With the caller's fp32 rows kept unscaled until they are used, and dBias stored without a wait: B = 4, S = 1, N = 1024, H = 32, D = 64, step 691 ->
 // 611 us; three waves per SIMD had hidden most of it elsewhere: S = N = 768, H = 4, D = 32 2311 -> 2284; S = 200, N = 640, H = 5, D = 64 1006 -> 987.)
-// (s_nop: five states between a vector instruction's write of a scalar register and its use as an address.)
+// (s_nop: five states between a vector instruction's write of a scalar register and its use as an address.  Clobbers: the address register m0, which
+// the compiler may want to keep something in, and memory, so that no read or write of the buffer that is filled moves across, with the waits' own.)
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, unsigned char *dst, int off) {
     const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)dst;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(base), "v"(off), "s"(rs));
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(base), "v"(off), "s"(rs) : "m0", "memory");
 }
 
 // Rows r0 .. r0 + ROWS - 1 of two arrays that share their strides, into LDS at `dst` and `dst` + ROWS rows: this wave's share

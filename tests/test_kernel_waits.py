@@ -46,6 +46,18 @@ def test_a_split_forwards_fetch_follows_the_reads_of_its_buffer(head_dim, tmp_pa
     assert seen >= 6      # two dtypes, three kinds of bias
 
 
+def test_a_load_into_lds_declares_what_it_changes():
+    """Written as an instruction that the compiler does not know, it sets m0 and writes LDS."""
+    seen = 0
+    for name in sorted(os.listdir(build.CSRC)):
+        with open(os.path.join(build.CSRC, name)) as f:
+            for statement in re.findall(r"asm volatile\((.*?)\);", f.read(), re.S):
+                if "m0" in statement.split(":")[0]:
+                    seen += 1
+                    assert statement.rstrip().endswith(': "m0", "memory"'), (name, statement)
+    assert seen >= 2
+
+
 VMEM = re.compile(r"(buffer|global|flat|scratch)_(load|store|atomic)")
 
 
