@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(256, 2) bwd_fused(EvoAttnParams p, Extra e, un
             auto dq_store = [&](int n) {
                 const f32x4 v = dq + before;
                 if (kb + 1 < nb) {
-                    // (no uniform offset: a store of 16 bytes with one was taken over by the next write of its registers in the last lanes)
+                    // (no uniform offset: see kFusedPast)
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4f, v), prs, (unsigned)poff + (n < 0 ? kFusedPast : (unsigned)(n * 32 * D * 4)), 0, 0);
                 } else {
                     v4 w;

@@ -191,7 +191,7 @@ __global__ void __launch_bounds__(256, KT == 2 ? 3 : 2) bwd_fused8(EvoAttnParams
             auto dq_store = [&](int n, int par) {
                 const f32x4 v = dq + before + *reinterpret_cast<const f32x4 *>(xch + par * 1024 + (wave & 1) * 512 + c * 32 + (j & 1) * 16);
                 if (kb + 1 < nb) {
-                    // (no uniform offset: a store of 16 bytes with one was taken over by the next write of its registers in the last lanes)
+                    // (no uniform offset: see kFusedPast)
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4f, v), prs, n < 0 ? kFusedPast : poff + (unsigned)(n * 32 * D * 4), 0, 0);
                 } else {
                     v4 w;

@@ -58,6 +58,18 @@ def test_a_load_into_lds_declares_what_it_changes():
     assert seen >= 2
 
 
+def test_no_wide_buffer_store_has_a_uniform_offset():
+    """The compiler puts no wait state between such a store and the next write of its data, which the store may still be reading."""
+    seen = 0
+    for name in sorted(os.listdir(build.CSRC)):
+        with open(os.path.join(build.CSRC, name)) as f:
+            for line in f:
+                if re.search(r"raw(_ptr)?_buffer_store_b(96|128)\(", line):
+                    seen += 1
+                    assert re.search(r", 0, 0\);\s*$", line), (name, line)
+    assert seen >= 2
+
+
 VMEM = re.compile(r"(buffer|global|flat|scratch)_(load|store|atomic)")
 
 
@@ -110,6 +122,7 @@ def test_a_stage_is_there_when_it_is_prepared(source, tmp_path):
     """The kernels that form dQ, dK and dV at once wait for all but so many of the youngest loads before they read what they had loaded into LDS: on every way
     through the kernel at least as many have been issued since."""
     text = _assembly(source, [], tmp_path)
+    assert not re.search(r"buffer_store_dwordx[34] .*, s\d+ offen", text)   # (see the test above)
     seen = 0
     for name, lines in _functions(text, "bwd_fused"):
         blocks, following = _blocks(lines)
