@@ -57,13 +57,17 @@ enum {
     EVO_FLAG_FORCE_GENERIC = 1, /* run the plain fp32-arithmetic kernels whatever the dtype */
     EVO_FLAG_PREP_VALID    = 2, /* evoattn_bwd: `prep` still holds what evoattn_fwd wrote for the
                                    same bias and mask; skip re-deriving it */
-    /* Measurement aids: enqueue a single phase of the matrix-core backward.  ONLY_DQ runs
+    /* Measurement aids: enqueue a single phase of a matrix-core backward of two kernels.  ONLY_DQ runs
      * the dQ kernel (dq, delta and the dBias partials, no final dBias sum); ONLY_DKDV runs
-     * the dK/dV kernel and needs the delta a previous full call left in the same workspace. */
+     * the dK/dV kernel and needs the delta a previous full call left in the same workspace.  Where a call without
+     * them forms dQ, dK and dV in one kernel or one launch, these are other kernels than its own: evoattn_kernels of
+     * the call with and without the flag says whether they are. */
     EVO_FLAG_ONLY_DQ       = 4,
     EVO_FLAG_ONLY_DKDV     = 8,
     /* Measurement aid: run the one-workgroup-per-(b,h,s) forms of the forward and dQ kernels
-     * also where the forms that walk over a chunk of S rows apply (same results). */
+     * also where the forms that walk over a chunk of S rows apply (same results).  One S row of an fp32 bias at head dim 64 whose rows
+     * start or end within a group of four entries, of 32 blocks of 128 queries or more, is read in place by one dQ kernel alone: neither this flag nor
+     * EVO_FLAG_DEBUG_NO_DQ_WIDE chooses another one there (EVO_FLAG_DEBUG_BIAS_TILES with them does). */
     EVO_FLAG_PER_PROBLEM   = 16,
     /* evoattn_fwd (and evoattn_prep_bytes of it): no evoattn_bwd will read this call's `prep`, which then may be left unwritten
      * and, where evoattn_prep_bytes says so, missing. */
@@ -78,7 +82,7 @@ enum {
                                              the other one: head dims 8 and 16, dK/dV also 32 */
     EVO_FLAG_DEBUG_NO_KV_RING   = 0x200,  /* dK/dV: the one-workgroup-per-problem kernel instead of the chunk-of-rows one */
     EVO_FLAG_DEBUG_FWD_BIAS_TILES = 0x400, /* chunk-of-rows forward: prepared bias tiles as C operands instead of the caller's 16-bit rows */
-    EVO_FLAG_DEBUG_BIAS_TILES   = 0x800,  /* S <= 4: prepare the bias tiles instead of reading the caller's bias */
+    EVO_FLAG_DEBUG_BIAS_TILES   = 0x800,  /* S <= 4 (forward and backward alike, `prep` differs): prepare the bias tiles instead of reading the caller's bias */
     EVO_FLAG_DEBUG_NO_DQ_WIDE   = 0x1000, /* dQ: the kernels that split a row's keys over the waves, also without a dBias sum */
     EVO_FLAG_DEBUG_NO_DQ_SPLIT  = 0x2000  /* dQ + dBias in one kernel, also where dQ and the dBias partials come from two */
 };

@@ -429,3 +429,18 @@ def test_forward_of_two_rows_where_it_pays(lib, shape, bias, pairs):
     p.bias_dtype = p.dtype if bias == "q" else _lib.EVO_F32
     p.flags = _lib.EVO_FLAG_DEBUG_BIAS_TILES if shape[1] <= 4 else 0
     assert (lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == b"mfma_fwd_pair") == pairs
+
+
+def test_flags_where_bias_rows_are_read_in_place(lib):
+    """One S row of an odd length at head dim 64, fp32 bias: the flags that choose among dQ kernels split the one launch in two, and choose another
+    kernel only together with the one that prepares tiles."""
+    p = good(4, 1, 251, 8, 64)
+    p.bias_dtype = _lib.EVO_F32
+
+    def names(flags):
+        p.flags = flags
+        return lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_BWD)
+    assert names(0) == b"mfma_dq_wide,mfma_dkdv(one launch)"
+    for flag in (_lib.EVO_FLAG_PER_PROBLEM, _lib.EVO_FLAG_DEBUG_NO_DQ_WIDE):
+        assert names(flag) == b"mfma_dq_wide,mfma_dkdv"
+        assert names(flag | _lib.EVO_FLAG_DEBUG_BIAS_TILES) == b"mfma_dq,mfma_dkdv"
