@@ -40,13 +40,11 @@ def _units():
     units = [("api", "api.hip", []), ("generic", "generic.hip", []), ("dispatch", "dispatch.hip", []),
              ("prep", "prep.hip", []), ("layernorm", "layernorm.hip", []), ("pair_bias", "pair_bias.hip", VGPR_FORM[:2]),
              ("linear", "linear.hip", VGPR_FORM[:2]), ("f32", "f32.hip", VGPR_FORM[:2]), ("mfma_bwd_fused", "mfma_bwd_fused.hip", VGPR_FORM),
-             ("mfma_bwd_fused8", "mfma_bwd_fused8.hip", VGPR_FORM), ("mfma_stream8", "mfma_stream8.hip", VGPR_FORM)]
+             ("mfma_bwd_fused8", "mfma_bwd_fused8.hip", VGPR_FORM), ("mfma_stream8", "mfma_stream8.hip", VGPR_FORM), ("mfma_dbias", "mfma_dbias.hip", VGPR_FORM)]
     for d in HEAD_DIMS:
         if d <= 16:
             units.append((f"mfma_fwd_d{d}", "mfma_fwd.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
             units.append((f"mfma_dqw_d{d}", "mfma_dq_wide.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
-            if d == 16:
-                units.append((f"mfma_dbias_d{d}", "mfma_dbias.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
         else:
             units.append((f"mfma_stream_d{d}", "mfma_stream.hip", [f"-DEVO_D={d}", *VGPR_FORM]))
         units.append((f"mfma_bwd_d{d}", "mfma_bwd.hip", [f"-DEVO_D={d}", *VGPR_FORM]))

@@ -1,11 +1,10 @@
-// dBias partials for rows of more than 256 keys, as a kernel of its own.
-// Compiled once per head dim (-DEVO_D=16; 8: mfma_stream8.hip, from 32 on: mfma_stream.hip).
+// dBias partials of long rows at head dim 16, as a kernel of its own (8: mfma_stream8.hip, from 32 on: mfma_stream.hip).
 //
 // dBias[b][h] is the sum over the S rows of dS = P * (dP - delta) (reference: the atomic add of
 // every dS tile, evoformer.py:458).  Summing it inside the dQ kernel ties every wave of that
 // kernel to a few (query tile, key tile) pairs for a whole chunk of S rows, and with many key
-// tiles per row that leaves a workgroup 32 queries for all the keys it stages (N = 768: dQ in
-// 1.67 ms against 0.68 ms without the sum).  For such rows dQ comes from the kernel that knows
+// tiles per row that leaves a workgroup 32 queries for all the keys it stages (H = 8, S = 512, N = 640: dQ with
+// dBias 1003 us, as two kernels 915).  For such rows dQ comes from the kernel that knows
 // nothing of dBias, and this kernel forms dS a second time: a workgroup of 4 waves owns a block
 // of 128 queries x 128 keys of one (b, h) for a chunk of S rows, a wave 32
 // queries x 4 key tiles, whose running sums (64 registers) and bias tiles (32, as 16-bit
@@ -18,16 +17,11 @@
 #include "bwd_common.h"
 #include "kernels.h"
 
-#ifndef EVO_D
-#error "compile with -DEVO_D=<head dim>"
-#endif
-
 namespace evo {
 
-template <int D>
 struct DbGeo {
-    static constexpr int C = D / 8;                          // 16-byte chunks per row
-    static constexpr int RPB = 16 / C > 0 ? 16 / C : 1;      // rows per 256 bytes
+    static constexpr int D = 16, C = D / 8;                  // 16-byte chunks per row
+    static constexpr int RPB = 16 / C;                       // rows per 256 bytes
     // key tiles per wave; keys, queries per workgroup
     static constexpr int TPW = 4, KB = TPW * 32, QB = 128;
     static constexpr int OFF_K = 0, OFF_V = KB * D * 2, OFF_AK = 2 * KB * D * 2;
@@ -37,10 +31,11 @@ struct DbGeo {
 
 // BF32: the bias is fp32 (its prepared tiles are fp32 in log2 units and stay resident as they are: twice the
 // registers of the 16-bit pairs, nothing to unpack)
-template <typename T, int D, bool BF32>
+template <typename T, bool BF32>
 __global__ void __launch_bounds__(256, 2) mfma_dbias(EvoAttnParams p, Extra e) {
+    typedef DbGeo R;
+    constexpr int D = R::D;
     typedef Geo<D> G;
-    typedef DbGeo<D> R;
     constexpr int KS = G::KS, KSD = G::KSD, AUGC = G::AUGC;
     constexpr int NTH = 256, KB = R::KB, C = R::C, TPW = R::TPW;
     constexpr int NIT = (KB * C + NTH - 1) / NTH;            // 16-byte pieces of K (and of V) per thread and row
@@ -249,22 +244,17 @@ __global__ void __launch_bounds__(256, 2) mfma_dbias(EvoAttnParams p, Extra e) {
     }
 }
 
-// Workgroups per chunk of S rows: one per (query block, key block, batch, head).
-int64_t EVO_CAT(mfma_dbias_blocks_d, EVO_D)(const EvoAttnParams &p) {
-    typedef DbGeo<EVO_D> R;
-    return (int64_t)((p.N + R::QB - 1) / R::QB) * ((p.N + R::KB - 1) / R::KB) * p.B * p.H;
-}
-
-int EVO_CAT(launch_mfma_dbias_d, EVO_D)(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
-    const int64_t grid = EVO_CAT(mfma_dbias_blocks_d, EVO_D)(p) * e.n_chunks;
+int launch_mfma_dbias_d16(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
+    typedef DbGeo R;
+    const int64_t grid = (int64_t)((p.N + R::QB - 1) / R::QB) * ((p.N + R::KB - 1) / R::KB) * p.B * p.H * e.n_chunks;   // one per (query block, key block, batch, head, chunk)
     if (grid <= 0 || grid > 0x7fffffff) return EVO_EOVERFLOW;
     const bool bf32 = p.bias_dtype == EVO_F32;
     if (p.dtype == EVO_BF16) {
-        if (bf32) mfma_dbias<bf16_t, EVO_D, true><<<(unsigned)grid, 256, 0, st>>>(p, e);
-        else mfma_dbias<bf16_t, EVO_D, false><<<(unsigned)grid, 256, 0, st>>>(p, e);
+        if (bf32) mfma_dbias<bf16_t, true><<<(unsigned)grid, 256, 0, st>>>(p, e);
+        else mfma_dbias<bf16_t, false><<<(unsigned)grid, 256, 0, st>>>(p, e);
     } else {
-        if (bf32) mfma_dbias<f16_t, EVO_D, true><<<(unsigned)grid, 256, 0, st>>>(p, e);
-        else mfma_dbias<f16_t, EVO_D, false><<<(unsigned)grid, 256, 0, st>>>(p, e);
+        if (bf32) mfma_dbias<f16_t, true><<<(unsigned)grid, 256, 0, st>>>(p, e);
+        else mfma_dbias<f16_t, false><<<(unsigned)grid, 256, 0, st>>>(p, e);
     }
     return hip_rc();
 }

@@ -1108,7 +1108,7 @@ __global__ void __launch_bounds__(256, 2) stream_bwd_one(EvoAttnParams p, Extra 
 
 // ------------------------------------------------------------------ dBias partials
 
-// What mfma_dbias.hip is for the smallest head dims: dS a second time, summed over a chunk of S rows in registers.  A
+// What mfma_dbias.hip is for head dim 16: dS a second time, summed over a chunk of S rows in registers.  A
 // workgroup has 128 queries x 64 keys (head dim 32: 128) of one (b, h), a wave 32 queries x all of the block's key tiles.  Keys (K, V, mask
 // columns) are shared and double-buffered in LDS; a wave's own rows of Q and dO come into LDS of its own, which it reads into registers at the
 // top of a row and refills at once, so they need no second buffer and no barrier.
