@@ -234,7 +234,7 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && 
 // as busy.  (The probabilities are stream_fwd's, their sums are added in another order.  Gated calls keep stream_fwd: the bias of a block's pair norm
 // has a gradient that is zero but for the rounding of O.)
 // us, stream_fwd / this: H = 4, S = N = 768 501 / 455, 512 168 / 153, 384 81 / 75; H = 8, S = 128, N = 384 53.7 / 50.6; S = 300, N = 224 54.5 / 51.1; with
-// an fp32 bias S = N = 768, H = 4 536 / 486.
+// an fp32 bias S = N = 768, H = 4 536 / 486.  (Three waves per SIMD cost 6 spilled registers, with an fp32 bias in bf16 23.)
 template <typename T, int BT>
 __global__ void __launch_bounds__(256, 3) stream_fwd_pair(EvoAttnParams p, Extra e) {
     constexpr int D = 32, NW = 4, KSD = D / 16, KS = KSD + 1;

@@ -15,7 +15,8 @@ namespace evo {
 // takes with 32.  A wave's 32 queries are two halves, for which K and V are read once.
 // Bound by vector issue, 0.92 (92 instructions per tile of 32 x 32 where there were 104, a third of them before and after the loop; each lane prepares one
 // row of Q and they are dealt out through LDS: 264 -> 248).  us, mfma_fwd.hip or, up to 256 keys, mfma_fwd_ring.hip / this, H = 8: S = 1024, N = 384 277 / 248;
-// S = 1000: N = 96 48 / 38, 192 104 / 95, 256 125 / 116, 768 967 / 818; with an fp32 bias S = 512, N = 384 169 / 152, N = 768 600 / 483.
+// S = 1000: N = 96 48 / 38, 192 104 / 95, 256 125 / 116, 768 967 / 818; with an fp32 bias S = 512, N = 384 169 / 152, N = 768 600 / 483.  (Three waves per SIMD
+// cost 4 spilled registers, with an fp32 bias up to 28.)
 struct Fwd8 {
     static constexpr int KS = 128, ARR = KS * 16, ROW = 3 * ARR, BYTES = 2 * ROW;   // keys per stage; K, V and the mask's columns of a row; two rows
 };
