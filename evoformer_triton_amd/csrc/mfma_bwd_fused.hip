@@ -10,8 +10,9 @@
 // lies in fp32 in a scratch of the workgroup's own (512 workgroups then share the problems), read back and added in the same order every time.
 // LSE rides in a matrix step with the mask (three 16-bit parts each, exact), -delta is the first C of dP.  delta = <dO, O> is formed where a wave
 // prepares a stage, and written for the dBias kernel.
-// Bounds: vector and matrix issue, .36 each, and LDS, .42, at two waves per SIMD (the registers of a wave's 64 keys); per wave, group and tile 42
-// vector and 12 matrix instructions.  S = N = 768, H = 4 without dBias 1292 -> 992 us (dQ and dK/dV kernels before), S = N = 384 180 -> 143,
+// No single bound: at S = N = 768, H = 4 the vector ALU is busy for .50 of the time, the matrix core .32, LDS .56, a fifth of that bank conflicts (counters, at
+// 2.1 GHz), at two waves per SIMD (the registers of a wave's 64 keys), which wait for .30 of their life; 3.6 GB of traffic where once through the tensors is 1.2.  Per wave,
+// group and tile 42 vector and 12 matrix instructions.  S = N = 768, H = 4 without dBias 1292 -> 992 us (dQ and dK/dV kernels before), S = N = 384 180 -> 143,
 // N = 256, S = 512, H = 8 281 -> 209.  Four tiles per wave spill 12 registers (with an fp32 bias 28, and three 9), read back once per
 // block of keys, outside the loop over queries.  Two tiles per wave and three waves per SIMD spill (1650); the next block's keys and first stage fetched
 // during this one's last: more scalar registers than there are, 1035; head dim 64, of 32-query stages, 960 against the two kernels' 560.

@@ -5,7 +5,8 @@
 // of the keys serves both products.  dK and dV of a tile are 8 registers, and a workgroup keeps up to 384 keys (KT = 6 tiles of 16 per wave):
 // rows up to that length are one block, their queries pass once.  A group's dQ is two tiles of 16 queries: two waves share one, each with half of the
 // keys, and meet in LDS.
-// Bound by vector issue, 0.69 (42 instructions per wave, tile and group, 16 of them for the bias), and matrix issue, 0.27, at two waves per SIMD.
+// Bound by the vector ALU, busy .79 of the time at S = 1024, N = 384, H = 8 (counters, at 2.1 GHz; 42 instructions per wave, tile and group, 16 of them for the bias); LDS
+// .50, a fifth of it bank conflicts, matrix core .32, at two waves per SIMD.
 // S = 1024, N = 384, H = 8, without dBias: dQ and dK/dV kernels 663 us, this 400.  Blocks of 192 keys (KT = 3) 495, at three waves per SIMD
 // with 29 registers spilled 575; KT = 2, three waves, 495; more workgroups than are resident at a time (768) 517.
 #include "fused_common.h"

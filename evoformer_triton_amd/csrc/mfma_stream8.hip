@@ -13,7 +13,7 @@ namespace evo {
 // matrix instruction is 16x16x32, whose 32 columns hold the scaled Q, the mask and what rounding the scaled Q left: one instruction per 16 x 16
 // scores (32x32x16: two per 32 x 32, the same time), and P V, of whose 16 rows the head dim fills half, takes half of the time it
 // takes with 32.  A wave's 32 queries are two halves, for which K and V are read once.
-// Bound by vector issue, 0.92 (92 instructions per tile of 32 x 32 where there were 104, a third of them before and after the loop; each lane prepares one
+// Bound by the vector ALU, busy all the time (92 instructions per tile of 32 x 32 where there were 104, a third of them before and after the loop; each lane prepares one
 // row of Q and they are dealt out through LDS: 264 -> 248).  us, mfma_fwd.hip or, up to 256 keys, mfma_fwd_ring.hip / this, H = 8: S = 1024, N = 384 277 / 248;
 // S = 1000: N = 96 48 / 38, 192 104 / 95, 256 125 / 116, 768 967 / 818; with an fp32 bias S = 512, N = 384 169 / 152, N = 768 600 / 483.  (Three waves per SIMD
 // cost 4 spilled registers, with an fp32 bias up to 28.)
@@ -340,7 +340,7 @@ int launch_stream_fwd8(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
 
 // stream_dbias (mfma_stream.hip) for this head dim: a workgroup has 128 queries x 128 keys of one (b, h) for a chunk of S rows, a wave 32
 // queries x 4 key tiles, whose sums and bias (fp32, log2 units: the first C of the score product) stay in registers.
-// Bound by vector and matrix issue together at two waves per SIMD.  S = 1024, N = 384, H = 8: mfma_dbias.hip's kernel 300 us (96 vector instructions per
+// The vector ALU is busy for .66 of the time, the matrix core .18, at two waves per SIMD.  S = 1024, N = 384, H = 8: mfma_dbias.hip's kernel 300 us (96 vector instructions per
 // tile and row), this 285 (34, and 75 per row to prepare the operands); two tiles per wave and three waves per SIMD 302; three tiles 475 (spills).
 struct Db8 {
     static constexpr int TPW = 4, KB = TPW * 32, QB = 128, ARR = KB * 16;   // K, V and the mask's columns
