@@ -156,13 +156,13 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && 
         for (int t = 0; t < AHEAD; ++t) bias.load(kt + AHEAD + t, ct[t]);
     };
     // ST tiles, from tile kt and row kb of the stage on
-    auto step = [&](const unsigned char *buf, int kt, int kb, const f32x16 *init) {
+    auto step = [&](const unsigned char *buf, int kt, int kb, const f32x16 *init, auto first) __attribute__((always_inline)) {
         const float used = mf;
         f32x16 a[ST];
 #pragma unroll
         for (int t = 0; t < ST; ++t) score(buf, kb + 32 * t, init[t], a[t]);
-        const bool lazy = kt != 0 && !__any(m != used);
-        if (!lazy) settle(kt == 0, a, used);
+        const bool lazy = !first && !__any(m != used);
+        if (!lazy) settle(first, a, used);
         v8 pf[2 * ST];
         float s = probs(a, pf);
         if (__builtin_expect(lazy && __any(!(s <= 8192.0f)), 0)) {   // some score stands far above m: once more, the long way
@@ -186,16 +186,16 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && 
     const int nst = (p.N + R::ROWS - 1) / R::ROWS;
     wait_loads();
     wait_lds_barrier();
-    for (int s = 0; s < nst; ++s) {
+    auto stage = [&](int s, auto first) __attribute__((always_inline)) {
         auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
         if (active) {
             const unsigned char *buf = lds[s & 1];
             f32x16 init[AHEAD];
             biases(2 * s, init, next);
-            step(buf, 2 * s, 0, init);
+            step(buf, 2 * s, 0, init, first);
             if (ST == 1 && 2 * s + 1 < NT) {
                 if (AHEAD == 1) biases(2 * s + 1, init, [] {});
-                step(buf, 2 * s + 1, 32, init + AHEAD - 1);
+                step(buf, 2 * s + 1, 32, init + AHEAD - 1, std::false_type());
             }
         } else {
             next();
@@ -204,6 +204,14 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && 
             wait_loads();
             wait_lds_barrier();
         }
+    };
+    // (Head dim 128, 16-bit tiles: the first stage by itself; with bf16 the compiler left its test in the loop otherwise.  us, S = 120, N = 58, H = 32 62.6 -> 59.7, S = 187,
+    // N = 56, H = 16 49.2 -> 47.2; some 600 calls of 33 to 64 keys .96 of the time at the median, longer ones 1.00.)
+    if constexpr (D == 128 && BT == 2) {
+        stage(0, std::true_type());
+        for (int s = 1; s < nst; ++s) stage(s, std::false_type());
+    } else {
+        for (int s = 0; s < nst; ++s) stage(s, s == 0);
     }
 
     if (!active) return;
