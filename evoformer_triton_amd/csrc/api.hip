@@ -97,7 +97,7 @@ static bool mfma_ok(const EvoAttnParams &p, int pass) {
     return true;
 }
 
-// fp32 on the fp32 matrix instruction (f32.hip): rows and their strides in whole 16-byte pieces.  Anything else in fp32 (and 16-bit tensors at odd addresses) takes the plain
+// fp32 on the matrix core (f32.hip): rows and their strides in whole 16-byte pieces.  Anything else in fp32 (and 16-bit tensors at odd addresses) takes the plain
 // kernels, one row per thread on the vector ALU.
 static bool f32_ok(const EvoAttnParams &p, int pass) {
     if (p.dtype != EVO_F32 || (p.flags & EVO_FLAG_FORCE_GENERIC)) return false;
