@@ -702,6 +702,7 @@ __global__ void __launch_bounds__(256, D == 32 ? 3 : D == 64 ? 2 : 1) split_fwd(
 // As mfma_dq_wide.hip, whose place it takes at these head dims: where dBias is no sum over S rows, or its sum comes from a
 // kernel of its own.  A wave has 32 queries for all keys; with WRITE_DS (S = 1) dBias is dS and goes out as it is formed.
 // Block `block` of 128 queries of problem `problem`, in `lds` of 2 R::BYTES.
+constexpr int kDsBytes = 32 * 32 * 4;   // a wave's tile of dS in fp32
 template <typename T, int D, int BT, bool WRITE_DS>
 __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, unsigned char *lds, unsigned problem, int block) {
     typedef StreamGeo<D> G;
@@ -767,6 +768,8 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
     const int64_t dsrow = (((int64_t)pr.b * p.H + pr.h) * p.N + qrow) * p.N;
     const bool ds_vec = (p.N & 3) == 0 && ((uintptr_t)p.dbias & 15) == 0, ds_f32 = p.dbias_dtype == EVO_F32;
 
+    float *const dstile = (float *)p.dbias + (((int64_t)pr.b * p.H + pr.h) * p.N + q0 + (lane >> 3)) * p.N + 4 * (lane & 7);   // (fp32; where this lane stores of a tile: its row of eight, its four columns)
+
     f32x16 dq[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -799,7 +802,34 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
             for (int dt = 0; dt < DT; ++dt) dq[dt] = Mfma<T>::mma(transposed<T, D>(buf, kb, ts, dt, lane), ds[ts], dq[dt]);
     };
     auto write = [&](int kt, const f32x16 &a) {
-        if (!WRITE_DS || q0 + li >= p.N) return;
+        if (!WRITE_DS) return;
+        if (PAIR && ds_f32) {   // through LDS of the wave's own, so that a store covers 128 bytes of eight rows each
+            unsigned char *const own = lds + 2 * R::BYTES + wave * kDsBytes;
+            auto at = [](int r, int c) { return r * 128 + ((c ^ (r >> 1 & 7)) << 4); };   // (two rows share the 64 banks)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+                f32x4 v;
+                v[0] = a[4 * rr]; v[1] = a[4 * rr + 1]; v[2] = a[4 * rr + 2]; v[3] = a[4 * rr + 3];
+                *reinterpret_cast<f32x4 *>(own + at(li, 2 * rr + g)) = v;
+            }
+            const int c = lane & 7, col = kt * 32 + 4 * c;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int r = 8 * j + (lane >> 3);
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(own + at(r, c));
+                if (q0 + r >= p.N) continue;
+                float *const d = dstile + (int64_t)(8 * j) * p.N + kt * 32;
+                if (col + 4 <= p.N) {
+                    *reinterpret_cast<f32x4_at4 *>(d) = v;   // (16 bytes wherever they start)
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (col + i < p.N) d[i] = v[i];
+                }
+            }
+            return;
+        }
+        if (q0 + li >= p.N) return;
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
             const int kg = kt * 32 + 8 * rr + 4 * g;   // registers 4 rr .. 4 rr + 3 hold keys kg .. kg + 3
@@ -838,16 +868,8 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
                 next();
                 bias.load(2 * s + 2, ct);
                 bias.load(2 * s + 3, c1);
-                f32x16 d0;
-                tile(buf, 0, b0, [&](const f32x16 &d) { d0 = d; });
-                if (2 * s + 1 < NT) {
-                    tile(buf, 32, b1, [&](const f32x16 &d) {
-                        write(2 * s, d0);
-                        write(2 * s + 1, d);
-                    });
-                } else {
-                    write(2 * s, d0);
-                }
+                tile(buf, 0, b0, [&](const f32x16 &d) { write(2 * s, d); });
+                if (2 * s + 1 < NT) tile(buf, 32, b1, [&](const f32x16 &d) { write(2 * s + 1, d); });
             } else {
                 next();
                 bias.load(2 * s + 1, ct);
@@ -862,9 +884,9 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
             next();
         }
         if (s + 1 < nst) {
-            // A stage before the last has two whole tiles: a wave that has queries stored at least eight pieces of dBias after it had asked
-            // for the next stage, and need not wait for them.
-            if (WRITE_DS && active) wait_loads_but<8>();
+            // A stage before the last has two whole tiles: a wave with 32 queries (with fewer, a store of eight rows may have none) stored at least
+            // eight pieces of dBias after it had asked for the next stage, and need not wait for them.
+            if (WRITE_DS && q0 + 32 <= p.N) wait_loads_but<8>();
             else wait_loads();
             wait_lds_barrier();
         }
@@ -878,7 +900,7 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
 
 template <typename T, int D, int BT, bool WRITE_DS>
 __global__ void __launch_bounds__(256, D == 32 ? 4 : D == 64 && BT < 3 ? 3 : 2) stream_dq(EvoAttnParams p, Extra e) {
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * FwdStream<D>::BYTES];
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * FwdStream<D>::BYTES + (D == 64 && BT >= 3 && WRITE_DS ? 4 * kDsBytes : 0)];
     const unsigned nqb = (p.N + 127) / 128, lid = xcd_remap(blockIdx.x, gridDim.x);
     dq_rows<T, D, BT, WRITE_DS>(p, e, lds, lid / nqb, lid % nqb);
 }
@@ -1402,7 +1424,7 @@ static int bwd_one_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st
     const unsigned grid = 2 * (unsigned)((p.N + 127) / 128) * (unsigned)(p.B * p.H);
     auto go = [&](auto kern) {
         constexpr int lds = KvStream<64, 4>::BYTES;
-        static_assert(lds >= 2 * FwdStream<64>::BYTES && lds <= 64 * 1024, "the larger of the two");
+        static_assert(lds >= 2 * FwdStream<64>::BYTES + 4 * kDsBytes && lds <= 64 * 1024, "the larger of the two");
         kern<<<grid, 256, lds, st>>>(p, e);
         return hip_rc();
     };
