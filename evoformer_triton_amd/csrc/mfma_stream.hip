@@ -1243,6 +1243,7 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
     fetch_queries(s_begin);
     for (int s = s_begin; s < s_end; ++s) {
         wait_loads();
+        asm volatile("" : "+v"(lse_n), "+v"(delta_n), "+v"(dead_n));   // (the compiler's own wait for them: here, not behind the next keys' loads)
         const bool dead = (D != 64 ? __builtin_amdgcn_readfirstlane(dead_n) : uniform_load(e.dead + b * p.S + s)) != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
         wait_lds_barrier();
         if (s + 1 < s_end) fetch_keys(s + 1);   // (everybody has left that buffer: it held row s - 1)
@@ -1288,6 +1289,8 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
                 a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (32 * j + li) * 16), qf[KSD], a);
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sum[j][r] += fast_exp2(a[r]) * dp[r];
+            } else {
+                asm volatile("");   // (a block of its own for the sums that stay: without one they are copied ahead of the branch, 16 moves a tile)
             }
             if (D < 128) __builtin_amdgcn_sched_barrier(0);   // (the next tile's operands would take the registers)
         }

@@ -424,6 +424,7 @@ __global__ void __launch_bounds__(256, 2) stream_dbias8(EvoAttnParams p, Extra e
     fetch_queries(s_begin);
     for (int s = s_begin; s < s_end; ++s) {
         wait_loads();
+        asm volatile("" : "+v"(q_n), "+v"(g_n), "+v"(lse_n), "+v"(delta_n), "+v"(dead_n));   // (the compiler's own wait for them: here, not behind the next keys' loads)
         const bool dead = __builtin_amdgcn_readfirstlane(dead_n) != 0, kill = dead && p.mask_kind == EVO_MASK_BOOL;
         wait_lds_barrier();
         if (s + 1 < s_end) fetch_keys(s + 1);   // (everybody has left that buffer: it held row s - 1)
@@ -437,25 +438,25 @@ __global__ void __launch_bounds__(256, 2) stream_dbias8(EvoAttnParams p, Extra e
         if (s + 1 < s_end) fetch_queries(s + 1);
         if (!active || kill) continue;
         const unsigned char *buf = lds + ((s - s_begin) & 1) * R::KEYS;
-        auto walk = [&](auto plain) {
 #pragma unroll
-            for (int j = 0; j < R::TPW; ++j) {
-                if (j < tiles) {   // uniform
-                    f32x16 z;
+        for (int j = 0; j < R::TPW; ++j) {
+            if (j < tiles) {   // uniform
+                f32x16 z;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) z[r] = 0.0f;
-                    const v8 k = *reinterpret_cast<const v8 *>(buf + ka + j * 512);
-                    f32x16 a = Mfma<T>::mma(k, qf, plain ? bias[j] : z), dp;                                // log2 P^T
-                    dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + va + j * 512), gf, z);          // dP^T - delta
-                    a = Mfma<T>::mma(k, ql, a);
+                for (int r = 0; r < 16; ++r) z[r] = 0.0f;
+                const v8 k = *reinterpret_cast<const v8 *>(buf + ka + j * 512);
+                f32x16 a;
+                if (__builtin_expect(!dead, 1)) a = Mfma<T>::mma(k, qf, bias[j]);                             // log2 P^T
+                else a = Mfma<T>::mma(k, qf, z);   // (a row with every key masked takes no bias)
+                const f32x16 dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + va + j * 512), gf, z);     // dP^T - delta
+                a = Mfma<T>::mma(k, ql, a);
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) sum[j][r] += fast_exp2(a[r]) * dp[r];
-                }
-                __builtin_amdgcn_sched_barrier(0);   // (the next tile's operands would take the registers)
+                for (int r = 0; r < 16; ++r) sum[j][r] += fast_exp2(a[r]) * dp[r];
+            } else {
+                asm volatile("");   // (a block of its own for the sums that stay: without one they are copied ahead of the branch, 16 moves a tile)
             }
-        };
-        if (!dead) walk(std::true_type());
-        else walk(std::false_type());   // (a row with every key masked takes no bias)
+            __builtin_amdgcn_sched_barrier(0);   // (the next tile's operands would take the registers)
+        }
     }
     // the partial of this chunk: lane = query li, registers 4 rr .. 4 rr + 3 = keys 8 rr + 4 g ..
     if (active && q0 + li < p.N) {
