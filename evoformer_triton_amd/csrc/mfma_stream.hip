@@ -148,19 +148,34 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && 
         return s;
     };
     // AHEAD tiles' bias, from tile kt on, and the next ones asked for; `between`: what is asked for once these have arrived
+    // (a tile that is a C operand as it lies: `step` asks for the next one where this one's chain has begun)
+    constexpr bool IN_PLACE = BT == 1;
     auto biases = [&](int kt, f32x16 (&init)[AHEAD], auto between) {
+        if constexpr (IN_PLACE) {
 #pragma unroll
-        for (int t = 0; t < AHEAD; ++t) init[t] = bias.take(ct[t]);
-        between();
+            for (int t = 0; t < AHEAD; ++t) bias.arrived(ct[t]);
+            between();
+        } else {
 #pragma unroll
-        for (int t = 0; t < AHEAD; ++t) bias.load(kt + AHEAD + t, ct[t]);
+            for (int t = 0; t < AHEAD; ++t) init[t] = bias.take(ct[t]);
+            between();
+#pragma unroll
+            for (int t = 0; t < AHEAD; ++t) bias.load(kt + AHEAD + t, ct[t]);
+        }
     };
     // ST tiles, from tile kt and row kb of the stage on
     auto step = [&](const unsigned char *buf, int kt, int kb, const f32x16 *init, auto first) __attribute__((always_inline)) {
         const float used = mf;
         f32x16 a[ST];
+        if constexpr (IN_PLACE) {
 #pragma unroll
-        for (int t = 0; t < ST; ++t) score(buf, kb + 32 * t, init[t], a[t]);
+            for (int t = 0; t < ST; ++t) score(buf, kb + 32 * t, ct[t], a[t]);
+#pragma unroll
+            for (int t = 0; t < ST; ++t) bias.refill(kt + ST + t, ct[t]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < ST; ++t) score(buf, kb + 32 * t, init[t], a[t]);
+        }
         const bool lazy = !first && !__any(m != used);
         if (!lazy) settle(first, a, used);
         v8 pf[2 * ST];
@@ -776,7 +791,7 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
 #pragma unroll
         for (int r = 0; r < 16; ++r) dq[dt][r] = 0.0f;
 
-    auto tile = [&](const unsigned char *buf, int kb, f32x16 a, auto leave) {   // `leave` takes dS
+    auto tile = [&](const unsigned char *buf, int kb, f32x16 a, auto begun, auto leave) {   // `begun`: the chains are; `leave` takes dS
         f32x16 dp;
 #pragma unroll
         for (int r = 0; r < 16; ++r) dp[r] = 0.0f;
@@ -788,6 +803,7 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
         }
         a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (kb + li) * 16), qf[KSD], a);
         dp = Mfma<T>::mma(vaug, gf[KSD], dp);
+        begun();
 #pragma unroll
         for (int r = 0; r < 16; ++r) a[r] = fast_exp2(a[r]) * dp[r];
         leave(a);
@@ -862,22 +878,27 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
         };
         if (active) {
             const unsigned char *buf = lds + (s & 1) * R::BYTES;
-            const f32x16 b0 = bias.take(ct);
             if constexpr (PAIR) {
-                const f32x16 b1 = bias.take(c1);
+                const f32x16 b0 = bias.take(ct), b1 = bias.take(c1);
                 next();
                 bias.load(2 * s + 2, ct);
                 bias.load(2 * s + 3, c1);
-                tile(buf, 0, b0, [&](const f32x16 &d) { write(2 * s, d); });
-                if (2 * s + 1 < NT) tile(buf, 32, b1, [&](const f32x16 &d) { write(2 * s + 1, d); });
+                tile(buf, 0, b0, [] {}, [&](const f32x16 &d) { write(2 * s, d); });
+                if (2 * s + 1 < NT) tile(buf, 32, b1, [] {}, [&](const f32x16 &d) { write(2 * s + 1, d); });
+            } else if constexpr (BT == 1) {
+                bias.arrived(ct);
+                next();
+                tile(buf, 0, ct, [&] { bias.refill(2 * s + 1, ct); }, [&](const f32x16 &d) { write(2 * s, d); });
+                if (2 * s + 1 < NT) tile(buf, 32, ct, [&] { bias.refill(2 * s + 2, ct); }, [&](const f32x16 &d) { write(2 * s + 1, d); });
             } else {
+                const f32x16 b0 = bias.take(ct);
                 next();
                 bias.load(2 * s + 1, ct);
-                tile(buf, 0, b0, [&](const f32x16 &d) { write(2 * s, d); });
+                tile(buf, 0, b0, [] {}, [&](const f32x16 &d) { write(2 * s, d); });
                 if (2 * s + 1 < NT) {
                     const f32x16 b1 = bias.take(ct);
                     bias.load(2 * s + 2, ct);
-                    tile(buf, 32, b1, [&](const f32x16 &d) { write(2 * s + 1, d); });
+                    tile(buf, 32, b1, [] {}, [&](const f32x16 &d) { write(2 * s + 1, d); });
                 }
             }
         } else {
@@ -958,9 +979,10 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
             nd = q < p.N ? -e.delta[pr.row0 + q] : 0.0f;
         }
     };
-    auto finish = [&](int stage) {   // what this wave fetched is there: its pieces of Q scaled, the extra columns
+    auto finish = [&](int stage, bool bias_behind) {   // what this wave fetched is there: its pieces of Q scaled, the extra columns
         unsigned char *buf = lds + (stage & 1) * R::STAGE;
-        wait_loads();
+        if (bias_behind) wait_loads_but<8>();   // (two tiles of the bias, in four pieces each, are younger than the stage)
+        else wait_loads();
         constexpr int PIECES = R::BLK / 1024;
 #pragma unroll
         for (int i = 0; i < (PIECES + NW - 1) / NW; ++i) {
@@ -1064,13 +1086,19 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
     };
 
     const int nst = (p.N + ROWS - 1) / ROWS;
-    finish(0);
+    finish(0, false);
     for (int s = 0; s < nst; ++s) {
         auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
         if (active) {
             const unsigned char *buf = lds + (s & 1) * R::STAGE;
             const int qt = s * (ROWS / 32);
-            if constexpr (TWO) {
+            if constexpr (TWO && BT == 1) {
+                bias.arrived(ct);
+                bias.arrived(c1);
+                next();
+                tile(buf, 0, [&] { return ct; }, [&] { bias.refill(qt + 2, ct); });
+                if (qt + 1 < NT) tile(buf, 32, [&] { return c1; }, [&] { bias.refill(qt + 3, c1); });
+            } else if constexpr (TWO) {
                 const f32x16 b0 = bias.take(ct), b1 = bias.take(c1);
                 next();
                 bias.load(qt + 2, ct);
@@ -1092,7 +1120,7 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
         } else {
             next();
         }
-        if (s + 1 < nst) finish(s + 1);
+        if (s + 1 < nst) finish(s + 1, TWO && BT == 1 && active);   // (a stage before the last has two tiles)
     }
 
     if (!active) return;

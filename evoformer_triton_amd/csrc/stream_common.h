@@ -174,6 +174,17 @@ struct BiasStream {
             return t;
         }
     }
+    // For a tile that is a C operand as it lies (BT = 1): the wait for it, here; and, once the chain that begins with it is under way, the next one
+    // into its registers (which that chain's first instruction must then not have taken for its result: 16 copies a tile otherwise).
+    __device__ __forceinline__ void arrived(Tile &t) const {
+        if constexpr (BT == 1) asm volatile("" : "+v"(t));
+    }
+    __device__ __forceinline__ void refill(int n, Tile &t) const {
+        if constexpr (BT == 1) {
+            asm volatile("" ::"v"(t));
+            load(n, t);
+        }
+    }
     // `value`, formed here: the wait for the tile stands before whatever the wave asks for next
     __device__ __forceinline__ f32x16 take(const Tile &t) const {
         f32x16 v = value(t);
@@ -193,6 +204,8 @@ struct BiasStream<T, 0, COLS> {
         return z;
     }
     __device__ __forceinline__ f32x16 take(const Tile &t) const { return value(t); }
+    __device__ __forceinline__ void arrived(Tile &) const {}
+    __device__ __forceinline__ void refill(int, Tile &) const {}
 };
 
 }  // namespace evo
