@@ -412,17 +412,20 @@ __global__ void __launch_bounds__(256, 3) stream_fwd_pair(EvoAttnParams p, Extra
     // a key tile of all (one or both) rows: kt, from row kb of the stage on
     auto step = [&](const unsigned char *buf, int kt, int kb, auto rows, auto plain, auto between) {
         constexpr int ROWS = decltype(rows)::value;
-        const f32x16 init = bias.take(ct);
+        f32x16 init;
+        if (BT == 1) bias.arrived(ct);   // (the C operand as it lies)
+        else init = bias.take(ct);
         between();
-        bias.load(kt + 1, ct);
+        if (BT != 1) bias.load(kt + 1, ct);
         f32x16 a[ROWS][1];
         float used[ROWS], s[ROWS];
         v8 pf[ROWS][2];
 #pragma unroll
         for (int j = 0; j < ROWS; ++j) {
             used[j] = mf[j];
-            score(j, plain, buf + j * R::BYTES, kb, init, a[j][0]);
+            score(j, plain, buf + j * R::BYTES, kb, bias.lies(ct, init), a[j][0]);
         }
+        if (BT == 1) bias.refill(kt + 1, ct);
         const bool lazy = !__any(m[0] != mf[0] || m[ROWS - 1] != mf[ROWS - 1]);
         if (!lazy)
 #pragma unroll

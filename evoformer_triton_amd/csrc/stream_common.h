@@ -177,13 +177,21 @@ struct BiasStream {
     // For a tile that is a C operand as it lies (BT = 1): the wait for it, here; and, once the chain that begins with it is under way, the next one
     // into its registers (which that chain's first instruction must then not have taken for its result: 16 copies a tile otherwise).
     __device__ __forceinline__ void arrived(Tile &t) const {
+#ifdef __HIP_DEVICE_COMPILE__   // (the host's own pass, which has no such registers, drops kernels' entries over it)
         if constexpr (BT == 1) asm volatile("" : "+v"(t));
+#endif
     }
     __device__ __forceinline__ void refill(int n, Tile &t) const {
         if constexpr (BT == 1) {
+#ifdef __HIP_DEVICE_COMPILE__
             asm volatile("" ::"v"(t));
+#endif
             load(n, t);
         }
+    }
+    __device__ __forceinline__ const f32x16 &lies(const Tile &t, const f32x16 &taken) const {
+        if constexpr (BT == 1) return t;
+        else return taken;
     }
     // `value`, formed here: the wait for the tile stands before whatever the wave asks for next
     __device__ __forceinline__ f32x16 take(const Tile &t) const {
