@@ -73,9 +73,10 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && 
         if (g == 0) qf[KSD][0] = qf[KSD][1] = qf[KSD][2] = (T)1.0f;
     }
     const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, dead, lane);
-    // AHEAD: tiles whose bias is asked for together, and ahead of a step.  Where few S rows leave the caller's bias rows as the traffic (head dim 64) it is
-    // both tiles of a stage, 256 bytes of a row at a time, which memory serves better than 128, at two waves per SIMD: B = 4, S = 1, N = 1024, H = 32,
-    // fp32 164 -> 148 us.  (Prepared tiles lie whole: S = 200, N = 640, H = 5, fp32 190 / 204.)
+    // AHEAD: tiles whose bias is asked for together.  Where few S rows leave the caller's bias rows as the traffic (head dim 64) it is
+    // both tiles of a stage, 256 bytes of a row at a time, which memory serves better than 128: B = 4, S = 1, N = 1024, H = 32, fp32 164 -> 148 us.  They are asked
+    // for when the stage before is half done: at its beginning they took 16 registers more than three waves per SIMD have (at two waves N = 1024 147 us, 768 89,
+    // 725 114; at three, so, 143, 84, 87; at three with what does not fit spilled 211, 106).  (Prepared tiles lie whole: S = 200, N = 640, H = 5, fp32 190 / 204.)
     constexpr int AHEAD = D == 64 && BT >= 3 ? 2 : ST;
     typename BiasStream<T, BT, false>::Tile ct[AHEAD];
 #pragma unroll
@@ -203,20 +204,33 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && 
     wait_lds_barrier();
     auto stage = [&](int s, auto first) __attribute__((always_inline)) {
         auto next = [&] { if (s + 1 < nst) fetch(s + 1); };
-        if (active) {
+        if (AHEAD > ST && active) {   // (the next stage's bias is asked for in the middle of this one, when both of this one's tiles have left their registers)
+            const unsigned char *buf = lds[s & 1];
+            f32x16 init = bias.take(ct[0]);
+            next();
+            step(buf, 2 * s, 0, &init, first);
+            if (2 * s + 1 < NT) {
+                init = bias.take(ct[AHEAD - 1]);
+                bias.load(2 * s + 2, ct[0]);
+                bias.load(2 * s + 3, ct[AHEAD - 1]);
+                step(buf, 2 * s + 1, 32, &init, std::false_type());
+            }
+        } else if (active) {
             const unsigned char *buf = lds[s & 1];
             f32x16 init[AHEAD];
             biases(2 * s, init, next);
             step(buf, 2 * s, 0, init, first);
             if (ST == 1 && 2 * s + 1 < NT) {
-                if (AHEAD == 1) biases(2 * s + 1, init, [] {});
-                step(buf, 2 * s + 1, 32, init + AHEAD - 1, std::false_type());
+                biases(2 * s + 1, init, [] {});
+                step(buf, 2 * s + 1, 32, init, std::false_type());
             }
         } else {
             next();
         }
         if (s + 1 < nst) {
-            wait_loads();
+            // (a stage before the last has two tiles, and the bias asked for there, four pieces or more for each, is younger than the rows)
+            if (AHEAD > ST && active) wait_loads_but<8>();
+            else wait_loads();
             wait_lds_barrier();
         }
     };
