@@ -607,7 +607,9 @@ static int fwd_launches(const EvoAttnParams &p, hipStream_t st) {
         e.bk16 = nullptr;
         e.bt = nullptr;
     }
-    if (const int rc = launch_prep(p, e, st, alone && ring && mfma_fwdr_reads_rows(p))) return rc;
+    // (that forward then has nothing to wait for: it reads the mask as given, too)
+    if (alone && ring && !fwd_pairs8_ok(p) && (!p.bias || mfma_fwdr_reads_rows(p))) e.m2a = nullptr;
+    else if (const int rc = launch_prep(p, e, st)) return rc;
     return fwd_pairs8_ok(p) ? launch_stream_fwd8(p, e, st) : ring ? launch_mfma_fwdr(p, e, st) : launch_mfma_fwd(p, e, st);
 }
 

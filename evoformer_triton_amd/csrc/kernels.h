@@ -17,7 +17,7 @@ int launch_dbias_reduce(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_gate_bwd(const EvoAttnParams &p, void *dout_ungated, float *delta, hipStream_t st);  // dO, dgate and delta from the gradient of the gated output
 int launch_mask_shift(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 
-int launch_prep(const EvoAttnParams &p, const Extra &e, hipStream_t st, bool masks_only = false);
+int launch_prep(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 int launch_mfma_fwd(const EvoAttnParams &p, const Extra &e, hipStream_t st);
 constexpr int kSplitFwdMaxN = 4096;   // (its mask row lies in LDS)
 int launch_split_fwd(const EvoAttnParams &p, hipStream_t st);  // the keys of a row split over waves; reads mask and bias as given

@@ -97,7 +97,10 @@ static __host__ __device__ inline bool fwdr_rows16(const EvoAttnParams &p) {
 // BIASK: 0 no bias, 1 fp32 tiles (x log2(e), accumulator order) as C operands, 2 the caller's 16-bit rows through the identity
 // GATED: the output gate in the epilogue (kernels of their own: the ungated one carries none of their registers);
 // 1: the gate's logits asked for in the epilogue, 2: copied into LDS while the row is computed (see gate_dma below)
-template <typename T, int D, int BIASK, int GATED>
+// OWN: the mask as the caller has it (a forward without a backward, whose prep kernel would write nothing else): waves 0 to 3 read a row's entries with the
+// rest of its stage, 64 keys each, and make its columns of them where they write the stage; what they found kept lies behind the stages. A launch and
+// 16 bytes per key less: S = 128, N = 251, H = 8, D = 32, fp16, gated 35.0 -> 32.7 us with the launch before it (the kernel itself 35.0 -> 36.3, traced).
+template <typename T, int D, int BIASK, int GATED, bool OWN>
 __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     typedef FwdRingGeo<D> R;
     constexpr int C = R::C;
@@ -216,7 +219,8 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     // (64 lanes x 16 bytes): K, V, then the mask columns; piece n belongs to wave n % 8.  Lane
     // i of piece m of K or V fills LDS slot 64 m + i of that block, which the swizzle assigns
     // to some chunk of some row.
-    u32x4 stg[IPW];
+    u32x4 stg[OWN ? IPW - 1 : IPW];
+    unsigned mraw = 0;   // (OWN: the mask's piece, an entry per lane)
     // K and V pieces are buffer loads: a resource (in scalar registers) that describes the K or V rows of
     // the S row asked for next, one lane offset that every K and V piece shares (a piece is 64 / C rows
     // of C 16-byte chunks; the swizzle depends on the row inside the piece only), and the piece's own
@@ -231,13 +235,42 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     // of the row that is asked for next (they stay at the chunk's last row)
     const unsigned char *krow = reinterpret_cast<const unsigned char *>((const T *)p.k + base0);
     const unsigned char *vrow = reinterpret_cast<const unsigned char *>((const T *)p.v + base0);
-    const unsigned char *arow = reinterpret_cast<const unsigned char *>(e.m2a + ((int64_t)b * p.S + s_begin) * np256);
+    // OWN: row s_begin of the mask itself, its entries of `mes` bytes (none: a row of something else, whose value is not used)
+    const unsigned mes = p.mask_kind == EVO_MASK_F32 ? 4 : p.mask_kind == EVO_MASK_BOOL ? 1 : 2;
+    const unsigned char *arow = OWN ? (const unsigned char *)(p.mask ? p.mask : p.q) + (p.mask ? ((int64_t)b * p.mask_stride_b + (int64_t)s_begin * p.mask_stride_s) * mes : 0)
+                                    : reinterpret_cast<const unsigned char *>(e.m2a + ((int64_t)b * p.S + s_begin) * np256);
+    const int64_t arow_step = OWN ? (p.mask ? p.mask_stride_s * mes : 0) : (int64_t)np256 * 16;
+    // An entry as it lies in memory (keys past the row: its last), by one load whatever its size: the four bytes, aligned, that it lies in.  (A branch over the kinds
+    // of mask here costs 20 registers, which are spilled.)  Its value: additive, not below the floor.
+    auto own_key = [&] {   // (formed where it is used: what follows from it would be kept in registers otherwise)
+        int key = (wave & 3) * 64 + lane;
+        asm volatile("" : "+v"(key));
+        return key;
+    };
+    auto mask_raw = [&](const unsigned char *row, int key) -> unsigned {
+        const unsigned low = (unsigned)(uintptr_t)row & 3u, o = (unsigned)min(key, p.N - 1) * mes + low;
+        return *reinterpret_cast<const unsigned *>(row - low + (o & ~3u));
+    };
+    auto mask_value = [&](const unsigned char *row, unsigned raw, int key) {
+        const unsigned x = raw >> (((((unsigned)(uintptr_t)row & 3u) + (unsigned)min(key, p.N - 1) * mes) & 3u) * 8u);
+        const float as16 = p.mask_kind == EVO_MASK_F16 ? (float)__builtin_bit_cast(f16_t, (unsigned short)x) : __uint_as_float(x << 16);
+        const float add = mes == 4 ? __uint_as_float(raw) : as16;
+        const float v = p.mask_kind == EVO_MASK_NONE ? 0.0f : p.mask_kind == EVO_MASK_BOOL ? ((x & 0xffu) ? 0.0f : -FLT_MAX) : add;
+        return key < p.N ? fmaxf(v, kMaskFloor) : kMaskFloor;
+    };
+    auto mask_chunk = [&](float v, int key) {   // (keys past the row carry the floor)
+        const uint2 a = pack_split3<T>(key < p.N ? fmaxf(v * kLog2e, kMaskFloor) : kMaskFloor);
+        const unsigned one = std::is_same<T, f16_t>::value ? 0x3C00u : 0x3F80u;
+        return u32x4{a.x, a.y | (one << 16), one | (one << 16), 0u};
+    };
+    int *const kept = reinterpret_cast<int *>(lds + gate_off + (GATED == 2 ? kGateBytes<D> : 0));   // [parity][piece]: some key of it is above the threshold
+    static_assert(R::I_ALL - 2 * R::I_K == 4 && 2 * R::I_K % 8 == 0 && IPW == R::I_K / 4 + 1, "piece m of the mask belongs to wave m, as its last one");
     int frow = 0;
     auto fetch_row = [&](int t) {   // moves the pointers to row min(t, nrows - 1); t grows by at most one per call
         if (t > frow && t < nrows) {
             krow += p.stride_s * 2;
             vrow += p.stride_s * 2;
-            arow += (int64_t)np256 * 16;
+            arow += arow_step;
             frow = t;
         }
     };
@@ -245,14 +278,16 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     // repeats a mask piece) so that the staging registers stay registers.
     auto fetch_piece = [&](int i) {
         const int n = wave + 8 * i;   // uniform
-        if (n < 2 * R::I_K) {
+        if (OWN && i == IPW - 1) {
+            mraw = mask_raw(arow, own_key());
+        } else if (n < 2 * R::I_K) {
             const bool isv = n >= R::I_K;
             const int m = isv ? n - R::I_K : n;
             const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)(isv ? vrow : krow), 0, kv_valid, 0x00020000);
-            stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)kv_voff, m * kv_piece, 0);
+            stg[OWN && i == IPW - 1 ? 0 : i] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)kv_voff, m * kv_piece, 0);
         } else {
             const int m = min(n, R::I_ALL - 1) - 2 * R::I_K;
-            stg[i] = *reinterpret_cast<const u32x4 *>(arow + m * 1024 + lane * 16);
+            stg[OWN && i == IPW - 1 ? 0 : i] = *reinterpret_cast<const u32x4 *>(arow + m * 1024 + lane * 16);
         }
     };
     auto fetch = [&](int t) {
@@ -265,8 +300,19 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
         if (t >= nrows) return;
         unsigned char *buf = lds + (t & 1) * R::BUF_BYTES + lds_piece0;
 #pragma unroll
-        for (int i = 0; i < IPW; ++i)
-            if (wave + 8 * i < R::I_ALL) *reinterpret_cast<u32x4 *>(buf + i * 8192) = stg[i];
+        for (int i = 0; i < IPW; ++i) {
+            const int n = wave + 8 * i;
+            if (OWN && i == IPW - 1) {
+                if (n >= R::I_ALL) continue;
+                const int key = own_key();
+                const float v = mask_value(arow, mraw, key);   // (the pointer stands at the row that was asked for last: this one)
+                *reinterpret_cast<u32x4 *>(buf + i * 8192) = mask_chunk(v, key);
+                const bool some = __any(v >= kShiftThreshold);
+                if (lane == 0) kept[(t & 1) * 4 + wave] = some;
+            } else if (n < R::I_ALL) {
+                *reinterpret_cast<u32x4 *>(buf + i * 8192) = stg[OWN && i == IPW - 1 ? 0 : i];
+            }
+        }
     };
     // this lane's half of its query row, straight from global memory
     v8 qraw[KSD], qnext[KSD];
@@ -307,10 +353,26 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     for (int t = 0; t < nrows; ++t) {
         const int s = s_begin + t;
         const unsigned pid = bh * (unsigned)p.S + s;
-        const bool dead = uniform_load(e.dead + b * p.S + s) != 0;
+        bool dead = false;
+        if (!OWN) dead = uniform_load(e.dead + b * p.S + s) != 0;
         EVO_TR(0);
         lds_barrier_f();   // the stage of this row is in LDS; everybody is done with the row before
         EVO_TR(1);
+        if (OWN && p.mask_kind != EVO_MASK_NONE) {
+            const int4 k = *reinterpret_cast<const int4 *>(kept + (t & 1) * 4);
+            dead = __builtin_amdgcn_readfirstlane(k.x | k.y | k.z | k.w) == 0;
+            if (__builtin_expect(dead, 0)) {   // (uniform over the workgroup) every key is masked: once more, less the row's largest entry
+                if (wave < 4) {
+                    const unsigned char *row = (const unsigned char *)p.mask + ((int64_t)b * p.mask_stride_b + (int64_t)s * p.mask_stride_s) * mes;
+                    float mx = kMaskFloor;
+                    for (int key = lane; key < p.N; key += 64) mx = fmaxf(mx, mask_value(row, mask_raw(row, key), key));
+                    mx = wave_max(mx);
+                    const int key = wave * 64 + lane;
+                    *reinterpret_cast<u32x4 *>(lds + (t & 1) * R::BUF_BYTES + R::OFF_A + wave * 1024 + lane * 16) = mask_chunk(mask_value(row, mask_raw(row, key), key) - mx, key);
+                }
+                lds_barrier_f();
+            }
+        }
         const unsigned char *buf = lds + (t & 1) * R::BUF_BYTES;
         if constexpr (GATED) {
             // The gate logits of the wave's own 32 query rows go to LDS by the load path itself (16 bytes per lane,
@@ -595,15 +657,16 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
 
 // ------------------------------------------------------------------ launcher
 
-template <typename T, int D, int BIASK, int GATED>
+template <typename T, int D, int BIASK, int GATED, bool OWN>
 static int fwdr_launch_g(const EvoAttnParams &p, const Extra &e0, hipStream_t st) {
     typedef FwdRingGeo<D> R;
     static PerDevice done{};
     int cus = 256;
-    auto kern = mfma_fwd_ring<T, D, BIASK, GATED>;
+    auto kern = mfma_fwd_ring<T, D, BIASK, GATED, OWN>;
+    constexpr int KEPT = OWN ? 32 : 0;
     constexpr int LDS_MOST = BIASK == 2 && R::LDS_BYTES < kBiasCopyBytes ? kBiasCopyBytes : R::LDS_BYTES;
-    if (const int rc = ensure_dynamic_lds((const void *)kern, LDS_MOST + (GATED == 2 ? kGateBytes<D> : 0), done, &cus)) return rc;
-    const int lds_bytes = (BIASK == 2 && !fwdr_rows16(p) ? LDS_MOST : R::LDS_BYTES) + (GATED == 2 ? kGateBytes<D> : 0);
+    if (const int rc = ensure_dynamic_lds((const void *)kern, LDS_MOST + (GATED == 2 ? kGateBytes<D> : 0) + KEPT, done, &cus)) return rc;
+    const int lds_bytes = (BIASK == 2 && !fwdr_rows16(p) ? LDS_MOST : R::LDS_BYTES) + (GATED == 2 ? kGateBytes<D> : 0) + KEPT;
     // one workgroup per CU: chunks of S rows such that (b, h, chunk) items about fill the chip
     Extra e = e0;
     const int bh = p.B * p.H;
@@ -617,8 +680,15 @@ static int fwdr_launch_g(const EvoAttnParams &p, const Extra &e0, hipStream_t st
 
 template <typename T, int D, int BIASK>
 static int fwdr_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
-    if (!p.gate) return fwdr_launch_g<T, D, BIASK, 0>(p, e, st);
-    return p.stride_h < p.stride_n ? fwdr_launch_g<T, D, BIASK, 2>(p, e, st) : fwdr_launch_g<T, D, BIASK, 1>(p, e, st);
+    auto with = [&](auto own) {
+        constexpr bool OWN = decltype(own)::value;
+        if (!p.gate) return fwdr_launch_g<T, D, BIASK, 0, OWN>(p, e, st);
+        return p.stride_h < p.stride_n ? fwdr_launch_g<T, D, BIASK, 2, OWN>(p, e, st) : fwdr_launch_g<T, D, BIASK, 1, OWN>(p, e, st);
+    };
+    if constexpr (BIASK != 1) {
+        if (!e.m2a) return with(std::true_type());   // (no mask was prepared)
+    }
+    return with(std::false_type());
 }
 
 template <typename T>

@@ -198,11 +198,11 @@ __global__ void __launch_bounds__(256) prep_kernel(EvoAttnParams p, Extra e, uns
     if (tid == 0) e.dead[row] = dead ? 1 : 0;
 }
 
-int launch_prep(const EvoAttnParams &p, const Extra &e, hipStream_t st, bool masks_only) {
+int launch_prep(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     const unsigned NT = (p.N + 31) / 32;
     // (no bias tiles where the kernels read the caller's tensor)
     const unsigned NS = (NT + kPrepStrip - 1) / kPrepStrip;
-    const unsigned nb = p.bias && !e.bias_direct && !masks_only ? (unsigned)e.bias_batches * p.H * NT * NS + 1u : 0u;
+    const unsigned nb = p.bias && !e.bias_direct ? (unsigned)e.bias_batches * p.H * NT * NS + 1u : 0u;
     const unsigned nm = (unsigned)(p.B * p.S);
     prep_kernel<<<nb + nm, 256, 0, st>>>(p, e, nb);
     hipError_t err = hipGetLastError();
