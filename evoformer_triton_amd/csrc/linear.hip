@@ -3,18 +3,20 @@
 //
 // Each is one launch (dW two: partial sums over slices of the rows, then their sum).  Through the library a product costs 18 to
 // 20 us of host time, which is what bounded the block (nine of them, 480 us per training step from the smallest shapes up to 32 768
-// rows), a stacked W a copy of the weights and of the bias, dW a sum of 16-bit partials.  The kernels themselves are bound by
-// memory and the wait for a stage (0.55 us from the request to the LDS, a stage's products 0.2 us) at these widths, K of 256 to
-// 1024.  Measured beside the library's, us: 32 768 rows, n = 1024, k = 256: y 34 (library 29), dx 27 (23), dW with bias gradient
-// 39 (32 and 11); n = k = 256: 11 (11.5), 11 (12), 24 (25 and 11); 1024 rows: 6 (5), 15 (8), 13 (10 and 6).  More and
-// smaller stages under way (five of 32) were no faster, nor all of a stage's operands read before its first product.
+// rows), a stacked W a copy of the weights and of the bias, dW a sum of 16-bit partials.  The kernels themselves are bound, at these
+// widths (K of 256 to 1024), by the path into LDS, which takes about 16 bytes per clock and CU: 32 KB per stage and workgroup, 0.75 us also where
+// a CU has one workgroup (four stages in a ring there: no change; operands or all of a stage through registers, one or two stages ahead: 2
+// to 8 % slower; a stage's operands all read before its first product: no change).  Measured beside the library's, us: 32 768 rows, n = 1024, k = 256: y
+// 28 (library 29), dx 25 (23), dW with bias gradient 42 (32 and 11); n = k = 256: 10 (11.5), 10 (12), 23 (25 and 11); 4096 rows, n = 1024: 8, 13, 19.
+// With the loads as a builtin, of which the compiler waits for the next stage's ahead of every transposing read, and outputs stored
+// 16 bytes of 64 rows at a time, those were 34, 32, 45; 11.5, 12, 24; 8, 18, 20 (a training step of the block, 32 768 rows of 256: 346, now 336).
 //
 // All three work in 128 x 128 tiles, four waves of 64 x 64 (2 x 2 accumulators of v_mfma_f32_32x32x16), 64 of the
 // contraction at a time, both operands brought by the load path into LDS (`global_load_lds_dwordx4`), the next stage on its way
 // while one is computed on: 64 KB, two workgroups per CU.  A 16-byte chunk of a staged row is stored at chunk ^ x(row)
 // (mfma_stream.hip), so that plain reads of 32 rows and transposing reads both touch all banks evenly.  Output tiles are formed
 // transposed (outputs along the accumulator's registers), with the 32 outputs of a tile dealt so that a lane ends up with 16
-// consecutive ones of a row: 32 bytes to store.  The contraction runs in ascending order, with one
+// consecutive ones of a row, and go to memory by way of LDS, 128 bytes of a row from eight lanes.  The contraction runs in ascending order, with one
 // rounding of the fp32 sum.
 //
 // Large products are the library's business: host.cpp has the lines and both sides.
@@ -34,10 +36,12 @@ __device__ __forceinline__ int swz128(int r) { return (r & 1) << 3 | ((r >> 1) &
 __device__ __forceinline__ int at128(int r, int c) { return r * 256 + ((c ^ swz128(r)) << 4); }
 __device__ __forceinline__ int swz64(int r) { return ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1); }
 
-__device__ __forceinline__ void lin_dma(const void *src, unsigned char *dst) {   // 16 bytes per lane, to dst + 16 * lane
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+// 16 bytes per lane, to dst (uniform) + 16 * lane, as an instruction that the compiler does not know: see dma16 in stream_common.h
+__device__ __forceinline__ void lin_dma(const void *src, unsigned char *dst) {
+    const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)dst;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(base), "v"(src) : "m0", "memory");
 }
-// this wave's loads have landed, everybody's have (and everybody is done with the stage before)
+// this wave's loads have landed, everybody's have, and everybody is done with the stage before
 __device__ __forceinline__ void lin_sync() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // output that row `r` of a 32-row accumulator tile holds: lane group g ends up with outputs 16g .. 16g+15 in register order
@@ -79,15 +83,8 @@ struct LinArgs {
     int M, N, K, bias_from;
 };
 
-// 16 consecutive outputs of row m from an accumulator tile
-template <typename T>
-__device__ __forceinline__ void lin_store(T *dst, const f32x16 &v) {
-    typename Mfma<T>::v8 o[2];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[i / 8][i % 8] = (T)v[i];
-    *reinterpret_cast<typename Mfma<T>::v8 *>(dst) = o[0];
-    *reinterpret_cast<typename Mfma<T>::v8 *>(dst + 8) = o[1];
-}
+// chunk c (8 outputs) of row r of a wave's 64 x 64 outputs on their way to memory
+__device__ __forceinline__ int lin_out_at(int r, int c) { return r * 128 + ((c ^ (r & 7)) << 4); }
 
 // FWD: y = x W^T + b, contraction over K, W rows dealt into LDS as outputs.  Else dx = dy W, contraction over N, W rows as
 // they come, read transposed.
@@ -153,14 +150,15 @@ __global__ void __launch_bounds__(256, 2) linear_rows(LinArgs<T> p) {
                 for (int u = 0; u < 2; ++u) acc[t][u] = Mfma<T>::mma(w[t], a[u], acc[t][u]);
         }
     }
+    // through LDS (the other stage's, which nobody reads any more), so that eight lanes store 128 bytes of a row
+    unsigned char *mine = lds[ns & 1] + wave * 8192;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const int o = o0 + wo + 32 * t + 16 * g;
-        if (o >= outs) continue;
         float b[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) b[i] = 0.0f;
-        if (FWD && p.bias && o >= p.bias_from) {
+        if (FWD && p.bias && o >= p.bias_from && o < outs) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const v8 v = ld8(p.bias + o - p.bias_from + 8 * h);
@@ -170,14 +168,21 @@ __global__ void __launch_bounds__(256, 2) linear_rows(LinArgs<T> p) {
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            const int m = m0 + wm + 32 * u + li;
-            if (m >= p.M) continue;
-            if (FWD) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) acc[t][u][i] += b[i];
+            for (int h = 0; h < 2; ++h) {
+                v8 v;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = (T)(FWD ? acc[t][u][8 * h + i] + b[8 * h + i] : acc[t][u][8 * h + i]);
+                *reinterpret_cast<v8 *>(mine + lin_out_at(32 * u + li, 4 * t + 2 * g + h)) = v;
             }
-            lin_store<T>(p.out + (int64_t)m * p.ldo + o, acc[t][u]);
         }
+    }
+    const int oc = o0 + wo + lane % 8 * 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int r = i * 8 + lane / 8, m = m0 + wm + r;
+        const v8 v = *reinterpret_cast<const v8 *>(mine + lin_out_at(r, lane % 8));
+        if (m < p.M && oc < outs) *reinterpret_cast<v8 *>(p.out + (int64_t)m * p.ldo + oc) = v;
     }
 }
 
