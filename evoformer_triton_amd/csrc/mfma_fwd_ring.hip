@@ -95,12 +95,12 @@ static __host__ __device__ inline bool fwdr_rows16(const EvoAttnParams &p) {
 }
 
 // BIASK: 0 no bias, 1 fp32 tiles (x log2(e), accumulator order) as C operands, 2 the caller's 16-bit rows through the identity
-// GATED: the output gate in the epilogue (kernels of their own: the ungated one carries none of their registers);
-// 1: the gate's logits asked for in the epilogue, 2: copied into LDS while the row is computed (see gate_dma below)
+// GATED: the output gate in the epilogue (kernels of their own: the ungated one carries none of their registers), its logits copied into LDS
+// while the row is computed
 // OWN: the mask as the caller has it (a forward without a backward, whose prep kernel would write nothing else): waves 0 to 3 read a row's entries with the
 // rest of its stage, 64 keys each, and make its columns of them where they write the stage; what they found kept lies behind the stages. A launch and
-// 16 bytes per key less: S = 128, N = 251, H = 8, D = 32, fp16, gated 35.0 -> 32.7 us with the launch before it (the kernel itself 35.0 -> 36.3, traced).
-template <typename T, int D, int BIASK, int GATED, bool OWN>
+// 16 bytes per key less: S = 128, N = 251, H = 8, D = 32, fp16, gated 35.0 -> 32.7 us with the launch before it (the waits of that time).
+template <typename T, int D, int BIASK, bool GATED, bool OWN>
 __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     typedef FwdRingGeo<D> R;
     constexpr int C = R::C;
@@ -121,7 +121,6 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     const int li = lane & 31, g = lane >> 5;
     const int NT = (p.N + 31) / 32;
     const int np256 = (p.N + 255) / 256 * 256;
-    const int nsteps = (p.N + 63) / 64;
     // Where the heads lie inside a token (the per-head layout) a cache line holds rows of several heads: the heads
     // of a chunk of S rows then run on one XCD, behind one L2 (consecutive workgroup ids go round the XCDs).
     const unsigned wid = p.stride_h < p.stride_n ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
@@ -130,6 +129,7 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     const int b = bh / p.H, h = bh % p.H;
     const int q0 = wave * 32;
     const bool qact = q0 < p.N;
+    const int nsteps = qact ? (p.N + 63) / 64 : 0;
     const int qrow = min(q0 + li, p.N - 1);
     const int64_t sn = p.stride_n;
     const float cscale = p.scale * kLog2e;
@@ -209,11 +209,6 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     // where the gated form's copy of the gate logits lies: behind the stages (and the bias rows' copy where that is used)
     constexpr int kStageMost = BIASK == 2 && R::LDS_BYTES < kBiasCopyBytes ? kBiasCopyBytes : R::LDS_BYTES;
     const int gate_off = BIASK == 2 && !fwdr_rows16(p) ? kStageMost : R::LDS_BYTES;
-    // Taken where a head's rows lie apart (heads inside a token: 8-byte pieces of 2 D bytes out of every row of
-    // the tensor; gated forward at S = 512, N = 256, H = 8, head dim 32: 144 against 157 us); where they lie one
-    // after the other the loads from the epilogue are as fast or faster (133 against 137 us).  Two kernels: one
-    // kernel with both ways spills more and runs the second case at 144 us.
-    constexpr bool gate_dma = GATED == 2;
 
     // ---- the stage of row s_begin + t lives in buffer t & 1.  It is a list of 1 KB pieces
     // (64 lanes x 16 bytes): K, V, then the mask columns; piece n belongs to wave n % 8.  Lane
@@ -263,7 +258,7 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
         const unsigned one = std::is_same<T, f16_t>::value ? 0x3C00u : 0x3F80u;
         return u32x4{a.x, a.y | (one << 16), one | (one << 16), 0u};
     };
-    int *const kept = reinterpret_cast<int *>(lds + gate_off + (GATED == 2 ? kGateBytes<D> : 0));   // [parity][piece]: some key of it is above the threshold
+    int *const kept = reinterpret_cast<int *>(lds + gate_off + (GATED ? kGateBytes<D> : 0));   // [parity][piece]: some key of it is above the threshold
     static_assert(R::I_ALL - 2 * R::I_K == 4 && 2 * R::I_K % 8 == 0 && IPW == R::I_K / 4 + 1, "piece m of the mask belongs to wave m, as its last one");
     int frow = 0;
     auto fetch_row = [&](int t) {   // moves the pointers to row min(t, nrows - 1); t grows by at most one per call
@@ -326,6 +321,16 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
         }
     };
 
+    // The compiler's wait for a row's queries, here and not where they are used: there requests of the next row's stage are under way in
+    // branches, which it cannot count, and it waited for these too, a memory latency per row.  With that and with no requests in a branch for waves
+    // without queries: S = 512, N = 256, H = 8, D = 32, bf16 91 -> 83 us, S = 128 30.2 -> 26.2.
+    auto arrived = [&](v8 (&x)[KSD]) {
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) asm volatile("" : "+v"(x[ks]));
+#endif
+    };
+
     fetch(0);
     fetch_q(0, qraw);
     if (BIASK == 2) {
@@ -349,6 +354,7 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
         }
     }
     stash(0);
+    arrived(qraw);
 
     for (int t = 0; t < nrows; ++t) {
         const int s = s_begin + t;
@@ -378,15 +384,17 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
             // The gate logits of the wave's own 32 query rows go to LDS by the load path itself (16 bytes per lane,
             // lane L to L * 16 of the wave's piece, no register in between) while the row is computed: asked for in
             // the epilogue they were waited for with nothing else to do, and asked for earlier into registers they
-            // cost registers the kernel does not have.  The wave alone writes and reads its piece.
-            if (qact && gate_dma) {
+            // cost registers the kernel does not have.  The wave alone writes and reads its piece.  The load is an instruction that the
+            // compiler does not know (dma16 in stream_common.h): it would wait for it, and for all that is younger, at the row's next transposing read.
+            // bf16, D = 32, H = 8, us, from the epilogue / so: S = 512, N = 256, heads inside a token 132 / 122 and one after the other 111 / 103; N = 200
+            // 101 / 89 and 95 / 87; D = 8, S = 1024, N = 256 150 / 143; D = 16, S = 512 86 / 83.
+            if (qact) {
 #pragma unroll
                 for (int i = 0; i < kGatePieces<D>; ++i) {
                     const int L = i * 64 + lane, row = min(L / C, 31), ch = L % C;
                     const T *src = (const T *)p.gate + base0 + (int64_t)t * p.stride_s + (int64_t)min(q0 + row, p.N - 1) * sn + ch * 8;
-                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
-                                                     (__attribute__((address_space(3))) void *)(lds + gate_off + wave * kGateWaveBytes<D> + i * 1024),
-                                                     16, 0, 0);
+                    const unsigned piece = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)(lds + gate_off + wave * kGateWaveBytes<D> + i * 1024);
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(piece), "v"(src) : "m0", "memory");
                 }
             }
         }
@@ -396,7 +404,7 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
         // carried in three 16-bit columns next to scores of order one)
         float m = 0.0f, mf = 0.0f, l = 0.0f;
         f32x16 oacc[DT];
-        if (qact) {
+        {   // (a wave without queries as well, with no steps: requests in a branch of its own would be waited for in the other, with all that is younger)
             v8 qf[KSD], qlo[KSD];
             const float cq = dead ? 0.0f : cscale;
             const float bscale = dead ? 0.0f : kLog2e;
@@ -605,15 +613,12 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
             }
 
         }
-        else {
-            fetch(t + 1);
-            fetch_q(t + 1, qnext);
-        }
         // The next stage goes into the other buffer, free since the barrier above.  This comes
         // before the row's own stores: what waits for the staged loads must not have the
         // stores in front of it (vector memory operations complete in order).
         EVO_TR(6);
         stash(t + 1);
+        arrived(qnext);
         EVO_TR(7);
         if (qact) {
             {   // the two lane groups hold the two halves of each query's sum
@@ -638,12 +643,8 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
                         for (int r = 0; r < 16; ++r) oacc[dt][r] *= inv;
                         // the wave's piece of the gate, in LDS since the top of the row (the compiler does not
                         // order the reads after that copy by itself)
-                        if (gate_dma) {
-                            if (dt == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                            gate_row_tile<T>((const T *)(lds + gate_off + wave * kGateWaveBytes<D>) + li * D, dt * 32, D, oacc[dt], g);
-                        } else {
-                            gate_row_tile<T>((const T *)p.gate + off, dt * 32, D, oacc[dt], g);
-                        }
+                        if (dt == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                        gate_row_tile<T>((const T *)(lds + gate_off + wave * kGateWaveBytes<D>) + li * D, dt * 32, D, oacc[dt], g);
                         store_row_tile<T>((T *)p.o_gated + off, dt * 32, D, oacc[dt], 1.0f, g);
                     }
                 }
@@ -657,7 +658,7 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
 
 // ------------------------------------------------------------------ launcher
 
-template <typename T, int D, int BIASK, int GATED, bool OWN>
+template <typename T, int D, int BIASK, bool GATED, bool OWN>
 static int fwdr_launch_g(const EvoAttnParams &p, const Extra &e0, hipStream_t st) {
     typedef FwdRingGeo<D> R;
     static PerDevice done{};
@@ -665,8 +666,8 @@ static int fwdr_launch_g(const EvoAttnParams &p, const Extra &e0, hipStream_t st
     auto kern = mfma_fwd_ring<T, D, BIASK, GATED, OWN>;
     constexpr int KEPT = OWN ? 32 : 0;
     constexpr int LDS_MOST = BIASK == 2 && R::LDS_BYTES < kBiasCopyBytes ? kBiasCopyBytes : R::LDS_BYTES;
-    if (const int rc = ensure_dynamic_lds((const void *)kern, LDS_MOST + (GATED == 2 ? kGateBytes<D> : 0) + KEPT, done, &cus)) return rc;
-    const int lds_bytes = (BIASK == 2 && !fwdr_rows16(p) ? LDS_MOST : R::LDS_BYTES) + (GATED == 2 ? kGateBytes<D> : 0) + KEPT;
+    if (const int rc = ensure_dynamic_lds((const void *)kern, LDS_MOST + (GATED ? kGateBytes<D> : 0) + KEPT, done, &cus)) return rc;
+    const int lds_bytes = (BIASK == 2 && !fwdr_rows16(p) ? LDS_MOST : R::LDS_BYTES) + (GATED ? kGateBytes<D> : 0) + KEPT;
     // one workgroup per CU: chunks of S rows such that (b, h, chunk) items about fill the chip
     Extra e = e0;
     const int bh = p.B * p.H;
@@ -682,8 +683,7 @@ template <typename T, int D, int BIASK>
 static int fwdr_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     auto with = [&](auto own) {
         constexpr bool OWN = decltype(own)::value;
-        if (!p.gate) return fwdr_launch_g<T, D, BIASK, 0, OWN>(p, e, st);
-        return p.stride_h < p.stride_n ? fwdr_launch_g<T, D, BIASK, 2, OWN>(p, e, st) : fwdr_launch_g<T, D, BIASK, 1, OWN>(p, e, st);
+        return p.gate ? fwdr_launch_g<T, D, BIASK, true, OWN>(p, e, st) : fwdr_launch_g<T, D, BIASK, false, OWN>(p, e, st);
     };
     if constexpr (BIASK != 1) {
         if (!e.m2a) return with(std::true_type());   // (no mask was prepared)
