@@ -11,7 +11,7 @@
 //     w / 4 and, of every block of keys, on the 32-key tiles (w % 4), (w % 4) + 4, ... (for
 //     rows of more than one key block: 32 query rows, wave w on the key tiles w, w + 8, ...);
 //   * K, V, the mask columns, and the slab's Q, dO and O rows of S row s+1 are requested
-//     (16 bytes per lane and load, 6 loads per wave at D = 32) before row s is computed out
+//     (16 bytes per lane and load, 6 loads per wave at D = 32) during row s - 1 or before row s is computed out
 //     of one LDS buffer, and written to the other buffer when that arithmetic is done; rows
 //     with more keys than one buffer holds go through it in blocks;
 //   * K^T fragments for dQ^T += K^T dS^T come from row-major K by transposing LDS reads
@@ -292,7 +292,7 @@ __global__ void __launch_bounds__(512) mfma_dq_ring(EvoAttnParams p, Extra e) {
         }
     };
     auto fetch = [&](Staged &stg, int t) { fetch_part(stg, t, 0, IPW); };
-    constexpr int SPLIT = IPW / 2;   // pieces asked for at the top of a row; the rest after its prologue
+    constexpr int SPLIT = IPW / 2;   // pieces written, and asked for again, between a row's tiles; the rest after them
     // What every wave of a query tile would otherwise redo in its prologue is done once, by
     // the wave that writes the piece: Q goes to LDS scaled by scale*log2(e) (where the scaled
     // Q is rounded once; with the rounding residue carried along it goes as given), zeroed
@@ -411,9 +411,11 @@ __global__ void __launch_bounds__(512) mfma_dq_ring(EvoAttnParams p, Extra e) {
     static_assert(NBLK == 1 || R::OWN_RED, "rows of several key blocks keep the partials out of the stage buffers");
     constexpr bool XBAR = NBLK == 1 && !R::TWO_RED;
     // With the partials out of the stage buffers, the buffer of the next stage is free from
-    // the stage barrier on: every wave asks for half of its pieces at the top of the row and
-    // writes them to LDS between its two tiles, while other waves compute; the other half it
-    // asks for after the row's prologue and writes after the tiles.
+    // the stage barrier on: every wave writes half of its pieces of the next stage to LDS between its two
+    // tiles, while other waves compute, and the other half after them, and asks for the same pieces of the
+    // stage after that as soon as their registers are free: a request has a whole row to arrive in.  Asked for and
+    // written within one row, in two halves, it had half of one, less than memory takes: S = 128, N = 256, H = 8, D = 32 with the gate's pass
+    // 56 -> 49 us, S = 512 146 -> 138; 8 to 12 registers, no spills.
     constexpr bool MID = NBLK == 1 && R::OWN_RED && TPW >= 2;
     // where the partials of the row that ended with stage `stage` lie; par: stage & 1 (one stage per row: the row's parity)
     auto red_of = [&](int stage, int par) {
@@ -425,6 +427,10 @@ __global__ void __launch_bounds__(512) mfma_dq_ring(EvoAttnParams p, Extra e) {
     fetch(sa, 0);
     fetch_advance(0);
     stash(sa, 0, 0);
+    if (MID) {
+        fetch(sa, 1);
+        fetch_advance(1);
+    }
 
     const uint2 one3 = ones3<T>();
     const uint2 zero3 = {0u, 0u};
@@ -458,13 +464,11 @@ __global__ void __launch_bounds__(512) mfma_dq_ring(EvoAttnParams p, Extra e) {
             EVO_TR(0);
             lds_barrier();   // stage t is in LDS; stage t-1 and the last reduction are done with
             EVO_TR(1);
-            // The CU's load path takes a stage's 48 requests (D = 32) at 16 clocks each: half of
-            // them go out now and half after the row's prologue rather than all queue up behind
-            // it (where the staging writes cannot be split, the waves take turns instead).  With
-            // few requests per wave there is nothing to gain.
+            // The CU's load path takes a stage's 48 requests (D = 32) at 16 clocks each: where the staging writes
+            // cannot be split, half of the waves send theirs now and half after the row's prologue rather
+            // than all queue up behind it.  With few requests per wave there is nothing to gain.
             const bool early = !(NBLK == 1 && IPW >= 4) || (wave & 1) == 0;
-            if (MID) fetch_part(nxt, t + 1, 0, SPLIT);
-            else if (early) fetch(nxt, t + 1);
+            if (!MID && early) fetch(nxt, t + 1);
             EVO_TR(2);
             const int par = PAR >= 0 ? PAR : (t & 1);
             buf = lds + par * R::BUF_BYTES;
@@ -515,9 +519,8 @@ __global__ void __launch_bounds__(512) mfma_dq_ring(EvoAttnParams p, Extra e) {
             }
 
             EVO_TR(4);
-            if (MID) fetch_part(nxt, t + 1, SPLIT, IPW);
-            else if (!early) fetch(nxt, t + 1);
-            fetch_advance(t + 1);
+            if (!MID && !early) fetch(nxt, t + 1);
+            if (!MID) fetch_advance(t + 1);
             EVO_TR(5);
             {
 #pragma unroll
@@ -536,6 +539,7 @@ __global__ void __launch_bounds__(512) mfma_dq_ring(EvoAttnParams p, Extra e) {
                     if (MID && jj == TPW - 1) {
                         EVO_TR(6);
                         stash_part(cur, t + 1, 0, SPLIT, par ^ 1);
+                        fetch_part(nxt, t + 2, 0, SPLIT);
                         EVO_TR(7);
                     }
                     // wave-uniform; no gradient goes through the scores of a row that a bool mask drops
@@ -612,8 +616,11 @@ __global__ void __launch_bounds__(512) mfma_dq_ring(EvoAttnParams p, Extra e) {
             }
             EVO_TR(8);
             // into the other buffer, free since the barrier above
-            if (MID) stash_part(cur, t + 1, SPLIT, IPW, par ^ 1);
-            else if (R::OWN_RED) stash(cur, t + 1, par ^ 1);
+            if (MID) {
+                stash_part(cur, t + 1, SPLIT, IPW, par ^ 1);
+                fetch_part(nxt, t + 2, SPLIT, IPW);
+                fetch_advance(t + 2);
+            } else if (R::OWN_RED) stash(cur, t + 1, par ^ 1);
         }
 
         // Partial dQ^T of this wave: lane = query li, register r = dim dt*32 + crow(r, g).  The
