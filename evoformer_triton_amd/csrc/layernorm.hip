@@ -10,6 +10,8 @@
 // stride.  The gradients of weight and bias are summed per lane over the rows a workgroup
 // visits, then over the workgroup in LDS, written as one partial per workgroup and added up
 // by a second small kernel in a fixed order: no atomics, bit-reproducible.
+#include <type_traits>
+
 #include "common.h"
 #include "bwd_common.h"
 #include "kernels.h"
@@ -18,8 +20,9 @@ namespace evo {
 
 constexpr int kLnThreads = 256;
 constexpr int kLnMaxPieces = 4;       // 16-byte pieces of a row per lane
-constexpr int kLnFwdBlocks = 4096;    // most workgroups of the forward
-constexpr int kLnBwdBlocks = 1024;    // most workgroups of the backward = partial sums of the weight and bias gradients
+// Most workgroups: of the forward (1024 to 4096 within 3 %), of the backward and of plain column sums = partial sums of the weight and bias gradients
+// (the backward with the partials' sum, 32 768 / 8192 / 98 304 rows of 256 bf16, 256 workgroups 18.1 / 11.9 / 52 us, 512 16.8 / 12.0 / 36, 1024 19.2 / 15.0 / 36).
+constexpr int kLnFwdBlocks = 2048, kLnBwdBlocks = 512, kLnSumBlocks = 1024;
 
 template <typename T>
 struct LnVec {
@@ -39,23 +42,50 @@ static LnShape ln_shape(int cols, int vec) {
     return {lpr, (n + lpr - 1) / lpr};
 }
 
-__device__ __forceinline__ float ln_group_sum(float s, int lpr) {
-    for (int o = lpr >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o);
+// The value of lane i ^ O, where the lanes of a group of LPR hold the same value with a period of 2 O lanes (sums made so far), or where O is 1 or 2.
+template <int O, int LPR>
+__device__ __forceinline__ float ln_other(float s) {
+    const int u = __float_as_int(s);
+    if constexpr (O == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(u, 0xB1, 0xF, 0xF, true));        // quad_perm 1 0 3 2
+    else if constexpr (O == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(u, 0x4E, 0xF, 0xF, true));   // quad_perm 2 3 0 1
+    else if constexpr (O == 4 && LPR >= 16) return __int_as_float(__builtin_amdgcn_mov_dpp(u, 0x124, 0xF, 0xF, true));   // row_ror 4
+    else if constexpr (O == 8) return __int_as_float(__builtin_amdgcn_mov_dpp(u, 0x128, 0xF, 0xF, true));  // row_ror 8
+    else return __shfl_xor(s, O);
+}
+
+// The sums over the LPR lanes of a group, by xor from half a group down: steps in the vector ALU instead of through LDS.
+template <int LPR>
+__device__ __forceinline__ float ln_group_sum(float s) {
+    if constexpr (LPR >= 64) {
+        const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+        s = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+    }
+    if constexpr (LPR >= 32) {
+        const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+        s = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+    }
+    if constexpr (LPR >= 16) s += ln_other<8, LPR>(s);
+    if constexpr (LPR >= 8) s += ln_other<4, LPR>(s);
+    if constexpr (LPR >= 4) s += ln_other<2, LPR>(s);
+    if constexpr (LPR >= 2) s += ln_other<1, LPR>(s);
     return s;
 }
 
-template <typename T, int PIECES>
+// Bound, where a row is long, by memory.  What a row costs beside its elements is kept low: lanes per row known when compiled, sums without LDS, a workgroup
+// over several rows with the next one's elements on their way.  32 768 rows of 256, bf16: 10.1 -> 8.5 us, backward with the
+// partials' sum 22.9 -> 16.8; 16 384 rows of 640 13.2 -> 10.6 and 27.7 -> 20.4.
+template <typename T, int PIECES, int LPR>
 __global__ void __launch_bounds__(kLnThreads)
 ln_fwd_kernel(const T *__restrict__ x, const T *__restrict__ gamma, const T *__restrict__ beta, T *__restrict__ y,
-              float *__restrict__ mean, float *__restrict__ rstd, int64_t rows, int cols, float eps, int lpr) {
-    constexpr int VEC = LnVec<T>::N;
+              float *__restrict__ mean, float *__restrict__ rstd, int64_t rows, int cols, float eps) {
+    constexpr int VEC = LnVec<T>::N, RPB = kLnThreads / LPR;
     typedef typename LnVec<T>::type vT;
-    const int tid = threadIdx.x, sub = tid % lpr, grp = tid / lpr, rpb = kLnThreads / lpr;
+    const int tid = threadIdx.x, sub = tid % LPR, grp = tid / LPR;
     const int npieces = cols / VEC;
     float g[PIECES][VEC], b[PIECES][VEC];
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-        const int pc = i * lpr + sub;
+        const int pc = i * LPR + sub;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
             g[i][e] = 1.0f;
@@ -75,29 +105,31 @@ ln_fwd_kernel(const T *__restrict__ x, const T *__restrict__ gamma, const T *__r
         }
     }
     const float inv = 1.0f / (float)cols;
-    for (int64_t row = (int64_t)blockIdx.x * rpb + grp; row < rows; row += (int64_t)gridDim.x * rpb) {
+    const int64_t step = (int64_t)gridDim.x * RPB;
+    vT raw[PIECES];
+    auto fetch = [&](int64_t row) {   // (lanes and rows past the end repeat the last)
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) raw[i] = *reinterpret_cast<const vT *>(x + min(row, rows - 1) * cols + min(i * LPR + sub, npieces - 1) * VEC);
+    };
+    fetch((int64_t)blockIdx.x * RPB + grp);
+    for (int64_t row = (int64_t)blockIdx.x * RPB + grp; row < rows; row += step) {
         float v[PIECES][VEC];
         float s = 0.0f;
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
-            const int pc = i * lpr + sub;
-            if (pc < npieces) {
-                const vT raw = *reinterpret_cast<const vT *>(x + row * cols + pc * VEC);
+            const bool in = i * LPR + sub < npieces;
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    v[i][e] = (float)raw[e];
-                    s += v[i][e];
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) v[i][e] = 0.0f;
+            for (int e = 0; e < VEC; ++e) {
+                v[i][e] = in ? (float)raw[i][e] : 0.0f;
+                s += v[i][e];
             }
         }
-        const float mu = ln_group_sum(s, lpr) * inv;
+        fetch(row + step);
+        const float mu = ln_group_sum<LPR>(s) * inv;
         float q = 0.0f;
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
-            if (i * lpr + sub < npieces) {
+            if (i * LPR + sub < npieces) {
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
                     const float d = v[i][e] - mu;
@@ -105,10 +137,10 @@ ln_fwd_kernel(const T *__restrict__ x, const T *__restrict__ gamma, const T *__r
                 }
             }
         }
-        const float r = 1.0f / sqrtf(ln_group_sum(q, lpr) * inv + eps);
+        const float r = 1.0f / sqrtf(ln_group_sum<LPR>(q) * inv + eps);
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
-            const int pc = i * lpr + sub;
+            const int pc = i * LPR + sub;
             if (pc < npieces) {
                 vT out;
 #pragma unroll
@@ -124,14 +156,14 @@ ln_fwd_kernel(const T *__restrict__ x, const T *__restrict__ gamma, const T *__r
 }
 
 // part: [gridDim.x][2][cols] fp32, the workgroup's sums of dy * xhat (weight) and of dy (bias)
-template <typename T, int PIECES>
+template <typename T, int PIECES, int LPR>
 __global__ void __launch_bounds__(kLnThreads)
 ln_bwd_kernel(const T *__restrict__ dy, const T *__restrict__ x, const T *__restrict__ gamma, const float *__restrict__ mean,
-              const float *__restrict__ rstd, T *__restrict__ dx, float *__restrict__ part, int64_t rows, int cols, int lpr) {
-    constexpr int VEC = LnVec<T>::N;
+              const float *__restrict__ rstd, T *__restrict__ dx, float *__restrict__ part, int64_t rows, int cols) {
+    constexpr int VEC = LnVec<T>::N, lpr = LPR, rpb = kLnThreads / LPR;
     typedef typename LnVec<T>::type vT;
     __shared__ float red[kLnThreads * PIECES * VEC];      // [rows per workgroup][lpr * PIECES * VEC]
-    const int tid = threadIdx.x, sub = tid % lpr, grp = tid / lpr, rpb = kLnThreads / lpr;
+    const int tid = threadIdx.x, sub = tid % lpr, grp = tid / lpr;
     const int npieces = cols / VEC;
     float g[PIECES][VEC], dg[PIECES][VEC], db[PIECES][VEC];
 #pragma unroll
@@ -150,20 +182,32 @@ ln_bwd_kernel(const T *__restrict__ dy, const T *__restrict__ x, const T *__rest
         }
     }
     const float inv = 1.0f / (float)cols;
-    for (int64_t row = (int64_t)blockIdx.x * rpb + grp; row < rows; row += (int64_t)gridDim.x * rpb) {
-        const float mu = mean[row], r = rstd[row];
+    const int64_t step = (int64_t)gridDim.x * rpb;
+    vT xr[PIECES], dr[PIECES];
+    float mu_next, r_next;
+    auto fetch = [&](int64_t row) {   // (lanes and rows past the end repeat the last)
+        row = min(row, rows - 1);
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int64_t at = row * cols + min(i * lpr + sub, npieces - 1) * VEC;
+            xr[i] = *reinterpret_cast<const vT *>(x + at);
+            dr[i] = *reinterpret_cast<const vT *>(dy + at);
+        }
+        mu_next = mean[row];
+        r_next = rstd[row];
+    };
+    fetch((int64_t)blockIdx.x * rpb + grp);
+    for (int64_t row = (int64_t)blockIdx.x * rpb + grp; row < rows; row += step) {
+        const float mu = mu_next, r = r_next;
         float xh[PIECES][VEC], gy[PIECES][VEC];
         float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
-            const int pc = i * lpr + sub;
-            if (pc < npieces) {
-                const vT xr = *reinterpret_cast<const vT *>(x + row * cols + pc * VEC);
-                const vT dr = *reinterpret_cast<const vT *>(dy + row * cols + pc * VEC);
+            if (i * lpr + sub < npieces) {
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
-                    const float d = (float)dr[e];
-                    xh[i][e] = ((float)xr[e] - mu) * r;
+                    const float d = (float)dr[i][e];
+                    xh[i][e] = ((float)xr[i][e] - mu) * r;
                     gy[i][e] = d * g[i][e];
                     s1 += gy[i][e];
                     s2 += gy[i][e] * xh[i][e];
@@ -175,8 +219,9 @@ ln_bwd_kernel(const T *__restrict__ dy, const T *__restrict__ x, const T *__rest
                 for (int e = 0; e < VEC; ++e) xh[i][e] = gy[i][e] = 0.0f;
             }
         }
+        fetch(row + step);
         if (dx) {   // uniform
-            const float c1 = ln_group_sum(s1, lpr) * inv, c2 = ln_group_sum(s2, lpr) * inv;
+            const float c1 = ln_group_sum<LPR>(s1) * inv, c2 = ln_group_sum<LPR>(s2) * inv;
 #pragma unroll
             for (int i = 0; i < PIECES; ++i) {
                 const int pc = i * lpr + sub;
@@ -305,17 +350,30 @@ static unsigned ln_blocks(int64_t rows, int lpr, int most) {
     return (unsigned)(want < most ? want : most);
 }
 
+// `go` with a row's pieces per lane and lanes as constants
+template <typename F>
+static void ln_forms(const LnShape &s, F go) {
+    typedef std::integral_constant<int, 1> One;
+    if (s.pieces > 2) go(std::integral_constant<int, 4>(), std::integral_constant<int, 64>());
+    else if (s.pieces == 2) go(std::integral_constant<int, 2>(), std::integral_constant<int, 64>());
+    else if (s.lpr == 64) go(One(), std::integral_constant<int, 64>());
+    else if (s.lpr == 32) go(One(), std::integral_constant<int, 32>());
+    else if (s.lpr == 16) go(One(), std::integral_constant<int, 16>());
+    else if (s.lpr == 8) go(One(), std::integral_constant<int, 8>());
+    else if (s.lpr == 4) go(One(), std::integral_constant<int, 4>());
+    else if (s.lpr == 2) go(One(), std::integral_constant<int, 2>());
+    else go(One(), One());
+}
+
 template <typename T>
 static int ln_fwd_launch(const void *x, const void *gamma, const void *beta, void *y, float *mean, float *rstd, int64_t rows,
                          int cols, float eps, hipStream_t st) {
     const LnShape s = ln_shape(cols, LnVec<T>::N);
     const unsigned grid = ln_blocks(rows, s.lpr, kLnFwdBlocks);
-    auto go = [&](auto kern) {
-        kern<<<grid, kLnThreads, 0, st>>>((const T *)x, (const T *)gamma, (const T *)beta, (T *)y, mean, rstd, rows, cols, eps, s.lpr);
-    };
-    if (s.pieces == 1) go(ln_fwd_kernel<T, 1>);
-    else if (s.pieces == 2) go(ln_fwd_kernel<T, 2>);
-    else go(ln_fwd_kernel<T, 4>);
+    ln_forms(s, [&](auto pieces, auto lpr) {
+        ln_fwd_kernel<T, decltype(pieces)::value, decltype(lpr)::value>
+            <<<grid, kLnThreads, 0, st>>>((const T *)x, (const T *)gamma, (const T *)beta, (T *)y, mean, rstd, rows, cols, eps);
+    });
     return hip_rc();
 }
 
@@ -325,14 +383,11 @@ static int ln_bwd_launch(const void *dy, const void *x, const void *gamma, const
     const LnShape s = ln_shape(cols, LnVec<T>::N);
     const unsigned grid = ln_blocks(rows, s.lpr, kLnBwdBlocks);
     const bool sums = dgamma || dbeta;
-    auto go = [&](auto kern) {
-        kern<<<grid, kLnThreads, 0, st>>>((const T *)dy, (const T *)x, (const T *)gamma, mean, rstd, (T *)dx, sums ? part : nullptr,
-                                          rows, cols, s.lpr);
-    };
     if (rows > 0) {
-        if (s.pieces == 1) go(ln_bwd_kernel<T, 1>);
-        else if (s.pieces == 2) go(ln_bwd_kernel<T, 2>);
-        else go(ln_bwd_kernel<T, 4>);
+        ln_forms(s, [&](auto pieces, auto lpr) {
+            ln_bwd_kernel<T, decltype(pieces)::value, decltype(lpr)::value>
+                <<<grid, kLnThreads, 0, st>>>((const T *)dy, (const T *)x, (const T *)gamma, mean, rstd, (T *)dx, sums ? part : nullptr, rows, cols);
+        });
         if (const int rc = hip_rc()) return rc;
     }
     if (sums) {   // (no rows: no partials, the sums are zero)
@@ -345,7 +400,7 @@ static int ln_bwd_launch(const void *dy, const void *x, const void *gamma, const
 template <typename T>
 static int colsum_launch(const void *a, void *out, float *part, int64_t rows, int cols, int64_t row_stride, hipStream_t st) {
     const LnShape s = ln_shape(cols, LnVec<T>::N);
-    const unsigned grid = ln_blocks(rows, s.lpr, kLnBwdBlocks);
+    const unsigned grid = ln_blocks(rows, s.lpr, kLnSumBlocks);
     auto go = [&](auto kern) { kern<<<grid, kLnThreads, 0, st>>>((const T *)a, part, rows, cols, row_stride, s.lpr); };
     if (rows > 0) {
         if (s.pieces == 1) go(colsum_kernel<T, 1>);
@@ -425,7 +480,7 @@ int evoattn_keep_mask(const float *keep, float *out, int64_t n, float inf, void 
 size_t evoattn_colsum_workspace_bytes(int64_t rows, int32_t cols, int32_t dtype) {
     using namespace evo;
     if (ln_check(rows, cols, dtype) != EVO_OK) return 0;
-    return (size_t)kLnBwdBlocks * (size_t)cols * sizeof(float);
+    return (size_t)kLnSumBlocks * (size_t)cols * sizeof(float);
 }
 
 int evoattn_colsum(const void *a, int64_t row_stride, void *out, void *workspace, size_t workspace_bytes, int64_t rows, int32_t cols,

@@ -1,0 +1,26 @@
+"""LayerNorm (csrc/layernorm.hip): every number of lanes per row it is built for, rows that do not fill their lanes, and several rows per group."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("rows,pieces", [(1, 1), (257, 2), (1025, 3), (300, 4), (9, 7), (50, 16), (70, 17), (16399, 32), (40, 64), (5, 65), (4, 200)])
+def test_rows_match_64_bits(gpu_device, rows, pieces, dtype):
+    from evoformer_triton_amd.block import _LayerNorm
+    cols = pieces * (16 // dtype.itemsize)   # a row's 16-byte pieces
+    g = torch.Generator().manual_seed(11)
+    x, dy = ((torch.randn((rows, cols), generator=g) + 0.3).to(dtype).to(gpu_device) for _ in range(2))
+    w, b = ((1.0 + 0.2 * torch.randn(cols, generator=g)).to(dtype).to(gpu_device) for _ in range(2))
+    leaves = [t.requires_grad_() for t in (x, w, b)]
+    y = _LayerNorm.apply(*leaves, 1e-5)
+    got = (y, *torch.autograd.grad(y, leaves, dy))
+    ref = [t.detach().double().requires_grad_() for t in leaves]
+    y64 = torch.nn.functional.layer_norm(ref[0], (cols,), ref[1], ref[2], 1e-5)
+    want = (y64, *torch.autograd.grad(y64, ref, dy.double()))
+    # one rounding of the result, and in fp32 the sums: rows + cols additions of 2^-24 at most, of terms up to the largest of |dy xhat|
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    for name, a, c in zip(("y", "dx", "dw", "db"), got, want):
+        terms = max(1.0, c.abs().max().item(), dy.abs().max().item() * (y64.abs().max().item() + 1.0) * (1.0 + rows ** 0.5 * (name in ("dw", "db"))))
+        assert (a.double() - c).abs().max().item() <= u * c.abs().max().item() + 2.0 ** -24 * (8 + (rows + cols) ** 0.5) * terms * (x.abs().max().item() + 1.0), name
