@@ -1169,7 +1169,7 @@ __global__ void __launch_bounds__(NW * 64, D == 32 ? 3 : 2) stream_dkdv(EvoAttnP
 // the memory-side cache, the one that waits for memory shares the chip with the one that computes, and a last round is
 // one instead of two.  dK/dV forms delta for itself.  The last problems come first: what the forward has left in the caches.
 // H = 32, fp32 bias, dQ and dK/dV one after the other / this, us: B = 1, N = 128 19.6 / 11.2, 256 28.7 / 16.8, 512 51 / 29, 1024 101 / 90; B = 3, N = 724
-// 220 / 171; B = 4, N = 1024 424 / 378 (4.8 TB/s past L2; problems in order the next call's forward takes 161 instead of 144;
+// 220 / 171; B = 4, N = 1024 424 / 378 (337 since dBias is stored 128 bytes of a row at a time, 5.3 TB/s past L2; problems in order the next call's forward takes 161 instead of 144;
 // sweeps turned so that both kinds meet in the same tile at the same time: no change); H = 8, B = 1, N = 2048 176 / 93.
 // Also without dBias (WRITE_DS) and with delta from the gate's pass (GIVEN), for rows that start or end within a group of four: as two launches, whose bias is read
 // entry by entry, these lost to the prepared tiles where there are few workgroups.

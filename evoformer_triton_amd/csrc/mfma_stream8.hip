@@ -341,7 +341,7 @@ int launch_stream_fwd8(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
 // stream_dbias (mfma_stream.hip) for this head dim: a workgroup has 128 queries x 128 keys of one (b, h) for a chunk of S rows, a wave 32
 // queries x 4 key tiles, whose sums and bias (fp32, log2 units: the first C of the score product) stay in registers.
 // The vector ALU is busy for .66 of the time, the matrix core .18, at two waves per SIMD.  S = 1024, N = 384, H = 8: mfma_dbias.hip's kernel 300 us (96 vector instructions per
-// tile and row), this 285 (34, and 75 per row to prepare the operands); two tiles per wave and three waves per SIMD 302; three tiles 475 (spills).
+// tile and row), this 285 (34, and 75 per row to prepare the operands) and 247 since no sum is copied around a tile's branch; two tiles per wave and three waves per SIMD 302; three tiles 475 (spills).
 struct Db8 {
     static constexpr int TPW = 4, KB = TPW * 32, QB = 128, ARR = KB * 16;   // K, V and the mask's columns
     static constexpr int KEYS = 3 * ARR;
