@@ -23,6 +23,8 @@ constexpr int kLnMaxPieces = 4;       // 16-byte pieces of a row per lane
 // Most workgroups: of the forward (1024 to 4096 within 3 %), of the backward and of plain column sums = partial sums of the weight and bias gradients
 // (the backward with the partials' sum, 32 768 / 8192 / 98 304 rows of 256 bf16, 256 workgroups 18.1 / 11.9 / 52 us, 512 16.8 / 12.0 / 36, 1024 19.2 / 15.0 / 36).
 constexpr int kLnFwdBlocks = 2048, kLnBwdBlocks = 512, kLnSumBlocks = 1024;
+constexpr int kLnPartials = 1024;   // that the workspace's size allows for: what callers of earlier builds were told, more than is written
+static_assert(kLnBwdBlocks <= kLnPartials && kLnSumBlocks <= kLnPartials, "a partial sum per workgroup");
 
 template <typename T>
 struct LnVec {
@@ -446,7 +448,7 @@ int evoattn_layernorm_fwd(const void *x, const void *gamma, const void *beta, vo
 size_t evoattn_layernorm_bwd_workspace_bytes(int64_t rows, int32_t cols, int32_t dtype) {
     using namespace evo;
     if (ln_check(rows, cols, dtype) != EVO_OK) return 0;
-    return (size_t)kLnBwdBlocks * 2 * (size_t)cols * sizeof(float);
+    return (size_t)kLnPartials * 2 * (size_t)cols * sizeof(float);
 }
 
 int evoattn_layernorm_bwd(const void *dy, const void *x, const void *gamma, const float *mean, const float *rstd, void *dx,
@@ -480,7 +482,7 @@ int evoattn_keep_mask(const float *keep, float *out, int64_t n, float inf, void 
 size_t evoattn_colsum_workspace_bytes(int64_t rows, int32_t cols, int32_t dtype) {
     using namespace evo;
     if (ln_check(rows, cols, dtype) != EVO_OK) return 0;
-    return (size_t)kLnSumBlocks * (size_t)cols * sizeof(float);
+    return (size_t)kLnPartials * (size_t)cols * sizeof(float);
 }
 
 int evoattn_colsum(const void *a, int64_t row_stride, void *out, void *workspace, size_t workspace_bytes, int64_t rows, int32_t cols,
