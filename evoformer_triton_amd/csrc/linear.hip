@@ -4,9 +4,10 @@
 // Each is one launch (dW two: partial sums over slices of the rows, then their sum).  Through the library a product costs 18 to
 // 20 us of host time, which is what bounded the block (nine of them, 480 us per training step from the smallest shapes up to 32 768
 // rows), a stacked W a copy of the weights and of the bias, dW a sum of 16-bit partials.  The kernels themselves are bound, at these
-// widths (K of 256 to 1024), by the path into LDS, which takes about 16 bytes per clock and CU: 32 KB per stage and workgroup, 0.75 us also where
-// a CU has one workgroup (four stages in a ring there: no change; operands or all of a stage through registers, one or two stages ahead: 2
-// to 8 % slower; a stage's operands all read before its first product: no change).  Measured beside the library's, us: 32 768 rows, n = 1024, k = 256: y
+// widths (K of 256 to 1024), by what a CU has under way from memory: 32 KB per stage and workgroup take 0.75 us, 18 bytes per clock, also where
+// a CU has one workgroup and however many stages are asked for (four in a ring: no change), where the same loads from L2 alone reach 55 bytes per clock in
+// any order of the chunks (operands or all of a stage through registers, one or two stages ahead: 2 to 8 % slower; a stage's operands all read
+// before its first product, tiles of 128 x 256: no change; a stage asked for between the products instead of ahead of them: 13 -> 15 to 19).  Measured beside the library's, us: 32 768 rows, n = 1024, k = 256: y
 // 28 (library 29), dx 25 (23), dW with bias gradient 42 (32 and 11); n = k = 256: 10 (11.5), 10 (12), 23 (25 and 11); 4096 rows, n = 1024: 8, 13, 19.
 // With the loads as a builtin, of which the compiler waits for the next stage's ahead of every transposing read, and outputs stored
 // 16 bytes of 64 rows at a time, those were 34, 32, 45; 11.5, 12, 24; 8, 18, 20 (a training step of the block, 32 768 rows of 256: 346, now 336).
