@@ -1270,13 +1270,16 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
             dma16(mrs, dst + R::OFF_A + wave * 1024, (wave * 64 + lane) * 16);
         }
     };
-    auto fetch_queries = [&](int s) {
+    auto fetch_query_pieces = [&](int s, int i0, int i1) __attribute__((always_inline)) {   // [i0, i1) of Q's and as many of dO's
         const __amdgpu_buffer_rsrc_t qrs = rows(p.q, s), grs = rows(p.dout, s);
 #pragma unroll
         for (int i = 0; i < R::QP; ++i) {
+            if (i < i0 || i >= i1) continue;
             dma16(qrs, own + i * 1024, qoff[i]);
             dma16(grs, own + 32 * G::ROW + i * 1024, qoff[i]);
         }
+    };
+    auto fetch_query_values = [&](int s) {
         const int64_t row0 = ((int64_t)bh * p.S + s) * p.N;
         lse_n = (p.lse + row0)[(unsigned)qrow];
         delta_n = (e.delta + row0)[(unsigned)qrow];
@@ -1285,7 +1288,8 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
         if (D != 64) dead_n = e.dead[b * p.S + s];
     };
     fetch_keys(s_begin);
-    fetch_queries(s_begin);
+    fetch_query_pieces(s_begin, 0, R::QP);
+    fetch_query_values(s_begin);
     for (int s = s_begin; s < s_end; ++s) {
         wait_loads();
         asm volatile("" : "+v"(lse_n), "+v"(delta_n), "+v"(dead_n));   // (the compiler's own wait for them: here, not behind the next keys' loads)
@@ -1304,7 +1308,10 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
 #pragma unroll
         for (int r = 0; r < 16; ++r) nd[r] = -delta_n;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (s + 1 < s_end) fetch_queries(s + 1);
+        if (s + 1 < s_end) {
+            if (!active || kill) fetch_query_pieces(s + 1, 0, R::QP);
+            fetch_query_values(s + 1);
+        }
 #pragma unroll
         for (int ks = 0; ks < KSD; ++ks) qf[ks] = scaled8<T>(qf[ks], dead ? 0.0f : cs);
         if (!active || kill) continue;
@@ -1315,10 +1322,18 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
             // not stored): 78 -> 74 us; at head dim 64 that is slower, 193 -> 205.
             if (D == 128 || j < tiles) {
                 f32x16 a, dp;
+                v8 k = *reinterpret_cast<const v8 *>(buf + G::at(32 * j + li, g)), v = *reinterpret_cast<const v8 *>(buf + R::OFF_V + G::at(32 * j + li, g));
 #pragma unroll
                 for (int ks = 0; ks < KSD; ++ks) {
-                    const int o = G::at(32 * j + li, 2 * ks + g);
-                    const v8 k = *reinterpret_cast<const v8 *>(buf + o);
+                    v8 k1, v1;
+                    if (ks + 1 < KSD) {
+                        const int o = G::at(32 * j + li, 2 * ks + 2 + g);
+                        k1 = *reinterpret_cast<const v8 *>(buf + o);
+                        v1 = *reinterpret_cast<const v8 *>(buf + R::OFF_V + o);
+                    }
+                    // The next row's queries a few pieces per step of the first tile: all at once they hold up the wave that asks, behind the CU's load
+                    // path.  S = 64, N = 512, H = 4, D = 128 (a wave per SIMD) 78 -> 74 us, S = N = 768, D = 32 468 -> 458, S = 200, N = 640, H = 5, D = 64 211 -> 209.
+                    if (j == 0 && s + 1 < s_end) fetch_query_pieces(s + 1, ks * R::QP / KSD, (ks + 1) * R::QP / KSD);
                     if (ks) {
                         a = Mfma<T>::mma(k, qf[ks], a);                                                        // log2 P^T
                     } else if (__builtin_expect(!dead, 1)) {
@@ -1329,7 +1344,11 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) stream_dbias(EvoAttnPara
                         for (int r = 0; r < 16; ++r) z[r] = 0.0f;
                         a = Mfma<T>::mma(k, qf[0], z);
                     }
-                    dp = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_V + o), gf[ks], ks ? dp : nd);         // dP^T - delta
+                    dp = Mfma<T>::mma(v, gf[ks], ks ? dp : nd);         // dP^T - delta
+                    if (ks + 1 < KSD) {
+                        k = k1;
+                        v = v1;
+                    }
                 }
                 a = Mfma<T>::mma(*reinterpret_cast<const v8 *>(buf + R::OFF_A + (32 * j + li) * 16), qf[KSD], a);
 #pragma unroll
