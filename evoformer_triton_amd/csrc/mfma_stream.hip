@@ -68,9 +68,7 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && 
     {
         const T *Q = (const T *)p.q + pr.base + (int64_t)qrow * p.stride_n;
 #pragma unroll
-        for (int ks = 0; ks < KSD; ++ks) qf[ks] = dead ? zero8<T>() : scaled8<T>(ld8(Q + ks * 16 + g * 8), c);
-        qf[KSD] = zero8<T>();
-        if (g == 0) qf[KSD][0] = qf[KSD][1] = qf[KSD][2] = (T)1.0f;
+        for (int ks = 0; ks < KSD; ++ks) qf[ks] = ld8(Q + ks * 16 + g * 8);
     }
     const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, dead, lane);
     // AHEAD: tiles whose bias is asked for together.  Where few S rows leave the caller's bias rows as the traffic (head dim 64) it is
@@ -81,6 +79,11 @@ __global__ void __launch_bounds__(256, D == 32 ? (BT == 0 ? 4 : 3) : D == 64 && 
     typename BiasStream<T, BT, false>::Tile ct[AHEAD];
 #pragma unroll
     for (int t = 0; t < AHEAD; ++t) bias.load(t, ct[t]);
+    asked_together<KSD>(qf);
+#pragma unroll
+    for (int ks = 0; ks < KSD; ++ks) qf[ks] = dead ? zero8<T>() : scaled8<T>(qf[ks], c);
+    qf[KSD] = zero8<T>();
+    if (g == 0) qf[KSD][0] = qf[KSD][1] = qf[KSD][2] = (T)1.0f;
 
     // m: the maximum the probabilities are relative to; mf: what the mask step subtracts inside the product (m, or 0 while
     // m is unknown or too large for three 16-bit columns): after the first step the scores arrive relative to m, and
@@ -323,14 +326,20 @@ __global__ void __launch_bounds__(256, 3) stream_fwd_pair(EvoAttnParams p, Extra
     for (int j = 0; j < 2; ++j) {
         const T *Q = (const T *)p.q + base[j] + (int64_t)qrow * p.stride_n;
 #pragma unroll
-        for (int ks = 0; ks < KSD; ++ks) qf[j][ks] = dead[j] ? zero8<T>() : scaled8<T>(ld8(Q + ks * 16 + g * 8), c);
-        qf[j][KSD] = zero8<T>();
-        if (g == 0) qf[j][KSD][0] = qf[j][KSD][1] = qf[j][KSD][2] = (T)1.0f;
+        for (int ks = 0; ks < KSD; ++ks) qf[j][ks] = ld8(Q + ks * 16 + g * 8);
     }
     const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, false, lane);
     typename BiasStream<T, BT, false>::Tile ct, c1;
     bias.load(0, ct);
     bias.load(1, c1);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        asked_together<KSD>(qf[j]);
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) qf[j][ks] = dead[j] ? zero8<T>() : scaled8<T>(qf[j][ks], c);
+        qf[j][KSD] = zero8<T>();
+        if (g == 0) qf[j][KSD][0] = qf[j][KSD][1] = qf[j][KSD][2] = (T)1.0f;
+    }
 
     float m[2] = {0.0f, 0.0f}, mf[2] = {0.0f, 0.0f}, l[2] = {0.0f, 0.0f};   // as in stream_fwd
     f32x16 o[2];
@@ -763,30 +772,18 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
 
     // this lane's half of the query row: Q (scaled), dO, and delta = <dO, O>
     const float cs = p.scale * kLog2e;
-    v8 qf[KS], gf[KS];
-    float dl = 0.0f;
-    {
-        const int64_t row = pr.base + (int64_t)qrow * p.stride_n + g * 8;
-        // (where delta is given, by the gate's pass, there may be no ungated O: dO is read in its place and the sum dropped)
-        const T *O = e.delta_given ? (const T *)p.dout : (const T *)p.o;
+    v8 qf[KS], gf[KS], of[KSD];
+    const int64_t row = pr.base + (int64_t)qrow * p.stride_n + g * 8;
+    // (where delta is given, by the gate's pass, there may be no ungated O: dO is read in its place and the sum dropped)
+    const T *O = e.delta_given ? (const T *)p.dout : (const T *)p.o;
 #pragma unroll
-        for (int ks = 0; ks < KSD; ++ks) {
-            qf[ks] = dead ? zero8<T>() : scaled8<T>(ld8((const T *)p.q + row + ks * 16), cs);
-            gf[ks] = ld8((const T *)p.dout + row + ks * 16);
-            dl = dot8<T>(gf[ks], ld8(O + row + ks * 16), dl);
-        }
-        dl += __shfl_xor(dl, 32);
-        if (e.delta_given) dl = e.delta[pr.row0 + qrow];
-        else if (g == 0 && q0 + li < p.N) e.delta[pr.row0 + q0 + li] = dl;
-        const float lse2 = p.lse[pr.row0 + qrow] * kLog2e;
-        const uint2 one3 = ones3<T>(), zero3 = {0u, 0u};
-        qf[KSD] = g == 0 ? aug8<T>(one3, pack_split3<T>(-lse2)) : zero8<T>();   // ones x mask, -lse x ones
-        gf[KSD] = g == 0 ? aug8<T>(pack_split3<T>(-dl), zero3) : zero8<T>();    // -delta x ones
-        if (kill) {   // no gradient through replaced scores: dP - delta is then zero, and dS with it
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) gf[ks] = zero8<T>();
-        }
+    for (int ks = 0; ks < KSD; ++ks) {
+        qf[ks] = ld8((const T *)p.q + row + ks * 16);
+        gf[ks] = ld8((const T *)p.dout + row + ks * 16);
+        of[ks] = ld8(O + row + ks * 16);
     }
+    float lse2 = p.lse[pr.row0 + qrow], dgiven = 0.0f;
+    if (e.delta_given) dgiven = e.delta[pr.row0 + qrow];
     const v8 vaug = aug8<T>(ones3<T>(), {0u, 0u});
     const BiasStream<T, BT, false> bias(p, e, pr, min(q0 >> 5, NT - 1), qrow, dead, lane);
     // PAIR: the caller's rows of a stage's two tiles are asked for together, and its dBias is stored together: 256 bytes of a row at a time (see
@@ -795,6 +792,28 @@ __device__ __forceinline__ void dq_rows(const EvoAttnParams &p, const Extra &e, 
     typename BiasStream<T, BT, false>::Tile ct, c1;
     bias.load(0, ct);
     if (PAIR) bias.load(1, c1);
+    {
+        asked_together<KSD>(qf);
+        asked_together<KSD>(gf);
+        asked_together<KSD>(of);
+        float dl = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks) {
+            qf[ks] = dead ? zero8<T>() : scaled8<T>(qf[ks], cs);
+            dl = dot8<T>(gf[ks], of[ks], dl);
+        }
+        dl += __shfl_xor(dl, 32);
+        if (e.delta_given) dl = dgiven;
+        else if (g == 0 && q0 + li < p.N) e.delta[pr.row0 + q0 + li] = dl;
+        lse2 *= kLog2e;
+        const uint2 one3 = ones3<T>(), zero3 = {0u, 0u};
+        qf[KSD] = g == 0 ? aug8<T>(one3, pack_split3<T>(-lse2)) : zero8<T>();   // ones x mask, -lse x ones
+        gf[KSD] = g == 0 ? aug8<T>(pack_split3<T>(-dl), zero3) : zero8<T>();    // -delta x ones
+        if (kill) {   // no gradient through replaced scores: dP - delta is then zero, and dS with it
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) gf[ks] = zero8<T>();
+        }
+    }
 
     // S = 1: this lane's row of dBias[b][h]
     const int64_t dsrow = (((int64_t)pr.b * p.H + pr.h) * p.N + qrow) * p.N;
@@ -1027,19 +1046,16 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
     fetch(0);
 
     // this wave's keys: K with the mask columns, V with ones against -delta
-    v8 kf[R::K_LDS ? 1 : KSD], vf[KSD], kaug, vaug;
+    v8 kf[KSD], vf[KSD], kaug, vaug;
+    uint2 mraw;
     {
         const int64_t row = pr.base + (int64_t)keyc * p.stride_n + g * 8;
 #pragma unroll
         for (int ks = 0; ks < KSD; ++ks) {
-            const v8 k = dead ? zero8<T>() : ld8((const T *)p.k + row + ks * 16);
-            if constexpr (R::K_LDS) *reinterpret_cast<v8 *>(lds + R::OFF_K + wave * 32 * G::ROW + G::at(li, 2 * ks + g)) = k;
-            else kf[ks] = k;
-            vf[ks] = kill ? zero8<T>() : ld8((const T *)p.v + row + ks * 16);   // (no gradient through replaced scores: dS is then zero)
+            kf[ks] = ld8((const T *)p.k + row + ks * 16);
+            vf[ks] = ld8((const T *)p.v + row + ks * 16);
         }
-        const uint2 mraw = e.m2[((int64_t)pr.b * p.S + pr.s) * (NT * 32) + min(key, NT * 32 - 1)];
-        kaug = g == 0 ? aug8<T>(mraw, one3) : zero8<T>();     // mask x ones, ones x -lse
-        vaug = g == 0 && !kill ? aug8<T>(one3, zero3) : zero8<T>();    // ones x -delta
+        mraw = e.m2[((int64_t)pr.b * p.S + pr.s) * (NT * 32) + min(key, NT * 32 - 1)];
     }
     const BiasStream<T, BT, true> bias(p, e, pr, min(key0 >> 5, NT - 1), keyc, dead, lane);
     // TWO: the bias of a stage's two tiles is asked for when the stage before begins, which its end waits for anyway, and nothing in a tile is waited
@@ -1050,6 +1066,16 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
     typename BiasStream<T, BT, true>::Tile ct, c1;
     bias.load(0, ct);
     if (TWO) bias.load(1, c1);
+    asked_together<KSD>(kf);
+    asked_together<KSD>(vf);
+#pragma unroll
+    for (int ks = 0; ks < KSD; ++ks) {
+        if (dead) kf[ks] = zero8<T>();
+        if (kill) vf[ks] = zero8<T>();   // (no gradient through replaced scores: dS is then zero)
+        if constexpr (R::K_LDS) *reinterpret_cast<v8 *>(lds + R::OFF_K + wave * 32 * G::ROW + G::at(li, 2 * ks + g)) = kf[ks];
+    }
+    kaug = g == 0 ? aug8<T>(mraw, one3) : zero8<T>();     // mask x ones, ones x -lse
+    vaug = g == 0 && !kill ? aug8<T>(one3, zero3) : zero8<T>();    // ones x -delta
     // (the dBias partials of the kernels before this one, summed on the way in where the caller asks for it)
     if (e.dbias_chunks > 0) sum_dbias_partials<NW * 64>(p, e, threadIdx.x);
 

@@ -40,6 +40,18 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, unsigned char *
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(base), "v"(off), "s"(rs) : "m0", "memory");
 }
 
+// The first N of `x`, loaded above, are wanted from here on: all are under way by now.  A load written where a condition decides about its use
+// (`dead ? zeros : scaled(load)`) is put into that branch, asked for there and waited for at once: KSD round trips to memory one after the other
+// ahead of a workgroup's first stage.  Training step, S = 64, N = 512, H = 4, D = 128 303 -> 294 us; S = 200, N = 640, H = 5, D = 64, fp32 bias 925 -> 921.
+template <int N, typename V, int M>
+__device__ __forceinline__ void asked_together(V (&x)[M]) {
+    static_assert(N <= M, "");
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i]));
+#endif
+}
+
 // Rows r0 .. r0 + ROWS - 1 of two arrays that share their strides, into LDS at `dst` and `dst` + ROWS rows: this wave's share
 // of the 1 KB pieces.  Rows at or beyond N repeat the last one (their keys carry the mask floor, their queries
 // probability zero).
