@@ -27,10 +27,17 @@
 
 namespace evo {
 
-// Two values as three bf16 pairs each whose sums are the values: every part is the rest rounded, so the third is exact (down to 2^-100; below, the
-// smaller parts run out of exponents).  A rest comes from one v_dot2c: x + (-1) part of this half + 0 part of the other.
+// Two values as three bf16 pairs each whose sums are the values: every part is the rest rounded, so the third is exact down to 2^-102; below, the
+// smaller parts run out of exponents.  A rest comes from one v_dot2c: x + (-1) part of this half + 0 part of the other.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 struct Parts2 { bf16x2 p[3]; };
+// So operands are split 2^24 times as large, every normal fp32 number whole, and results divided by it: of a dO or a V around 1e-36 nothing is lost, and dS,
+// formed of the two, is 2^48 times itself (split as they are, dQ of a dO around 1e-34 was 6 times, around 1e-36 600 times as far from 64 bits as by the fp32
+// instruction).  A score's two factors can't both be: the staged one is, the other one is split 2^24 times as small.  Where that takes a value of it
+// below 2^-102 (`begin`; the dBias kernel, which stages both, asks whether the larger one is so large that it could tell), `either_way` has the fp32 instruction.
+// Of the probabilities the forward's are relative to a sum in which one is 2^-8 at least; dV's, where a key may have only small ones, are split 2^24 times as
+// large as well.
+constexpr float kUp = 0x1p24f, kDown = 0x1p-24f, kUp2 = 0x1p48f, kDown2 = 0x1p-48f, kDown3 = 0x1p-72f, kWhole = 0x1p-102f, kMostStaged = 0x1p84f;
 __device__ __forceinline__ Parts2 parts2(float x, float y) {
     // (-1, 0) and (0, -1), kept from the compiler: it writes the first as the inline constant -1.0, which the instruction reads as (0, -1)
     unsigned lo = 0x0000bf80u, hi = 0xbf800000u;
@@ -87,6 +94,16 @@ struct Split {
             }
         return r;
     }
+    // Zero, or not a number where a value's parts are not all of it once it has been multiplied by `scale`: what the lane's sums begin with, so that they are
+    // not finite then (kept beside them, the answer cost the kernels with a bias 16 registers).
+    static __device__ __forceinline__ float begin(const f32x4 (&v)[NP], float scale) {
+        bool lacks = false;
+#pragma unroll
+        for (int j = 0; j < NP; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) lacks |= fabsf(v[j][i] * scale) < kWhole && v[j][i] != 0.0f;
+        return lacks && scale != 0.0f ? __int_as_float(0x7fc00000) : 0.0f;
+    }
     static __device__ __forceinline__ v8 operand(const unsigned char *tile, int part, int ks, int lane) {
         return *reinterpret_cast<const v8 *>(tile + part * PLANE + G::at(lane & 31, 2 * ks + (lane >> 5)));
     }
@@ -113,11 +130,11 @@ struct Split {
         }
         return c;
     }
-    static __device__ __forceinline__ void cols(const unsigned char *tile, int lane, const f32x16 &w, f32x16 (&acc)[DT]) {
+    static __device__ __forceinline__ void cols(const unsigned char *tile, int lane, const f32x16 &w, f32x16 (&acc)[DT], float scale = 1.0f) {
         v8 b[3][2];
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
-            const Parts2 a = parts2(w[r], w[r + 1]);
+            const Parts2 a = parts2(w[r] * scale, w[r + 1] * scale);
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
                 b[i][r >> 3][r & 7] = a.p[i][0];
@@ -162,12 +179,14 @@ __device__ __forceinline__ uint2 parts_of(float x) { return pack_split3<bf16_t>(
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_of(const void *base, const EvoAttnParams &p) {
     return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)(((unsigned)(p.N - 1) * (unsigned)p.stride_n + (unsigned)p.D) * 4u), 0x00020000);
 }
-// ROWS rows of two arrays through registers into LDS: `load` asks for rows r0 .. (r0 < N), `put` splits and writes them (the first array's times `scale`).
-template <int D, int THREADS, int ROWS = 32>
+// ROWS rows of two arrays through registers into LDS: `load` asks for rows r0 .. (r0 < N), `put` splits and writes them, times a factor for each array;
+// HUGE_TOO: `huge`, the lanes that have written a value of the first array of kMostStaged or more so far (lacking 2^-102 of the other factor they might show it).
+template <int D, int THREADS, int ROWS = 32, bool HUGE_TOO = false>
 struct SplitStage {
     typedef Split<D> E;
     static constexpr int PIECES = ROWS * D / 4, PER = (2 * PIECES + THREADS - 1) / THREADS;   // (of one array: a multiple of 64)
     f32x4 v[PER];
+    unsigned long long huge = 0;
     __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t a, __amdgpu_buffer_rsrc_t b, unsigned stride_n, int r0) {
         const int first = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);
 #pragma unroll
@@ -178,14 +197,15 @@ struct SplitStage {
                                                                                  (unsigned)r0 * stride_n * 4u, 0));
         }
     }
-    __device__ __forceinline__ void put(unsigned char *dst0, unsigned char *dst1, float scale = 1.0f) const {
+    __device__ __forceinline__ void put(unsigned char *dst0, unsigned char *dst1, float scale0, float scale1) {
         const int first = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const int k0 = first + i * THREADS, k = (k0 & (PIECES - 1)) + (threadIdx.x & 63);
             if (2 * PIECES % THREADS != 0 && k0 >= 2 * PIECES) break;
-            f32x4 x = v[i];
-            if (k0 < PIECES) x *= scale;
+            const f32x4 x = v[i] * (k0 < PIECES ? scale0 : scale1);
+            if (HUGE_TOO && k0 < PIECES)
+                huge |= __builtin_amdgcn_ballot_w64(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))) >= kMostStaged);
             E::put(k0 < PIECES ? dst0 : dst1, k / (D / 4), k % (D / 4) * 4, x);
         }
     }
@@ -271,8 +291,8 @@ template <int D, bool SPLITS> constexpr int shared_bytes() {
     else return DirectShared<D>::BYTES;
 }
 // A kernel forms its results in parts and, where some result of the workgroup is then not finite, once more on the fp32 instruction: parts of an infinite
-// operand, or of one beyond bf16's range, are not numbers, where the value itself may give a number, or an infinite result.
-// (`split` tells whether a result of this thread's is not finite.)
+// operand, or of one that is beyond bf16's range when 2^24 times as large, are not numbers, where the value itself may give a number, or an infinite result.
+// The same where a score's factors might not be whole (above).  (`split` tells whether this thread has found one or the other.)
 template <bool SPLITS, class A, class B>
 __device__ __forceinline__ void either_way(A split, B direct) {
     if constexpr (SPLITS) {
@@ -302,18 +322,19 @@ __device__ __forceinline__ bool split_body_fwd(const EvoAttnParams &p, unsigned 
     const float shift = uniform(block_shift<W>(p, pr.b, pr.s, sh.red()));
     const bool dead = shift != 0.0f;   // (of such a row the scores are the mask's)
     BiasAhead<BIAS, true> bias(p, pr.b, pr.h, rowc, dead, l);
-    const typename E::Frag q = E::frag(qv, dead ? 0.0f : p.scale * kLog2e);
+    const float qscale = dead ? 0.0f : p.scale * kLog2e * kDown;
+    const typename E::Frag q = E::frag(qv, qscale);
     const uint2 ones = ones3<bf16_t>(), none = make_uint2(0, 0);
     uint4 extra = g == 0 ? chunk_of(ones, none) : make_uint4(0, 0, 0, 0);   // against (mask, 1): adds mask - mf
     f32x16 acc[E::DT];
 #pragma unroll
     for (int t = 0; t < E::DT; ++t) acc[t] = zero16();
     // Maximum (log2 units), what of it the extra step subtracts (not where it is so low that a score would be lost beside it), sum.
-    float m = 0.0f, mf = 0.0f, sum = 0.0f;
+    float m = 0.0f, mf = 0.0f, sum = E::begin(qv, qscale);
     const int nt = (p.N + 31) / 32;
     for (int kt = 0; kt < nt; ++kt) {
         const int buf = kt & 1;
-        st.put(sh.tile(buf, 0), sh.tile(buf, 1));
+        st.put(sh.tile(buf, 0), sh.tile(buf, 1), kUp, kUp);
         if (threadIdx.x < 32) sh.chunk(buf)[threadIdx.x] = chunk_of(parts_of(mask_got(p, mk, kt * 32 + threadIdx.x, shift) * kLog2e), ones);
         __syncthreads();
         if (kt + 1 < nt) {
@@ -354,7 +375,7 @@ __device__ __forceinline__ bool split_body_fwd(const EvoAttnParams &p, unsigned 
     }
     sum = both_halves(sum);
     if (row < p.N) {
-        const float inv = 1.0f / sum;
+        const float inv = kDown / sum;
 #pragma unroll
         for (int t = 0; t < E::DT; ++t)
 #pragma unroll
@@ -422,16 +443,18 @@ __device__ __forceinline__ bool split_body_dq(const EvoAttnParams &p, float *del
     const bool dead = shift != 0.0f;
     BiasAhead<BIAS, true> bias(p, pr.b, pr.h, rowc, dead, l);
     const float ll = ds_blocked(p, shift) ? kMaskFloor : -lse * kLog2e;   // (no gradient through replaced scores: dS is zero)
-    const typename E::Frag q = E::frag(qv, dead ? 0.0f : p.scale * kLog2e), go = E::frag(gv, 1.0f);
+    const float qscale = dead ? 0.0f : p.scale * kLog2e * kDown;
+    const typename E::Frag q = E::frag(qv, qscale), go = E::frag(gv, kUp);
     const uint2 ones = ones3<bf16_t>(), none = make_uint2(0, 0);
-    const uint4 zero = make_uint4(0, 0, 0, 0), xs = g == 0 ? chunk_of(ones, parts_of(ll)) : zero, xd = g == 0 ? chunk_of(none, parts_of(-dl)) : zero;   // against (mask, 1)
+    const uint4 zero = make_uint4(0, 0, 0, 0), xs = g == 0 ? chunk_of(ones, parts_of(ll)) : zero, xd = g == 0 ? chunk_of(none, parts_of(-dl * kUp2)) : zero;   // against (mask, 1)
     f32x16 acc[E::DT];
 #pragma unroll
     for (int t = 0; t < E::DT; ++t) acc[t] = zero16();
+    acc[0][0] = E::begin(qv, qscale);
     const int nt = (p.N + 31) / 32;
     for (int kt = 0; kt < nt; ++kt) {
         const int buf = kt & 1;
-        st.put(sh.tile(buf, 0), sh.tile(buf, 1));
+        st.put(sh.tile(buf, 0), sh.tile(buf, 1), kUp, kUp);
         if (threadIdx.x < 32) sh.chunk(buf)[threadIdx.x] = chunk_of(parts_of(mask_got(p, mk, kt * 32 + threadIdx.x, shift) * kLog2e), ones);
         __syncthreads();
         if (kt + 1 < nt) {
@@ -458,7 +481,7 @@ __device__ __forceinline__ bool split_body_dq(const EvoAttnParams &p, float *del
                 if (c >= D) continue;
                 f32x4 o;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = acc[t][4 * j + i] * p.scale;
+                for (int i = 0; i < 4; ++i) o[i] = acc[t][4 * j + i] * (p.scale * kDown3);
                 put4((float *)p.dq + pr.base, off + c, o);
             }
     }
@@ -503,21 +526,22 @@ __device__ __forceinline__ bool split_body_dkdv(const EvoAttnParams &p, const Ex
     const bool dead = shift != 0.0f, blocked = ds_blocked(p, shift);   // (blocked: dP - delta is zero)
     BiasAhead<BIAS, false> bias(p, pr.b, pr.h, keyc, dead, l);
     const float mk = mask_entry(p, pr.b, pr.s, keyc, shift) * kLog2e;
-    const typename E::Frag k = E::frag(kv, dead ? 0.0f : 1.0f), v = E::frag(vv, blocked ? 0.0f : 1.0f);
+    const float kscale = dead ? 0.0f : kDown;
+    const typename E::Frag k = E::frag(kv, kscale), v = E::frag(vv, blocked ? 0.0f : kUp);
     const uint2 ones = ones3<bf16_t>(), none = make_uint2(0, 0);
     // against a row's chunk, (-LSE, -delta), and in the upper half's columns ones: LSE and mask; delta
     const uint4 zero = make_uint4(0, 0, 0, 0), xs = chunk_of(g == 0 ? ones : parts_of(mk), none), xd = g == 0 && !blocked ? chunk_of(none, ones) : zero;
     f32x16 dk[E::DT], dv[E::DT];
 #pragma unroll
     for (int t = 0; t < E::DT; ++t) dk[t] = dv[t] = zero16();
-    float dm = 0.0f;
+    float dm = E::begin(kv, kscale);
     const int nt = (p.N + 31) / 32;
     for (int qt = 0; qt < nt; ++qt) {
         const int buf = qt & 1;
-        st.put(sh.tile(buf, 0), sh.tile(buf, 1), p.scale * kLog2e);
+        st.put(sh.tile(buf, 0), sh.tile(buf, 1), p.scale * kLog2e * kUp, kUp);
         if (threadIdx.x < 32) {   // (rows at and beyond N: probability zero)
             const bool in = qt * 32 + (int)threadIdx.x < p.N;
-            sh.chunk(buf)[threadIdx.x] = chunk_of(parts_of(in ? -lse * kLog2e : kMaskFloor), parts_of(in ? -dl : 0.0f));
+            sh.chunk(buf)[threadIdx.x] = chunk_of(parts_of(in ? -lse * kLog2e : kMaskFloor), parts_of(in ? -dl * kUp2 : 0.0f));
         }
         __syncthreads();
         if (qt + 1 < nt) {
@@ -532,7 +556,7 @@ __device__ __forceinline__ bool split_body_dkdv(const EvoAttnParams &p, const Ex
         x = E::M::mma(row, as_operand(xs), x);
 #pragma unroll
         for (int r = 0; r < 16; ++r) x[r] = fast_exp2(x[r]);
-        E::cols(sh.tile(buf, 1), l, x, dv);
+        E::cols(sh.tile(buf, 1), l, x, dv, kUp);
         f32x16 ds = E::M::mma(row, as_operand(xd), E::rows(sh.tile(buf, 1), l, v));
 #pragma unroll
         for (int r = 0; r < 16; ++r) ds[r] *= x[r];
@@ -544,7 +568,7 @@ __device__ __forceinline__ bool split_body_dkdv(const EvoAttnParams &p, const Ex
     }
     dm = both_halves(dm);
     if (key < p.N) {
-        if (p.dmask && g == 0) e.dmask_part[pr.row0 + key] = dm;
+        if (p.dmask && g == 0) e.dmask_part[pr.row0 + key] = dm * kDown2;
 #pragma unroll
         for (int t = 0; t < E::DT; ++t)
 #pragma unroll
@@ -554,8 +578,8 @@ __device__ __forceinline__ bool split_body_dkdv(const EvoAttnParams &p, const Ex
                 f32x4 a, o;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    a[i] = dk[t][4 * j + i] * kLn2;   // (of Q as scaled)
-                    o[i] = dv[t][4 * j + i];
+                    a[i] = dk[t][4 * j + i] * (kLn2 * kDown3);   // (of Q as scaled)
+                    o[i] = dv[t][4 * j + i] * kDown2;
                 }
                 put4((float *)p.dk + pr.base, off + c, a);
                 put4((float *)p.dv + pr.base, off + c, o);
@@ -610,7 +634,8 @@ __device__ __forceinline__ bool split_body_dbias(const EvoAttnParams &p, const f
     const int s0 = ck * chunk, s1 = min(s0 + chunk, p.S);
     const uint2 ones = ones3<bf16_t>(), none = make_uint2(0, 0);
     if (threadIdx.x == 0) *one = chunk_of(ones, none);
-    SplitStage<D, TH, ROWS> sq, sk;
+    SplitStage<D, TH, ROWS> sq;
+    SplitStage<D, TH, ROWS, true> sk;
     float lse = 0.0f, dl = 0.0f, shift = 0.0f, next_shift = 0.0f;
     unsigned mk = 0;
     auto load = [&](int s) {
@@ -636,11 +661,11 @@ __device__ __forceinline__ bool split_body_dbias(const EvoAttnParams &p, const f
         __syncthreads();
         shift = next_shift;
         const bool dead = shift != 0.0f;
-        sq.put(lds, lds + ARRAY, dead ? 0.0f : p.scale * kLog2e);
-        sk.put(lds + 2 * ARRAY, lds + 3 * ARRAY);
+        sq.put(lds, lds + ARRAY, dead ? 0.0f : p.scale * kLog2e * kDown, kUp);
+        sk.put(lds + 2 * ARRAY, lds + 3 * ARRAY, kUp, kUp);
         {
             const int i = threadIdx.x;
-            if (i < ROWS) qchunk[i] = chunk_of(parts_of(q0 + i < p.N ? -lse * kLog2e : kMaskFloor), parts_of(q0 + i < p.N ? -dl : 0.0f));
+            if (i < ROWS) qchunk[i] = chunk_of(parts_of(q0 + i < p.N ? -lse * kLog2e : kMaskFloor), parts_of(q0 + i < p.N ? -dl * kUp2 : 0.0f));
             else if (i < 2 * ROWS) qchunk[i] = chunk_of(parts_of(mask_got(p, mk, k0 + i - ROWS, shift) * kLog2e), none);   // (the keys': behind the rows')
         }
         __syncthreads();
@@ -671,10 +696,10 @@ __device__ __forceinline__ bool split_body_dbias(const EvoAttnParams &p, const f
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int q = q0 + qw + crow(r, g);
-            if (q < p.N) out[(int64_t)q * p.N] = acc[kt][r];
+            if (q < p.N) out[(int64_t)q * p.N] = acc[kt][r] * kDown2;
         }
     }
-    return active && !(finite_check(acc) == 0.0f);
+    return sk.huge != 0 || (active && !(finite_check(acc) == 0.0f));
 }
 template <int D, int KT, bool SPLITS, bool BIAS>
 __global__ void __launch_bounds__((64 * DBiasGeo<D, KT>::W), D <= 64 ? 2 : 1) f32_dbias(EvoAttnParams p, const float *delta, const float *shift_tab, float *part, int chunk) {

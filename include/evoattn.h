@@ -40,7 +40,10 @@ enum {
     EVO_NONE = -1,
     EVO_BF16 = 0,
     EVO_F16  = 1,
-    EVO_F32  = 2   /* every product and sum in fp32, on the fp32 matrix instruction where rows lie in whole 16-byte pieces */
+    EVO_F32  = 2   /* operands, sums and results in fp32.  Where rows lie in whole 16-byte pieces the products are the fp32 matrix instruction's or, at head
+                      dim 32 and above 64 keys at 8, 16 and 64, sums of six products of three bf16 parts each: no further from 64 bits, over all of
+                      fp32's normal range.  Results that are then not finite, and scores of factors that no common scale holds whole, are
+                      formed once more by the fp32 instruction. */
 };
 
 /* row-mask encodings; mask is indexed [b][s][key], key contiguous */

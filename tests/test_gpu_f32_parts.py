@@ -40,6 +40,41 @@ def test_no_further_from_64_bits_than_fp32(gpu_device, shape):
         assert ours <= 3.0 * plain, (name, ours, plain)
 
 
+def _errors(got, x):
+    """Distance from 64 bits, ours and that of the formula in fp32, and the result itself: norms of each row of a tensor's last dimension."""
+    ref = {t: eager.attention_fwd_bwd(*(y.to(t) for y in x), compute_dtype=t) for t in (torch.float64, torch.float32)}
+    for name, y in got.items():
+        exact = ref[torch.float64][name]
+        yield name, (y.double() - exact).norm(dim=-1), (ref[torch.float32][name].double() - exact).norm(dim=-1), exact.norm(dim=-1)
+
+
+# A part below 2^-126 is not there, or has lost bits: operands, dS and results from where that begins to where an operand itself ends, and a score's factors
+# of which one is small and the other large.  The bound: 20 units of 2^-24, three times what such calls show at ordinary sizes (sums of up to 257 terms, each
+# rounded; P of scores of up to 5 in size).  Split as they are, the least of these cases is 24 units off, most are thousands.
+@pytest.mark.parametrize("small", [{"do": 1e-34}, {"do": 1e-36}, {"v": 1e-34}, {"v": 1e-36}, {"v": 1e-18, "do": 1e-18}, {"k": 1e-36}, {"q": 1e-36},
+                                   {"q": 1e30, "k": 1e-34}, {"q": 1e-34, "k": 1e30}, {"q": 1e-24, "k": 1e20}, {"q": 1e20, "k": 1e-24}],
+                         ids=lambda s: "-".join(f"{n}{x:g}" for n, x in s.items()))
+@pytest.mark.parametrize("shape", [(1, 3, 63, 2, 32), (1, 2, 96, 3, 8), (1, 3, 140, 2, 16), (1, 193, 257, 1, 32), (1, 3, 127, 2, 64)], ids=lambda s: "x".join(map(str, s)))
+def test_small_operands(gpu_device, shape, small):
+    x = list(_inputs(*shape))
+    for n, f in small.items():
+        x["q k v mask bias do".split().index(n)] *= f
+    for name, ours, _, size in _errors(_run(gpu_device, *x), x):
+        assert ours.norm() <= 20 * 2.0 ** -24 * size.norm(), (name, (ours.norm() / size.norm()).item())
+
+
+@pytest.mark.parametrize("shape", [(1, 3, 64, 2, 32), (1, 2, 96, 3, 8), (1, 3, 140, 2, 64)], ids=lambda s: "x".join(map(str, s)))
+def test_keys_of_small_probabilities(gpu_device, shape):
+    """dK and dV of keys that every query gives the same some 2^-115 to 2^-124: as far from 64 bits, relative to themselves, as the formula's."""
+    q, k, v, mask, bias, do = _inputs(*shape)
+    keys = torch.arange(0, shape[2], 5)
+    bias.zero_()[..., keys] = -torch.linspace(76.0, 82.0, len(keys))
+    x = (0.01 * q, k, v, torch.zeros_like(mask), bias, do)
+    for name, ours, plain, size in _errors(_run(gpu_device, *x), x):
+        if name in ("dK", "dV"):
+            assert (ours / size).max() <= 3.0 * (plain / size).max(), (name, (ours / size).max().item(), (plain / size).max().item())
+
+
 @pytest.mark.parametrize("what", ["v inf", "v -inf", "v large", "k inf", "q inf", "do inf", "do large"])
 @pytest.mark.parametrize("shape", [(1, 2, 40, 2, 32), (1, 3, 140, 1, 16), (1, 385, 130, 1, 32), (1, 2, 100, 2, 64)], ids=lambda s: "x".join(map(str, s)))
 def test_infinite_and_large_operands(gpu_device, shape, what):
