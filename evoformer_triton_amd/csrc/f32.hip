@@ -292,11 +292,12 @@ template <int D, bool SPLITS> constexpr int shared_bytes() {
 }
 // A kernel forms its results in parts and, where some result of the workgroup is then not finite, once more on the fp32 instruction: parts of an infinite
 // operand, or of one that is beyond bf16's range when 2^24 times as large, are not numbers, where the value itself may give a number, or an infinite result.
-// The same where a score's factors might not be whole (above).  (`split` tells whether this thread has found one or the other.)
+// The same where a score's factors might not be whole (above).  `split` returns, for the whole workgroup, whether one or the other is so, and then has written nothing
+// over an operand: these are read again, and O may lie where Q does, dQ where O does, dK and dV where K and V do (a workgroup writes only the rows it alone reads).
 template <bool SPLITS, class A, class B>
 __device__ __forceinline__ void either_way(A split, B direct) {
     if constexpr (SPLITS) {
-        if (!__syncthreads_or(split())) return;
+        if (!split()) return;
     }
     direct();
 }
@@ -374,6 +375,7 @@ __device__ __forceinline__ bool split_body_fwd(const EvoAttnParams &p, unsigned 
         E::cols(sh.tile(buf, 1), l, x, acc);
     }
     sum = both_halves(sum);
+    if (__syncthreads_or(active && !(fmaf(sum, 0.0f, finite_check(acc)) == 0.0f))) return true;
     if (row < p.N) {
         const float inv = kDown / sum;
 #pragma unroll
@@ -395,7 +397,7 @@ __device__ __forceinline__ bool split_body_fwd(const EvoAttnParams &p, unsigned 
             }
         if (g == 0) p.lse[pr.row0 + row] = fmaf(m, kLn2, logf(sum));
     }
-    return active && !(fmaf(sum, 0.0f, finite_check(acc)) == 0.0f);
+    return false;
 }
 template <int D, int W, bool BIAS>
 __global__ void __launch_bounds__(64 * W, D <= 32 && W >= 4 ? (W == 8 ? 4 : 3) : D <= 64 ? 2 : 1) f32_fwd(EvoAttnParams p, int vec) {
@@ -472,6 +474,7 @@ __device__ __forceinline__ bool split_body_dq(const EvoAttnParams &p, float *del
         for (int r = 0; r < 16; ++r) x[r] = fast_exp2(x[r]) * dp[r];
         E::cols(sh.tile(buf, 0), l, x, acc);
     }
+    if (__syncthreads_or(active && !(finite_check(acc) == 0.0f))) return true;
     if (row < p.N) {
 #pragma unroll
         for (int t = 0; t < E::DT; ++t)
@@ -485,7 +488,7 @@ __device__ __forceinline__ bool split_body_dq(const EvoAttnParams &p, float *del
                 put4((float *)p.dq + pr.base, off + c, o);
             }
     }
-    return active && !(finite_check(acc) == 0.0f);
+    return false;
 }
 template <int D, int W, bool BIAS>
 __global__ void __launch_bounds__(64 * W, D <= 64 ? 2 : 1) f32_dq(EvoAttnParams p, int vec, float *delta, float *shift_tab, int delta_given) {
@@ -567,6 +570,7 @@ __device__ __forceinline__ bool split_body_dkdv(const EvoAttnParams &p, const Ex
         E::cols(sh.tile(buf, 0), l, ds, dk);
     }
     dm = both_halves(dm);
+    if (__syncthreads_or(active && !(fmaf(dm, 0.0f, finite_check(dk) + finite_check(dv)) == 0.0f))) return true;
     if (key < p.N) {
         if (p.dmask && g == 0) e.dmask_part[pr.row0 + key] = dm * kDown2;
 #pragma unroll
@@ -585,7 +589,7 @@ __device__ __forceinline__ bool split_body_dkdv(const EvoAttnParams &p, const Ex
                 put4((float *)p.dv + pr.base, off + c, o);
             }
     }
-    return active && !(fmaf(dm, 0.0f, finite_check(dk) + finite_check(dv)) == 0.0f);
+    return false;
 }
 template <int D, int W, bool BIAS>
 __global__ void __launch_bounds__(64 * W, D <= 64 ? 2 : 1) f32_dkdv(EvoAttnParams p, Extra e) {
@@ -699,7 +703,7 @@ __device__ __forceinline__ bool split_body_dbias(const EvoAttnParams &p, const f
             if (q < p.N) out[(int64_t)q * p.N] = acc[kt][r] * kDown2;
         }
     }
-    return sk.huge != 0 || (active && !(finite_check(acc) == 0.0f));
+    return __syncthreads_or(sk.huge != 0 || (active && !(finite_check(acc) == 0.0f)));   // (dBias lies where nothing is read any more; asked before the stores, 16 to 38 registers more)
 }
 template <int D, int KT, bool SPLITS, bool BIAS>
 __global__ void __launch_bounds__((64 * DBiasGeo<D, KT>::W), D <= 64 ? 2 : 1) f32_dbias(EvoAttnParams p, const float *delta, const float *shift_tab, float *part, int chunk) {

@@ -95,3 +95,40 @@ def test_infinite_and_large_operands(gpu_device, shape, what):
             continue
         big = want[n][ok].abs().max().item()
         assert ((a - want[n])[ok].abs() <= 1e-5 * want[n][ok].abs().clamp_min(1.0) + 1e-6 * big).all(), n
+
+
+@pytest.mark.parametrize("shape", [(1, 3, 60, 2, 32), (1, 2, 140, 2, 16), (1, 200, 260, 1, 32), (1, 2, 100, 2, 64)], ids=lambda s: "x".join(map(str, s)))
+def test_results_in_the_place_of_operands(gpu_device, shape):
+    """O over Q, dQ over O, dK and dV over K and V, through the C ABI, with workgroups that form their results twice: the bits of results elsewhere."""
+    import ctypes
+    import evoformer_triton_amd.evoformer as E
+    from evoformer_triton_amd import _lib
+    B, S, N, H, D = shape
+    lib, dev = _lib.load(), gpu_device
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    q0, k0, v0, mask, bias, do0 = (t.to(dev) for t in _inputs(*shape))
+    v0[0, 1, 7, 0, 3] = 3.4e38        # beyond what bf16 holds, and O and dP with it
+    do0[0, 1, 5] *= 1e-30
+
+    def call(in_place):
+        q, k, v, do, q2 = (t.clone() for t in (q0, k0, v0, do0, q0))
+        mz, mk, mstr = E._prep_mask(mask, B, S, N, dev)
+        bz, bdt, bstr = E._prep_bias(bias, B, H, N, q.dtype, dev)
+        o, lse = q if in_place else torch.empty_like(q), torch.empty((B, H, S, N), device=dev)
+        p = E._params(q, k, v, mz, mk, mstr, bz, bdt, bstr, o, lse, "reference")
+        assert lib.evoattn_kernels(ctypes.byref(p), _lib.EVO_PASS_FWD) == b"f32_fwd"
+        prep = torch.empty(max(1, lib.evoattn_prep_bytes(ctypes.byref(p))), dtype=torch.uint8, device=dev)
+        p.prep, p.prep_bytes = prep.data_ptr(), prep.numel()
+        assert lib.evoattn_fwd(ctypes.byref(p), st) == 0
+        kept = o.clone()
+        p.q = q2.data_ptr()
+        dq, dk, dv = (o, k, v) if in_place else (torch.empty_like(q) for _ in range(3))
+        p.dout, p.dq, p.dk, p.dv = do.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
+        ws = torch.empty(lib.evoattn_bwd_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8, device=dev)
+        p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+        assert lib.evoattn_bwd(ctypes.byref(p), st) == 0
+        torch.cuda.synchronize()
+        return kept, dq, dk, dv
+
+    for name, a, b in zip(("O", "dQ", "dK", "dV"), call(False), call(True)):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32)), name
