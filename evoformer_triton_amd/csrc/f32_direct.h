@@ -437,13 +437,16 @@ __device__ __forceinline__ void direct_dkdv(const EvoAttnParams &p, const Extra 
 #pragma unroll
     for (int t = 0; t < E::DT; ++t) dk[t] = dv[t] = zero16();
     float dm = 0.0f;
-    float b[16] = {};   // of the next tile: asked for once this one's are used
+    float b[16] = {};
     auto ask_bias = [&](int qt) {
         if (!BIAS || dead) return;
 #pragma unroll
         for (int r = 0; r < 16; ++r) b[r] = at1(bmat, (unsigned)min(qt * 32 + crow(r, g), p.N - 1) * (unsigned)p.bias_stride_row + (unsigned)keyc);
     };
-    ask_bias(0);
+    // The bias a tile ahead, but not at head dim 64: its 16 registers are then live beside dP and dV, and 29 spilled (S = 512, N = 64, H = 8, a step: 367 us without,
+    // 393 with; N = 32 196 / 208.  D = 128, N = 64 811 with, 882 without, D = 16 131 / 138, D = 8 114 / 118).
+    constexpr bool AHEAD = D != 64;
+    if (AHEAD) ask_bias(0);
     const int nt = (p.N + 31) / 32;
     for (int qt = 0; qt < nt; ++qt) {
         const int buf = NB == 2 ? qt & 1 : 0;
@@ -455,6 +458,11 @@ __device__ __forceinline__ void direct_dkdv(const EvoAttnParams &p, const Extra 
             st.load(src, stride_n, (qt + 1) * 32, p.N);
             rv = row_ask((qt + 1) * 32);
         }
+        if (!AHEAD) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) b[r] = 0.0f;
+            ask_bias(qt);
+        }
         f32x16 x = zero16();
         E::rows(sh.tile(buf, 0), l, k, x);
 #pragma unroll
@@ -463,7 +471,8 @@ __device__ __forceinline__ void direct_dkdv(const EvoAttnParams &p, const Extra 
 #pragma unroll
             for (int i = 0; i < 4; ++i) x[4 * j + i] = exp_less(fmaf(x[4 * j + i], scale, BIAS ? b[4 * j + i] : 0.0f) + mk, lse[i]);
         }
-        if (qt + 1 < nt) ask_bias(qt + 1);
+        if (AHEAD && qt + 1 < nt) ask_bias(qt + 1);
+        if (!AHEAD) __builtin_amdgcn_sched_barrier(0);   // (the bias is used up before dP takes its registers)
         E::cols(sh.tile(buf, 1), l, x, dv);
         f32x16 ds = zero16();
         E::rows(sh.tile(buf, 1), l, v, ds);
