@@ -238,11 +238,14 @@ struct BiasAhead {
     __device__ __forceinline__ void ask(int t) {
         if (!BIAS) return;
         const int c = min(32 * t, (N - 1) & ~31);
-        if (c + 32 <= N) {   // (uniform)
+        // (uniform; a last tile's pieces that lie beyond the row are the row's last.  An entry at a time there: S = 64, N = 120 / 248, H = 8, D = 32 forward
+        // 18 / 42 us, so 14 / 35, where the fp32 instruction took 17 / 48.  As a branch of its own it is waited for: N = 250, S = 4, D = 8 15 -> 16 us.)
+        if (c + 32 <= N || (ROW && N % 4 == 0)) {
+            const unsigned last = at - 16u * g + 4u * (unsigned)(N - 4);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 if (ROW) {
-                    const f32x4 x = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, at + 32u * j, 4u * c, 0));
+                    const f32x4 x = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, min(at + 4u * c + 32u * j, last), 0, 0));
 #pragma unroll
                     for (int i = 0; i < 4; ++i) v[4 * j + i] = x[i];
                 } else {

@@ -132,3 +132,22 @@ def test_results_in_the_place_of_operands(gpu_device, shape):
 
     for name, a, b in zip(("O", "dQ", "dK", "dV"), call(False), call(True)):
         assert torch.equal(a.view(torch.int32), b.view(torch.int32)), name
+
+
+@pytest.mark.parametrize("shape", [(1, 3, 4, 2, 32), (1, 3, 40, 2, 32), (1, 2, 60, 1, 32), (2, 2, 72, 2, 8), (1, 2, 100, 2, 16), (1, 3, 130, 1, 32), (1, 130, 140, 3, 64), (1, 97, 252, 4, 32)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_a_bias_ends_where_its_rows_do(gpu_device, shape):
+    """Rows of a wider array that holds no numbers beside them: the bits of the same rows without a gap, also in the last tile's pieces of four."""
+    B, S, N, H, D = shape
+    q, k, v, mask, bias, do = (t.to(gpu_device) for t in _inputs(*shape))
+    wide = torch.full((B, 1, H, N, N + 4), float("nan"), device=gpu_device)
+    wide[..., :N] = bias
+    from evoformer_triton_amd import EvoformerAttention
+    out = []
+    for b in (bias, wide[..., :N]):
+        leaves = [t.detach().clone().requires_grad_() for t in (q, k, v)]
+        b = b.detach().requires_grad_()
+        o = EvoformerAttention.apply(*leaves, mask, b)
+        out.append((o, *torch.autograd.grad(o, (*leaves, b), do)))
+    for a, c in zip(*out):
+        assert torch.equal(a, c) and torch.isfinite(a).all()
