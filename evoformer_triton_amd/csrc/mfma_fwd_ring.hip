@@ -236,7 +236,7 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
                                     : reinterpret_cast<const unsigned char *>(e.m2a + ((int64_t)b * p.S + s_begin) * np256);
     const int64_t arow_step = OWN ? (p.mask ? p.mask_stride_s * mes : 0) : (int64_t)np256 * 16;
     // An entry as it lies in memory (keys past the row: its last), by one load whatever its size: the four bytes, aligned, that it lies in.  (A branch over the kinds
-    // of mask here costs 20 registers, which are spilled.)  Its value: additive, not below the floor.
+    // of mask here costs 20 registers, which are spilled.)  Its value: additive, not below the floor (which an entry that is no number has, too).
     auto own_key = [&] {   // (formed where it is used: what follows from it would be kept in registers otherwise)
         int key = (wave & 3) * 64 + lane;
         asm volatile("" : "+v"(key));
@@ -251,7 +251,9 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
         const float as16 = p.mask_kind == EVO_MASK_F16 ? (float)__builtin_bit_cast(f16_t, (unsigned short)x) : __uint_as_float(x << 16);
         const float add = mes == 4 ? __uint_as_float(raw) : as16;
         const float v = p.mask_kind == EVO_MASK_NONE ? 0.0f : p.mask_kind == EVO_MASK_BOOL ? ((x & 0xffu) ? 0.0f : -FLT_MAX) : add;
-        return key < p.N ? fmaxf(v, kMaskFloor) : kMaskFloor;
+        // (by its bits: this unit is compiled as if no NaN came, and the hardware's maximum keeps a signalling one)
+        const unsigned bits = __float_as_uint(v);
+        return key < p.N && bits <= __float_as_uint(kMaskFloor) && (int)bits <= 0x7f800000 ? v : kMaskFloor;
     };
     auto mask_chunk = [&](float v, int key) {   // (keys past the row carry the floor)
         const uint2 a = pack_split3<T>(key < p.N ? fmaxf(v * kLog2e, kMaskFloor) : kMaskFloor);

@@ -48,3 +48,31 @@ def test_same_bits_as_with_a_backward(gpu_device, case, bias):
     both = call(True)
     assert torch.isfinite(both).all()
     assert torch.equal(alone, both)
+
+
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("bits", [0x7FC0, 0xFFC0, 0x7F81, 0xFF81], ids=hex)
+@pytest.mark.parametrize("kind", ["f32", "bf16", "f16"])
+def test_a_mask_entry_that_is_no_number_drops_its_key(gpu_device, kind, bits, gated):
+    """Quiet and signalling, of either sign: the key gets the floor that a prepared mask gives it; a row of nothing else is a row with every key masked."""
+    from evoformer_triton_amd import evoformer_attention
+    g = torch.Generator().manual_seed(9)
+    q, k, v, gate = (torch.randn((1, 7, 150, 2, 32), generator=g).to(torch.float16 if kind == "f16" else torch.bfloat16).to(gpu_device) for _ in range(4))
+    m = torch.randn((1, 7, 1, 1, 150), generator=g)
+    drop = torch.rand(m.shape, generator=g) < 0.2
+    drop[..., 0] = False
+    drop[0, 3] = True
+    if kind == "f32":
+        none = torch.tensor(bits << 16 | 1, dtype=torch.int64).to(torch.int32)
+        m = torch.where(drop, none, m.view(torch.int32)).view(torch.float32)
+    elif kind == "bf16":
+        m = torch.where(drop, torch.tensor(bits).to(torch.int16), m.bfloat16().view(torch.int16)).view(torch.bfloat16)
+    else:
+        m = torch.where(drop, torch.tensor({0x7FC0: 0x7E00, 0xFFC0: 0xFE00, 0x7F81: 0x7C01, 0xFF81: 0xFC01}[bits]).to(torch.int16), m.half().view(torch.int16)).view(torch.float16)
+    assert torch.isnan(m[drop]).all()
+    m = m.to(gpu_device)
+    out = []
+    for grad in (False, True):
+        qq = q.clone().requires_grad_(grad)
+        out.append(evoformer_attention(qq, k, v, m, None, layout="ds4sci", **({"gate": gate} if gated else {})).detach())
+    assert torch.isfinite(out[1]).all() and torch.equal(*out)
