@@ -97,10 +97,11 @@ static __host__ __device__ inline bool fwdr_rows16(const EvoAttnParams &p) {
 // BIASK: 0 no bias, 1 fp32 tiles (x log2(e), accumulator order) as C operands, 2 the caller's 16-bit rows through the identity
 // GATED: the output gate in the epilogue (kernels of their own: the ungated one carries none of their registers), its logits copied into LDS
 // while the row is computed
-// OWN: the mask as the caller has it (a forward without a backward, whose prep kernel would write nothing else): waves 0 to 3 read a row's entries with the
+// OWN: 0, or, in a forward without a backward, whose prep kernel would write nothing but the mask's columns, the bytes of an entry of the mask, which it then reads as
+// the caller has it (a kernel for each size: see mask_raw): waves 0 to 3 read a row's entries with the
 // rest of its stage, 64 keys each, and make its columns of them where they write the stage; what they found kept lies behind the stages. A launch and
 // 16 bytes per key less: S = 128, N = 251, H = 8, D = 32, fp16, gated 35.0 -> 32.7 us with the launch before it (the waits of that time).
-template <typename T, int D, int BIASK, bool GATED, bool OWN>
+template <typename T, int D, int BIASK, bool GATED, int OWN>
 __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     typedef FwdRingGeo<D> R;
     constexpr int C = R::C;
@@ -230,27 +231,30 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
     // of the row that is asked for next (they stay at the chunk's last row)
     const unsigned char *krow = reinterpret_cast<const unsigned char *>((const T *)p.k + base0);
     const unsigned char *vrow = reinterpret_cast<const unsigned char *>((const T *)p.v + base0);
-    // OWN: row s_begin of the mask itself, its entries of `mes` bytes (none: a row of something else, whose value is not used)
-    const unsigned mes = p.mask_kind == EVO_MASK_F32 ? 4 : p.mask_kind == EVO_MASK_BOOL ? 1 : 2;
-    const unsigned char *arow = OWN ? (const unsigned char *)(p.mask ? p.mask : p.q) + (p.mask ? ((int64_t)b * p.mask_stride_b + (int64_t)s_begin * p.mask_stride_s) * mes : 0)
+    // OWN: row s_begin of the mask itself, its entries of OWN bytes (none: a row of something else, of which nothing is read)
+    const unsigned char *arow = OWN ? (const unsigned char *)(p.mask ? p.mask : p.q) + (p.mask ? ((int64_t)b * p.mask_stride_b + (int64_t)s_begin * p.mask_stride_s) * OWN : 0)
                                     : reinterpret_cast<const unsigned char *>(e.m2a + ((int64_t)b * p.S + s_begin) * np256);
-    const int64_t arow_step = OWN ? (p.mask ? p.mask_stride_s * mes : 0) : (int64_t)np256 * 16;
-    // An entry as it lies in memory (keys past the row: its last), by one load whatever its size: the four bytes, aligned, that it lies in.  (A branch over the kinds
-    // of mask here costs 20 registers, which are spilled.)  Its value: additive, not below the floor (which an entry that is no number has, too).
+    const int64_t arow_step = OWN ? (p.mask ? p.mask_stride_s * OWN : 0) : (int64_t)np256 * 16;
+    // An entry as it lies in memory (keys past the row, and without a mask: zero), by a load of its own size.  (Of any size in one kernel: by the aligned four bytes that
+    // it lies in, up to three beside the mask are read; by three loads of which two find nothing a gated forward is 2 to 4 % slower; a branch costs 20
+    // registers, which are spilled.)  Its value: additive, not below the floor (which an entry that is no number has, too).
     auto own_key = [&] {   // (formed where it is used: what follows from it would be kept in registers otherwise)
         int key = (wave & 3) * 64 + lane;
         asm volatile("" : "+v"(key));
         return key;
     };
+    const int mask_bytes = p.mask_kind == EVO_MASK_NONE ? 0 : p.N * OWN;
     auto mask_raw = [&](const unsigned char *row, int key) -> unsigned {
-        const unsigned low = (unsigned)(uintptr_t)row & 3u, o = (unsigned)min(key, p.N - 1) * mes + low;
-        return *reinterpret_cast<const unsigned *>(row - low + (o & ~3u));
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)row, 0, mask_bytes, 0x00020000);
+        if constexpr (OWN == 1) return __builtin_amdgcn_raw_buffer_load_b8(rs, key, 0, 0);
+        else if constexpr (OWN == 2) return __builtin_amdgcn_raw_buffer_load_b16(rs, key * 2, 0, 0);
+        else return __builtin_amdgcn_raw_buffer_load_b32(rs, key * 4, 0, 0);
     };
-    auto mask_value = [&](const unsigned char *row, unsigned raw, int key) {
-        const unsigned x = raw >> (((((unsigned)(uintptr_t)row & 3u) + (unsigned)min(key, p.N - 1) * mes) & 3u) * 8u);
-        const float as16 = p.mask_kind == EVO_MASK_F16 ? (float)__builtin_bit_cast(f16_t, (unsigned short)x) : __uint_as_float(x << 16);
-        const float add = mes == 4 ? __uint_as_float(raw) : as16;
-        const float v = p.mask_kind == EVO_MASK_NONE ? 0.0f : p.mask_kind == EVO_MASK_BOOL ? ((x & 0xffu) ? 0.0f : -FLT_MAX) : add;
+    auto mask_value = [&](unsigned raw, int key) {
+        float v;
+        if constexpr (OWN == 1) v = p.mask_kind == EVO_MASK_NONE || raw ? 0.0f : -FLT_MAX;
+        else if constexpr (OWN == 2) v = p.mask_kind == EVO_MASK_F16 ? (float)__builtin_bit_cast(f16_t, (unsigned short)raw) : __uint_as_float(raw << 16);
+        else v = __uint_as_float(raw);
         // (by its bits: this unit is compiled as if no NaN came, and the hardware's maximum keeps a signalling one)
         const unsigned bits = __float_as_uint(v);
         return key < p.N && bits <= __float_as_uint(kMaskFloor) && (int)bits <= 0x7f800000 ? v : kMaskFloor;
@@ -302,7 +306,7 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
             if (OWN && i == IPW - 1) {
                 if (n >= R::I_ALL) continue;
                 const int key = own_key();
-                const float v = mask_value(arow, mraw, key);   // (the pointer stands at the row that was asked for last: this one)
+                const float v = mask_value(mraw, key);
                 *reinterpret_cast<u32x4 *>(buf + i * 8192) = mask_chunk(v, key);
                 const bool some = __any(v >= kShiftThreshold);
                 if (lane == 0) kept[(t & 1) * 4 + wave] = some;
@@ -371,12 +375,12 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
             dead = __builtin_amdgcn_readfirstlane(k.x | k.y | k.z | k.w) == 0;
             if (__builtin_expect(dead, 0)) {   // (uniform over the workgroup) every key is masked: once more, less the row's largest entry
                 if (wave < 4) {
-                    const unsigned char *row = (const unsigned char *)p.mask + ((int64_t)b * p.mask_stride_b + (int64_t)s * p.mask_stride_s) * mes;
+                    const unsigned char *row = (const unsigned char *)p.mask + ((int64_t)b * p.mask_stride_b + (int64_t)s * p.mask_stride_s) * OWN;
                     float mx = kMaskFloor;
-                    for (int key = lane; key < p.N; key += 64) mx = fmaxf(mx, mask_value(row, mask_raw(row, key), key));
+                    for (int key = lane; key < p.N; key += 64) mx = fmaxf(mx, mask_value(mask_raw(row, key), key));
                     mx = wave_max(mx);
                     const int key = wave * 64 + lane;
-                    *reinterpret_cast<u32x4 *>(lds + (t & 1) * R::BUF_BYTES + R::OFF_A + wave * 1024 + lane * 16) = mask_chunk(mask_value(row, mask_raw(row, key), key) - mx, key);
+                    *reinterpret_cast<u32x4 *>(lds + (t & 1) * R::BUF_BYTES + R::OFF_A + wave * 1024 + lane * 16) = mask_chunk(mask_value(mask_raw(row, key), key) - mx, key);
                 }
                 lds_barrier_f();
             }
@@ -660,7 +664,7 @@ __global__ void __launch_bounds__(512) mfma_fwd_ring(EvoAttnParams p, Extra e) {
 
 // ------------------------------------------------------------------ launcher
 
-template <typename T, int D, int BIASK, bool GATED, bool OWN>
+template <typename T, int D, int BIASK, bool GATED, int OWN>
 static int fwdr_launch_g(const EvoAttnParams &p, const Extra &e0, hipStream_t st) {
     typedef FwdRingGeo<D> R;
     static PerDevice done{};
@@ -684,13 +688,17 @@ static int fwdr_launch_g(const EvoAttnParams &p, const Extra &e0, hipStream_t st
 template <typename T, int D, int BIASK>
 static int fwdr_launch(const EvoAttnParams &p, const Extra &e, hipStream_t st) {
     auto with = [&](auto own) {
-        constexpr bool OWN = decltype(own)::value;
+        constexpr int OWN = decltype(own)::value;
         return p.gate ? fwdr_launch_g<T, D, BIASK, true, OWN>(p, e, st) : fwdr_launch_g<T, D, BIASK, false, OWN>(p, e, st);
     };
     if constexpr (BIASK != 1) {
-        if (!e.m2a) return with(std::true_type());   // (no mask was prepared)
+        if (!e.m2a) {   // (no mask was prepared)
+            if (p.mask_kind == EVO_MASK_F32) return with(std::integral_constant<int, 4>());
+            if (p.mask_kind == EVO_MASK_BF16 || p.mask_kind == EVO_MASK_F16) return with(std::integral_constant<int, 2>());
+            return with(std::integral_constant<int, 1>());
+        }
     }
-    return with(std::false_type());
+    return with(std::integral_constant<int, 0>());
 }
 
 template <typename T>

@@ -46,6 +46,20 @@ def test_a_split_forwards_fetch_follows_the_reads_of_its_buffer(head_dim, tmp_pa
     assert seen >= 6      # two dtypes, three kinds of bias
 
 
+@pytest.mark.parametrize("head_dim", [8, 16, 32])
+def test_a_mask_is_read_by_its_own_entries(head_dim, tmp_path):
+    """The forward that reads a mask as given: by loads of an entry's size, of a resource that ends with the row, and none of the four bytes around an entry."""
+    text = _assembly("mfma_fwd_ring.hip", [f"-DEVO_D={head_dim}"], tmp_path)
+    seen = 0
+    for name, lines in _functions(text, "mfma_fwd_ring"):
+        size = int(re.search(r"ELi(\d)EEEv", name).group(1))
+        loads = re.findall(r"^\s+((?:global|buffer)_load_(?:ubyte|ushort|dword))\b", "\n".join(lines), re.M)
+        assert "global_load_dword" not in loads, name
+        assert {x for x in loads if x.startswith("buffer")} == {0: set(), 1: {"buffer_load_ubyte"}, 2: {"buffer_load_ushort"}, 4: {"buffer_load_dword"}}[size], name
+        seen += size != 0
+    assert seen == 24      # two dtypes, bias or none, gate or none, three sizes of entry
+
+
 def test_a_load_into_lds_declares_what_it_changes():
     """Written as an instruction that the compiler does not know, it sets m0 and writes LDS."""
     seen = 0
