@@ -22,9 +22,12 @@ constexpr int kLnThreads = 256;
 constexpr int kLnMaxPieces = 4;       // 16-byte pieces of a row per lane
 // Most workgroups: of the forward (1024 to 4096 within 3 %), of the backward and of plain column sums = partial sums of the weight and bias gradients
 // (the backward with the partials' sum, 32 768 / 8192 / 98 304 rows of 256 bf16, 256 workgroups 18.1 / 11.9 / 52 us, 512 16.8 / 12.0 / 36, 1024 19.2 / 15.0 / 36).
-constexpr int kLnFwdBlocks = 2048, kLnBwdBlocks = 512, kLnSumBlocks = 1024;
+// In fp32 1024, too: of 512 each adds up twice as many rows one after the other, and where there are many the result was 1.1 times as far from 64 bits (98 304 rows
+// of 256; 3 000 000 of 4: 1.24; in 16 bits the result's own rounding is a thousand times that).
+constexpr int kLnFwdBlocks = 2048, kLnSumBlocks = 1024;
+template <typename T> constexpr int kLnBwdBlocks = sizeof(T) == 4 ? 1024 : 512;
 constexpr int kLnPartials = 1024;   // that the workspace's size allows for: what callers of earlier builds were told, more than is written
-static_assert(kLnBwdBlocks <= kLnPartials && kLnSumBlocks <= kLnPartials, "a partial sum per workgroup");
+static_assert(kLnBwdBlocks<float> <= kLnPartials && kLnSumBlocks <= kLnPartials, "a partial sum per workgroup");
 
 template <typename T>
 struct LnVec {
@@ -383,7 +386,7 @@ template <typename T>
 static int ln_bwd_launch(const void *dy, const void *x, const void *gamma, const float *mean, const float *rstd, void *dx,
                          void *dgamma, void *dbeta, float *part, int64_t rows, int cols, hipStream_t st) {
     const LnShape s = ln_shape(cols, LnVec<T>::N);
-    const unsigned grid = ln_blocks(rows, s.lpr, kLnBwdBlocks);
+    const unsigned grid = ln_blocks(rows, s.lpr, kLnBwdBlocks<T>);
     const bool sums = dgamma || dbeta;
     if (rows > 0) {
         ln_forms(s, [&](auto pieces, auto lpr) {

@@ -24,3 +24,18 @@ def test_rows_match_64_bits(gpu_device, rows, pieces, dtype):
     for name, a, c in zip(("y", "dx", "dw", "db"), got, want):
         terms = max(1.0, c.abs().max().item(), dy.abs().max().item() * (y64.abs().max().item() + 1.0) * (1.0 + rows ** 0.5 * (name in ("dw", "db"))))
         assert (a.double() - c).abs().max().item() <= u * c.abs().max().item() + 2.0 ** -24 * (8 + (rows + cols) ** 0.5) * terms * (x.abs().max().item() + 1.0), name
+
+
+def test_weight_gradients_in_fp32_come_from_1024_partial_sums(gpu_device):
+    """With half as many each is a sum of twice as many rows one after the other, and further from 64 bits: read from what the call leaves in its workspace."""
+    import ctypes
+    from evoformer_triton_amd import _lib
+    lib, rows, cols = _lib.load(), 8192, 256
+    x, dy = (torch.randn((rows, cols), device=gpu_device) for _ in range(2))
+    mean, rstd, dw, db = x.mean(1), 1.0 / x.std(1), torch.empty(cols, device=gpu_device), torch.empty(cols, device=gpu_device)
+    n = lib.evoattn_layernorm_bwd_workspace_bytes(rows, cols, _lib.EVO_F32)
+    ws = torch.full((n // 4,), float("nan"), device=gpu_device)
+    assert lib.evoattn_layernorm_bwd(dy.data_ptr(), x.data_ptr(), None, mean.data_ptr(), rstd.data_ptr(), None, dw.data_ptr(), db.data_ptr(), ws.data_ptr(), n, rows, cols,
+                                     _lib.EVO_F32, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    assert torch.isfinite(ws).sum().item() == 1024 * 2 * cols and torch.isfinite(dw).all()
