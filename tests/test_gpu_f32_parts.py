@@ -24,28 +24,27 @@ def _run(dev, q, k, v, mask, bias, do):
     return dict(zip(("O", "dQ", "dK", "dV", "dBias"), (t.detach().cpu() for t in (o, *torch.autograd.grad(o, (q, k, v, bias), do.to(dev))))))
 
 
-# rows of one, two and three tiles with and without a remainder; two, four and eight waves; dBias blocks of 64 and 128; every head dim that takes parts
-@pytest.mark.parametrize("shape", [(1, 3, 31, 2, 32), (1, 2, 64, 2, 16), (2, 5, 65, 2, 32), (1, 3, 96, 3, 8), (1, 2, 127, 2, 64), (1, 9, 129, 2, 16),
-                                   (1, 97, 130, 4, 32), (1, 96, 256, 4, 32), (1, 2, 257, 2, 32), (1, 3, 63, 1, 64), (1, 384, 144, 1, 64), (1, 400, 161, 1, 8)],
-                         ids=lambda s: "x".join(map(str, s)))
-def test_no_further_from_64_bits_than_fp32(gpu_device, shape):
-    x = _inputs(*shape)
-    got = _run(gpu_device, *x)
-    ref = {t: eager.attention_fwd_bwd(*(y.to(t) for y in x), compute_dtype=t) for t in (torch.float64, torch.float32)}
-    for name, t in got.items():
-        exact = ref[torch.float64][name]
-        ours, plain = ((y.double() - exact).norm().item() for y in (t, ref[torch.float32][name]))
-        # Three times the formula's own in fp32: its sums are blocked, and with the fp32 matrix instruction (64 and fewer keys at head dims other than 32, where
-        # nothing is split) a gradient is up to 2.6 times as far as its; in parts 2.3.
-        assert ours <= 3.0 * plain, (name, ours, plain)
-
-
 def _errors(got, x):
     """Distance from 64 bits, ours and that of the formula in fp32, and the result itself: norms of each row of a tensor's last dimension."""
     ref = {t: eager.attention_fwd_bwd(*(y.to(t) for y in x), compute_dtype=t) for t in (torch.float64, torch.float32)}
     for name, y in got.items():
         exact = ref[torch.float64][name]
         yield name, (y.double() - exact).norm(dim=-1), (ref[torch.float32][name].double() - exact).norm(dim=-1), exact.norm(dim=-1)
+
+
+# Rows of one, two and three tiles with and without a remainder; two, four and eight waves; dBias blocks of 64 and 128; every head dim that takes parts.  Beside a shape:
+# how far O, dQ, dK, dV and dBias of these inputs are from 64 bits by the fp32 matrix instruction alone (norms, in 2^-24 of the result's).
+@pytest.mark.parametrize("shape,instruction", [
+    ((1, 3, 31, 2, 32), (3.0, 5.2, 5.2, 4.8, 4.9)), ((1, 2, 64, 2, 16), (3.5, 5.9, 5.7, 5.5, 5.4)), ((2, 5, 65, 2, 32), (3.8, 6.2, 6.2, 5.8, 5.8)),
+    ((1, 3, 96, 3, 8), (4.0, 6.5, 6.6, 6.7, 5.9)), ((1, 2, 127, 2, 64), (5.5, 8.4, 8.3, 8.1, 7.6)), ((1, 9, 129, 2, 16), (4.8, 7.9, 7.8, 7.9, 6.9)),
+    ((1, 97, 130, 4, 32), (5.0, 8.1, 8.1, 7.9, 7.8)), ((1, 96, 256, 4, 32), (6.9, 10.6, 10.6, 10.6, 9.6)), ((1, 2, 257, 2, 32), (7.1, 11.8, 11.3, 11.1, 10.7)),
+    ((1, 3, 63, 1, 64), (4.1, 6.1, 6.0, 5.7, 5.6)), ((1, 384, 144, 1, 64), (5.8, 9.0, 9.1, 8.8, 8.9)), ((1, 400, 161, 1, 8), (5.1, 8.7, 8.6, 8.5, 8.3))],
+    ids=lambda s: "x".join(map(str, s)) if isinstance(s[0], int) else "")
+def test_no_further_from_64_bits_than_the_fp32_instruction(gpu_device, shape, instruction):
+    x = _inputs(*shape)
+    for (name, ours, _, size), former in zip(_errors(_run(gpu_device, *x), x), instruction):
+        off = (ours.norm() / size.norm()).item() * 2 ** 24
+        assert off <= former + 0.1, (name, off, former)     # (0.1: the table's last place, twice)
 
 
 # A part below 2^-126 is not there, or has lost bits: operands, dS and results from where that begins to where an operand itself ends, and a score's factors
@@ -88,9 +87,9 @@ def test_infinite_and_large_operands(gpu_device, shape, what):
     o, w = got["O"], want["O"]
     assert torch.equal(torch.isnan(o), torch.isnan(w)) and torch.equal(torch.isinf(o), torch.isinf(w)) and torch.equal(o[torch.isinf(o)], w[torch.isinf(w)])
     for n, a in got.items():
-        ok = torch.isfinite(a) & torch.isfinite(want[n])
-        if name in ("q", "k", "do") or n == "O":   # (dS of an infinite dP has no sign that two orders of its sums would agree on)
-            assert torch.equal(torch.isfinite(a), torch.isfinite(want[n])) or n != "O", n
+        # a number wherever the formula has one; elsewhere too only where a large operand's products overflow in the order of the formula's sums alone
+        ok = torch.isfinite(want[n])
+        assert torch.isfinite(a)[ok].all() and (kind == "large" or torch.equal(torch.isfinite(a), ok)), n
         if not ok.any():
             continue
         big = want[n][ok].abs().max().item()
