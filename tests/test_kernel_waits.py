@@ -1,6 +1,7 @@
 """Waits that no result shows to be missing, read from the compiled kernels' own assembly (built here; no GPU)."""
 import os
 import re
+import shutil
 import subprocess
 
 import pytest
@@ -8,10 +9,11 @@ import pytest
 from evoformer_triton_amd import build
 
 
-def _assembly(source, defines, tmp_path):
+def _assembly(source, defines, tmp_path, csrc=build.CSRC):
     out = str(tmp_path / "kernel.s")
-    subprocess.check_call([build._hipcc(), *build.HIPCC_FLAGS, *defines, *build.VGPR_FORM, "-S", "--cuda-device-only",
-                           os.path.join(build.CSRC, source), "-o", out], stderr=subprocess.DEVNULL)
+    flags = [x for x in build.HIPCC_FLAGS if x != "-I" + build.CSRC] + ["-I" + str(csrc)]
+    subprocess.check_call([build._hipcc(), *flags, *defines, *build.VGPR_FORM, "-S", "--cuda-device-only",
+                           os.path.join(csrc, source), "-o", out], stderr=subprocess.DEVNULL)
     with open(out) as f:
         return f.read()
 
@@ -137,8 +139,14 @@ def test_a_stage_is_there_when_it_is_prepared(source, tmp_path):
     through the kernel at least as many have been issued since."""
     text = _assembly(source, [], tmp_path)
     assert not re.search(r"buffer_store_dwordx[34] .*, s\d+ offen", text)   # (see the test above)
+    # two dtypes, three kinds of bias, three widths or more, the first stage and the others
+    assert _waits_behind_loads(text, "bwd_fused") >= 36
+
+
+def _waits_behind_loads(text, kernels):
+    """How many waits written by hand the kernels have; each finds every load into LDS done, on every way to it."""
     seen = 0
-    for name, lines in _functions(text, "bwd_fused"):
+    for name, lines in _functions(text, kernels):
         blocks, following = _blocks(lines)
         into = {"entry": None}
         todo = ["entry"]
@@ -159,4 +167,33 @@ def test_a_stage_is_there_when_it_is_prepared(source, tmp_path):
         for b in blocks:
             if b in into:
                 _after(blocks[b], into[b], check)
-    assert seen >= 36     # two dtypes, three kinds of bias, three widths or more, the first stage and the others
+    return seen
+
+
+# What holds in every stage but a row's last, for a wave with 32 queries: the stage has a second tile, whose rows of the bias are whole, and all of dBias is stored
+WHOLE_STAGES = {
+    "mfma_stream.hip": [("const bool active = q0 < p.N;", "const bool active = true;", 4), ("const bool active = key0 < p.N;", "const bool active = true;", 1),
+                        ("            if (2 * s + 1 < NT) {\n                init = bias.take(ct[AHEAD - 1]);", "            if (true) {\n                init = bias.take(ct[AHEAD - 1]);", 1),
+                        ("if (2 * s + 1 < NT) tile(", "if (true) tile(", 2),
+                        ("                if (2 * s + 1 < NT) {\n                    const f32x16 b1 = bias.take(ct);", "                if (true) {\n                    const f32x16 b1 = bias.take(ct);", 1),
+                        ("if (qt + 1 < NT) tile(", "if (true) tile(", 2),
+                        ("if (q0 + r >= p.N) continue;", "", 1), ("if (col + 4 <= p.N) {", "if (true) {", 1), ("if (q0 + li >= p.N) return;\n#pragma unroll\n        for (int rr", "#pragma unroll\n        for (int rr", 1),
+                        ("if ((ds_vec || ds_f32) && kg + 4 <= p.N) {", "if (ds_vec || ds_f32) {", 1), ("if (kg + i < p.N) {", "{", 1)],
+    "stream_common.h": [("if (BT == 5 && !COLS && t * 32 + 32 > N) {", "if (false) {", 1)],
+}
+
+
+def test_a_stage_is_there_when_it_is_computed_on(tmp_path):
+    """The kernels at head dim 64 that wait for all but the eight youngest loads and stores between stages: on every way from one stage to the next, at least eight are
+    younger than what the stage's rows were loaded into LDS by.  (On the kernel as it is for stages before the last: the ways to a last stage's end lead to no wait.)"""
+    csrc = tmp_path / "csrc"
+    shutil.copytree(build.CSRC, csrc)
+    for source, changes in WHOLE_STAGES.items():
+        text = (csrc / source).read_text()
+        for old, new, times in changes:
+            assert text.count(old) == times, (source, old)
+            text = text.replace(old, new)
+        (csrc / source).write_text(text)
+    text = _assembly("mfma_stream.hip", ["-DEVO_D=64"], tmp_path, csrc)
+    seen = sum(_waits_behind_loads(text, k) for k in ("stream_fwd", "stream_dq", "stream_dkdv", "stream_bwd_one"))
+    assert seen >= 100 and text.count("s_waitcnt vmcnt(8)") >= 10, seen
