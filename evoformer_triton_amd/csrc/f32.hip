@@ -770,15 +770,16 @@ static int bwd_launch(const EvoAttnParams &p, const Extra &e, int vec, hipStream
     return p.dmask ? launch_dmask_reduce(p, e, st) : EVO_OK;
 }
 
-// Waves, of 32 rows each, that share what a workgroup stages: two for short rows, else four; eight in a forward of more than 128 queries where even such
-// workgroups fill the chip (us, eight / four, D = 32: S = 64, N = 256, H = 8 36.9 / 38.8, S = 100, N = 160, H = 4 19.8 / 24.7, S = 32, N = 250, H = 4 22.0 / 15.8;
-// the backward of the first: 161 / 154).
+// Waves, of 32 rows each, that share what a workgroup stages: two for short rows, else four; eight in a forward of more than 128 queries and more than 384 workgroups so:
+// twice as many of four waves are more than three on each of 256 CUs, what fits at once, while two of eight fit there.  us, H = 4, workgroups of eight waves 320 / 384 / 448 / 512,
+// D = 32, N = 256: eight 31 / 33 / 34 / 36, four 28 / 30 / 37 / 39; N = 1 000 97 / 101 / 109 / 112 and 87 / 93 / 119 / 124; D = 8, N = 250 30 / 30 / 30 / 30 and 25 / 25 / 34 / 34; D = 64, N = 400
+// 73 / 74 / 75 / 79 and 65 / 66 / 79 / 83.  (193 to 256, one each: eight 4 to 13 % faster at D = 8 and 64, 0 to 9 at 32.  The backward: S = 64, N = 256, H = 8 161 / 154.)
 template <int D, bool FWD, class F>
 static int by_rows(const EvoAttnParams &p, F go) {
     auto with = [&](auto w) { return p.bias_dtype != EVO_NONE ? go(w, std::true_type()) : go(w, std::false_type()); };
     if (p.N <= 64) return with(std::integral_constant<int, 2>());
     if constexpr (FWD && D <= 64)
-        if (p.N > 128 && (int64_t)((p.N + 255) / 256) * p.B * p.H * p.S >= 384) return with(std::integral_constant<int, 8>());
+        if (p.N > 128 && (int64_t)((p.N + 255) / 256) * p.B * p.H * p.S > 384) return with(std::integral_constant<int, 8>());
     return with(std::integral_constant<int, 4>());
 }
 #define EVO_F32_DISPATCH(FWD, fn, ...) \
