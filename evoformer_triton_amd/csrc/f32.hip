@@ -284,6 +284,17 @@ __device__ __forceinline__ float finite_check(const f32x16 (&acc)[DT]) {
         for (int r = 0; r < 16; ++r) x = fmaf(acc[t][r], 0.0f, x);
     return x;
 }
+// Whether a thread of the workgroup's says so (__syncthreads_or takes three times as long: 0.3 us of a call of 5).
+template <int W>
+__device__ __forceinline__ bool any_wave(bool x, float *red) {
+    const bool mine = __any(x);
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = mine ? 1.0f : 0.0f;
+    __syncthreads();
+    float r = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) r += red[w];
+    return uniform(r) != 0.0f;
+}
 // Which calls form products out of parts, all of a call's kernels or none (P and the LSE then have the same roundings; with two kinds dV of large scores
 // was twice as far from 64 bits); the others stay on the fp32 instruction alone.  Head dim 128 has no registers for three parts of every operand.  Rows of up to
 // 64, which two waves share: head dims 8 and 16 have little to multiply (S = 256, N = 64, H = 8 forward 13.9 and 15.1 us, in parts 15.5 and 16.4),
@@ -300,7 +311,7 @@ template <int D, bool SPLITS> constexpr int shared_bytes() {
 template <bool SPLITS, class A, class B>
 __device__ __forceinline__ void either_way(A split, B direct) {
     if constexpr (SPLITS) {
-        if (!split()) return;
+        if (__builtin_expect(!split(), 1)) return;
     }
     direct();
 }
@@ -378,7 +389,7 @@ __device__ __forceinline__ bool split_body_fwd(const EvoAttnParams &p, unsigned 
         E::cols(sh.tile(buf, 1), l, x, acc);
     }
     sum = both_halves(sum);
-    if (__syncthreads_or(active && !(fmaf(sum, 0.0f, finite_check(acc)) == 0.0f))) return true;
+    if (__builtin_expect(any_wave<W>(active && !(fmaf(sum, 0.0f, finite_check(acc)) == 0.0f), sh.red()), 0)) return true;
     if (row < p.N) {
         const float inv = kDown / sum;
 #pragma unroll
@@ -477,7 +488,7 @@ __device__ __forceinline__ bool split_body_dq(const EvoAttnParams &p, float *del
         for (int r = 0; r < 16; ++r) x[r] = fast_exp2(x[r]) * dp[r];
         E::cols(sh.tile(buf, 0), l, x, acc);
     }
-    if (__syncthreads_or(active && !(finite_check(acc) == 0.0f))) return true;
+    if (__builtin_expect(any_wave<W>(active && !(finite_check(acc) == 0.0f), sh.red()), 0)) return true;
     if (row < p.N) {
 #pragma unroll
         for (int t = 0; t < E::DT; ++t)
@@ -573,7 +584,7 @@ __device__ __forceinline__ bool split_body_dkdv(const EvoAttnParams &p, const Ex
         E::cols(sh.tile(buf, 0), l, ds, dk);
     }
     dm = both_halves(dm);
-    if (__syncthreads_or(active && !(fmaf(dm, 0.0f, finite_check(dk) + finite_check(dv)) == 0.0f))) return true;
+    if (__builtin_expect(any_wave<W>(active && !(fmaf(dm, 0.0f, finite_check(dk) + finite_check(dv)) == 0.0f), sh.red()), 0)) return true;
     if (key < p.N) {
         if (p.dmask && g == 0) e.dmask_part[pr.row0 + key] = dm * kDown2;
 #pragma unroll
@@ -609,7 +620,7 @@ __global__ void __launch_bounds__(64 * W, D <= 64 ? 2 : 1) f32_dkdv(EvoAttnParam
 template <int D, int KT, bool SPLITS>
 struct DBias : DBiasGeo<D, KT> {
     static constexpr int BLK = DBiasGeo<D, KT>::BLK, DIRECT = 4 * (BLK / 32) * Direct<D>::TILE + 3 * BLK * 4;
-    static constexpr int CHUNKS = SPLITS ? 4 * (BLK / 32) * Split<D <= 64 ? D : 64>::TILE : 0, SPLIT = CHUNKS + (2 * BLK + 1) * 16;   // Q, dO, K, V; rows' and keys' chunks, ones
+    static constexpr int CHUNKS = SPLITS ? 4 * (BLK / 32) * Split<D <= 64 ? D : 64>::TILE : 0, SPLIT = CHUNKS + (2 * BLK + 1) * 16 + 64;   // Q, dO, K, V; rows' and keys' chunks, ones, a value per wave
     static constexpr int BYTES = SPLITS && SPLIT > DIRECT ? SPLIT : DIRECT;
 };
 template <int D, int KT, bool BIAS>
@@ -706,7 +717,7 @@ __device__ __forceinline__ bool split_body_dbias(const EvoAttnParams &p, const f
             if (q < p.N) out[(int64_t)q * p.N] = acc[kt][r] * kDown2;
         }
     }
-    return __syncthreads_or(sk.huge != 0 || (active && !(finite_check(acc) == 0.0f)));   // (dBias lies where nothing is read any more; asked before the stores, 16 to 38 registers more)
+    return any_wave<R::W>(sk.huge != 0 || (active && !(finite_check(acc) == 0.0f)), reinterpret_cast<float *>(one + 1));   // (dBias lies where nothing is read any more; asked before the stores, 16 to 38 registers more)
 }
 template <int D, int KT, bool SPLITS, bool BIAS>
 __global__ void __launch_bounds__((64 * DBiasGeo<D, KT>::W), D <= 64 ? 2 : 1) f32_dbias(EvoAttnParams p, const float *delta, const float *shift_tab, float *part, int chunk) {
