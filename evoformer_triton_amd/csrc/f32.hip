@@ -672,7 +672,7 @@ __device__ __forceinline__ bool split_body_dbias(const EvoAttnParams &p, const f
         }
     };
     static_assert(TH >= 2 * ROWS, "a thread for each row's and each key's chunk");
-    E::clear(lds, 4 * ROWS, TH);
+    if (D < 16) E::clear(lds, 4 * ROWS, TH);   // (no columns beyond 16 are read)
     load(s0);
     const bf16x8 xd = g == 0 ? as_operand(chunk_of(none, ones)) : zero8<bf16_t>();
     for (int s = s0; s < s1; ++s) {

@@ -574,8 +574,7 @@ __device__ __forceinline__ void direct_dbias(const EvoAttnParams &p, const float
             else if (k < 3 * ROWS) small[k] = mask_got(p, sv[j], k0 + i, shift);
         }
     };
-    E::clear(lds, 4 * ROWS, TH);
-    load(s0);
+    load(s0);   // (nothing reads the columns beyond D)
     for (int s = s0; s < s1; ++s) {
         __syncthreads();
         sq.put(lds, lds + ARRAY);
