@@ -191,8 +191,8 @@ struct SplitStage {
         const int first = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int k0 = first + i * THREADS, k = (k0 & (PIECES - 1)) + (threadIdx.x & 63);   // (k0: the same for the wave)
-            if (2 * PIECES % THREADS != 0 && k0 >= 2 * PIECES) break;
+            // (k0: the same for the wave; where there are more waves than pieces, some ask for the others' again: behind a branch the load is waited for at once)
+            const int k0 = (first + i * THREADS) & (2 * PIECES - 1), k = (k0 & (PIECES - 1)) + (threadIdx.x & 63);
             v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(k0 < PIECES ? a : b, ((unsigned)(k / (D / 4)) * stride_n + (unsigned)(k % (D / 4) * 4)) * 4u,
                                                                                  (unsigned)r0 * stride_n * 4u, 0));
         }
