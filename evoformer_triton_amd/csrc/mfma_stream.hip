@@ -1046,14 +1046,23 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
     fetch(0);
 
     // this wave's keys: K with the mask columns, V with ones against -delta
+    // (all asked for before any is used, but not where the caller's bias rows come to head dim 128 as well: the loop then spills others, dK/dV of one row, N = 1 008, H = 4,
+    // fp32 90 -> 100 us; a step of it so 170 and with all together 184, of 16 bits at N = 2 048, H = 2 362 and 377.  With prepared tiles S = 64, N = 512 294 / 285.)
+    constexpr bool TOGETHER = !(D == 128 && BT >= 3);
     v8 kf[KSD], vf[KSD], kaug, vaug;
     uint2 mraw;
     {
         const int64_t row = pr.base + (int64_t)keyc * p.stride_n + g * 8;
 #pragma unroll
         for (int ks = 0; ks < KSD; ++ks) {
-            kf[ks] = ld8((const T *)p.k + row + ks * 16);
-            vf[ks] = ld8((const T *)p.v + row + ks * 16);
+            if constexpr (TOGETHER) {
+                kf[ks] = ld8((const T *)p.k + row + ks * 16);
+                vf[ks] = ld8((const T *)p.v + row + ks * 16);
+            } else {
+                kf[ks] = dead ? zero8<T>() : ld8((const T *)p.k + row + ks * 16);
+                *reinterpret_cast<v8 *>(lds + R::OFF_K + wave * 32 * G::ROW + G::at(li, 2 * ks + g)) = kf[ks];
+                vf[ks] = kill ? zero8<T>() : ld8((const T *)p.v + row + ks * 16);
+            }
         }
         mraw = e.m2[((int64_t)pr.b * p.S + pr.s) * (NT * 32) + min(key, NT * 32 - 1)];
     }
@@ -1066,13 +1075,15 @@ __device__ __forceinline__ void dkdv_rows(const EvoAttnParams &p, const Extra &e
     typename BiasStream<T, BT, true>::Tile ct, c1;
     bias.load(0, ct);
     if (TWO) bias.load(1, c1);
-    asked_together<KSD>(kf);
-    asked_together<KSD>(vf);
+    if constexpr (TOGETHER) {
+        asked_together<KSD>(kf);
+        asked_together<KSD>(vf);
+    }
 #pragma unroll
     for (int ks = 0; ks < KSD; ++ks) {
-        if (dead) kf[ks] = zero8<T>();
-        if (kill) vf[ks] = zero8<T>();   // (no gradient through replaced scores: dS is then zero)
-        if constexpr (R::K_LDS) *reinterpret_cast<v8 *>(lds + R::OFF_K + wave * 32 * G::ROW + G::at(li, 2 * ks + g)) = kf[ks];
+        if (TOGETHER && dead) kf[ks] = zero8<T>();
+        if (TOGETHER && kill) vf[ks] = zero8<T>();   // (no gradient through replaced scores: dS is then zero)
+        if constexpr (TOGETHER && R::K_LDS) *reinterpret_cast<v8 *>(lds + R::OFF_K + wave * 32 * G::ROW + G::at(li, 2 * ks + g)) = kf[ks];
     }
     kaug = g == 0 ? aug8<T>(mraw, one3) : zero8<T>();     // mask x ones, ones x -lse
     vaug = g == 0 && !kill ? aug8<T>(one3, zero3) : zero8<T>();    // ones x -delta
