@@ -301,8 +301,9 @@ __device__ __forceinline__ bool any_wave(bool x, float *red) {
 // at 64 the backward spills (171, 190).
 constexpr bool splits(int D, int W) { return D == 32 || (D <= 64 && W > 2); }
 template <int D, bool SPLITS> constexpr int shared_bytes() {
-    if constexpr (SPLITS) return SplitShared<D>::BYTES > DirectShared<D>::BYTES ? SplitShared<D>::BYTES : DirectShared<D>::BYTES;
-    else return DirectShared<D>::BYTES;
+    // (the second forming writes none of the vote's words, which a wave may still be reading when another has begun with it)
+    if constexpr (SPLITS) static_assert(DirectShared<D>::BYTES <= SplitShared<D>::BYTES - 64, "");
+    return SPLITS ? SplitShared<D <= 64 ? D : 64>::BYTES : DirectShared<D>::BYTES;
 }
 // A kernel forms its results in parts and, where some result of the workgroup is then not finite, once more on the fp32 instruction: parts of an infinite
 // operand, or of one that is beyond bf16's range when 2^24 times as large, are not numbers, where the value itself may give a number, or an infinite result.
@@ -621,7 +622,8 @@ template <int D, int KT, bool SPLITS>
 struct DBias : DBiasGeo<D, KT> {
     static constexpr int BLK = DBiasGeo<D, KT>::BLK, DIRECT = 4 * (BLK / 32) * Direct<D>::TILE + 3 * BLK * 4;
     static constexpr int CHUNKS = SPLITS ? 4 * (BLK / 32) * Split<D <= 64 ? D : 64>::TILE : 0, SPLIT = CHUNKS + (2 * BLK + 1) * 16 + 64;   // Q, dO, K, V; rows' and keys' chunks, ones, a value per wave
-    static constexpr int BYTES = SPLITS && SPLIT > DIRECT ? SPLIT : DIRECT;
+    static_assert(!SPLITS || D > 64 || DIRECT <= SPLIT - 64, "the second forming writes none of the vote's words");
+    static constexpr int BYTES = SPLITS ? SPLIT : DIRECT;
 };
 template <int D, int KT, bool BIAS>
 __device__ __forceinline__ bool split_body_dbias(const EvoAttnParams &p, const float *delta, const float *shift_tab, float *part, int chunk, unsigned char *lds) {
