@@ -16,9 +16,10 @@
 // keeps a small call at one launch forward and three or four backward.  Bias, mask and rows of the next tile are asked for before this one is computed on
 // and nothing is done to them until then: with a conversion behind a load, every tile waited for memory (forward 56 -> 39 us of the case below).
 //
-// us, fp32 instruction / this, B = 1: S = 64, N = 256, H = 8, D = 32 forward 51 / 36, backward 218 / 155 (counters: a forward's SIMD is busy 67 k clocks, 33 k of
-// them with vector and 26 k with matrix instructions; with one tile of keys instead of eight 22 k); S = 4, N = 1 024, H = 4 74 / 46, 224 / 142; S = 100, N = 160, H = 4 32 / 20, 134 / 103;
-// D = 64, S = 64, N = 256, H = 8 92 / 62, 383 / 319.  Not taken up: 64 rows per stage, all of a tile's operands read ahead, a priority of half
+// us, fp32 instruction / this, B = 1: S = 64, N = 256, H = 8, D = 32 forward 48 / 36, backward 228 / 151 (counters: a forward's SIMD is busy 67 k clocks, 33 k of
+// them with vector and 26 k with matrix instructions; with one tile of keys instead of eight 22 k; in dQ, dBias and dK/dV, at 1.6 waves per SIMD, vector instructions
+// take 0.31 to 0.33 of the time and matrix instructions 0.28 to 0.34); S = 4, N = 1 024, H = 4 76 / 47, 231 / 139; S = 100, N = 160, H = 4 31 / 19, 135 / 103;
+// D = 64, S = 64, N = 256, H = 8 90 / 62, 384 / 330.  Not taken up: 64 rows per stage, all of a tile's operands read ahead, a priority of half
 // the waves (each within 3 %), eight waves in the backward (161 / 154).
 // Error against 64 bits over that of the fp32 instruction, N = 32 to 256, 160 calls: .65 to .78 at the median for every result, none above 1.
 //
@@ -298,7 +299,9 @@ __device__ __forceinline__ bool any_wave(bool x, float *red) {
 // Which calls form products out of parts, all of a call's kernels or none (P and the LSE then have the same roundings; with two kinds dV of large scores
 // was twice as far from 64 bits); the others stay on the fp32 instruction alone.  Head dim 128 has no registers for three parts of every operand.  Rows of up to
 // 64, which two waves share: head dims 8 and 16 have little to multiply (S = 256, N = 64, H = 8 forward 13.9 and 15.1 us, in parts 15.5 and 16.4),
-// at 64 the backward spills (171, 190).
+// at 64 the backward spills (171, 190).  Above 64 keys parts win at every head dim up to 64, whatever the registers: 131 forwards and steps of 65 to 1 000 keys take
+// 0.55 to 0.87 of the instruction's time (S = 64, N = 256, H = 8 a step at D = 8 164 / 124 us with dK/dV at two waves per SIMD instead of four, D = 16 194 / 133, D = 64 472 / 391
+// with 36 registers of dK/dV spilled).
 constexpr bool splits(int D, int W) { return D == 32 || (D <= 64 && W > 2); }
 template <int D, bool SPLITS> constexpr int shared_bytes() {
     // (the second forming writes none of the vote's words, which a wave may still be reading when another has begun with it)

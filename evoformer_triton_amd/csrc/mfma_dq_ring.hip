@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(512) mfma_dq_ring(EvoAttnParams p, Extra e) {
     // tiles, while other waves compute, and the other half after them, and asks for the same pieces of the
     // stage after that as soon as their registers are free: a request has a whole row to arrive in.  Asked for and
     // written within one row, in two halves, it had half of one, less than memory takes: S = 128, N = 256, H = 8, D = 32 with the gate's pass
-    // 56 -> 49 us, S = 512 146 -> 138; 8 to 12 registers, no spills.
+    // 56 -> 49 us, S = 512 146 -> 138; 8 to 12 registers, none spilled but one more (two) in the form of 384 keys at head dim 16.
     constexpr bool MID = NBLK == 1 && R::OWN_RED && TPW >= 2;
     // where the partials of the row that ended with stage `stage` lie; par: stage & 1 (one stage per row: the row's parity)
     auto red_of = [&](int stage, int par) {
